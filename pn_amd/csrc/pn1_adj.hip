@@ -204,10 +204,11 @@ struct Fp64Scope {
     ~Fp64Scope() { c->mode = mode; }
 };
 
+// The first `last` evaluations of a step, the first of them prepared.
 int enqueue_stages(pn1_ctx* c, int last, const Phys& P)
 {
     for (int stage = 1; stage <= last; ++stage) {
-        int rc = enqueue_force(c, stage, P);
+        int rc = enqueue_eval(c, stage, P);
         if (rc) return rc;
     }
     return PN1_OK;
@@ -270,6 +271,7 @@ int pn1_adjoint_forward(pn1_ctx* c, int steps, int interval)
     Fp64Scope fp64(c);
     drop_graph(c);
     const Phys P = make_phys(c);
+    if ((rc = enqueue_prep(c, P))) return rc;
     for (int t = 0; t < steps; ++t) {
         if (t % interval == 0 && (rc = copy6(c, a->ckpt + (size_t)(t / interval) * s6, c->X)))
             return rc;
@@ -306,6 +308,7 @@ int pn1_adjoint_backward(pn1_ctx* c, const double* gx, const double* gv, double*
         // the segment's states: per step s, Y1 = H1 and Y2 = H2 (the last
         // step runs two stages only: its end state is not needed)
         if ((rc = copy6(c, c->X, a->ckpt + (size_t)k * s6))) return rc;
+        if ((rc = enqueue_prep(c, P))) return rc;
         for (int t = t0; t < t1; ++t) {
             double* st = a->seg + 3 * (size_t)(t - t0) * s6;
             if ((rc = copy6(c, st, c->X))) return rc;
@@ -686,7 +689,7 @@ struct EnsFp64Scope {
 int ens_stages(pn1_ens* e, int last, const Phys& P)
 {
     for (int stage = 1; stage <= last; ++stage) {
-        int rc = ens_enqueue_force(e, stage, P);
+        int rc = ens_enqueue_eval(e, stage, P);
         if (rc) return rc;
     }
     return PN1_OK;
@@ -742,6 +745,7 @@ int pn1_ens_adjoint_forward(pn1_ens* e, int steps, int interval)
     EnsFp64Scope fp64(e);
     edrop_graph(e);
     const Phys P = ens_phys(e);
+    if ((rc = ens_enqueue_prep(e, P))) return rc;
     for (int t = 0; t < steps; ++t) {
         if (t % interval == 0 && (rc = ens_copy6(e, a->ckpt + (size_t)(t / interval) * s6, e->X)))
             return rc;
@@ -778,6 +782,7 @@ int pn1_ens_adjoint_backward(pn1_ens* e, const double* gx, const double* gv, dou
     for (int k = nck - 1; k >= 0; --k) {
         const int t0 = k * a->interval, t1 = std::min(a->steps, t0 + a->interval);
         if ((rc = ens_copy6(e, e->X, a->ckpt + (size_t)k * s6))) return rc;
+        if ((rc = ens_enqueue_prep(e, P))) return rc;
         for (int t = t0; t < t1; ++t) {
             double* st = a->seg + 3 * (size_t)(t - t0) * s6;
             if ((rc = ens_copy6(e, st, e->X))) return rc;

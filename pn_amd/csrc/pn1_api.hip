@@ -8,7 +8,7 @@
 //   Y[6][cap]   stage input (the reference's x1, v1)
 //   H1, H2      stage states 1 and 2 (the reference's hx[1..2], hv[1..2])
 //   m[cap], acc[3][cap]
-//   j64[cap] / j32[cap]   per-evaluation j-records (AoS)
+//   j64[3][cap + 2], j32[cap + 2]   per-evaluation j-records (AoS)
 //   part        pair partials: FP64 [S][16][cap]; mixed [S][16 + 3][cap] floats
 //               (the sums, then the Kahan compensations of the Newtonian sums)
 // Device memory is allocated by pn1_create, and grown by pn1_upload,
@@ -92,6 +92,7 @@ void plan(pn1_ctx* c)
 {
     const int nst = c->n - 1;
     c->nblk = nblocks(nst);
+    c->nrow = nst > 0 ? (nst + RB - 1) / RB : 1;
     c->nIblk = nst > 0 ? (nst + WG - 1) / WG : 0;
     int S = c->jsplit_req;
     if (S <= 0) {
@@ -205,117 +206,136 @@ bool ready(pn1_ctx* c, int* rc)
 }
 
 // ---- one force evaluation (+ stage update) ------------------------------
-template <int MODE, int STAGE>
-void launch_fin(pn1_ctx* c, const double* in, const Phys& P)
+JRec64* rec_buf(const pn1_ctx* c, int k) { return c->j64 + (size_t)k * ((size_t)c->cap + 2); }
+
+// ticket false: the sums over the rows are left to k_gsum / k_bh, or not
+// needed (an i shard).
+RowBufs row_bufs(const pn1_ctx* c, bool ticket = true)
 {
-    // the cancellation ratios are refreshed by plain evaluations and the
-    // first stage of each step (the pair kernel accumulated their sums)
-    float* kout = (MODE == 1 && STAGE <= 1) ? c->kr : nullptr;
-    hipLaunchKernelGGL((k_fin<MODE, STAGE>), dim3(c->nblk), dim3(WG), 0, c->st, in, c->X, c->Y,
-                       c->H1, c->H2, c->m, (const void*)c->part, part_slots(c, c->S), c->gs,
-                       c->acc, c->bhblk,
-                       kout, (const int*)c->fn, (const double*)c->xp, (const int*)c->fl,
-                       (const double*)c->xh, P, 1, c->n);
-    hipLaunchKernelGGL((k_bh<STAGE>), dim3(1), dim3(WG), 0, c->st, c->bhblk, c->nblk, c->gs, c->X,
-                       c->Y, c->H1, c->H2, c->acc, P);
+    RowBufs R;
+    R.rows = c->rows;
+    R.fmask = c->fmask;
+    R.hmask = c->hmask;
+    R.gs = c->gs;
+    R.flist = c->flist;
+    R.fn = c->fn;
+    R.ticket = ticket ? c->ticket : nullptr;
+    return R;
+}
+
+// The mixed form's prep inputs (FP64 form: none).
+MixPrep mix_prep(const pn1_ctx* c, const Phys& P)
+{
+    MixPrep M;
+    const bool mixed = c->mode == PN1_MIXED;
+    M.j32 = mixed ? c->j32 : nullptr;
+    M.thr = mixed ? c->thr : nullptr;
+    M.mmax = mixed ? c->mmax : 0.0;
+    M.tauf = mixed ? c->tauf : 0.0;
+    M.lam = mixed ? P.lam : 0.0;
+    return M;
+}
+
+// Waves per row of k_fin: FG up to FIN_ROWS rows, which one wave per row
+// would leave most of the chip idle on; 1 above.
+constexpr int FIN_ROWS = 1024;
+
+// Stars i0 .. i1 - 1 (all: every star and the BH).
+template <int MODE, int STAGE>
+void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int S, int i0, int i1, bool all)
+{
+    FinBufs F;
+    F.in = in;
+    F.X = c->X;
+    F.Y = c->Y;
+    F.H1 = c->H1;
+    F.H2 = c->H2;
+    F.m = c->m;
+    F.acc = c->acc;
+    F.kr = c->kr;
+    F.xr = c->xr;
+    F.j64 = rec_buf(c, STAGE <= 1 ? 0 : STAGE - 1);
+    F.jnext = rec_buf(c, STAGE % 3);
+    const int row0 = (i0 - 1) / RB, rows = std::max(1, (i1 - i0 + RB - 1) / RB);
+    const RowBufs R = row_bufs(c, all);
+    const int slots = part_slots(c, S);
+    if (c->nrow <= FIN_ROWS)
+        hipLaunchKernelGGL((k_fin<MODE, STAGE, FG>), dim3(rows), dim3(FWG), 0, c->st, F, R,
+                           (const void*)c->part, slots, mix_prep(c, P), P, row0, i1, c->nrow);
+    else
+        hipLaunchKernelGGL((k_fin<MODE, STAGE, 1>), dim3((rows + FG - 1) / FG), dim3(FWG), 0,
+                           c->st, F, R, (const void*)c->part, slots, mix_prep(c, P), P, row0, i1,
+                           c->nrow);
 }
 
 // The pair kernel over i blocks ib0 .. ib0 + nib - 1 against every star,
 // with the j range split in S chunks.  ts (mixed form): also accumulate the
 // sums behind the stars' cancellation ratios.
-void launch_pair(pn1_ctx* c, const double* in, const Phys& P, int ib0, int nib, int S, bool ts)
+void launch_pair(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int ib0, int nib,
+                 int S, bool ts)
 {
     const bool mixed = c->mode == PN1_MIXED;
     const dim3 g(pair_grid(S, nib)), blk(WG);
     const int variant = kernel_variant(c);
     if (mixed) {
-        launch_pair32(c, in, P, ib0, nib, S, pair32_form(variant, ts, c->eqm));
+        launch_pair32(c, j64, in, P, ib0, nib, S, pair32_form(variant, ts, c->eqm));
     } else if (variant & 1) {
-        hipLaunchKernelGGL(k_pair64<1>, g, blk, 0, c->st, c->j64, in, (double*)c->part, P, S, nib,
+        hipLaunchKernelGGL(k_pair64<1>, g, blk, 0, c->st, j64, in, (double*)c->part, P, S, nib,
                            ib0);
     } else {
-        hipLaunchKernelGGL(k_pair64<0>, g, blk, 0, c->st, c->j64, in, (double*)c->part, P, S, nib,
+        hipLaunchKernelGGL(k_pair64<0>, g, blk, 0, c->st, j64, in, (double*)c->part, P, S, nib,
                            ib0);
     }
 }
 
-// k_prep's mixed-form inputs (prev: the thresholds from the previous
-// evaluation; false: none, the first pass after an upload).
-MixPrep mix_prep(const pn1_ctx* c, const Phys& P, bool prev)
+// The records and sums of an evaluation on X; FP64: whatever the mode, the
+// FP64 form's only (energy).
+int prep_x(pn1_ctx* c, const Phys& P, bool fp64)
 {
-    MixPrep M;
-    M.j32 = c->j32;
-    M.thr = c->thr;
-    M.aprev = prev ? c->acc : nullptr;
-    M.kprev = prev ? c->kr : nullptr;
-    M.mmax = c->mmax;
-    M.tauf = c->tauf;
-    M.lam = P.lam;
-    M.hard_rows = 1;
-    return M;
+    MixPrep M = mix_prep(c, P);
+    if (fp64) M.j32 = nullptr;
+    const bool prev = M.j32 && c->acc_ok;
+    hipLaunchKernelGGL(k_prep, dim3((c->nrow + FG - 1) / FG), dim3(FWG), 0, c->st,
+                       (const double*)c->X, c->m, P, c->nrow, rec_buf(c, 0), row_bufs(c), M,
+                       prev ? (const double*)c->acc : nullptr, prev ? (const float*)c->kr : nullptr);
+    HIPCHK(c, hipGetLastError());
+    return PN1_OK;
 }
 
-MixPrep fp64_prep()
-{
-    MixPrep M;
-    M.j32 = nullptr;
-    M.thr = nullptr;
-    M.aprev = nullptr;
-    M.kprev = nullptr;
-    M.mmax = M.tauf = M.lam = 0.0;
-    M.hard_rows = 0;
-    return M;
-}
-
-// The records and separable sums of one evaluation on `in`; mixed form:
-// also the list of stars taken out of the FP32 pass and the FP64 sums of
-// their pairs.
-void launch_prep(pn1_ctx* c, const double* in, const Phys& P)
-{
-    const bool mixed = c->mode == PN1_MIXED;
-    const MixPrep M = mixed ? mix_prep(c, P, c->acc_ok) : fp64_prep();
-    hipLaunchKernelGGL(k_prep, dim3(c->nblk), dim3(WG), 0, c->st, in, c->m, P, c->j64, c->gblk, M,
-                       c->fl, c->fblk);
-    hipLaunchKernelGGL((k_rows_sum<NGS>), dim3(1), dim3(WG), 0, c->st, c->gblk, c->nblk, c->gs);
-    if (mixed) {
-        hipLaunchKernelGGL(k_flist, dim3(1), dim3(WG), 0, c->st, (const int*)c->fl,
-                           (const int*)c->fblk, c->nblk, c->n, c->flist, c->hlist, c->fn);
-        hipLaunchKernelGGL(k_pair_fl, dim3(c->nblk), dim3(WG), 0, c->st, (const JRec64*)c->j64,
-                           in, (const int*)c->flist, (const int*)c->fn, c->xp, P);
-        hipLaunchKernelGGL(k_hard_rows, dim3(c->hgrid), dim3(HWG), 0, c->st,
-                           (const JRec64*)c->j64, in, (const int*)c->hlist, (const int*)c->fn,
-                           c->xh, c->hseg, P);
-        hipLaunchKernelGGL(k_hard_sum, dim3((HCAP * (NACC + 1) + WG - 1) / WG), dim3(WG), 0,
-                           c->st, (const int*)c->hlist, (const int*)c->fn,
-                           (const double*)c->hseg, c->xh, c->cap);
-    }
-}
+int enqueue_prep(pn1_ctx* c, const Phys& P) { return prep_x(c, P, false); }
 
 // stage 0: plain evaluation on X; stages 1..3: the driver's force calls.
-int enqueue_force(pn1_ctx* c, int stage, const Phys& P)
+int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
 {
     const double* in = stage <= 1 ? c->X : c->Y;
     const bool mixed = c->mode == PN1_MIXED;
-    launch_prep(c, in, P);
     if (c->n > 1) {
         hipEvent_t e1 = nullptr;
         if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
-        launch_pair(c, in, P, 0, c->nIblk, c->S, stage <= 1);
+        launch_pair(c, rec_buf(c, stage <= 1 ? 0 : stage - 1), in, P, 0, c->nIblk, c->S,
+                    stage <= 1);
         if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     }
     switch (stage * 2 + (mixed ? 1 : 0)) {
-    case 0: launch_fin<0, 0>(c, in, P); break;
-    case 1: launch_fin<1, 0>(c, in, P); break;
-    case 2: launch_fin<0, 1>(c, in, P); break;
-    case 3: launch_fin<1, 1>(c, in, P); break;
-    case 4: launch_fin<0, 2>(c, in, P); break;
-    case 5: launch_fin<1, 2>(c, in, P); break;
-    case 6: launch_fin<0, 3>(c, in, P); break;
-    default: launch_fin<1, 3>(c, in, P); break;
+    case 0: launch_fin<0, 0>(c, in, P, c->S, 1, c->n, true); break;
+    case 1: launch_fin<1, 0>(c, in, P, c->S, 1, c->n, true); break;
+    case 2: launch_fin<0, 1>(c, in, P, c->S, 1, c->n, true); break;
+    case 3: launch_fin<1, 1>(c, in, P, c->S, 1, c->n, true); break;
+    case 4: launch_fin<0, 2>(c, in, P, c->S, 1, c->n, true); break;
+    case 5: launch_fin<1, 2>(c, in, P, c->S, 1, c->n, true); break;
+    case 6: launch_fin<0, 3>(c, in, P, c->S, 1, c->n, true); break;
+    default: launch_fin<1, 3>(c, in, P, c->S, 1, c->n, true); break;
     }
     HIPCHK(c, hipGetLastError());
     c->acc_ok = mixed;
     return PN1_OK;
+}
+
+// One plain force evaluation of X.
+int enqueue_force(pn1_ctx* c, const Phys& P)
+{
+    const int rc = enqueue_prep(c, P);
+    return rc ? rc : enqueue_eval(c, 0, P);
 }
 
 int ensure_prev_acc(pn1_ctx* c, const Phys& P)
@@ -323,15 +343,17 @@ int ensure_prev_acc(pn1_ctx* c, const Phys& P)
     if (c->mode != PN1_MIXED || c->acc_ok) return PN1_OK;
     const bool prof = c->prof;      // not one of the caller's timed launches
     c->prof = false;
-    const int rc = enqueue_force(c, 0, P);
+    const int rc = enqueue_force(c, P);
     c->prof = prof;
     return rc;
 }
 
+// One step of the driver, its first evaluation prepared (by enqueue_prep or
+// the step before).
 int enqueue_step(pn1_ctx* c, const Phys& P)
 {
     for (int stage = 1; stage <= 3; ++stage) {
-        int rc = enqueue_force(c, stage, P);
+        int rc = enqueue_eval(c, stage, P);
         if (rc) return rc;
     }
     return PN1_OK;
@@ -352,19 +374,17 @@ int fetch3(pn1_ctx* c, const double* dsrc, double* out)
 
 // ---- scratch of pn1_force_noalloc -----------------------------------------
 // Sized for n <= PN1_NOALLOC_MAX_N and a j split of at most NA_MAXS chunks:
-// j-records, per-block separable sums, their totals, pair partials and the
-// per-block BH partials of one FP64 force evaluation, each part 256-byte
+// j-records, pair partials, the rows' values and the separable sums of one FP64 force evaluation, each part 256-byte
 // aligned (offsets in doubles).
 constexpr int NA_MAXS = 32;
-constexpr int NA_MAXB = (PN1_NOALLOC_MAX_N + WG - 1) / WG;
+constexpr int NA_MAXB = (PN1_NOALLOC_MAX_N + RB - 1) / RB;
 constexpr size_t na_round(size_t d) { return (d + 31) & ~(size_t)31; }
 constexpr size_t NA_J64 = 0;
 constexpr size_t NA_PART =
     NA_J64 + na_round((size_t)PN1_NOALLOC_MAX_N * (sizeof(JRec64) / sizeof(double)));
-constexpr size_t NA_GBLK = NA_PART + na_round((size_t)NA_MAXS * NACC * PN1_NOALLOC_MAX_N);
-constexpr size_t NA_GS = NA_GBLK + na_round((size_t)NA_MAXB * NGS);
-constexpr size_t NA_BH = NA_GS + na_round(NGS);
-constexpr size_t NA_TOTAL = NA_BH + na_round((size_t)NA_MAXB * 3);
+constexpr size_t NA_ROWS = NA_PART + na_round((size_t)NA_MAXS * NACC * PN1_NOALLOC_MAX_N);
+constexpr size_t NA_GS = NA_ROWS + na_round((size_t)NA_MAXB * RV);
+constexpr size_t NA_TOTAL = NA_GS + na_round(NGS);
 static_assert(sizeof(JRec64) % sizeof(double) == 0, "JRec64 in doubles");
 
 // j split of pn1_force_noalloc: NA_MAXS chunks, halved while a chunk would
@@ -427,15 +447,14 @@ void pn1_destroy(pn1_ctx* c)
         (void)hipEventDestroy(e.first);
         (void)hipEventDestroy(e.second);
     }
-    double* bufs[] = {c->X, c->Y, c->H1, c->H2, c->m, c->acc, c->gblk, c->gs, c->bhblk, c->eblk,
-                      c->eout};
+    double* bufs[] = {c->X, c->Y, c->H1, c->H2, c->m, c->acc, c->rows, c->gs, c->eblk, c->eout};
     for (double* b : bufs)
         if (b) (void)hipFree(b);
     if (c->j64) (void)hipFree(c->j64);
     if (c->j32) (void)hipFree(c->j32);
     if (c->thr) (void)hipFree(c->thr);
     if (c->kr) (void)hipFree(c->kr);
-    void* fbufs[] = {c->fl, c->fblk, c->flist, c->fn, c->xp, c->hlist, c->xh, c->hseg};
+    void* fbufs[] = {c->fmask, c->hmask, c->flist, c->fn, c->ticket, c->xr};
     for (void* b : fbufs)
         if (b) (void)hipFree(b);
     if (c->part) (void)hipFree(c->part);
@@ -469,6 +488,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     }
     const size_t cap = (size_t)capacity;
     const size_t nb = (size_t)nblocks(capacity) + 1;
+    const size_t nr = (cap + RB - 1) / RB + 1;          // rows of 64 stars
     int rc = PN1_OK;
     if (!rc) rc = dalloc(c, &c->X, 6 * cap);
     if (!rc) rc = dalloc(c, &c->Y, 6 * cap);
@@ -476,24 +496,23 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->H2, 6 * cap);
     if (!rc) rc = dalloc(c, &c->m, cap);
     if (!rc) rc = dalloc(c, &c->acc, 3 * cap);
-    if (!rc) rc = dalloc(c, &c->gblk, nb * NGS);
+    if (!rc) rc = dalloc(c, &c->rows, nr * RV);
     if (!rc) rc = dalloc(c, &c->gs, 16);
-    if (!rc) rc = dalloc(c, &c->bhblk, nb * 3);
     if (!rc) rc = dalloc(c, &c->eblk, nb * NEB);
     if (!rc) rc = dalloc(c, &c->eout, 8);
     // two records more than particles: the pair loops fetch up to jr[j + 2]
-    if (!rc) rc = dalloc(c, &c->j64, cap + 2);
+    if (!rc) rc = dalloc(c, &c->j64, 3 * (cap + 2));
     if (!rc) rc = dalloc(c, &c->j32, cap + 2);
     if (!rc) rc = dalloc(c, &c->thr, cap);
     if (!rc) rc = dalloc(c, &c->kr, cap);
-    if (!rc) rc = dalloc(c, &c->fl, cap);
-    if (!rc) rc = dalloc(c, &c->fblk, 2 * nb);
+    if (!rc) rc = dalloc(c, &c->fmask, nr);
+    if (!rc) rc = dalloc(c, &c->hmask, nr);
+    if (!rc) rc = dalloc(c, &c->xr, (size_t)(NACC + 1) * cap);
     if (!rc) rc = dalloc(c, &c->flist, cap);
-    if (!rc) rc = dalloc(c, &c->hlist, cap);
-    if (!rc) rc = dalloc(c, &c->xh, (size_t)(NACC + 1) * cap);
-    if (!rc) rc = dalloc(c, &c->hseg, (size_t)HCAP * HSEG * (NACC + 1));
     if (!rc) rc = dalloc(c, &c->fn, 4);
-    if (!rc) rc = dalloc(c, &c->xp, (size_t)(NACC + 1) * cap);
+    if (!rc) rc = dalloc(c, &c->ticket, 1);
+    if (!rc && hipMemsetAsync(c->ticket, 0, sizeof(unsigned int), c->st) != hipSuccess)
+        rc = PN1_EDEVICE;
     if (!rc && host_malloc((void**)&c->h_stage, 7 * cap * sizeof(double)) != hipSuccess) {
         c->h_stage = nullptr;
         rc = PN1_ENOMEM;
@@ -626,7 +645,7 @@ int pn1_force(pn1_ctx* c, double* a)
     if (!a) return seterr(c, PN1_EINVAL, "null output");
     const Phys P = make_phys(c);
     if ((rc = ensure_prev_acc(c, P))) return rc;
-    if ((rc = enqueue_force(c, 0, P))) return rc;
+    if ((rc = enqueue_force(c, P))) return rc;
     return fetch3(c, c->acc, a);
 }
 
@@ -658,22 +677,15 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
     if ((rc = ensure_part(c, S))) return rc;
     // every star's j-record and the separable sums: what a sharded run would
     // all-gather and all-reduce before its pair kernel
-    launch_prep(c, in, P);
+    if ((rc = enqueue_prep(c, P))) return rc;
     hipEvent_t e1 = nullptr;
     if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
-    launch_pair(c, in, P, (i0 - 1) / WG, nib, S, true);
+    launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
-    const dim3 gf(nib);
     if (mixed)
-        hipLaunchKernelGGL((k_fin<1, 0>), gf, dim3(WG), 0, c->st, in, c->X, c->Y, c->H1, c->H2,
-                           c->m, (const void*)c->part, part_slots(c, S), c->gs, c->acc, c->bhblk, c->kr,
-                           (const int*)c->fn, (const double*)c->xp, (const int*)c->fl,
-                           (const double*)c->xh, P, i0, i1);
+        launch_fin<1, 0>(c, in, P, S, i0, i1, false);
     else
-        hipLaunchKernelGGL((k_fin<0, 0>), gf, dim3(WG), 0, c->st, in, c->X, c->Y, c->H1, c->H2,
-                           c->m, (const void*)c->part, part_slots(c, S), c->gs, c->acc, c->bhblk, c->kr,
-                           (const int*)c->fn, (const double*)c->xp, (const int*)c->fl,
-                           (const double*)c->xh, P, i0, i1);
+        launch_fin<0, 0>(c, in, P, S, i0, i1, false);
     if (!mixed) c->acc_ok = false;
     HIPCHK(c, hipGetLastError());
     const size_t cap = (size_t)c->cap, cnt = (size_t)(i1 - i0);
@@ -692,9 +704,7 @@ int pn1_energy(pn1_ctx* c, pn1_energy_t* out)
     if (!ready(c, &rc)) return rc;
     if (!out) return seterr(c, PN1_EINVAL, "null output");
     const Phys P = make_phys(c);
-    hipLaunchKernelGGL(k_prep, dim3(c->nblk), dim3(WG), 0, c->st, c->X, c->m, P, c->j64,
-                       c->gblk, fp64_prep(), c->fl, c->fblk);
-    hipLaunchKernelGGL((k_rows_sum<NGS>), dim3(1), dim3(WG), 0, c->st, c->gblk, c->nblk, c->gs);
+    if ((rc = prep_x(c, P, true))) return rc;
     if (c->n > 1)
         hipLaunchKernelGGL(k_epair64, dim3(c->pair_grid), dim3(WG), 0, c->st, c->j64, c->X,
                            (double*)c->part, P, c->S, c->nIblk);
@@ -722,6 +732,7 @@ int pn1_step(pn1_ctx* c, int steps)
     if (steps == 0) return PN1_OK;
     const Phys P = make_phys(c);
     if ((rc = ensure_prev_acc(c, P))) return rc;
+    if ((rc = enqueue_prep(c, P))) return rc;
     if (c->prof) {
         for (int s = 0; s < steps; ++s)
             if ((rc = enqueue_step(c, P))) return rc;
@@ -828,9 +839,9 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
         c->tile_req = keep_tile;
         plan(c);
         int r = ensure_part(c);
-        if (!r) r = enqueue_force(c, 0, P);                      // warm-up
+        if (!r) r = enqueue_force(c, P);                         // warm-up
         if (!r && hipEventRecord(ea, c->st) != hipSuccess) r = seterr(c, PN1_EDEVICE, "hipEventRecord failed");
-        for (int k = 0; k < reps && !r; ++k) r = enqueue_force(c, 0, P);
+        for (int k = 0; k < reps && !r; ++k) r = enqueue_force(c, P);
         if (!r && hipEventRecord(eb, c->st) != hipSuccess) r = seterr(c, PN1_EDEVICE, "hipEventRecord failed");
         float ms = 0.0f;
         if (!r && (hipEventSynchronize(eb) != hipSuccess || hipEventElapsedTime(&ms, ea, eb) != hipSuccess))
@@ -905,28 +916,29 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
     P.cap = n;
     JRec64* j64 = (JRec64*)(base + NA_J64);
     double* part = base + NA_PART;
-    double* gblk = base + NA_GBLK;
-    double* gs = base + NA_GS;
-    double* bhblk = base + NA_BH;
-    const int nst = n - 1, nblk = nblocks(nst), nib = (nst + WG - 1) / WG;
+    RowBufs R = {};
+    R.rows = base + NA_ROWS;
+    R.gs = base + NA_GS;
+    MixPrep M = {};
+    FinBufs F = {};
+    F.in = st;
+    F.m = m;
+    F.acc = acc;
+    F.j64 = j64;
+    const int nst = n - 1, nib = (nst + WG - 1) / WG;
+    const int nrow = nst > 0 ? (nst + RB - 1) / RB : 1;
     const int S = na_split(nst);
-    hipLaunchKernelGGL(k_prep, dim3(nblk), dim3(WG), 0, s, st, m, P, j64, gblk, fp64_prep(),
-                       (int*)nullptr, (int*)nullptr);
-    hipLaunchKernelGGL((k_rows_sum<NGS>), dim3(1), dim3(WG), 0, s, (const double*)gblk, nblk, gs);
-    if (nst > 0) {
-        int grid = S * nib;
-        if (S <= 8 && 8 % S == 0) grid = 8 * ((nib + 8 / S - 1) / (8 / S));
-        hipLaunchKernelGGL(k_pair64<0>, dim3(grid), dim3(WG), 0, s, (const JRec64*)j64, st, part,
-                           P, S, nib, 0);
-    }
-    hipLaunchKernelGGL((k_fin<0, 0>), dim3(nblk), dim3(WG), 0, s, st, (double*)nullptr,
-                       (double*)nullptr, (double*)nullptr, (double*)nullptr, m,
-                       (const void*)part, S, (const double*)gs, acc, bhblk, (float*)nullptr,
-                       (const int*)nullptr, (const double*)nullptr, (const int*)nullptr,
-                       (const double*)nullptr, P, 1, n);
-    hipLaunchKernelGGL((k_bh<0>), dim3(1), dim3(WG), 0, s, (const double*)bhblk, nblk,
-                       (const double*)gs, (double*)nullptr, (double*)nullptr, (double*)nullptr,
-                       (double*)nullptr, acc, P);
+    // no ticket counter here: a call that overlapped another one against the
+    // contract would leave it wrong for every later call
+    hipLaunchKernelGGL(k_prep, dim3((nrow + FG - 1) / FG), dim3(FWG), 0, s, st, m, P, nrow, j64, R,
+                       M, (const double*)nullptr, (const float*)nullptr);
+    hipLaunchKernelGGL(k_gsum, dim3(1), dim3(FWG), 0, s, R, nrow);
+    if (nst > 0)
+        hipLaunchKernelGGL(k_pair64<0>, dim3(pair_grid(S, nib)), dim3(WG), 0, s,
+                           (const JRec64*)j64, st, part, P, S, nib, 0);
+    hipLaunchKernelGGL((k_fin<0, 0, FG>), dim3(nrow), dim3(FWG), 0, s, F, R, (const void*)part, S,
+                       M, P, 0, n, nrow);
+    hipLaunchKernelGGL(k_bh, dim3(1), dim3(FWG), 0, s, F, R, nrow, P);
     return hipGetLastError() == hipSuccess ? PN1_OK : PN1_EDEVICE;
 }
 

@@ -15,7 +15,8 @@ constexpr int NEB = 4;      // energy per-block partials
 // sqrt(3/2): stored velocities are pre-scaled by it, so that the pair term
 // 1.5 (v_j.r)^2 w^2 is a plain square of (s_j.r) w with s_j = sqrt(3/2) v_j.
 #define PN1_SQ15 1.2247448713915890491
-// 4 / sqrt(3/2) and 3 / sqrt(3/2) = sqrt(6)
+// 1 / sqrt(3/2), 4 / sqrt(3/2) and 3 / sqrt(3/2) = sqrt(6)
+#define PN1_ISQ15 0.81649658092772603
 #define PN1_4OSQ15 3.2659863237109041
 #define PN1_SQ6 2.4494897427831781
 
@@ -107,12 +108,11 @@ struct Phys {
 // A star whose previous evaluation had mscale * A_TS > PN1_HARD_K |a| (its
 // pair terms cancel to 1/30 of their magnitudes or less) takes every pair in
 // FP64: the FP32 rounding of the terms, ~0.1 u of their magnitudes once
-// averaged, would otherwise near 1e-6 of |a|.  With MixPrep::hard_rows the
-// star's whole row is evaluated in FP64 by a pass of its own (k_hard_rows,
-// one workgroup per such star) and its FP32 lane does no extra work
-// (rc2 = dn2 = 0; k_fin takes the FP64 row instead); otherwise its FP32 lane
-// takes the FP64 branch for every pair (rc2 = FLT_MAX), which makes its whole
-// wave several times slower than the others.
+// averaged, would otherwise near 1e-6 of |a|.  Its whole row is evaluated in
+// FP64 by k_fin, in the workgroup that finishes the star, and its FP32 lane
+// does no extra work (rc2 = dn2 = 0).  An FP64 branch in the lane for every
+// pair instead would make its whole wave several times slower than the
+// others.
 // Without a previous evaluation (after an upload) the thresholds are
 // rc2 = 0 and dn2 = FLT_MAX: no FP64 pairs, lo parts everywhere.
 #define PN1_CLOSE_KAPPA 0.25
@@ -132,20 +132,17 @@ struct __align__(8) Thr {
 // lam m_j e_j^2 > tauf, tauf = PN1_FLAG_ETA / (6 u D), D twice the
 // farthest star from the BH at upload, is taken out of the FP32 pass (its
 // mixed record is neutralised: far away, zero mass, zero 1PN fields) and
-// its pairs with every star are evaluated in FP64 by k_pair_fl, whose sums
-// k_fin adds.  Such stars are rare (none in the benchmark's Plummer sphere
-// at N = 131072 within |d| < 3e-3).
+// its pairs with every star are evaluated in FP64 by k_fin.  Such stars are
+// rare (none in the benchmark's Plummer sphere at N = 131072 within
+// |d| < 3e-3).
 #define PN1_FLAG_ETA 1e-8
 #define PN1_FAR 1e18f
-// What k_prep needs for the mixed form besides the FP64 records.
+// What the mixed form's prep needs besides the FP64 records.
 struct MixPrep {
     JRec32* j32;            // null: FP64 form (nothing below is used)
     Thr* thr;
-    const double* aprev;    // previous evaluation (both null after an upload)
-    const float* kprev;
     double mmax, tauf;      // the cluster's largest |m| of its stars; BH-close threshold
     double lam;
-    int hard_rows;          // stars beyond PN1_HARD_K get FP64 rows of their own
 };
 
 // ---------------------------------------------------------------------

@@ -28,23 +28,22 @@ struct pn1_ctx {
     int S = 1, nIblk = 0, pair_grid = 0, nblk = 1, tile = 64;
     // device buffers
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr;
-    double *m = nullptr, *acc = nullptr, *gblk = nullptr, *gs = nullptr;
-    double *bhblk = nullptr, *eblk = nullptr, *eout = nullptr;
+    double *m = nullptr, *acc = nullptr, *rows = nullptr, *gs = nullptr;
+    double *eblk = nullptr, *eout = nullptr;
+    // three buffers of cap + 2 records: each of a step's evaluations reads
+    // one and prepares the next
     pn1dev::JRec64* j64 = nullptr;
     pn1dev::JRec32* j32 = nullptr;
     pn1dev::Thr* thr = nullptr; // mixed form's per-star pair thresholds
     float* kr = nullptr;        // mixed form's per-star cancellation ratios
-    // mixed form: stars taken out of the FP32 pass (flags, per-block counts,
-    // their list and number) and the FP64 sums of their pairs
-    int *fl = nullptr, *fblk = nullptr, *flist = nullptr, *fn = nullptr;
-    double* xp = nullptr;
-    // hard stars (PN1_HARD_K): their list, FP64 rows [NACC + 1][cap] and the
-    // segment sums of the split rows [HCAP][HSEG][NACC + 1]; hgrid
-    // workgroups of k_hard_rows take the work units in turn
-    int* hlist = nullptr;
-    double* xh = nullptr;
-    double* hseg = nullptr;
-    int hgrid = 1024;
+    // per row of 64 stars: its values of the sums over all stars (rows) and,
+    // mixed form, the masks of its BH-close and hard stars; the list of
+    // BH-close stars and its length; the O(n) kernels' ticket counter
+    int nrow = 1;
+    unsigned long long *fmask = nullptr, *hmask = nullptr;
+    int *flist = nullptr, *fn = nullptr;
+    unsigned int* ticket = nullptr;
+    double* xr = nullptr;       // FP64 sums for hard stars and BH-close pairs [NACC + 1][cap]
     // acc and kr hold the last mixed evaluation of the uploaded run (cleared
     // by pn1_upload and by FP64 evaluations): the mixed form's thresholds
     // read them
@@ -66,9 +65,12 @@ namespace pn1host {
 
 int seterr(pn1_ctx* c, int code, const char* fmt, ...);
 pn1dev::Phys make_phys(const pn1_ctx* c);
-// Launches one force evaluation (stage 0: plain, on X; 1..3: the stage
-// driver's calls, with their state updates) on the context's stream.
-int enqueue_force(pn1_ctx* c, int stage, const pn1dev::Phys& P);
+// The records and sums of a plain evaluation or a step's first one, on X.
+int enqueue_prep(pn1_ctx* c, const pn1dev::Phys& P);
+// One prepared evaluation on the context's stream (stage 0: plain, on X;
+// 1..3: the stage driver's calls, with their state updates, each preparing
+// the next; stage 3 the next step's first).
+int enqueue_eval(pn1_ctx* c, int stage, const pn1dev::Phys& P);
 // Mixed form after an upload: one evaluation with the pair thresholds off
 // (no previous accelerations yet), so that the next has them.
 int ensure_prev_acc(pn1_ctx* c, const pn1dev::Phys& P);

@@ -6,7 +6,9 @@
 //   coff[nc + 1]   first particle of each cluster
 //   cm0[nc]        BH mass of each cluster
 //   cmmax[nc]      largest star mass of each cluster
-//   blk[nb], cblk[nc + 1]   256-star blocks of the O(n) kernels, per cluster
+//   blk[nb], cblk[nc + 1]   256-star blocks, per cluster (energy, adjoint)
+//   row[nrow], crow[nc + 1]   64-star rows of the force's O(n) kernels, per
+//                  cluster; pblk[npblk]: groups of FG of them (k_ens_prep)
 //   items[nitems]  pair work items in 8 per-XCD queues (qoff[9]): whole
 //                  clusters go to the least-loaded queue, largest first;
 //                  each queue is sorted by decreasing pair count
@@ -32,7 +34,7 @@ struct pn1_ens {
     int L_req = 0, tile_req = 0, variant_req = -1;
     int L = 512, tile = 64;
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr, *m = nullptr, *acc = nullptr;
-    double *gblk = nullptr, *gs = nullptr, *bhblk = nullptr, *eblk = nullptr, *eout = nullptr;
+    double *rows = nullptr, *gs = nullptr, *eblk = nullptr, *eout = nullptr;
     double* cm0 = nullptr;
     double* cmmax = nullptr;      // each cluster's largest star mass
     pn1dev::Thr* thr = nullptr;   // mixed form's per-star pair thresholds
@@ -40,20 +42,19 @@ struct pn1_ens {
     bool acc_ok = false;          // acc, kr hold the last mixed evaluation
     bool eqm = false;             // each cluster's stars have one mass
     double* ctauf = nullptr;      // each cluster's BH-close threshold (PN1_FLAG_ETA)
-    // mixed form: stars taken out of the FP32 pass (flags, per-block counts
-    // [nb_cap], lists at each cluster's offset, per-cluster numbers) and the
-    // FP64 sums of their pairs [NACC + 1][cap]
-    int *fl = nullptr, *fblk = nullptr, *flist = nullptr, *fn = nullptr;
-    double* xp = nullptr;
-    // hard stars (PN1_HARD_K): per-cluster lists, all clusters' (star,
-    // cluster) pairs [cap] (their number in counter[NXCD]), FP64 rows
-    // [NACC + 1][cap] and the segment sums of the split rows
-    // [HCAP][HSEG][NACC + 1]
-    int* hlist = nullptr;
-    int2* hall = nullptr;
-    double* xh = nullptr;
-    double* hseg = nullptr;
-    int fblk_cap = 0, gblk_cap = 0, bhblk_cap = 0, eblk_cap = 0;
+    // per row: its values of the sums over all stars (rows) and, mixed form,
+    // the masks of its BH-close and hard stars; BH-close stars (lists at each
+    // cluster's offset, per-cluster numbers); the O(n) kernels' tickets
+    unsigned long long *fmask = nullptr, *hmask = nullptr;
+    int *flist = nullptr, *fn = nullptr;
+    unsigned int* ticket = nullptr;
+    double* xr = nullptr;         // as in pn1_ctx
+    pn1dev::EBlk *row = nullptr, *pblk = nullptr;
+    int* crow = nullptr;
+    int nrow = 0, npblk = 0;
+    int fmask_cap = 0, hmask_cap = 0, row_cap = 0, pblk_cap = 0;
+    int rows_cap = 0, eblk_cap = 0;
+    // three buffers of cap + 2 records, as in pn1_ctx
     pn1dev::JRec64* j64 = nullptr;
     pn1dev::JRec32* j32 = nullptr;
     int *coff = nullptr, *cblk = nullptr, *qoff = nullptr;
@@ -82,9 +83,9 @@ namespace pn1host {
 
 int eerr(pn1_ens* e, int code, const char* fmt, ...);
 pn1dev::Phys ens_phys(const pn1_ens* e);
-// One force evaluation of every cluster (stage 0: plain, on X; 1..3: the
-// stage driver's calls with their state updates), on the ensemble's stream.
-int ens_enqueue_force(pn1_ens* e, int stage, const pn1dev::Phys& P);
+// As enqueue_prep and enqueue_eval, for every cluster.
+int ens_enqueue_prep(pn1_ens* e, const pn1dev::Phys& P);
+int ens_enqueue_eval(pn1_ens* e, int stage, const pn1dev::Phys& P);
 // Mixed form after an upload: one evaluation with the pair thresholds off.
 int ens_ensure_prev_acc(pn1_ens* e, const pn1dev::Phys& P);
 int ens_fetch3(pn1_ens* e, const double* dsrc, double* out);

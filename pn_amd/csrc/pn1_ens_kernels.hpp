@@ -2,21 +2,20 @@
 //
 // All clusters live in one state (SoA stride cap).  Cluster c occupies
 // particles [coff[c], coff[c + 1]); its BH is particle coff[c], its stars
-// follow.  One force evaluation of the whole ensemble is five launches:
+// follow.  One force evaluation of the whole ensemble is two launches, after
+// one that prepares the first (as in a single context):
 //
-//   k_ens_prep   per-star j-records and per-block separable sums; blocks
-//                come from a block table, each inside one cluster
-//   k_ens_gsum   one workgroup per cluster: that cluster's separable sums;
-//                also resets the work counters of the pair kernel and the
-//                count of the mixed form's hard stars
+//   k_ens_prep   per-star j-records and the clusters' separable sums;
+//                workgroups come from a table, each inside one cluster, and
+//                a cluster's last one adds its sums (a ticket per cluster)
 //   k_ens_pair*  ONE persistent launch for all clusters: workgroups take
 //                (cluster, 256-star i-block, j-chunk) items from per-XCD
 //                queues (atomic counters), items sorted by decreasing cost
 //                on the host; every item writes its partial sums to its own
 //                slot, so the result does not depend on which workgroup ran
 //                which item
-//   k_ens_fin    per star, as k_fin, with its cluster's sums and BH
-//   k_ens_bh     one workgroup per cluster: its BH
+//   k_ens_fin    per row of 64 stars, as k_fin, with its cluster's sums and
+//                BH; it also resets the pair kernel's queues
 //
 // The pair arithmetic is the single-cluster kernels' (body64 / body32),
 // and so is the order of each lane's j loop: with one chunk per cluster
@@ -181,124 +180,99 @@ void k_ens_pair32x(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64
     ens_pair32<PP, TS, EQ>(jr, j64, thr, st, part, items, counter, qoff, cmmax, P, tile);
 }
 
-// M: the mixed form's inputs (M.j32 null: FP64), with each cluster's largest
-// star mass cmmax[c] and BH-close threshold ctauf[c] in place of M.mmax,
-// M.tauf; fl, fblk: as k_prep.
-inline __global__ __launch_bounds__(WG) void k_ens_prep(const double* __restrict__ st,
-                                                const double* __restrict__ m,
-                                                const double* __restrict__ cm0,
-                                                const int* __restrict__ coff,
-                                                const EBlk* __restrict__ blk, Phys P,
-                                                JRec64* __restrict__ j64,
-                                                double* __restrict__ gblk, MixPrep M,
-                                                const double* __restrict__ cmmax,
-                                                const double* __restrict__ ctauf,
-                                                int* __restrict__ fl, int* __restrict__ fblk)
+// Per-cluster buffers.  Cluster c's rows of 64 stars are [crow[c],
+// crow[c + 1]) (at least one, also without stars).
+struct EnsBufs {
+    const double* cm0;
+    const int* coff;
+    const int* crow;
+    const double *cmmax, *ctauf;
+    unsigned int* counter;        // the pair kernel's queues
+};
+
+__device__ __forceinline__ void reset_queues(unsigned int* counter)
 {
-    const EBlk b = blk[blockIdx.x];
-    const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
-    const int li = b.first + (int)threadIdx.x;
-    double g[NGS];
+    if (blockIdx.x == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
+}
+
+// As k_prep, one workgroup per FG rows of a cluster (pblk: its cluster and
+// first local star).  M.mmax, M.tauf: per cluster, from E; R.ticket, R.gs and
+// R.fn: one entry (or NGS) per cluster.
+inline __global__ __launch_bounds__(FWG) void k_ens_prep(const double* __restrict__ st,
+                                                const double* __restrict__ m, Phys P, EnsBufs E,
+                                                const EBlk* __restrict__ pblk,
+                                                JRec64* __restrict__ j64, RowBufs R, MixPrep M,
+                                                const double* __restrict__ aprev,
+                                                const float* __restrict__ kprev)
+{
+    reset_queues(E.counter);
+    const EBlk b = pblk[blockIdx.x];
+    const int off = E.coff[b.c], nst = E.coff[b.c + 1] - off - 1;
+    const int r0 = E.crow[b.c], r1 = E.crow[b.c + 1];
+    const int row = r0 + b.first / RB + (int)(threadIdx.x >> 6);
+    const size_t cap = (size_t)P.cap;
+    if (M.j32) {
+        M.mmax = E.cmmax[b.c];
+        M.tauf = E.ctauf[b.c];
+    }
+    if (row < r1) {
+        const int li = b.first + (int)threadIdx.x;
+        double g[NGS];
+        bool f = false, hard = false;
+        const bool ok = li < nst;
+        if (ok) {
+            const int p = off + 1 + li;
+            const double x[3] = {st[p], st[cap + p], st[2 * cap + p]};
+            const double v[3] = {st[3 * cap + p], st[4 * cap + p], st[5 * cap + p]};
+            const double x0[3] = {st[off], st[cap + off], st[2 * cap + off]};
+            double a[3] = {0.0, 0.0, 0.0};
+            float kr = 0.0f;
+            if (aprev) {
 #pragma unroll
-    for (int k = 0; k < NGS; ++k) g[k] = 0.0;
-    if (M.j32) {
-        M.mmax = cmmax[b.c];
-        M.tauf = ctauf[b.c];
-    }
-    bool f = false, hard = false;
-    if (li < nst) {
-        f = prep_star(st, m, P.cap, off + 1 + li, off, cm0[b.c], P.eps2, j64, g, M, hard);
-        hard = hard && M.hard_rows;
-        if (M.j32) fl[off + 1 + li] = (f ? 1 : 0) | (hard ? 2 : 0);
-    }
-    block_sum<NGS>(g, gblk + (size_t)blockIdx.x * NGS);
-    if (M.j32) {
-        const int cnt = __syncthreads_count(f);
-        const int hcnt = __syncthreads_count(hard);
-        if (threadIdx.x == 0) {
-            fblk[2 * blockIdx.x] = cnt;
-            fblk[2 * blockIdx.x + 1] = hcnt;
+                for (int k = 0; k < 3; ++k) a[k] = aprev[k * cap + p];
+                kr = kprev[p];
+            }
+            f = prep_star(x, v, x0, m[p], p, E.cm0[b.c], P.eps2, j64, g, M, aprev != nullptr, a,
+                          kr, hard);
         }
+        const double cb[3] = {0.0, 0.0, 0.0};
+        put_row<false, true>(row, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
+                             R.hmask);
     }
+    if (last_block(R.ticket + b.c, (unsigned)((r1 - r0 + FG - 1) / FG)))
+        close_prep(R, M.j32 != nullptr, r0, r1, off + 1, R.gs + (size_t)b.c * NGS, R.flist + off,
+                   R.fn + b.c);
 }
 
-// One workgroup per cluster: its BH-close stars, in increasing order, at
-// flist[coff[c] ..), their number in fn[c]; its hard stars likewise at
-// hlist[coff[c] ..), their number in hn[c], and appended as (star,
-// cluster) pairs to the evaluation's list of every cluster's hard stars,
-// hall[0 .. *hcount) (k_ens_gsum zeroes *hcount).  The clusters' order in
-// hall depends on which workgroup reserves its range first; each hard row
-// is computed on its own, so the results do not.
-inline __global__ __launch_bounds__(WG) void k_ens_flist(const int* __restrict__ fl,
-                                                 const int* __restrict__ fblk,
-                                                 const int* __restrict__ cblk,
-                                                 const int* __restrict__ coff,
-                                                 int* __restrict__ flist, int* __restrict__ fn,
-                                                 int* __restrict__ hlist, int* __restrict__ hn,
-                                                 int2* __restrict__ hall,
-                                                 unsigned int* __restrict__ hcount)
+// As k_fin: one workgroup per row of the ensemble (G = FG, blk the row
+// table) or per FG rows of a cluster (G = 1, blk = pblk).
+template <int MODE, int STAGE, int G>
+__global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
+               const void* __restrict__ part, const long long* __restrict__ poff, int L,
+               MixPrep M, Phys P)
 {
-    __shared__ int s_at;
-    const int c = blockIdx.x;
-    list_flagged<0, 2>(fl, fblk, cblk[c], cblk[c + 1], coff[c] + 1, coff[c + 1],
-                       flist + coff[c], fn + c);
-    const int nh = list_flagged<1, 2>(fl, fblk, cblk[c], cblk[c + 1], coff[c] + 1,
-                                      coff[c + 1], hlist + coff[c], hn + c);
-    if (nh == 0) return;                     // uniform: every thread holds the count
-    if (threadIdx.x == 0) s_at = (int)atomicAdd(hcount, (unsigned int)nh);
-    __syncthreads();                         // s_at, and the list written above
-    for (int k = (int)threadIdx.x; k < nh; k += WG)
-        hall[s_at + k] = make_int2(hlist[coff[c] + k], c);
-}
-
-// FP64 rows of every cluster's hard stars (as k_hard_rows, j over the
-// star's own cluster): every entry of hall in HSEG units (into hseg), or,
-// beyond HCAP entries, every one whole; the workgroups take the units in
-// turn.  With at most HCAP hard stars in the ensemble, each row is summed
-// as a single-cluster run sums it.
-inline __global__ __launch_bounds__(HWG) void k_ens_hard_rows(const JRec64* __restrict__ jr,
-                                                      const double* __restrict__ st,
-                                                      const int* __restrict__ coff,
-                                                      const int2* __restrict__ hall,
-                                                      const unsigned int* __restrict__ hcount,
-                                                      double* __restrict__ xh,
-                                                      double* __restrict__ hseg, Phys P)
-{
-    const int nh = (int)*hcount, ns = hard_split(nh), nu = ns * HSEG + (nh - ns);
-    for (int u = blockIdx.x; u < nu; u += gridDim.x) {
-        const int2 w = hall[u < ns * HSEG ? u / HSEG : ns + (u - ns * HSEG)];
-        hard_unit(jr, st, P.cap, P.eps2, u, ns, w.x, coff[w.y] + 1, coff[w.y + 1], xh, hseg);
-    }
-}
-
-// The split rows' segment sums, in segment order (as k_hard_sum).
-inline __global__ __launch_bounds__(WG) void k_ens_hard_sum(const int2* __restrict__ hall,
-                                                    const unsigned int* __restrict__ hcount,
-                                                    const double* __restrict__ hseg,
-                                                    double* __restrict__ xh, int cap)
-{
-    const int t = blockIdx.x * WG + threadIdx.x;
-    const int ns = hard_split((int)*hcount);
-    if (t < ns * (NACC + 1)) hard_sum(hseg, t, hall[t / (NACC + 1)].x, cap, xh);
-}
-
-// Per star block: its stars' FP64 pairs with their cluster's flagged stars
-// (k_pair_fl per cluster), into xp [NACC + 1][cap] at the star's index.
-inline __global__ __launch_bounds__(WG) void k_ens_pair_fl(const JRec64* __restrict__ jr,
-                                                   const double* __restrict__ st,
-                                                   const int* __restrict__ coff,
-                                                   const EBlk* __restrict__ blk,
-                                                   const int* __restrict__ flist,
-                                                   const int* __restrict__ fn,
-                                                   double* __restrict__ xp, Phys P)
-{
+    reset_queues(E.counter);
     const EBlk b = blk[blockIdx.x];
-    const int nf = fn[b.c];
-    const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
-    const int li = b.first + (int)threadIdx.x;
-    if (nf == 0 || li >= nst) return;
-    const int i = off + 1 + li;
-    flagged_pairs(jr, st, P.cap, i, P.eps2, flist + off, nf, xp, (size_t)P.cap, i);
+    const int off = E.coff[b.c], nst = E.coff[b.c + 1] - off - 1;
+    const int r0 = E.crow[b.c], r1 = E.crow[b.c + 1];
+    const Row q = {off, nst, b.first, r0 + b.first / RB};
+    double* gs = R.gs + (size_t)b.c * NGS;
+    if (MODE == 1) {
+        M.mmax = E.cmmax[b.c];
+        M.tauf = E.ctauf[b.c];
+    }
+    if (nst > 0) {
+        const void* base = MODE == 0 ? (const void*)((const double*)part + poff[b.c] * NACC)
+                                     : (const void*)((const float*)part + poff[b.c] * MROWS);
+        fin_rows<MODE, STAGE, G>(F, R, q, base, ens_nchunks(nst, L), (size_t)nst, 0, gs,
+                                 R.flist + off, R.fn + b.c, E.cm0[b.c], M, P);
+    } else {
+        empty_row(R, q.row, MODE == 1);
+    }
+    const unsigned nblk = (unsigned)(G == 1 ? (r1 - r0 + FG - 1) / FG : r1 - r0);
+    if (last_block(R.ticket + b.c, nblk))
+        fin_close<MODE, STAGE>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P);
 }
 
 // One workgroup per cluster: rows [cblk[c], cblk[c+1]) of `rows` (N wide).
@@ -312,81 +286,6 @@ __device__ __forceinline__ void cluster_rows_sum(const double* __restrict__ rows
     for (int b = cblk[c] + (int)threadIdx.x; b < cblk[c + 1]; b += WG)
 #pragma unroll
         for (int k = 0; k < N; ++k) g[k] += rows[(size_t)b * N + k];
-}
-
-inline __global__ __launch_bounds__(WG) void k_ens_gsum(const double* __restrict__ gblk,
-                                                const int* __restrict__ cblk,
-                                                double* __restrict__ gs,
-                                                unsigned int* __restrict__ counter)
-{
-    const int c = blockIdx.x;
-    if (c == 0 && threadIdx.x <= NXCD) counter[threadIdx.x] = 0u;   // queues, hard stars
-    double g[NGS];
-    cluster_rows_sum<NGS>(gblk, cblk, c, g);
-    block_sum<NGS>(g, gs + (size_t)c * NGS);
-}
-
-template <int MODE, int STAGE>
-__global__ __launch_bounds__(WG) void k_ens_fin(const double* in, double* X, double* Y,
-                                               double* H1, double* H2,
-                                               const double* __restrict__ m,
-                                               const double* __restrict__ cm0,
-                                               const int* __restrict__ coff,
-                                               const EBlk* __restrict__ blk,
-                                               const void* __restrict__ part,
-                                               const long long* __restrict__ poff,
-                                               const double* __restrict__ gs,
-                                               double* __restrict__ acc,
-                                               double* __restrict__ bhblk,
-                                               const double* __restrict__ cmmax,
-                                               float* __restrict__ kout,
-                                               const int* __restrict__ fn,
-                                               const double* __restrict__ xp,
-                                               const int* __restrict__ fl,
-                                               const double* __restrict__ xh, Phys P,
-                                               EConst E)
-{
-    const EBlk b = blk[blockIdx.x];
-    const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
-    const int li = b.first + (int)threadIdx.x;
-    double cb[3] = {0.0, 0.0, 0.0};
-    if (li < nst) {
-        double S_[NACC], ts, a[3];
-        if (MODE == 1 && (fl[off + 1 + li] & 2)) {
-            load_row(xh, (size_t)P.cap, off + 1 + li, S_, ts);
-        } else {
-            const void* base = MODE == 0
-                                   ? (const void*)((const double*)part + poff[b.c] * NACC)
-                                   : (const void*)((const float*)part + poff[b.c] * MROWS);
-            gather_acc<MODE, (STAGE <= 1)>(base, ens_nchunks(nst, E.L), (size_t)nst, li,
-                             MODE == 1 ? cmmax[b.c] : 1.0, S_, ts);
-            if (MODE == 1 && fn[b.c] > 0) add_flagged(xp, (size_t)P.cap, off + 1 + li, S_, ts);
-        }
-        fin_star<STAGE>(in, X, Y, H1, H2, m, P.cap, off + 1 + li, off, S_,
-                        gs + (size_t)b.c * NGS, fin_consts(P, cm0[b.c]), acc, cb, a);
-        if (MODE == 1 && kout) kout[off + 1 + li] = cancel_ratio(ts, a);
-    }
-    block_sum<3>(cb, bhblk + (size_t)blockIdx.x * 3);
-}
-
-template <int STAGE>
-__global__ __launch_bounds__(WG) void k_ens_bh(const double* __restrict__ bhblk,
-                                              const int* __restrict__ cblk,
-                                              const int* __restrict__ coff,
-                                              const double* __restrict__ gs, double* X,
-                                              double* Y, double* H1, double* H2,
-                                              double* __restrict__ acc, Phys P)
-{
-    const int c = blockIdx.x;
-    double s[3];
-    cluster_rows_sum<3>(bhblk, cblk, c, s);
-    __shared__ double tot[3];
-    block_sum<3>(s, tot);
-    if (threadIdx.x == 0) {
-        const double t[3] = {tot[0], tot[1], tot[2]};
-        bh_finish<STAGE>(t, gs + (size_t)c * NGS, coff[c], P.cap, P.lam, P.dt, X, Y, H1, H2,
-                         acc);
-    }
 }
 
 // ---------------------------------------------------------------------

@@ -1,17 +1,21 @@
 // pn1_kernels.hpp -- device code of libpn1 (gfx950, wave64).
 //
 // One force evaluation of Limit-sticky9's force() (Limit-sticky9.c:21-424)
-// is five launches on one stream:
+// is two launches on one stream, after one that prepares the first:
 //
 //   k_prep    O(n)   per-star BH geometry (d, |d|^2, e = (|d|^2+eps^2)^-1/2)
-//                    written once as an AoS j-record, plus per-block
-//                    partials of the separable sums (sum m e, sum m e^3 d, ...)
-//   k_gsum    1 WG   fixed-order reduction of those partials
+//                    written once as an AoS j-record, and the separable sums
+//                    (sum m e, sum m e^3 d, ...)
 //   k_pair*   O(n^2) the star-star pair sums, one rsqrt per pair
 //   k_fin     O(n)   star accelerations from the pair sums and the O(n)
-//                    closed forms; the stage update of the RK driver; per-block
-//                    partials of the BH's 1PN acceleration
-//   k_bh      1 WG   BH acceleration and its stage update
+//                    closed forms, the BH's acceleration, the stage update of
+//                    the RK driver and, inside a step, all that k_prep does
+//                    for the driver's next evaluation
+//
+// A step of the driver is therefore k_prep once and then (k_pair, k_fin)
+// three times per step.  The O(n) kernels end with the sums over all stars:
+// their workgroups take a ticket when done, and the last one adds the
+// per-row partials and finishes the BH (last_block).
 //
 // Pair kernels: i-particle per lane in VGPRs; the j loop has wave-uniform
 // bounds, so each j-record is fetched with scalar loads into SGPRs and
@@ -30,97 +34,268 @@
 #include "pn1_common.hpp"
 
 namespace pn1dev {
-// Stage update of the reference's RK driver for particle p, given its
-// acceleration a (Limit-sticky9.c:853-891).  STAGE 1..3 follow the three
-// force calls; STAGE 0 (plain force evaluation) does nothing.  FMA
-// contraction is off so each line rounds exactly as the reference's.
+// What the stage update of the reference's RK driver (Limit-sticky9.c:853-891)
+// reads of particle p: its state in this force call (x, v) and, from stage 2
+// on, at the start of the step (X, V); stage 3 also the sums of the two
+// stage states (hx, hv).  Loaded ahead of the acceleration it needs.
+struct StageIn {
+    double x[3], v[3], X[3], V[3], hx[3], hv[3];
+};
+
+// Of components row0 .. row0 + n - 1, in s from index 0 on.
 template <int STAGE>
-__device__ __forceinline__ void stage_update(int p, int cap, const double (&a)[3],
-                                             double* X, double* Y, double* H1,
-                                             double* H2, double dt)
+__device__ __forceinline__ StageIn stage_load(const double* in, const double* X,
+                                              const double* H1, const double* H2, int cap, int p,
+                                              int row0 = 0, int n = 3)
+{
+    StageIn s;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (k >= n) break;
+        const size_t ix = (size_t)(row0 + k) * cap + p, iv = (size_t)(3 + row0 + k) * cap + p;
+        s.x[k] = in[ix];
+        s.v[k] = in[iv];
+        if (STAGE >= 2) {
+            s.X[k] = X[ix];
+            s.V[k] = X[iv];
+        }
+        if (STAGE == 3) {
+            s.hx[k] = H1[ix] + H2[ix];
+            s.hv[k] = H1[iv] + H2[iv];
+        }
+    }
+    return s;
+}
+
+// The position the driver's next force call takes (its velocities are known
+// before this call's acceleration), component k.  FMA contraction is off
+// here and below so each line rounds exactly as the reference's.
+template <int STAGE>
+__device__ __forceinline__ double stage_pos(const StageIn& s, double dt, int k)
+{
+#pragma clang fp contract(off)
+    if (STAGE == 1) return s.x[k] + 0.5 * s.v[k] * dt;
+    if (STAGE == 2) return s.X[k] + 0.5 * s.v[k] * dt;   // v1 of stage 1
+    if (STAGE == 3) {
+        const double hx3 = s.X[k] + s.v[k] * dt;         // v1 of stage 2
+        return (s.X[k] + hx3 + 2.0 * s.hx[k]) / 6.0;
+    }
+    return s.x[k];
+}
+
+// Stage update of component k of particle p (row `row` of the SoA state, k
+// of s), given its acceleration a; STAGE 1..3 follow the three force calls,
+// STAGE 0 (plain force evaluation) does nothing.  nx, nv receive the state
+// the driver's next force call takes (Y after stages 1 and 2, X after
+// stage 3).
+template <int STAGE>
+__device__ __forceinline__ void stage_update(int p, int cap, const StageIn& s, int k, int row,
+                                             double a, double* X, double* Y, double* H1,
+                                             double* H2, double dt, double& nx, double& nv)
 {
 #pragma clang fp contract(off)
     if (STAGE == 0) return;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const size_t ix = (size_t)k * cap + p, iv = (size_t)(3 + k) * cap + p;
-        const double x = X[ix], v = X[iv];
-        if (STAGE == 1) {
-            const double x1 = x + 0.5 * v * dt;
-            const double v1 = v + 0.5 * a[k] * dt;
-            Y[ix] = x1; Y[iv] = v1; H1[ix] = x1; H1[iv] = v1;
-        } else if (STAGE == 2) {
-            const double v1o = Y[iv];            // v1 of stage 1
-            const double x1 = x + 0.5 * v1o * dt;
-            const double v1 = v + 0.5 * a[k] * dt;
-            Y[ix] = x1; Y[iv] = v1; H2[ix] = x1; H2[iv] = v1;
-        } else {
-            const double v1o = Y[iv];            // v1 of stage 2
-            const double hx3 = x + v1o * dt;
-            const double hv3 = v + a[k] * dt;
-            X[ix] = (x + hx3 + 2.0 * (H1[ix] + H2[ix])) / 6.0;
-            X[iv] = (v + hv3 + 2.0 * (H1[iv] + H2[iv])) / 6.0;
-        }
+    const size_t ix = (size_t)row * cap + p, iv = (size_t)(3 + row) * cap + p;
+    nx = stage_pos<STAGE>(s, dt, k);
+    if (STAGE == 1) {
+        nv = s.v[k] + 0.5 * a * dt;
+        Y[ix] = nx; Y[iv] = nv; H1[ix] = nx; H1[iv] = nv;
+    } else if (STAGE == 2) {
+        nv = s.V[k] + 0.5 * a * dt;
+        Y[ix] = nx; Y[iv] = nv; H2[ix] = nx; H2[iv] = nv;
+    } else {
+        const double hv3 = s.V[k] + a * dt;
+        nv = (s.V[k] + hv3 + 2.0 * s.hv[k]) / 6.0;
+        X[ix] = nx;
+        X[iv] = nv;
     }
+}
+
+// ---------------------------------------------------------------------
+// rows: the O(n) kernels take the stars in rows of 64 (one per lane of a
+// wave), FG waves to a workgroup
+// ---------------------------------------------------------------------
+constexpr int RB = 64;
+constexpr int FG = 8;
+constexpr int FWG = FG * RB;
+// A row's share of the sums over all stars: RV doubles, the BH's 1PN
+// acceleration (3), then the NGS separable sums of the next evaluation.
+constexpr int RV = 16;
+constexpr int RV_G = 3;
+static_assert(RV_G + NGS <= RV, "a row's values");
+
+// Sum over the wave, in every lane (xor butterfly: the same bits in each).
+__device__ __forceinline__ double wave_sum(double t)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    return t;
+}
+
+// lo = {a in the lower half (G = 32) or the even rows of 16 (G = 16), b's
+// other half moved there}, and hi the rest: adding both sums a over lane
+// pairs l, l ^ G in the lanes without that bit and b in the others.
+template <int G>
+__device__ __forceinline__ double swap_sum(double a, double b)
+{
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    const unsigned long long ua = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long ub = (unsigned long long)__double_as_longlong(b);
+    u32x2 l, h;
+    if (G == 32) {
+        l = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+        h = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+    } else {
+        l = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
+        h = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+    }
+    const double x = __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0]));
+    const double y = __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+    return x + y;
+}
+
+// The wave's sums of 16 values: lane l gets the sum of v[l >> 2] over all
+// lanes.  Halving the values at each exchange takes 15 of them instead of
+// the 16 x 6 of one butterfly per value, and half the code, which in kernels
+// that run each instruction once is most of their time.
+__device__ __forceinline__ double wave_sums16(const double (&v)[16])
+{
+    const int lane = threadIdx.x & 63;
+    double a[8], b[4], c[2];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a[k] = swap_sum<32>(v[k], v[8 + k]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b[k] = swap_sum<16>(a[k], a[4 + k]);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const bool up = lane & 8;
+        const double keep = up ? b[2 + k] : b[k], send = up ? b[k] : b[2 + k];
+        c[k] = keep + __shfl_xor(send, 8, 64);
+    }
+    const bool up = lane & 4;
+    double t = (up ? c[1] : c[0]) + __shfl_xor(up ? c[0] : c[1], 4, 64);
+    t += __shfl_xor(t, 2, 64);
+    t += __shfl_xor(t, 1, 64);
+    return t;
+}
+
+// Values that one workgroup hands to another within a launch (the rows' sums
+// and masks, to the last workgroup): stored and loaded at device scope, past
+// the XCD's own L2.  A release fence would do the same for ordinary stores,
+// but it writes back every dirty line of that L2, per workgroup (measured on
+// MI355X: 0.14 us each, 1.4 ms of an ensemble's 9864 workgroups).
+template <typename T>
+__device__ __forceinline__ void hand_over(T* p, T v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T take_over(const T* p)
+{
+    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Fixed-order sums of rows [b0, b1), by a workgroup of FWG threads, into
+// tot[RV] (LDS), for every thread of it: thread t adds value t % RV of rows
+// t / RV, t / RV + FWG / RV, ...
+__device__ __forceinline__ void rows_total(const double* rows, int b0, int b1, double* tot)
+{
+    __shared__ double sh[FG][RV];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double t = 0.0;
+#pragma unroll 8
+    for (int b = b0 + (int)threadIdx.x / RV; b < b1; b += FWG / RV)
+        t += take_over(&rows[(size_t)b * RV + (threadIdx.x & (RV - 1))]);
+    t += __shfl_xor(t, 16, 64);
+    t += __shfl_xor(t, 32, 64);
+    if (lane < RV) sh[wid][lane] = t;
+    __syncthreads();
+    if (threadIdx.x < RV) {
+        t = sh[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < FG; ++w) t += sh[w][threadIdx.x];
+        tot[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+
+// Whether this workgroup is the last of `nblk` to get here (the counter goes
+// back to 0 for the next launch).  What the others handed over before is
+// visible to it: every wave waits for its own stores to complete before the
+// workgroup takes its ticket, and the last ticket is taken after all others.
+// Every thread of the workgroup calls it.
+__device__ __forceinline__ bool last_block(unsigned int* cnt, unsigned int nblk)
+{
+    __shared__ bool s_last;
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned int t =
+            __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = t == nblk - 1;
+        if (s_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    return s_last;
 }
 
 // ---------------------------------------------------------------------
 // k_prep: per-star BH geometry + separable sums
 // ---------------------------------------------------------------------
 // Mixed form's pair thresholds of a star at x from its BH whose previous
-// evaluation gave the acceleration aprev and cancellation ratio kprev
-// (null: none known), for star masses up to mmax (see Thr).
-__device__ __forceinline__ Thr pair_thresholds(double x, double y, double z,
-                                               const double* aprev, const float* kprev,
-                                               size_t cap, int p, double mmax, bool rows,
+// evaluation gave the acceleration a and cancellation ratio kr (known:
+// false if there was none), for star masses up to mmax (see Thr).
+__device__ __forceinline__ Thr pair_thresholds(const double (&x)[3], bool known,
+                                               const double (&a)[3], float kr, double mmax,
                                                bool& hard)
 {
     Thr t;
     hard = false;
-    if (!aprev) {
+    if (!known) {
         t.rc2 = 0.0f;
         t.dn2 = __FLT_MAX__;
         return t;
     }
-    hard = !(kprev[p] <= (float)PN1_HARD_K);                   // NaN too
-    if (hard && rows) {          // the FP32 lane's sums are not used
+    hard = !(kr <= (float)PN1_HARD_K);                         // NaN too
+    if (hard) {                  // the FP32 lane's sums are not used
         t.rc2 = t.dn2 = 0.0f;
         return t;
     }
-    const double ax = aprev[p], ay = aprev[cap + p], az = aprev[2 * cap + p];
-    const double A = sqrt(ax * ax + ay * ay + az * az);
-    const double X = sqrt(x * x + y * y + z * z);
-    const double rc2 = mmax / (PN1_CLOSE_KAPPA * A);            // +inf if A == 0
-    const double dn3 = 6.0 * 0x1p-24 * X * mmax / (PN1_LAZY_ETA * A);
-    const double dn2 = cbrt(dn3 * dn3);
-    t.rc2 = hard ? __FLT_MAX__ : (float)fmin(rc2, (double)__FLT_MAX__);
-    // close pairs are found inside the lo-part branch: dn2 >= rc2
-    t.dn2 = fmaxf((float)fmin(dn2, (double)__FLT_MAX__), t.rc2);
+    // 1 / |a| and |x| from one reciprocal square root each, and the power
+    // 2/3 from the FP32 logarithm and exponential (dn2 to ~1e-6: it only says
+    // where the lo parts start to matter)
+    const double A2 = a[0] * a[0] + a[1] * a[1] + a[2] * a[2];
+    const double X2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
+    const double q = mmax * rsq64(A2);                          // NaN if A2 == 0
+    const float rc2 = (float)fmin(q * (1.0 / PN1_CLOSE_KAPPA), (double)__FLT_MAX__);
+    const float dn3 = (float)(6.0 * 0x1p-24 / PN1_LAZY_ETA * q * (X2 * rsq64(X2)));
+    const float dn2 = __builtin_amdgcn_exp2f((2.0f / 3.0f) * __builtin_amdgcn_logf(dn3));
+    t.rc2 = rc2;
+    // no acceleration to compare with: every pair is close
+    t.dn2 = A2 > 0.0 ? fmaxf(fminf(dn2, __FLT_MAX__), rc2) : __FLT_MAX__;
     return t;
 }
 
-// Star p (SoA stride cap) of a cluster whose BH sits at index b0 and has
-// mass m0: writes its j-records and adds its terms of the separable sums
-// to g.  Mixed form (M.j32 set): also its pair thresholds, from its previous
-// acceleration M.aprev (SoA [3][cap]) and cancellation ratio M.kprev, and
-// its mixed record in units of the cluster's largest star mass M.mmax;
-// returns whether the star is close enough to the BH to be taken out of the
-// FP32 pass (see PN1_FLAG_ETA), in which case its mixed record is neutral;
-// hard: whether its pair terms cancel beyond PN1_HARD_K.
-__device__ __forceinline__ bool prep_star(const double* __restrict__ st,
-                                          const double* __restrict__ m, int cap, int p,
-                                          int b0, double m0, double eps2,
-                                          JRec64* __restrict__ j64, double (&g)[NGS],
-                                          const MixPrep& M, bool& hard)
+// Star p at x, velocity v, of a cluster whose BH sits at x0 and has mass m0:
+// writes its j-records and its terms of the separable sums, g.  Mixed form
+// (M.j32 set): also its pair thresholds, from its previous acceleration a
+// and cancellation ratio kr (`known`: there was one), and its mixed record
+// in units of the cluster's largest star mass M.mmax; returns whether the
+// star is close enough to the BH to be taken out of the FP32 pass (see
+// PN1_FLAG_ETA), in which case its mixed record is neutral; hard: whether
+// its pair terms cancel beyond PN1_HARD_K.
+__device__ __forceinline__ bool prep_star(const double (&xp)[3], const double (&vp)[3],
+                                          const double (&x0)[3], double mp, int p, double m0,
+                                          double eps2, JRec64* __restrict__ j64,
+                                          double (&g)[NGS], const MixPrep& M, bool known,
+                                          const double (&a)[3], float kr, bool& hard)
 {
 #pragma clang fp contract(off)
     hard = false;
-    const double x = st[p], y = st[cap + p], z = st[2 * cap + p];
-    const double vx = st[3 * cap + p], vy = st[4 * cap + p], vz = st[5 * cap + p];
-    const double mp = m[p];
-    const double dx = x - st[b0], dy = y - st[cap + b0], dz = z - st[2 * cap + b0];
+    const double x = xp[0], y = xp[1], z = xp[2], vx = vp[0], vy = vp[1], vz = vp[2];
+    const double dx = x - x0[0], dy = y - x0[1], dz = z - x0[2];
     const double D2 = dx * dx + dy * dy + dz * dz;
-    const double e = 1.0 / sqrt(D2 + eps2);     // as Limit-sticky9.c:106-108
+    const double e = rsq64(D2 + eps2);
     const double E3 = e * e * e;
     const double q = mp * E3;
     const double V2 = vx * vx + vy * vy + vz * vz;
@@ -162,46 +337,50 @@ __device__ __forceinline__ bool prep_star(const double* __restrict__ st,
         h.Qdx = (float)r.Qdx; h.Qdy = (float)r.Qdy; h.Qdz = (float)r.Qdz;
     }
     M.j32[p] = h;
-    M.thr[p] = pair_thresholds(dx, dy, dz, M.aprev, M.kprev, (size_t)cap, p, M.mmax,
-                               M.hard_rows != 0, hard);
+    const double d[3] = {dx, dy, dz};
+    M.thr[p] = pair_thresholds(d, known, a, kr, M.mmax, hard);
     return flagged;
 }
 
-// Mixed form: fl per star, bit 0 whether it is taken out of the FP32 pass
-// (BH-close), bit 1 whether it gets an FP64 row of its own (hard); fblk per
-// block the number of each, [2 b] and [2 b + 1].  The BH mass is m[0].
-inline __global__ __launch_bounds__(WG) void k_prep(const double* __restrict__ st,
-                                            const double* __restrict__ m, Phys P,
-                                            JRec64* __restrict__ j64,
-                                            double* __restrict__ gblk, MixPrep M,
-                                            int* __restrict__ fl, int* __restrict__ fblk)
+// One row of stars' share of the sums over all stars, by its wave (ok: the
+// lane holds a star): the BH shares cb (BH) and the separable sums g (NEXT),
+// and, in the mixed form, the bit masks of its BH-close and its hard stars.
+template <bool BH, bool NEXT>
+__device__ __forceinline__ void put_row(int row, bool ok, const double (&cb)[3],
+                                        const double (&g)[NGS], double* __restrict__ rows,
+                                        bool mixed, bool flagged, bool hard,
+                                        unsigned long long* __restrict__ fmask,
+                                        unsigned long long* __restrict__ hmask)
 {
-    const int p = blockIdx.x * WG + threadIdx.x + 1;
-    double g[NGS];
+    const int lane = threadIdx.x & 63;
+    double v[RV];
 #pragma unroll
-    for (int k = 0; k < NGS; ++k) g[k] = 0.0;
-    bool f = false, hard = false;
-    if (p < P.n) {
-        f = prep_star(st, m, P.cap, p, 0, m[0], P.eps2, j64, g, M, hard);
-        hard = hard && M.hard_rows;
-        if (M.j32) fl[p] = (f ? 1 : 0) | (hard ? 2 : 0);
+    for (int k = 0; k < RV; ++k) v[k] = 0.0;
+    if (ok) {
+        if (BH)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) v[k] = cb[k];
+        if (NEXT)
+#pragma unroll
+            for (int k = 0; k < NGS; ++k) v[RV_G + k] = g[k];
     }
-    block_sum<NGS>(g, gblk + (size_t)blockIdx.x * NGS);
-    if (M.j32) {
-        const int cnt = __syncthreads_count(f);
-        const int hcnt = __syncthreads_count(hard);
-        if (threadIdx.x == 0) {
-            fblk[2 * blockIdx.x] = cnt;
-            fblk[2 * blockIdx.x + 1] = hcnt;
+    const double t = wave_sums16(v);
+    if ((lane & 3) == 0) hand_over(&rows[(size_t)row * RV + (lane >> 2)], t);
+    if (NEXT && mixed) {
+        const unsigned long long f = __builtin_amdgcn_ballot_w64(ok && flagged);
+        const unsigned long long h = __builtin_amdgcn_ballot_w64(ok && hard);
+        if (lane == 0) {
+            hand_over(&fmask[row], f);
+            hmask[row] = h;
         }
     }
 }
 
-// Exclusive prefix sum of one value per thread over the workgroup, in
-// thread order; *total receives the sum.
+// Exclusive prefix sum of one value per thread over the workgroup (FWG
+// threads), in thread order; *total receives the sum.
 __device__ __forceinline__ int block_excl_scan(int v, int* total)
 {
-    __shared__ int wsum[WG / 64];
+    __shared__ int wsum[FG];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     int incl = v;
 #pragma unroll
@@ -211,72 +390,106 @@ __device__ __forceinline__ int block_excl_scan(int v, int* total)
     }
     if (lane == 63) wsum[wid] = incl;
     __syncthreads();
-    int base = 0;
+    int base = 0, all = 0;
 #pragma unroll
-    for (int w = 0; w < WG / 64; ++w) base += w < wid ? wsum[w] : 0;
-    *total = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    for (int w = 0; w < FG; ++w) {
+        base += w < wid ? wsum[w] : 0;
+        all += wsum[w];
+    }
+    *total = all;
     __syncthreads();
     return base + incl - v;
 }
 
-// The stars with bit BIT of fl set in blocks [b0, b1) (block b covers the
-// stars p0 + (b - b0) * WG .. + WG - 1, its count of them at
-// fblk[b * STRIDE + BIT]) listed in increasing order at out[0 ..), their
-// number in *nout and returned to every thread.  One workgroup.
-template <int BIT = 0, int STRIDE = 1>
-__device__ __forceinline__ int list_flagged(const int* __restrict__ fl,
-                                             const int* __restrict__ fblk, int b0, int b1,
-                                             int p0, int pend, int* __restrict__ out,
+// The stars whose bit is set in the masks of rows [b0, b1) (row b0 starts at
+// star p0), in increasing order, at out[0 ..), their number in *nout.  One
+// workgroup of FWG threads.
+__device__ __forceinline__ void list_flagged(const unsigned long long* mask, int b0, int b1,
+                                             int p0, int* __restrict__ out,
                                              int* __restrict__ nout)
 {
     int base = 0;
-    for (int bb = b0; bb < b1; bb += WG) {
+    for (int bb = b0; bb < b1; bb += FWG) {
         const int b = bb + (int)threadIdx.x;
-        const int cnt = b < b1 ? fblk[b * STRIDE + BIT] : 0;
+        unsigned long long f = b < b1 ? take_over(&mask[b]) : 0ull;
+        if (!__syncthreads_or(f != 0ull)) continue;     // hardly ever any
         int total;
-        const int at = base + block_excl_scan(cnt, &total);
-        if (cnt > 0) {
-            // the block's flags 16 at a time: 16 loads in flight, not one
-            int k = at;
-            const int q0 = p0 + (b - b0) * WG, qe = min(q0 + WG, pend);
-            for (int q = q0; q < qe; q += 16) {
-                int f[16];
-#pragma unroll
-                for (int u = 0; u < 16; ++u) f[u] = fl[min(q + u, qe - 1)];
-#pragma unroll
-                for (int u = 0; u < 16; ++u)
-                    if (q + u < qe && ((f[u] >> BIT) & 1)) out[k++] = q + u;
-            }
+        int at = base + block_excl_scan(__popcll(f), &total);
+        while (f) {
+            out[at++] = p0 + (b - b0) * RB + __builtin_ctzll(f);
+            f &= f - 1;
         }
         base += total;
     }
     if (threadIdx.x == 0) *nout = base;
-    return base;
 }
 
-// The BH-close stars (flist, fn[0]) and the hard stars (hlist, fn[1]) of
-// k_prep's flags.
-inline __global__ __launch_bounds__(WG) void k_flist(const int* __restrict__ fl,
-                                             const int* __restrict__ fblk, int nblk, int n,
-                                             int* __restrict__ flist, int* __restrict__ hlist,
-                                             int* __restrict__ fn)
+// The buffers of the O(n) kernels' sums over all stars.
+struct RowBufs {
+    double* rows;                          // per row: its RV values
+    unsigned long long *fmask, *hmask;     // per row: BH-close and hard stars
+    double* gs;                            // separable sums of the evaluation
+    int *flist, *fn;                       // its BH-close stars and their number
+    unsigned int* ticket;                  // last_block's counter (null: the sums are
+                                           // added by k_gsum and k_bh instead)
+};
+
+// After the last row of a prep: the separable sums, and the BH-close list of
+// rows [b0, b1) (p0: row b0's first star).
+__device__ __forceinline__ void close_prep(const RowBufs& R, bool mixed, int b0, int b1, int p0,
+                                           double* __restrict__ gs, int* __restrict__ flist,
+                                           int* __restrict__ fn)
 {
-    list_flagged<0, 2>(fl, fblk, 0, nblk, 1, n, flist, fn);
-    list_flagged<1, 2>(fl, fblk, 0, nblk, 1, n, hlist, fn + 1);
+    __shared__ double tot[RV];
+    rows_total(R.rows, b0, b1, tot);
+    if (threadIdx.x < NGS) gs[threadIdx.x] = tot[RV_G + threadIdx.x];
+    if (mixed) list_flagged(R.fmask, b0, b1, p0, flist, fn);
 }
 
-// Fixed-order sum of nblk rows of N doubles (one workgroup).
-template <int N>
-__global__ __launch_bounds__(WG) void k_rows_sum(const double* __restrict__ rows, int nblk,
-                                                double* __restrict__ out)
+// Records, separable sums and (mixed form) thresholds, BH-close and hard
+// stars of the state st.  aprev, kprev (mixed form): each star's previous
+// acceleration (SoA [3][cap]) and cancellation ratio, null after an upload.
+// The BH mass is m[0].
+inline __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ st,
+                                             const double* __restrict__ m, Phys P, int nrow,
+                                             JRec64* __restrict__ j64, RowBufs R, MixPrep M,
+                                             const double* __restrict__ aprev,
+                                             const float* __restrict__ kprev)
 {
-    double g[N];
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * FG + (int)(threadIdx.x >> 6);
+    const int p = 1 + row * RB + lane;
+    const size_t cap = (size_t)P.cap;
+    if (row < nrow) {
+        double g[NGS];
+        bool f = false, hard = false;
+        const bool ok = p < P.n;
+        if (ok) {
+            const double x[3] = {st[p], st[cap + p], st[2 * cap + p]};
+            const double v[3] = {st[3 * cap + p], st[4 * cap + p], st[5 * cap + p]};
+            const double x0[3] = {st[0], st[cap], st[2 * cap]};
+            double a[3] = {0.0, 0.0, 0.0};
+            float kr = 0.0f;
+            if (aprev) {
 #pragma unroll
-    for (int k = 0; k < N; ++k) g[k] = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += WG)
-#pragma unroll
-        for (int k = 0; k < N; ++k) g[k] += rows[(size_t)b * N + k];
-    block_sum<N>(g, out);
+                for (int k = 0; k < 3; ++k) a[k] = aprev[k * cap + p];
+                kr = kprev[p];
+            }
+            f = prep_star(x, v, x0, m[p], p, m[0], P.eps2, j64, g, M, aprev != nullptr, a, kr,
+                          hard);
+        }
+        const double cb[3] = {0.0, 0.0, 0.0};
+        put_row<false, true>(row, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
+                             R.hmask);
+    }
+    if (R.ticket && last_block(R.ticket, gridDim.x))
+        close_prep(R, M.j32 != nullptr, 0, nrow, 1, R.gs, R.flist, R.fn);
+}
+
+// The separable sums of the rows (one workgroup), where k_prep leaves them.
+inline __global__ __launch_bounds__(FWG) void k_gsum(RowBufs R, int nrow)
+{
+    close_prep(R, false, 0, nrow, 1, R.gs, R.flist, R.fn);
 }
 
 // ---------------------------------------------------------------------
@@ -818,230 +1031,149 @@ void k_pair32q(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
 }
 
 // ---------------------------------------------------------------------
-// k_fin: star accelerations, stage update, BH partials
+// k_fin: star accelerations, stage update, BH, the next evaluation's prep
 // ---------------------------------------------------------------------
-// The pairs of every star i with the stars taken out of the FP32 pass
-// (flist[0 .. nf), see PN1_FLAG_ETA), in FP64 with the FP64 form's body:
-// per star the NACC sums and sum m_j w^2, written to xp [NACC + 1][stride]
-// at idx.  Nothing when nf is 0.
-__device__ __forceinline__ void flagged_pairs(const JRec64* __restrict__ jr,
-                                              const double* __restrict__ st, int cap, int i,
-                                              double eps2, const int* __restrict__ flist,
-                                              int nf, double* __restrict__ xp, size_t stride,
-                                              int idx)
+// The local stars [first, first + 64 nrow) of a cluster (BH at off, nst
+// stars) whose sums need more than the FP32 pass gave, mixed form: x at the
+// star's index gets, [NACC + 1][cap] (the NACC sums and sum m_j w^2, from the
+// FP64 form's body),
+//   a hard star (hmask of the rows, see PN1_HARD_K): its whole row over the
+//     cluster's records (BH-close stars included, with their full records),
+//     reduced over the workgroup's FWG lanes in a fixed order;
+//   any other star: its pairs with the nf BH-close stars (flist, see
+//     PN1_FLAG_ETA), if there are any.
+// Row r's star part runs in wave r (wave 0 if nrow is 1).  Every thread of
+// the workgroup calls it.  A call, not inlined, ahead of k_fin's own work: it
+// is rare, and inlined its registers would halve k_fin's occupancy.
+__attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ jr,
+                                                    const double* __restrict__ st, int cap,
+                                                    double eps2, int off, int nst, int first,
+                                                    int nrow,
+                                                    const unsigned long long* __restrict__ hmask,
+                                                    const int* __restrict__ flist, int nf,
+                                                    double* __restrict__ x)
 {
-    const I64 I = load_i64(jr, st, cap, i, eps2);
-    double a[NACC], ts = 0.0;
-#pragma unroll
-    for (int k = 0; k < NACC; ++k) a[k] = 0.0;
-    for (int f = 0; f < nf; ++f) {
-        const int j = flist[f];
-        body64<true>(jr[j], j, i, I, a, eps2);
-        if (j != i) {
-            const double rx = jr[j].x - I.x, ry = jr[j].y - I.y, rz = jr[j].z - I.z;
-            ts += jr[j].m / (rx * rx + ry * ry + rz * rz + eps2);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < NACC; ++k) xp[(size_t)k * stride + idx] = a[k];
-    xp[(size_t)NACC * stride + idx] = ts;
-}
-
-inline __global__ __launch_bounds__(WG) void k_pair_fl(const JRec64* __restrict__ jr,
-                                               const double* __restrict__ st,
-                                               const int* __restrict__ flist,
-                                               const int* __restrict__ fn,
-                                               double* __restrict__ xp, Phys P)
-{
-    const int nf = *fn;
-    const int i = blockIdx.x * WG + threadIdx.x + 1;
-    if (nf == 0 || i >= P.n) return;
-    flagged_pairs(jr, st, P.cap, i, P.eps2, flist, nf, xp, (size_t)P.cap, i);
-}
-
-// FP64 sums of hard star i (see PN1_HARD_K) over the records [j0, j1)
-// with the FP64 form's body (BH-close stars included, with their full
-// records): the NACC sums and sum m_j w^2, reduced over the workgroup's HWG
-// lanes in a fixed order and written to out[k * stride + idx], k <= NACC.
-// Two records per lane in flight (the loads of a row are not shared by
-// other lanes, so their latency is hidden only by having many in flight).
-constexpr int HWG = 256;
-// A hard star's row is split in HSEG segments of the j range, each a work
-// unit of its own: one workgroup streaming a whole row (16 MB of records
-// at n = 131073) took ~460 us on one CU, on the critical path of every
-// mixed evaluation; 32 units on 32 CUs take ~1/32 of that.  The segments'
-// sums go to a scratch of HCAP stars x HSEG x (NACC + 1) and are added in
-// segment order (k_hard_sum).  An evaluation with more than HCAP hard
-// stars takes every row in one unit: whether a row is split depends only
-// on the count, never on a star's place in the list (which in an ensemble
-// follows the order the clusters' workgroups appended them).
-constexpr int HSEG = 32;
-constexpr int HCAP = 1024;
-
-__device__ __forceinline__ int hard_split(int nh) { return nh <= HCAP ? nh : 0; }
-
-__device__ __forceinline__ void hard_row(const JRec64* __restrict__ jr,
-                                         const double* __restrict__ st, int cap, double eps2,
-                                         int i, int j0, int j1, double* __restrict__ out,
-                                         size_t stride, size_t idx)
-{
-    __shared__ double wsum[NACC + 1][HWG / 64];
-    const I64 I = load_i64(jr, st, cap, i, eps2);
-    double a[NACC], ts = 0.0;
-#pragma unroll
-    for (int k = 0; k < NACC; ++k) a[k] = 0.0;
-    auto pair = [&](const JRec64& J, int j) {
+    __shared__ double wsum[NACC + 1][FG];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double a[NACC], ts;
+    auto pair = [&](int j, int i, const I64& I) {
+        const JRec64& J = jr[j];
         body64<true>(J, j, i, I, a, eps2);
         if (j != i) {
             const double rx = J.x - I.x, ry = J.y - I.y, rz = J.z - I.z;
             ts += J.m / (rx * rx + ry * ry + rz * rz + eps2);
         }
     };
-    for (int j = j0 + (int)threadIdx.x; j < j1; j += 2 * HWG) {
-        const int jb = j + HWG;
-        const JRec64 A = jr[j];
-        const JRec64 B = jr[jb < j1 ? jb : j];
-        pair(A, j);
-        if (jb < j1) pair(B, jb);
+    if (nf > 0 && wid < nrow && first + (int)threadIdx.x < nst) {
+        const int i = off + 1 + first + (int)threadIdx.x;
+        const I64 I = load_i64(jr, st, cap, i, eps2);
+        ts = 0.0;
+#pragma unroll
+        for (int k = 0; k < NACC; ++k) a[k] = 0.0;
+        for (int f = 0; f < nf; ++f) pair(flist[f], i, I);
+#pragma unroll
+        for (int k = 0; k < NACC; ++k) x[(size_t)k * cap + i] = a[k];
+        x[(size_t)NACC * cap + i] = ts;
     }
-    double v[NACC + 1];
+    for (int r = 0; r < nrow && first + r * RB < nst; ++r) {
+        unsigned long long hm = hmask[r];
+        while (hm) {
+            const int h = r * RB + __builtin_ctzll(hm), i = off + 1 + first + h;
+            hm &= hm - 1;
+            const I64 I = load_i64(jr, st, cap, i, eps2);
+            ts = 0.0;
 #pragma unroll
-    for (int k = 0; k < NACC; ++k) v[k] = a[k];
-    v[NACC] = ts;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+            for (int k = 0; k < NACC; ++k) a[k] = 0.0;
+            for (int j = off + 1 + (int)threadIdx.x; j <= off + nst; j += FWG) pair(j, i, I);
 #pragma unroll
-    for (int k = 0; k <= NACC; ++k) {
-        double t = v[k];
+            for (int k = 0; k <= NACC; ++k) {
+                const double t = wave_sum(k < NACC ? a[k] : ts);
+                if (lane == 0) wsum[k][wid] = t;
+            }
+            __syncthreads();
+            if ((int)threadIdx.x == h)
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-        if (lane == 0) wsum[k][wid] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x <= NACC) {
-        double t = 0.0;
-#pragma unroll
-        for (int w = 0; w < HWG / 64; ++w) t += wsum[threadIdx.x][w];
-        out[(size_t)threadIdx.x * stride + idx] = t;
-    }
-    __syncthreads();
-}
-
-// Work unit u of the rows of the hard stars, ns = hard_split(nh) of them
-// split (unit h * HSEG + g: star h, segment g, into hseg), for a star of a
-// cluster whose stars are [p0, pend); the units past ns * HSEG are whole
-// rows (into xh).
-__device__ __forceinline__ void hard_unit(const JRec64* __restrict__ jr,
-                                          const double* __restrict__ st, int cap, double eps2,
-                                          int u, int ns, int star, int p0, int pend,
-                                          double* __restrict__ xh, double* __restrict__ hseg)
-{
-    if (u < ns * HSEG) {
-        const int g = u % HSEG, len = (pend - p0 + HSEG - 1) / HSEG;
-        const int j0 = min(pend, p0 + g * len), j1 = min(pend, j0 + len);
-        hard_row(jr, st, cap, eps2, star, j0, j1, hseg + (size_t)u * (NACC + 1), 1, 0);
-    } else {
-        hard_row(jr, st, cap, eps2, star, p0, pend, xh, (size_t)cap, (size_t)star);
+                for (int k = 0; k <= NACC; ++k) {
+                    double t = 0.0;
+                    for (int w = 0; w < FG; ++w) t += wsum[k][w];
+                    x[(size_t)k * cap + i] = t;
+                }
+            __syncthreads();
+        }
     }
 }
 
-// The hard stars hlist[0 .. fn[1]): all in HSEG units each, or, beyond
-// HCAP of them, all whole; the workgroups take the units in turn.
-inline __global__ __launch_bounds__(HWG) void k_hard_rows(const JRec64* __restrict__ jr,
-                                                  const double* __restrict__ st,
-                                                  const int* __restrict__ hlist,
-                                                  const int* __restrict__ fn,
-                                                  double* __restrict__ xh,
-                                                  double* __restrict__ hseg, Phys P)
+// Sum of the S chunk partials of one row of stars, by G waves (G = 1 or FG):
+// wave g adds chunks g, g + G, ... of the lane's star, and the waves' sums
+// are added pairwise in a fixed order; the result is in wave 0 of the G.
+// `part` points at the cluster's partial area, `stride` is its per-sum
+// stride and `idx` the star's index in it (any valid one for a lane without
+// a star).  FP64: [S][NACC][stride]; mixed: [S][MROWS][stride] floats (the
+// NACC32 sums, then the Newtonian Kahan compensations), whose sums built
+// from the record's mass m_j / mscale are scaled back by mscale; A[NACC] is
+// the mixed form's A_TS sum (TS: the stages whose pair kernels write it).
+template <int MODE, bool TS, int G>
+__device__ __forceinline__ void gather_row(const void* __restrict__ part, int S, size_t stride,
+                                           size_t idx, double mscale, double (&A)[NACC + 1])
 {
-    const int nh = fn[1], ns = hard_split(nh), nu = ns * HSEG + (nh - ns);
-    for (int u = blockIdx.x; u < nu; u += gridDim.x) {
-        const int h = u < ns * HSEG ? u / HSEG : ns + (u - ns * HSEG);
-        hard_unit(jr, st, P.cap, P.eps2, u, ns, hlist[h], 1, P.n, xh, hseg);
-    }
-}
-
-// Row value k of split hard star h (t = h * (NACC + 1) + k, h < ns): its
-// HSEG segment sums added in segment order, into xh at the star.
-__device__ __forceinline__ void hard_sum(const double* __restrict__ hseg, int t, int star,
-                                         int cap, double* __restrict__ xh)
-{
-    const int h = t / (NACC + 1), k = t % (NACC + 1);
-    const double* q = hseg + (size_t)h * HSEG * (NACC + 1) + k;
-    double s = 0.0;
-    for (int g = 0; g < HSEG; ++g) s += q[(size_t)g * (NACC + 1)];
-    xh[(size_t)k * cap + star] = s;
-}
-
-inline __global__ __launch_bounds__(WG) void k_hard_sum(const int* __restrict__ hlist,
-                                                const int* __restrict__ fn,
-                                                const double* __restrict__ hseg,
-                                                double* __restrict__ xh, int cap)
-{
-    const int t = blockIdx.x * WG + threadIdx.x;
-    const int ns = hard_split(fn[1]);
-    if (t < ns * (NACC + 1)) hard_sum(hseg, t, hlist[t / (NACC + 1)], cap, xh);
-}
-
-// Sum of the S chunk partials of one star.  `part` points at the
-// cluster's partial area, `stride` is its per-sum stride and `idx` the
-// star's index in it.  FP64: [S][NACC][stride]; mixed: [S][MROWS][stride]
-// floats (the NACC32 sums, then the Newtonian Kahan compensations), whose
-// sums built from the record's mass m_j / mscale are scaled back by mscale;
-// ts is the mixed form's A_TS sum (0 for FP64, and without TS: the stages
-// whose pair kernels do not write that row).
-template <int MODE, bool TS = true>
-__device__ __forceinline__ void gather_acc(const void* __restrict__ part, int S, size_t stride,
-                                           int idx, double mscale, double (&A)[NACC], double& ts)
-{
+    constexpr int NV = MODE == 1 && TS ? NACC + 1 : NACC;
+    const int lane = threadIdx.x & 63;
+    const int g = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 #pragma unroll
-    for (int k = 0; k < NACC; ++k) A[k] = 0.0;
-    ts = 0.0;
+    for (int k = 0; k <= NACC; ++k) A[k] = 0.0;
     if (MODE == 0) {
         const double* pp = (const double*)part;
-        for (int s = 0; s < S; ++s)
+        for (int s = g; s < S; s += G) {
+            double L[NACC];
 #pragma unroll
-            for (int k = 0; k < NACC; ++k) A[k] += pp[(size_t)(s * NACC + k) * stride + idx];
+            for (int k = 0; k < NACC; ++k)
+                L[k] = __builtin_nontemporal_load(&pp[(size_t)(s * NACC + k) * stride + idx]);
+            __builtin_amdgcn_sched_barrier(0);       // all of a chunk's loads in flight
+#pragma unroll
+            for (int k = 0; k < NACC; ++k) A[k] += L[k];
+        }
     } else {
         const float* pp = (const float*)part;
-        for (int s = 0; s < S; ++s) {
+        for (int s = g; s < S; s += G) {
             const float* ps = pp + (size_t)s * MROWS * stride + idx;
+            float L[NV], C[3];
 #pragma unroll
-            for (int k = 0; k < NACC; ++k) A[k] += (double)ps[(size_t)k * stride];
-            if (TS) ts += (double)ps[(size_t)A_TS * stride];
+            for (int k = 0; k < NV; ++k)
+                L[k] = __builtin_nontemporal_load(&ps[(size_t)k * stride]);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) A[A_NX + k] -= (double)ps[(size_t)(NACC32 + k) * stride];
+            for (int k = 0; k < 3; ++k)
+                C[k] = __builtin_nontemporal_load(&ps[(size_t)(NACC32 + k) * stride]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < NV; ++k) A[k] += (double)L[k];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) A[A_NX + k] -= (double)C[k];
         }
 #pragma unroll
-        for (int k = 0; k < NACC; ++k)
-            if (k <= A_UZ || k == A_KS || k == A_PHI || k == A_W3) A[k] *= mscale;
-        ts *= mscale;
+        for (int k = 0; k < NV; ++k)
+            if (k <= A_UZ || k == A_KS || k == A_PHI || k == A_W3 || k == A_TS) A[k] *= mscale;
     }
-}
-
-// A hard star's FP64 row (k_hard_rows).
-__device__ __forceinline__ void load_row(const double* __restrict__ xh, size_t stride, int idx,
-                                         double (&A)[NACC], double& ts)
-{
+    if (G > 1) {
+        __shared__ double sh[G > 1 ? G / 2 : 1][NV][RB];
 #pragma unroll
-    for (int k = 0; k < NACC; ++k) A[k] = xh[(size_t)k * stride + idx];
-    ts = xh[(size_t)NACC * stride + idx];
-}
-
-// Adds one star's FP64 sums of its pairs with the stars taken out of the
-// FP32 pass (k_pair_fl) to its gathered sums.
-__device__ __forceinline__ void add_flagged(const double* __restrict__ xp, size_t stride, int idx,
-                                            double (&A)[NACC], double& ts)
-{
+        for (int h = G / 2; h >= 1; h >>= 1) {
+            if (g >= h && g < 2 * h)
 #pragma unroll
-    for (int k = 0; k < NACC; ++k) A[k] += xp[(size_t)k * stride + idx];
-    ts += xp[(size_t)NACC * stride + idx];
+                for (int k = 0; k < NV; ++k) sh[g - h][k][lane] = A[k];
+            __syncthreads();
+            if (g < h)
+#pragma unroll
+                for (int k = 0; k < NV; ++k) A[k] += sh[g][k][lane];
+            __syncthreads();
+        }
+    }
 }
 
 // Mixed form: the star's cancellation ratio for the next evaluation's
-// thresholds, sum m_j w^2 / |a| (+inf for a = 0).
+// thresholds, sum m_j w^2 / |a| (NaN for a = 0, which counts as hard).
 __device__ __forceinline__ float cancel_ratio(double ts, const double (&a)[3])
 {
-    return (float)(ts / sqrt(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]));
+    return (float)(ts * rsq64(a[0] * a[0] + a[1] * a[1] + a[2] * a[2]));
 }
 
 // Run constants shared by the O(n) passes of one cluster.
@@ -1049,28 +1181,23 @@ struct FinC {
     double m0, eps, eps2, ws, lam, dt;
 };
 
-// Star p (BH of its cluster at index b0): its acceleration from its pair
-// sums S_ and the cluster's separable sums gs, the stage update, and its
-// share cb of the BH's 1PN acceleration (a1 + a1c).
+// Star p (BH of its cluster at x0) of mass mp in state st, with |d|^2 = D2 and
+// e from its record: its acceleration
+// from its pair sums S_ and the cluster's separable sums gs, the stage update
+// (nx, nv: the state of the driver's next force call), and its share cb of
+// the BH's 1PN acceleration (a1 + a1c).
 template <int STAGE>
-__device__ __forceinline__ void fin_star(const double* in, double* X, double* Y, double* H1,
-                                         double* H2, const double* __restrict__ m, int cap,
-                                         int p, int b0, const double (&S_)[NACC],
-                                         const double* __restrict__ gs, const FinC& C,
+__device__ __forceinline__ void fin_star(const StageIn& st, const double (&x0)[3], double mp,
+                                         double D2, double e,
+                                         double* X, double* Y, double* H1, double* H2, int cap,
+                                         int p, const double (&S_)[NACC + 1],
+                                         const double (&gs)[NGS], const FinC& C,
                                          double* __restrict__ acc, double (&cb)[3],
-                                         double (&a)[3])
+                                         double (&a)[3], double (&nx)[3], double (&nv)[3])
 {
-    const double m0 = C.m0, mp = m[p], eps2 = C.eps2;
-    const double x[3] = {in[p], in[cap + p], in[2 * cap + p]};
-    const double v[3] = {in[3 * cap + p], in[4 * cap + p], in[5 * cap + p]};
-    const double x0[3] = {in[b0], in[cap + b0], in[2 * cap + b0]};
-    double d[3], D2, e;
-    {
-#pragma clang fp contract(off)
-        for (int k = 0; k < 3; ++k) d[k] = x[k] - x0[k];
-        D2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-        e = 1.0 / sqrt(D2 + eps2);
-    }
+    const double m0 = C.m0, eps2 = C.eps2;
+    const double (&x)[3] = st.x, (&v)[3] = st.v;
+    const double d[3] = {x[0] - x0[0], x[1] - x0[1], x[2] - x0[2]};
     const double E3 = e * e * e, q = mp * E3;
     const double G1 = gs[G_G1];
     const double M1[3] = {gs[G_M1X], gs[G_M1Y], gs[G_M1Z]};
@@ -1091,7 +1218,7 @@ __device__ __forceinline__ void fin_star(const double* in, double* X, double* Y,
         const double B = -m0 * E3 * (d[k] * cB + 4.0 * vd * v[k]);
         const double Sg = cS * d[k] + 7.0 * mp * E3 * vd * v[k];
         const double t4 = E3 * (4.0 * vP * d[k] - 3.0 * Pd * v[k] - 4.0 * vd * Pp[k]);
-        const double ru = S_[A_UX + k] / PN1_SQ15 - v[k] * S_[A_KS];
+        const double ru = S_[A_UX + k] * PN1_ISQ15 - v[k] * S_[A_KS];
         const double t3 = S_[A_TX + k] - 3.5 * m0 * e * (M1[k] - q * d[k]);
         const double rr = S_[A_RX + k] + cB * S_[A_NX + k];
         const double pn = B + Sg + rr + ru + c1 * d[k] + t3 + t4;
@@ -1119,7 +1246,7 @@ __device__ __forceinline__ void fin_star(const double* in, double* X, double* Y,
     const double cC2 = mE3 * (4.0 * (G1 - mp * e) + 1.25 * S_[A_PHI] + 0.25 * xi
                               + mp * self_br);
     const double cQ2 = mp * mp * E3 * (4.0 * e + 1.25 * C.eps);
-    const double vm = mE3 / m0, vm2 = mp * mp * E3 / m0;
+    const double vm = mE3 / m0, vm2 = mp * vm;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const double A1 = cA1 * d[k] + 3.0 * mE3 * vd * v[k];
@@ -1128,7 +1255,9 @@ __device__ __forceinline__ void fin_star(const double* in, double* X, double* Y,
         const double Q2 = cQ2 * d[k] - vm2 * (4.0 * V2 * d[k] - 7.0 * vd * v[k]);
         cb[k] = A1 + cC0 * d[k] + C2 + Q2;
     }
-    stage_update<STAGE>(p, cap, a, X, Y, H1, H2, C.dt);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        stage_update<STAGE>(p, cap, st, k, k, a[k], X, Y, H1, H2, C.dt, nx[k], nv[k]);
 }
 
 __device__ __forceinline__ FinC fin_consts(const Phys& P, double m0)
@@ -1143,75 +1272,178 @@ __device__ __forceinline__ FinC fin_consts(const Phys& P, double m0)
     return C;
 }
 
-// Stars p0 .. p1 - 1 (p0 = 1, p1 = n: every star; a sub-range is one i shard
-// of a plain evaluation, STAGE 0); the BH mass is m[0].
-// kout (mixed form, evaluations that accumulated A_TS; else null): each
-// star's cancellation ratio, for the next evaluations' pair thresholds.
-// Mixed form: plus the FP64 sums xp of the pairs with the stars taken out of
-// the FP32 pass (when fn[0] > 0); a hard star (fl bit 1) takes its FP64 row
-// xh instead of both.
-template <int MODE, int STAGE>
-__global__ __launch_bounds__(WG) void k_fin(const double* in, double* X, double* Y, double* H1,
-                                           double* H2, const double* __restrict__ m,
-                                           const void* __restrict__ part, int S,
-                                           const double* __restrict__ gs,
-                                           double* __restrict__ acc,
-                                           double* __restrict__ bhblk, float* __restrict__ kout,
-                                           const int* __restrict__ fn,
-                                           const double* __restrict__ xp,
-                                           const int* __restrict__ fl,
-                                           const double* __restrict__ xh, Phys P, int p0,
-                                           int p1)
+// What k_fin works on besides the partial sums.  kr (mixed form): each
+// star's cancellation ratio, written by the evaluations that accumulated
+// A_TS (plain ones and the first stage of a step) and read by the others.
+struct FinBufs {
+    const double* in;
+    double *X, *Y, *H1, *H2;
+    const double* m;
+    double* acc;
+    float* kr;
+    double* xr;          // rare_rows' sums (mixed form)
+    const JRec64* j64;   // this evaluation's records
+    JRec64* jnext;       // the next one's (another buffer: other rows may
+                         // still read this evaluation's)
+};
+
+// One row of a cluster's stars: local stars first .. first + 63 of nst, BH
+// at index off, its rows from row0 on; row: this one's index among all rows.
+struct Row {
+    int off, nst, first, row;
+};
+
+// The workgroup's rows of a cluster: row q.row by all FG waves (G = FG), or
+// rows q.row .. q.row + FG - 1 by one wave each (G = 1; q.first: the first
+// star of the workgroup's).  Accelerations, stage update and BH shares, and,
+// inside a step (STAGE 1..3), the records and row sums of the driver's next
+// evaluation on the state the stage update gives.  Every thread calls this.
+//
+// G = FG is for few rows: one wave adding all S chunks of its stars leaves
+// most of the chip idle (at n = 10241, S = 128 that took as long as the pair
+// kernel).  With many rows the chip is full either way, and the star part
+// behind the gather, which one wave runs, counts: G = 1 keeps all FG busy.
+template <int MODE, int STAGE, int G>
+__device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, const Row& q,
+                                         const void* __restrict__ part, int S, size_t stride,
+                                         size_t idx0, const double* __restrict__ gsp,
+                                         const int* __restrict__ flist,
+                                         const int* __restrict__ fn, double m0, const MixPrep& M,
+                                         const Phys& P)
 {
-    const int p = p0 + blockIdx.x * WG + threadIdx.x;
-    double cb[3] = {0.0, 0.0, 0.0};
-    if (p < p1) {
-        double S_[NACC], ts, a[3];
-        if (MODE == 1 && (fl[p] & 2)) {
-            load_row(xh, (size_t)P.cap, p, S_, ts);
-        } else {
-            gather_acc<MODE, (STAGE <= 1)>(part, S, (size_t)P.cap, p, P.mmax, S_, ts);
-            if (MODE == 1 && fn[0] > 0) add_flagged(xp, (size_t)P.cap, p, S_, ts);
+    constexpr bool TS = STAGE <= 1;
+    const int lane = threadIdx.x & 63, cap = P.cap;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int mine = G == 1 ? wid : 0;              // this wave's row of the workgroup's
+    const int lf = q.first + mine * RB;             // its first star
+    const int li = lf + lane;
+    const bool ok = li < q.nst;
+    const int lc = ok ? li : min(q.first, q.nst - 1);
+    const int p = q.off + 1 + lc;
+    const bool star = G == 1 ? lf < q.nst : wid == 0;   // this wave runs the star part
+    int nf = 0;
+    bool is_hard = false;
+    if (MODE == 1) {
+        nf = *fn;
+        unsigned long long any = 0ull;
+#pragma unroll
+        for (int r = 0; r < (G == 1 ? FG : 1); ++r)
+            if (q.first + r * RB < q.nst) {
+                const unsigned long long hm = R.hmask[q.row + r];
+                any |= hm;
+                if (r == mine) is_hard = (hm >> lane) & 1;
+            }
+        if (nf > 0 || any)
+            rare_rows(F.j64, F.in, cap, P.eps2, q.off, q.nst, q.first, G == 1 ? FG : 1,
+                      R.hmask + q.row, flist, nf, F.xr);
+    }
+    // everything the star part reads, requested ahead of the partial sums
+    StageIn st, b0;
+    double gs[NGS], mp = 0.0, D2 = 0.0, e = 0.0;
+    float kr = 0.0f;
+    if (star) {
+        D2 = F.j64[p].D2;
+        e = F.j64[p].e;
+        st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, p);
+        b0 = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, q.off);
+        mp = F.m[p];
+#pragma unroll
+        for (int k = 0; k < NGS; ++k) gs[k] = gsp[k];
+        if (MODE == 1 && !TS) kr = F.kr[p];
+    }
+    double A[NACC + 1];
+    if (G > 1 || star) gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+    if (MODE == 1 && star && ok && (is_hard || nf > 0)) {
+        // a hard star: its FP64 row instead of the gathered sums; another
+        // one: plus its pairs with the BH-close stars
+#pragma unroll
+        for (int k = 0; k <= NACC; ++k)
+            A[k] = (is_hard ? 0.0 : A[k]) + F.xr[(size_t)k * cap + p];
+    }
+    if (!star) return;
+    double cb[3] = {0.0, 0.0, 0.0}, a[3], nx[3], nv[3], g[NGS];
+    bool f = false, hard = false;
+    if (ok) {
+        fin_star<STAGE>(st, b0.x, mp, D2, e, F.X, F.Y, F.H1, F.H2, cap, p, A, gs,
+                        fin_consts(P, m0), F.acc, cb, a, nx, nv);
+        if (MODE == 1 && TS) {
+            kr = cancel_ratio(A[NACC], a);
+            F.kr[p] = kr;
         }
-        fin_star<STAGE>(in, X, Y, H1, H2, m, P.cap, p, 0, S_, gs, fin_consts(P, m[0]), acc, cb, a);
-        if (MODE == 1 && kout) kout[p] = cancel_ratio(ts, a);
+        if (STAGE > 0) {
+            const double x0[3] = {stage_pos<STAGE>(b0, P.dt, 0), stage_pos<STAGE>(b0, P.dt, 1),
+                                  stage_pos<STAGE>(b0, P.dt, 2)};
+            f = prep_star(nx, nv, x0, mp, p, m0, P.eps2, F.jnext, g, M, true, a, kr, hard);
+        }
     }
-    block_sum<3>(cb, bhblk + (size_t)blockIdx.x * 3);
+    put_row<true, (STAGE > 0)>(q.row + mine, ok, cb, g, R.rows, MODE == 1, f, hard, R.fmask,
+                               R.hmask);
 }
 
-// BH at index b0: Newton sum_j m_j e_j^3 d_j plus lam times the star shares
-// tot; stage update.  Thread 0 only.
-template <int STAGE>
-__device__ __forceinline__ void bh_finish(const double (&tot)[3], const double* __restrict__ gs,
-                                          int b0, int cap, double lam, double dt, double* X,
-                                          double* Y, double* H1, double* H2,
-                                          double* __restrict__ acc)
+// A cluster without stars: its one row of zeros.
+__device__ __forceinline__ void empty_row(const RowBufs& R, int row, bool mixed)
 {
-    double a0[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        a0[k] = gs[G_M1X + k] + lam * tot[k];
-        acc[(size_t)k * cap + b0] = a0[k];
+    if (threadIdx.x < RV) hand_over(&R.rows[(size_t)row * RV + threadIdx.x], 0.0);
+    if (mixed && threadIdx.x == 0) {
+        hand_over(&R.fmask[row], 0ull);
+        R.hmask[row] = 0ull;
     }
-    stage_update<STAGE>(b0, cap, a0, X, Y, H1, H2, dt);
 }
 
-template <int STAGE>
-__global__ __launch_bounds__(WG) void k_bh(const double* __restrict__ bhblk, int nblk,
-                                          const double* __restrict__ gs, double* X, double* Y,
-                                          double* H1, double* H2, double* __restrict__ acc,
-                                          Phys P)
+// After the last row of an evaluation: the BH at b0, its acceleration Newton
+// sum_j m_j e_j^3 d_j plus lam times the rows' shares and its stage update
+// (thread k: component k), and the next evaluation's separable sums and
+// BH-close list.
+template <int MODE, int STAGE>
+__device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, int b0row,
+                                          int b1row, int b0, double* __restrict__ gs,
+                                          int* __restrict__ flist, int* __restrict__ fn,
+                                          const Phys& P)
 {
-    double s[3] = {0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblk; b += WG)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s[k] += bhblk[(size_t)b * 3 + k];
-    __shared__ double tot[3];
-    block_sum<3>(s, tot);
-    if (threadIdx.x == 0) {
-        const double t[3] = {tot[0], tot[1], tot[2]};
-        bh_finish<STAGE>(t, gs, 0, P.cap, P.lam, P.dt, X, Y, H1, H2, acc);
+    __shared__ double tot[RV];
+    const int t = threadIdx.x;
+    StageIn st;
+    double nwt = 0.0;
+    if (t < 3) {
+        st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, P.cap, b0, t, 1);
+        nwt = gs[G_M1X + t];
     }
+    rows_total(R.rows, b0row, b1row, tot);
+    if (t < 3) {
+        double nx, nv;
+        const double a = nwt + P.lam * tot[t];
+        F.acc[(size_t)t * P.cap + b0] = a;
+        stage_update<STAGE>(b0, P.cap, st, 0, t, a, F.X, F.Y, F.H1, F.H2, P.dt, nx, nv);
+    }
+    if (STAGE > 0) {
+        __syncthreads();                       // gs has been read
+        if (t < NGS) gs[t] = tot[RV_G + t];
+        if (MODE == 1) list_flagged(R.fmask, b0row, b1row, b0 + 1, flist, fn);
+    }
+}
+
+// Rows from row0 on, up to star p1 (all: the BH too, by the last workgroup;
+// a sub-range is one i shard of a plain evaluation); the BH mass is m[0].
+template <int MODE, int STAGE, int G>
+__global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M, Phys P,
+           int row0, int p1, int nrow)
+{
+    const int row = row0 + (int)blockIdx.x * (G == 1 ? FG : 1);
+    const Row q = {0, p1 - 1, row * RB, row};
+    if (P.n > 1)
+        fin_rows<MODE, STAGE, G>(F, R, q, part, S, (size_t)P.cap, 1, R.gs, R.flist, R.fn, F.m[0],
+                                 M, P);
+    else
+        empty_row(R, 0, MODE == 1);
+    if (R.ticket && last_block(R.ticket, gridDim.x))
+        fin_close<MODE, STAGE>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P);
+}
+
+// The BH from the rows' shares (one workgroup), where k_fin leaves it.
+inline __global__ __launch_bounds__(FWG) void k_bh(FinBufs F, RowBufs R, int nrow, Phys P)
+{
+    fin_close<0, 0>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P);
 }
 
 // ---------------------------------------------------------------------

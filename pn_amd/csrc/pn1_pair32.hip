@@ -18,18 +18,19 @@ namespace pn1host {
 namespace {
 
 template <int PP, bool TS, bool EQ>
-void launch32(pn1_ctx* c, const double* in, const Phys& P, int ib0, int nib, int S)
+void launch32(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int ib0, int nib,
+              int S)
 {
     if (quad_pairs(c, S))
         hipLaunchKernelGGL((k_pair32q<PP, TS, EQ>), dim3(pair_grid(S / QSUB, nib)), dim3(WGQ), 0,
-                           c->st, c->j32, c->j64, c->thr, in, (float*)c->part, P, S, nib, ib0,
+                           c->st, c->j32, j64, c->thr, in, (float*)c->part, P, S, nib, ib0,
                            c->tile);
     else
         hipLaunchKernelGGL((k_pair32<PP, TS, EQ>), dim3(pair_grid(S, nib)), dim3(WG), 0, c->st,
-                           c->j32, c->j64, c->thr, in, (float*)c->part, P, S, nib, ib0, c->tile);
+                           c->j32, j64, c->thr, in, (float*)c->part, P, S, nib, ib0, c->tile);
 }
 
-using Launch32 = void (*)(pn1_ctx*, const double*, const Phys&, int, int, int);
+using Launch32 = void (*)(pn1_ctx*, const JRec64*, const double*, const Phys&, int, int, int);
 const Launch32 k_launch32[16] = {
     launch32<0, false, false>, launch32<0, false, true>, launch32<0, true, false>,
     launch32<0, true, true>,   launch32<1, false, false>, launch32<1, false, true>,
@@ -39,19 +40,19 @@ const Launch32 k_launch32[16] = {
     launch32<3, true, true>};
 
 template <int PP, bool TS, bool EQ>
-void ens_launch32(pn1_ens* e, const double* in, const Phys& P, dim3 g)
+void ens_launch32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g)
 {
     if constexpr ((PP & 1) != 0)
-        hipLaunchKernelGGL((k_ens_pair32x<PP, TS, EQ>), g, dim3(WG), 0, e->st, e->j32, e->j64,
+        hipLaunchKernelGGL((k_ens_pair32x<PP, TS, EQ>), g, dim3(WG), 0, e->st, e->j32, j64,
                            e->thr, in, (float*)e->part, e->items, e->counter, e->qoff, e->cmmax,
                            P, e->tile);
     else
-        hipLaunchKernelGGL((k_ens_pair32<PP, TS, EQ>), g, dim3(WG), 0, e->st, e->j32, e->j64,
+        hipLaunchKernelGGL((k_ens_pair32<PP, TS, EQ>), g, dim3(WG), 0, e->st, e->j32, j64,
                            e->thr, in, (float*)e->part, e->items, e->counter, e->qoff, e->cmmax,
                            P, e->tile);
 }
 
-using EnsLaunch32 = void (*)(pn1_ens*, const double*, const Phys&, dim3);
+using EnsLaunch32 = void (*)(pn1_ens*, const JRec64*, const double*, const Phys&, dim3);
 const EnsLaunch32 k_ens_launch32[16] = {
     ens_launch32<0, false, false>, ens_launch32<0, false, true>, ens_launch32<0, true, false>,
     ens_launch32<0, true, true>,   ens_launch32<1, false, false>, ens_launch32<1, false, true>,
@@ -62,14 +63,16 @@ const EnsLaunch32 k_ens_launch32[16] = {
 
 }  // namespace
 
-void launch_pair32(pn1_ctx* c, const double* in, const Phys& P, int ib0, int nib, int S, int form)
+void launch_pair32(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int ib0,
+                   int nib, int S, int form)
 {
-    k_launch32[form & 15](c, in, P, ib0, nib, S);
+    k_launch32[form & 15](c, j64, in, P, ib0, nib, S);
 }
 
-void launch_ens_pair32(pn1_ens* e, const double* in, const Phys& P, dim3 g, int form)
+void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g,
+                       int form)
 {
-    k_ens_launch32[form & 15](e, in, P, g);
+    k_ens_launch32[form & 15](e, j64, in, P, g);
 }
 
 hipError_t ens_pair32_occupancy(int var, int* per_cu)

@@ -20,10 +20,11 @@ inline int pair32_form(int variant, bool ts, bool eqm)
 
 // Single cluster: i blocks ib0 .. ib0 + nib - 1 against every star, the j
 // range split in S chunks (pn1_pair32.hip).
-void launch_pair32(pn1_ctx* c, const double* in, const pn1dev::Phys& P, int ib0, int nib, int S,
-                   int form);
+void launch_pair32(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
+                   const pn1dev::Phys& P, int ib0, int nib, int S, int form);
 // Ensemble: one persistent launch of grid g over the work queues.
-void launch_ens_pair32(pn1_ens* e, const double* in, const pn1dev::Phys& P, dim3 g, int form);
+void launch_ens_pair32(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
+                       const pn1dev::Phys& P, dim3 g, int form);
 // Resident workgroups per CU of the ensemble kernel of loop variant var
 // (0..3), in its form with the cancellation sums (the one with the most
 // registers).
