@@ -146,10 +146,12 @@ int  pn1_sync(pn1_ctx *ctx);
 const char *pn1_last_error(const pn1_ctx *ctx);
 
 /* Launch shape of the pair kernels: the j range is split into `jsplit`
- * chunks (0 = automatic; a split of 32 or more, a multiple of 8, ends in 16
- * chunks an eighth as long as the others, which the launch runs last, so
- * that it does not wait long on its last workgroups), the mixed kernel
- * compensates its FP32 sums every
+ * chunks, one per 256-star workgroup (0 = automatic: up to 192 parts, eight
+ * of them to a workgroup of 64 stars, which adds their sums; `variant` then
+ * stays -1, else the split is an automatic one of the 256-star kernels).  A
+ * split of 32 or more, a multiple of 8, ends in 16 chunks an eighth as long
+ * as the others, which the launch runs last, so that it does not wait long
+ * on its last workgroups.  The mixed kernel compensates its FP32 sums every
  * `tile` pairs (0 = default), and `variant` picks the kernel form (-1 =
  * automatic per mode): bit 0 the j loop (clear: one j-record at a time,
  * set: two in flight), bit 1 (mixed form) one Newton step on the FP32

@@ -87,54 +87,74 @@ double flag_threshold(double dmax)
     return PN1_FLAG_ETA / (6.0 * 0x1p-24 * 2.0 * dmax);
 }
 
-// j split S and grid of the pair kernels for the current n.
+// j split of the 256-star kernels where none is set explicitly (i shards,
+// energy): many short rounds of workgroups, chunks of at least 64 records.
+int auto_split(int nst)
+{
+    const int nib = nst > 0 ? (nst + WG - 1) / WG : 0;
+    int S = 1;
+    while (S < 128 && (long)S * nib < 32768 && (nst + 2 * S - 1) / (2 * S) >= 64) S *= 2;
+    return nst > 0 && S > nst ? nst : S;
+}
+
+// Partials per star of the automatic plan: from 8192 stars on the tapered
+// split's 24 (16 long chunks and 8 short ones), below 16, fewer while a
+// wave's part would hold fewer than 4 records.  Short parts balance the launch
+// and fill the chip, partials cost k_fin.  Measured on MI355X (one evaluation,
+// FP64 / mixed, us; 24 is the tapered one):
+//   slots       4     8          16           24           32         64
+//   n = 1025    25/28 18.6/22.7  18.0/19.7                 21.5/22.4  30/28
+//   n = 2049    35/41 23.3/28.7  23.5/23.7                 27/26      37/34
+//   n = 10241         178/128    177/111      178/108      182/113    201/130
+//   n = 131073                   24850/12860  24808/12715
+int auto_slots(int nst)
+{
+    if (nst >= 8192) return TLONG + TSHORT;
+    int s = TLONG;
+    while (s > 1 && nst < 4 * s * PW) s >>= 1;
+    return s;
+}
+
+// Launch plan of the pair kernels for the current n.
 void plan(pn1_ctx* c)
 {
     const int nst = c->n - 1;
     c->nblk = nblocks(nst);
     c->nrow = nst > 0 ? (nst + RB - 1) / RB : 1;
     c->nIblk = nst > 0 ? (nst + WG - 1) / WG : 0;
-    int S = c->jsplit_req;
-    if (S <= 0) {
-        // Many short rounds of workgroups: the last, partly filled round of
-        // a grid costs little when there are tens of rounds (measured on
-        // MI355X at n = 131073: the mixed pair kernel takes 13.3 ms at split
-        // 64, 14.4 ms at 16 and 22.9 ms at 4; at n = 10241 split 128 is 1.2x
-        // faster than 32).  Chunks stay >= 64 records.
-        S = 1;
-        while (S < 128 && (long)S * c->nIblk < 32768 && (nst + 2 * S - 1) / (2 * S) >= 64) S *= 2;
-    }
-    if (nst > 0 && S > nst) S = nst;
-    if (S < 1) S = 1;
-    c->S = S;
-    if (S <= 8 && 8 % S == 0) {
-        const int per = 8 / S;
-        c->pair_grid = 8 * ((c->nIblk + per - 1) / per);
+    c->slots = 0;
+    if (c->jsplit_req > 0) {
+        c->S = std::max(1, std::min(c->jsplit_req, std::max(nst, 1)));
+    } else if (c->variant_req >= 0 || nst < 1) {
+        c->S = auto_split(nst);
     } else {
-        c->pair_grid = S * c->nIblk;
+        c->slots = auto_slots(nst);
+        c->S = c->slots * PW;
     }
     c->tile = c->tile_req > 0 ? (c->tile_req < 2 ? 2 : c->tile_req) : 64;
 }
 
-// Bytes of pair partials a j split of S chunks needs (0: the plan's).
-size_t part_need(const pn1_ctx* c, int split = 0)
+// Bytes of pair partials of `slots` chunks per star (0: the plan's).
+size_t part_need(const pn1_ctx* c, int slots = 0)
 {
-    const size_t cap = (size_t)c->cap, S = (size_t)(split > 0 ? split : c->S);
+    const size_t cap = (size_t)c->cap;
+    const size_t S = (size_t)(slots > 0 ? slots : c->slots ? c->slots : c->S);
+    const size_t SE = (size_t)std::max(c->slots ? auto_split(c->n - 1) : c->S, 1);
     size_t need = S * NACC * cap * sizeof(double);
-    const size_t needE = S * NACCE * cap * sizeof(double);
+    const size_t needE = SE * NACCE * cap * sizeof(double);
     const size_t need32 = S * MROWS * cap * sizeof(float);
     if (needE > need) need = needE;
     if (need32 > need) need = need32;
     return need;
 }
 
-// Partial-sum buffer for a j split of S chunks (default: the plan's).  The
+// Partial-sum buffer for `slots` chunks per star (default: the plan's).  The
 // new buffer is allocated before the old one is freed: if the allocation
 // is refused, the old buffer stays (ready() then refuses launches of a
 // plan it does not cover).
-int ensure_part(pn1_ctx* c, int split = 0)
+int ensure_part(pn1_ctx* c, int slots = 0)
 {
-    const size_t need = part_need(c, split);
+    const size_t need = part_need(c, slots);
     if (need <= c->part_bytes) return PN1_OK;
     void* p = nullptr;
     if (dev_malloc(&p, need) != hipSuccess)
@@ -164,7 +184,7 @@ bool quad_pairs(const pn1_ctx* c, int S)
     return c->mode == PN1_MIXED && S >= QSUB && S % QSUB == 0 && (kernel_variant(c) & 4);
 }
 
-// Partial-sum slots per star of a launch split in S chunks.
+// Partials per star of a launch of the 256-star kernels split in S chunks.
 int part_slots(const pn1_ctx* c, int S) { return quad_pairs(c, S) ? S / QSUB : S; }
 
 // Workgroups of a pair launch over nib i blocks with `slots` chunks each
@@ -240,9 +260,9 @@ MixPrep mix_prep(const pn1_ctx* c, const Phys& P)
 // would leave most of the chip idle on; 1 above.
 constexpr int FIN_ROWS = 1024;
 
-// Stars i0 .. i1 - 1 (all: every star and the BH).
+// Stars i0 .. i1 - 1 (all: every star and the BH), `slots` partials each.
 template <int MODE, int STAGE>
-void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int S, int i0, int i1, bool all)
+void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, int i1, bool all)
 {
     FinBufs F;
     F.in = in;
@@ -258,7 +278,6 @@ void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int S, int i0, int 
     F.jnext = rec_buf(c, STAGE % 3);
     const int row0 = (i0 - 1) / RB, rows = std::max(1, (i1 - i0 + RB - 1) / RB);
     const RowBufs R = row_bufs(c, all);
-    const int slots = part_slots(c, S);
     if (c->nrow <= FIN_ROWS)
         hipLaunchKernelGGL((k_fin<MODE, STAGE, FG>), dim3(rows), dim3(FWG), 0, c->st, F, R,
                            (const void*)c->part, slots, mix_prep(c, P), P, row0, i1, c->nrow);
@@ -309,22 +328,29 @@ int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
 {
     const double* in = stage <= 1 ? c->X : c->Y;
     const bool mixed = c->mode == PN1_MIXED;
+    const int slots = c->slots ? c->slots : part_slots(c, c->S);
     if (c->n > 1) {
         hipEvent_t e1 = nullptr;
         if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
-        launch_pair(c, rec_buf(c, stage <= 1 ? 0 : stage - 1), in, P, 0, c->nIblk, c->S,
-                    stage <= 1);
+        const JRec64* j64 = rec_buf(c, stage <= 1 ? 0 : stage - 1);
+        if (!c->slots)
+            launch_pair(c, j64, in, P, 0, c->nIblk, c->S, stage <= 1);
+        else if (mixed)
+            launch_pair32w(c, j64, in, P, c->slots, stage <= 1);
+        else
+            hipLaunchKernelGGL(k_pair64w, dim3(c->slots * c->nrow), dim3(PW * RB), 0, c->st, j64,
+                               in, (double*)c->part, P, c->slots, c->nrow);
         if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     }
     switch (stage * 2 + (mixed ? 1 : 0)) {
-    case 0: launch_fin<0, 0>(c, in, P, c->S, 1, c->n, true); break;
-    case 1: launch_fin<1, 0>(c, in, P, c->S, 1, c->n, true); break;
-    case 2: launch_fin<0, 1>(c, in, P, c->S, 1, c->n, true); break;
-    case 3: launch_fin<1, 1>(c, in, P, c->S, 1, c->n, true); break;
-    case 4: launch_fin<0, 2>(c, in, P, c->S, 1, c->n, true); break;
-    case 5: launch_fin<1, 2>(c, in, P, c->S, 1, c->n, true); break;
-    case 6: launch_fin<0, 3>(c, in, P, c->S, 1, c->n, true); break;
-    default: launch_fin<1, 3>(c, in, P, c->S, 1, c->n, true); break;
+    case 0: launch_fin<0, 0>(c, in, P, slots, 1, c->n, true); break;
+    case 1: launch_fin<1, 0>(c, in, P, slots, 1, c->n, true); break;
+    case 2: launch_fin<0, 1>(c, in, P, slots, 1, c->n, true); break;
+    case 3: launch_fin<1, 1>(c, in, P, slots, 1, c->n, true); break;
+    case 4: launch_fin<0, 2>(c, in, P, slots, 1, c->n, true); break;
+    case 5: launch_fin<1, 2>(c, in, P, slots, 1, c->n, true); break;
+    case 6: launch_fin<0, 3>(c, in, P, slots, 1, c->n, true); break;
+    default: launch_fin<1, 3>(c, in, P, slots, 1, c->n, true); break;
     }
     HIPCHK(c, hipGetLastError());
     c->acc_ok = mixed;
@@ -665,10 +691,9 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
     const int nib = (i1 - i0 + WG - 1) / WG;
     // The j split: an explicit one (pn1_set_tuning, pn1_autotune) as set,
     // which keeps the rows bitwise equal to pn1_force's; otherwise the
-    // shard's own plan, the full launch's split doubled while the shard's
-    // grid has fewer than 16384 workgroups (chunks of >= 64 records, at most
-    // 512 chunks).
-    int S = c->S;
+    // shard's own plan, auto_split doubled while the shard's grid has fewer
+    // than 16384 workgroups (chunks of >= 64 records, at most 512 chunks).
+    int S = c->jsplit_req > 0 ? c->S : auto_split(n - 1);
     if (c->jsplit_req <= 0) {
         const int nst = n - 1;
         while (S < 512 && (long)S * nib < 16384 && (nst + 2 * S - 1) / (2 * S) >= 64) S *= 2;
@@ -683,9 +708,9 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
     launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     if (mixed)
-        launch_fin<1, 0>(c, in, P, S, i0, i1, false);
+        launch_fin<1, 0>(c, in, P, part_slots(c, S), i0, i1, false);
     else
-        launch_fin<0, 0>(c, in, P, S, i0, i1, false);
+        launch_fin<0, 0>(c, in, P, part_slots(c, S), i0, i1, false);
     if (!mixed) c->acc_ok = false;
     HIPCHK(c, hipGetLastError());
     const size_t cap = (size_t)c->cap, cnt = (size_t)(i1 - i0);
@@ -705,11 +730,12 @@ int pn1_energy(pn1_ctx* c, pn1_energy_t* out)
     if (!out) return seterr(c, PN1_EINVAL, "null output");
     const Phys P = make_phys(c);
     if ((rc = prep_x(c, P, true))) return rc;
+    const int S = c->slots ? auto_split(c->n - 1) : c->S;
     if (c->n > 1)
-        hipLaunchKernelGGL(k_epair64, dim3(c->pair_grid), dim3(WG), 0, c->st, c->j64, c->X,
-                           (double*)c->part, P, c->S, c->nIblk);
+        hipLaunchKernelGGL(k_epair64, dim3(pair_grid(S, c->nIblk)), dim3(WG), 0, c->st, c->j64,
+                           c->X, (double*)c->part, P, S, c->nIblk);
     hipLaunchKernelGGL(k_efin, dim3(c->nblk), dim3(WG), 0, c->st, c->X, c->m,
-                       (const double*)c->part, c->n > 1 ? c->S : 0, c->gs, c->eblk, P);
+                       (const double*)c->part, c->n > 1 ? S : 0, c->gs, c->eblk, P);
     hipLaunchKernelGGL(k_ered, dim3(1), dim3(WG), 0, c->st, c->eblk, c->nblk, c->X, c->m, c->gs,
                        c->eout, P);
     HIPCHK(c, hipGetLastError());
@@ -815,7 +841,7 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
     const int nst = c->n - 1;
     const bool was_prof = c->prof;
     const int keep_tile = c->tile_req, keep_S = c->jsplit_req, keep_var = c->variant_req;
-    std::vector<int> splits = {0};                  // 0 = the automatic plan
+    std::vector<int> splits = {0};    // 0 = the automatic plan, which has one form
     for (int S = 8; S <= 256; S *= 2)
         if (S <= std::max(1, nst / 64)) splits.push_back(S);
     const Phys P = make_phys(c);
@@ -835,7 +861,7 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
     }
     auto time_shape = [&](int S, int var, double* avg) {
         c->jsplit_req = S;
-        c->variant_req = var;
+        c->variant_req = S ? var : -1;
         c->tile_req = keep_tile;
         plan(c);
         int r = ensure_part(c);
@@ -850,13 +876,13 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
         return r;
     };
     for (int S : splits) {
-        for (int var = 0; var < 2 && !rc; ++var) {
+        for (int var = 0; var < (S ? 2 : 1) && !rc; ++var) {
             double avg = 0.0;
             rc = time_shape(S, var, &avg);
             if (!rc && avg < best) {
                 best = avg;
-                bS = c->S;
-                bV = var;
+                bS = S;
+                bV = c->variant_req;
             }
         }
         if (rc) break;
@@ -933,7 +959,15 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
     hipLaunchKernelGGL(k_prep, dim3((nrow + FG - 1) / FG), dim3(FWG), 0, s, st, m, P, nrow, j64, R,
                        M, (const double*)nullptr, (const float*)nullptr);
     hipLaunchKernelGGL(k_gsum, dim3(1), dim3(FWG), 0, s, R, nrow);
-    if (nst > 0)
+    // The two-in-flight form gives the same sums; with few waves per SIMD it
+    // hides more of its loads' latency, and above 8192 stars the one-record
+    // form's 7 waves make two rounds of the grid (measured on MI355X, pair
+    // launch, one record / two: n = 4097 58/60 us, 12000 287/268, 16384
+    // 482/438).
+    if (nst > 8192)
+        hipLaunchKernelGGL(k_pair64<1>, dim3(pair_grid(S, nib)), dim3(WG), 0, s,
+                           (const JRec64*)j64, st, part, P, S, nib, 0);
+    else if (nst > 0)
         hipLaunchKernelGGL(k_pair64<0>, dim3(pair_grid(S, nib)), dim3(WG), 0, s,
                            (const JRec64*)j64, st, part, P, S, nib, 0);
     hipLaunchKernelGGL((k_fin<0, 0, FG>), dim3(nrow), dim3(FWG), 0, s, F, R, (const void*)part, S,

@@ -25,7 +25,9 @@ struct pn1_ctx {
     double tauf = 0.0;          // BH-close threshold of the mixed form (PN1_FLAG_ETA)
     int jsplit_req = 0, tile_req = 0, variant_req = -1;
     // launch plan for the current n
-    int S = 1, nIblk = 0, pair_grid = 0, nblk = 1, tile = 64;
+    // j split (S parts); slots: partials per star of the automatic plan's pair
+    // kernels, which give each PW parts (0: the explicit split's kernels)
+    int S = 1, slots = 0, nIblk = 0, nblk = 1, tile = 64;
     // device buffers
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr;
     double *m = nullptr, *acc = nullptr, *rows = nullptr, *gs = nullptr;

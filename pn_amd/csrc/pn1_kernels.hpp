@@ -620,6 +620,109 @@ __global__ __launch_bounds__(WG) void k_pair64(const JRec64* __restrict__ jr,
     }
 }
 
+// The automatic plan's form: a workgroup takes 64 stars, one per lane in each
+// of its PW waves, and chunk s of S; wave w takes part w of the chunk (part
+// s PW + w of the j range split in S PW), and the waves' sums are added
+// pairwise in LDS and written as one partial.  Against one part per 256-star
+// workgroup (k_pair64 / k_pair32, explicit splits) it gives short parts
+// without as many partials: 16 or 24 per star instead of 64 to 128, which
+// k_fin then reads in a fraction of the time, and enough waves at small n.
+// Measured on MI355X, FP64 / mixed evaluation (pair and k_fin), us:
+//   n         65    257   1025  2049  4097  8193     10241    32769
+//   256 stars 23/31 25/29 28/31 43/60 55/56 147/98   209/130  1683/903
+//   this form 13/15 15/18 18/20 24/24 44/35 121/81   176/111  1578/841
+// PW = 4 and 16 were within 3% up to n = 2049; above, 16 waves leave a
+// compute unit idle between workgroups (up to +30%).
+constexpr int PW = 8;
+
+// Workgroup -> chunk s of S and row ig of 64 stars, and the bounds of wave
+// w's part of the chunk with the window that can contain j == i.  A split of
+// TLONG + TSHORT chunks is tapered: the last TSHORT are an eighth as long
+// and run after all others, so that the launch does not wait long on its last
+// workgroups.
+constexpr int TLONG = 16, TSHORT = 8;
+__device__ __forceinline__ JRange j_part(int bid, int S, int nrow, int wave, int n, int& s,
+                                         int& ig)
+{
+    const int nst = n - 1;
+    int len;
+    JRange R;
+    if (S <= TLONG) {
+        s = bid % S;
+        ig = bid / S;
+        len = (nst + S * PW - 1) / (S * PW);
+        R.j0 = 1 + (s * PW + wave) * len;
+    } else {
+        const int lp = (nst + (TLONG + 1) * PW - 1) / ((TLONG + 1) * PW);
+        const int t = bid - TLONG * nrow;
+        if (t < 0) {
+            s = bid % TLONG;
+            ig = bid / TLONG;
+            len = lp;
+            R.j0 = 1 + (s * PW + wave) * len;
+        } else {
+            const int q = t % TSHORT;
+            s = TLONG + q;
+            ig = t / TSHORT;
+            len = (lp + 7) / 8;
+            R.j0 = 1 + TLONG * PW * lp + (q * PW + wave) * len;
+        }
+    }
+    R.j0 = min(n, R.j0);
+    R.j1 = min(n, R.j0 + len);
+    R.w0 = max(R.j0, ig * RB + 1);
+    R.w1 = min(R.j1, ig * RB + 1 + RB);
+    return R;
+}
+
+// Adds the PW waves' v pairwise in a fixed order; the sums are in wave 0.
+// Every thread of the workgroup calls it.
+template <int N>
+__device__ __forceinline__ void waves_total(double (&v)[N], int wave, int lane)
+{
+    __shared__ double sh[PW / 2][N][RB];
+#pragma unroll
+    for (int h = PW / 2; h >= 1; h >>= 1) {
+        if (wave >= h && wave < 2 * h)
+#pragma unroll
+            for (int k = 0; k < N; ++k) sh[wave - h][k][lane] = v[k];
+        __syncthreads();
+        if (wave < h)
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k] += sh[wave][k][lane];
+        if (h > 1) __syncthreads();
+    }
+}
+
+// Held to k_pair64's 7 waves per SIMD (72 VGPRs; 80 otherwise).
+inline __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(7, 8)))
+void k_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
+               double* __restrict__ part, Phys P, int S, int nrow)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    int s, ig;
+    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
+    const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
+    const I64 I = load_i64(jr, st, P.cap, i, P.eps2);
+    const double eps2 = P.eps2;
+    double a[NACC];
+#pragma unroll
+    for (int k = 0; k < NACC; ++k) a[k] = 0.0;
+    if (R.w0 < R.w1) {
+        run64<false, 0>(jr, R.j0, R.w0, i, I, a, eps2);
+        run64<true, 0>(jr, R.w0, R.w1, i, I, a, eps2);
+        run64<false, 0>(jr, R.w1, R.j1, i, I, a, eps2);
+    } else {
+        run64<false, 0>(jr, R.j0, R.j1, i, I, a, eps2);
+    }
+    waves_total(a, wave, lane);
+    if (wave == 0 && li < n) {
+#pragma unroll
+        for (int k = 0; k < NACC; ++k) stream_out(a[k], &part[(size_t)(s * NACC + k) * P.cap + li]);
+    }
+}
+
 // ---------------------------------------------------------------------
 // force pair kernel, mixed: FP32 pair arithmetic on double-single
 // positions, FP32 tile sums folded into Kahan-compensated FP32 totals, and
@@ -1026,6 +1129,56 @@ void k_pair32q(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
 #pragma unroll
             for (int q = 0; q < QSUB - 1; ++q) t += (double)red[q][k][col];
             stream_out((float)t, &ps[k * cap]);
+        }
+    }
+}
+
+// k_pair64w's form of the mixed kernel.  The waves' sums are added in FP64:
+// the Newtonian totals s - c are written as a hi/lo float pair (s = hi,
+// c = -lo, so that k_fin's s - c is the FP64 total to ~2^-48), the other sums
+// rounded once to FP32.
+template <bool TS, bool EQ>
+__global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
+               const Thr* __restrict__ thr, const double* __restrict__ st,
+               float* __restrict__ part, Phys P, int S, int nrow, int tile)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    int s, ig;
+    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
+    const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
+    const I32 I = load_i32(j64, thr, st, P.cap, i, 0, P.eps2);
+    const float eps2 = P.eps2f;
+    const double eps2d = P.eps2, rscale = 1.0 / P.mmax;
+    float a[NACC32], sumN[3], cmpN[3];
+#pragma unroll
+    for (int k = 0; k < NACC32; ++k) a[k] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) sumN[k] = cmpN[k] = 0.0f;
+    int cnt = 0;
+    if (R.w0 < R.w1) {
+        run32<false, 0, TS, EQ>(jr, j64, R.j0, R.w0, i, I, a, eps2, eps2d, rscale, sumN, cmpN, tile, cnt);
+        run32<true, 0, TS, EQ>(jr, j64, R.w0, R.w1, i, I, a, eps2, eps2d, rscale, sumN, cmpN, tile, cnt);
+        run32<false, 0, TS, EQ>(jr, j64, R.w1, R.j1, i, I, a, eps2, eps2d, rscale, sumN, cmpN, tile, cnt);
+    } else {
+        run32<false, 0, TS, EQ>(jr, j64, R.j0, R.j1, i, I, a, eps2, eps2d, rscale, sumN, cmpN, tile, cnt);
+    }
+    fold_newton(a, sumN, cmpN);
+    constexpr int NV = TS ? NACC32 : NACC;
+    double v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+        v[k] = k <= A_NZ ? (double)sumN[k] - (double)cmpN[k] : (double)a[k];
+    waves_total(v, wave, lane);
+    if (wave == 0 && li < n) {
+        const size_t cap = (size_t)P.cap;
+        float* ps = part + (size_t)s * MROWS * cap + li;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            const float hi = (float)v[k];
+            stream_out(hi, &ps[k * cap]);
+            if (k <= A_NZ) stream_out(-(float)(v[k] - (double)hi), &ps[(NACC32 + k) * cap]);
         }
     }
 }

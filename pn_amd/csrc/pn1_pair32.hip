@@ -39,6 +39,13 @@ const Launch32 k_launch32[16] = {
     launch32<3, false, false>, launch32<3, false, true>,  launch32<3, true, false>,
     launch32<3, true, true>};
 
+template <bool TS, bool EQ>
+void launch32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots)
+{
+    hipLaunchKernelGGL((k_pair32w<TS, EQ>), dim3(slots * c->nrow), dim3(PW * RB), 0, c->st, c->j32,
+                       j64, c->thr, in, (float*)c->part, P, slots, c->nrow, c->tile);
+}
+
 template <int PP, bool TS, bool EQ>
 void ens_launch32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g)
 {
@@ -67,6 +74,15 @@ void launch_pair32(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& 
                    int nib, int S, int form)
 {
     k_launch32[form & 15](c, j64, in, P, ib0, nib, S);
+}
+
+void launch_pair32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots,
+                    bool ts)
+{
+    if (ts)
+        (c->eqm ? launch32w<true, true> : launch32w<true, false>)(c, j64, in, P, slots);
+    else
+        (c->eqm ? launch32w<false, true> : launch32w<false, false>)(c, j64, in, P, slots);
 }
 
 void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g,
