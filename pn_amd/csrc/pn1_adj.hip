@@ -39,8 +39,9 @@ using namespace pn1host;
 struct pn1_adj {
     int cap = 0;
     double *mu = nullptr, *out = nullptr, *L = nullptr, *LY1 = nullptr, *LY2 = nullptr;
-    double *T = nullptr, *blk = nullptr, *gm0 = nullptr;
+    double *gm0 = nullptr, *sums = nullptr;
     ARec* rec = nullptr;
+    double* jd = nullptr;       // the pair kernel's records (RevD), [REVD_F][cap]
     double* rpart = nullptr;    // pair kernel partials, rpart_n doubles
     size_t rpart_n = 0;
     double* ckpt = nullptr;     // nck states of 6 x cap
@@ -58,7 +59,7 @@ void adj_free(pn1_ctx* c)
 {
     pn1_adj* a = c ? c->adj : nullptr;
     if (!a) return;
-    void* bufs[] = {a->mu, a->out, a->L, a->LY1, a->LY2, a->T, a->blk, a->gm0, a->rec, a->rpart,
+    void* bufs[] = {a->mu, a->out, a->L, a->LY1, a->LY2, a->gm0, a->sums, a->rec, a->jd, a->rpart,
                     a->ckpt, a->seg};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -88,16 +89,15 @@ int adj_get(pn1_ctx* c, pn1_adj** out)
         c->adj = a;
         a->cap = c->cap;
         const size_t s6 = 6 * (size_t)c->cap;
-        const size_t nb = (size_t)((c->cap + WG - 1) / WG + 1);
         int rc = PN1_OK;
         if (!rc) rc = aalloc(c, &a->mu, s6);
         if (!rc) rc = aalloc(c, &a->out, s6);
         if (!rc) rc = aalloc(c, &a->L, s6);
         if (!rc) rc = aalloc(c, &a->LY1, s6);
         if (!rc) rc = aalloc(c, &a->LY2, s6);
-        if (!rc) rc = aalloc(c, &a->T, s6);
-        if (!rc) rc = aalloc(c, &a->blk, nb * 4);
         if (!rc) rc = aalloc(c, &a->gm0, 2);
+        if (!rc) rc = aalloc(c, &a->sums, RV);
+        if (!rc) rc = aalloc(c, &a->jd, (size_t)REVD_F * c->cap);
         if (!rc) rc = aalloc(c, &a->rec, (size_t)c->cap + 2);
         if (rc) {
             adj_free(c);
@@ -108,13 +108,12 @@ int adj_get(pn1_ctx* c, pn1_adj** out)
     return PN1_OK;
 }
 
-int nblk_of(const pn1_ctx* c) { return c->n > 1 ? (c->n - 1 + WG - 1) / WG : 1; }
-
 // j chunk L of the single-pass pair kernel for nst stars in nIb blocks of
 // 256: whole 64-record tiles, the longest that still gives about
 // PN1_ADJ_BLOCKS workgroups (several rounds of the whole device), within
-// [128, 2048].  At n = 16385, L = 128 ... 1024 time within 2% of each
-// other.  The partials take ceil(nst / L) * 7 + nIb * 6 rows of cap doubles:
+// [64, 2048].  At n = 16385, L = 128 ... 1024 time within 2% of each
+// other; at n = 2049, 64-record chunks (a tile per wave, the least there is)
+// put twice the workgroups of 128-record ones on the chip (52 -> 32 us).  The partials take ceil(nst / L) * 7 + nIb * 6 rows of cap doubles:
 // the j-side rows (one per 256-star block) dominate, ~n^2 / 5.3 bytes.
 #ifndef PN1_ADJ_BLOCKS
 #define PN1_ADJ_BLOCKS 2048
@@ -124,16 +123,21 @@ int adj_chunk(int nst, int nIb)
     const int s0 = std::max(1, (PN1_ADJ_BLOCKS + nIb - 1) / std::max(nIb, 1));
     int L = (nst + s0 - 1) / s0;
     L = (L + 63) / 64 * 64;
-    return std::min(std::max(L, 128), 2048);
+    return std::min(std::max(L, 64), 2048);
 }
 
-// out = J_F(y)^T mu for the state y (SoA 6 x cap); d/dm0 to gm0[1], added
-// to gm0[0].  FP64.
-int enqueue_vjp(pn1_ctx* c, pn1_adj* a, const double* y, const double* mu, double* out,
-                const Phys& P)
+// Rows up to which k_adj_fin's workgroups share a row among their waves (as
+// k_fin's).
+constexpr int ADJ_FIN_ROWS = 1024;
+
+// out = z + J_F(y)^T mu for the state y (SoA 6 x cap) and the cotangent mu = l
+// (z: nothing if null); d/dm0 to gm0[1], added to gm0[0].  FP64.
+int enqueue_vjp(pn1_ctx* c, pn1_adj* a, const double* y, const AdjLin& l, const AdjAdd& z,
+                double* out, const Phys& P)
 {
-    const int nblk = nblk_of(c);
     int S = 0, nIb = 0;
+    hipLaunchKernelGGL(k_adj_prep, dim3((c->nrow + FG - 1) / FG), dim3(FWG), 0, c->st, y, l, a->mu,
+                       c->m, P, c->nrow, a->rec, a->jd, c->rows, a->sums, c->ticket);
     if (c->n > 1) {
         // an explicit j split (pn1_set_tuning, pn1_autotune) sets the chunk
         // count, rounded to whole tiles; otherwise the VJP picks its own
@@ -151,23 +155,19 @@ int enqueue_vjp(pn1_ctx* c, pn1_adj* a, const double* y, const double* mu, doubl
             if (rc) return rc;
             a->rpart_n = need;
         }
-        hipLaunchKernelGGL(k_adj_prep, dim3(nblk), dim3(WG), 0, c->st, y, mu, c->m, P, a->rec);
-        hipLaunchKernelGGL(k_adj_rev, dim3(S * nIb), dim3(WG), 0, c->st, a->rec, y, mu, c->m,
-                           a->rpart, P, L, S);
+        hipLaunchKernelGGL(k_adj_rev, dim3(S * nIb), dim3(WG), 0, c->st, a->rec, a->jd, y, a->mu,
+                           c->m, a->rpart, P, L, S);
     }
-    hipLaunchKernelGGL(k_adj_fin, dim3(nblk), dim3(WG), 0, c->st, a->rec, y, mu, c->m,
-                       (const double*)a->rpart, S, nIb, out, a->blk, P);
-    hipLaunchKernelGGL(k_adj_bh, dim3(1), dim3(WG), 0, c->st, a->blk, nblk, mu, out, a->gm0, P);
+    if (c->nrow <= ADJ_FIN_ROWS)
+        hipLaunchKernelGGL(k_adj_fin<FG>, dim3(c->nrow), dim3(FWG), 0, c->st, a->rec, y, a->mu,
+                           c->m, (const double*)a->rpart, S, nIb, a->sums, z, out, a->gm0,
+                           c->nrow, c->rows, c->ticket, P);
+    else
+        hipLaunchKernelGGL(k_adj_fin<1>, dim3((c->nrow + FG - 1) / FG), dim3(FWG), 0, c->st,
+                           a->rec, y, a->mu, c->m, (const double*)a->rpart, S, nIb, a->sums, z,
+                           out, a->gm0, c->nrow, c->rows, c->ticket, P);
     HIPCHK(c, hipGetLastError());
     return PN1_OK;
-}
-
-void lin(pn1_ctx* c, double* out, double ca, const double* A, double cb = 0.0,
-         const double* B = nullptr, double cc = 0.0, const double* C = nullptr, double cd = 0.0,
-         const double* D = nullptr)
-{
-    hipLaunchKernelGGL(k_adj_lin, dim3((c->n + WG - 1) / WG), dim3(WG), 0, c->st, out, c->n,
-                       c->cap, ca, A, cb, B, cc, C, cd, D);
 }
 
 // AoS host [n][3] pair (x part, v part) -> SoA device 6 x cap.
@@ -226,9 +226,10 @@ int pn1_force_vjp(pn1_ctx* c, const double* u, double* gx, double* gv, double* g
     pn1_adj* a;
     if ((rc = adj_get(c, &a))) return rc;
     const Phys P = make_phys(c);
-    if ((rc = put6(c, nullptr, u, a->mu))) return rc;
+    if ((rc = put6(c, nullptr, u, a->L))) return rc;
     HIPCHK(c, hipMemsetAsync(a->gm0, 0, 2 * sizeof(double), c->st));
-    if ((rc = enqueue_vjp(c, a, c->X, a->mu, a->out, P))) return rc;
+    const AdjLin mu = {a->L, nullptr, 1.0, 0.0};
+    if ((rc = enqueue_vjp(c, a, c->X, mu, AdjAdd{}, a->out, P))) return rc;
     const size_t cap = (size_t)c->cap;
     if ((rc = fetch3(c, a->out, gx))) return rc;
     if ((rc = fetch3(c, a->out + 3 * cap, gv))) return rc;
@@ -318,13 +319,13 @@ int pn1_adjoint_backward(pn1_ctx* c, const double* gx, const double* gv, double*
         }
         for (int t = t1 - 1; t >= t0; --t) {
             const double* st = a->seg + 3 * (size_t)(t - t0) * s6;
-            lin(c, a->mu, dt / 6.0, a->L);
-            if ((rc = enqueue_vjp(c, a, st + 2 * s6, a->mu, a->LY2, P))) return rc;
-            lin(c, a->mu, dt / 6.0, a->L, dt / 2.0, a->LY2);
-            if ((rc = enqueue_vjp(c, a, st + s6, a->mu, a->LY1, P))) return rc;
-            lin(c, a->mu, dt / 6.0, a->L, dt / 2.0, a->LY1);
-            if ((rc = enqueue_vjp(c, a, st, a->mu, a->T, P))) return rc;
-            lin(c, a->L, 1.0, a->L, 1.0, a->LY2, 1.0, a->LY1, 1.0, a->T);
+            const AdjLin m2 = {a->L, nullptr, dt / 6.0, 0.0};
+            const AdjLin m1 = {a->L, a->LY2, dt / 6.0, dt / 2.0};
+            const AdjLin m0 = {a->L, a->LY1, dt / 6.0, dt / 2.0};
+            const AdjAdd sum = {a->L, a->LY2, a->LY1};
+            if ((rc = enqueue_vjp(c, a, st + 2 * s6, m2, AdjAdd{}, a->LY2, P))) return rc;
+            if ((rc = enqueue_vjp(c, a, st + s6, m1, AdjAdd{}, a->LY1, P))) return rc;
+            if ((rc = enqueue_vjp(c, a, st, m0, sum, a->L, P))) return rc;
         }
     }
     if ((rc = copy6(c, c->X, a->ckpt))) return rc;          // leave the initial state
@@ -350,22 +351,36 @@ int pn1_adjoint_backward(pn1_ctx* c, const double* gx, const double* gv, double*
 // =========================================================================
 namespace pn1dev {
 
-__global__ __launch_bounds__(WG) void k_ens_adj_prep(const double* __restrict__ y,
-                                                    const double* __restrict__ mu,
-                                                    const double* __restrict__ m,
-                                                    const int* __restrict__ coff,
-                                                    const EBlk* __restrict__ blk, Phys P,
-                                                    ARec* __restrict__ rec)
+// As k_adj_prep, one workgroup per FG rows of a cluster (pblk; crow: its
+// rows); it also resets the pair kernel's queues.
+__global__ __launch_bounds__(FWG) void k_ens_adj_prep(const double* __restrict__ y, AdjLin l,
+                                                     double* __restrict__ mu,
+                                                     const double* __restrict__ m,
+                                                     const int* __restrict__ coff,
+                                                     const int* __restrict__ crow,
+                                                     const EBlk* __restrict__ pblk, Phys P,
+                                                     ARec* __restrict__ rec,
+                                                     double* __restrict__ jd,
+                                                     double* __restrict__ rows,
+                                                     double* __restrict__ sums,
+                                                     unsigned int* __restrict__ ticket,
+                                                     unsigned int* __restrict__ counter)
 {
-    const EBlk b = blk[blockIdx.x];
+    __shared__ double tot[RV];
+    if (blockIdx.x == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
+    const EBlk b = pblk[blockIdx.x];
     const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
+    const int r0 = crow[b.c], r1 = crow[b.c + 1];
+    const int row = r0 + b.first / RB + (int)(threadIdx.x >> 6);
     const int li = b.first + (int)threadIdx.x;
-    if (li < nst) adj_prep_star(y, mu, m, (size_t)P.cap, P.eps2, off + 1 + li, off, rec);
-}
-
-__global__ void k_ens_adj_reset(unsigned int* __restrict__ counter)
-{
-    if (threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
+    if (row < r1)
+        adj_prep_row(y, l, mu, m, (size_t)P.cap, P.eps2, P.lam, off + 1 + li, li < nst, off, rec,
+                     jd, rows, row);
+    if (b.first == 0) adj_prep_bh(l, mu, (size_t)P.cap, off);
+    if (last_block(ticket + b.c, (unsigned)((r1 - r0 + FG - 1) / FG))) {
+        rows_total(rows, r0, r1, tot);
+        if (threadIdx.x < RV) sums[(size_t)b.c * RV + threadIdx.x] = tot[threadIdx.x];
+    }
 }
 
 // Persistent single-pass pair kernel over the ensemble's work items.  Item
@@ -374,6 +389,7 @@ __global__ void k_ens_adj_reset(unsigned int* __restrict__ counter)
 // stride nst: i side (s*NADJ1 + k), s < S_c; then j side
 // (S_c*NADJ1 + ib*NADJ2 + k).  Every item writes its own rows.
 __global__ __launch_bounds__(WG) void k_ens_adj_rev(const ARec* __restrict__ rec,
+                                                   const double* __restrict__ jd,
                                                    const double* __restrict__ y,
                                                    const double* __restrict__ mu,
                                                    const double* __restrict__ m,
@@ -383,9 +399,6 @@ __global__ __launch_bounds__(WG) void k_ens_adj_rev(const ARec* __restrict__ rec
                                                    unsigned int* __restrict__ counter,
                                                    const int* __restrict__ qoff, Phys P, int L)
 {
-    __shared__ double sh[NADJ2][4][64];
-    __shared__ double tls[4][REVJ_F][64];
-    const int wv = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     int q = 0;
     for (;;) {
         const int it = ens_take(counter, qoff, q);
@@ -395,33 +408,17 @@ __global__ __launch_bounds__(WG) void k_ens_adj_rev(const ARec* __restrict__ rec
         const int li = w.ib * WG + (int)threadIdx.x;
         const bool iok = li < nst;
         const bool live = w.ib * WG + (__builtin_amdgcn_readfirstlane((int)threadIdx.x) & ~63) < nst;
-        const int i = w.off + 1 + (iok ? li : nst - 1);
-        const ABH B = load_abh(y, mu, m, P.cap, w.off);
-        const RevU U = rev_uniform(B, P.eps2, P.lam);
-        const ARec me = rec[i];
-        const RevI I = rev_setup(me, U);
-        RevIAcc ai;
-        rev_zero(ai);
+        const RevU U = rev_uniform(load_abh(y, mu, m, P.cap, w.off), P.eps2, P.lam);
         const int S = ens_nchunks(nst, L), s = (w.j0 - w.off - 1) / L;
         double* base = apart + aoff[w.c];
-        double* pj = base + (size_t)S * NADJ1 * nst;
-        for (int jt = w.j0; jt < w.j1; jt += 64) {
-            double g[NADJ2];
-            rev_tile(rec, I, U, i, iok, live, jt, w.j1, ai, g, tls[wv]);
-#pragma unroll
-            for (int k = 0; k < NADJ2; ++k) sh[k][wv][lane] = g[k];
-            __syncthreads();
-            const int jl = jt + lane;
-            if (wv == 0 && jl < w.j1) {
-#pragma unroll
-                for (int k = 0; k < NADJ2; ++k)
-                    pj[((size_t)w.ib * NADJ2 + k) * nst + (jl - w.off - 1)] =
-                        ((sh[k][0][lane] + sh[k][1][lane]) + sh[k][2][lane]) + sh[k][3][lane];
-            }
-            __syncthreads();
-        }
+        double* pj = base + ((size_t)S * NADJ1 + (size_t)w.ib * NADJ2) * nst;
         double g[NADJ1];
-        rev_ifin(me, U, ai, g);
+        rev_chunk(rec, jd, (size_t)P.cap, U, w.off + 1 + (iok ? li : nst - 1), iok, live, w.j0,
+                  w.j1, g, [&](int j, const double (&gj)[NADJ2]) {
+#pragma unroll
+                      for (int k = 0; k < NADJ2; ++k)
+                          pj[(size_t)k * nst + (j - w.off - 1)] = gj[k];
+                  });
         if (iok) {
 #pragma unroll
             for (int k = 0; k < NADJ1; ++k) base[((size_t)s * NADJ1 + k) * nst + li] = g[k];
@@ -429,80 +426,48 @@ __global__ __launch_bounds__(WG) void k_ens_adj_rev(const ARec* __restrict__ rec
     }
 }
 
-__global__ __launch_bounds__(WG) void k_ens_adj_fin(const ARec* __restrict__ rec,
-                                                   const double* __restrict__ y,
-                                                   const double* __restrict__ mu,
-                                                   const double* __restrict__ m,
-                                                   const int* __restrict__ coff,
-                                                   const EBlk* __restrict__ blk,
-                                                   const double* __restrict__ apart,
-                                                   const long long* __restrict__ aoff,
-                                                   double* __restrict__ out,
-                                                   double* __restrict__ ablk, Phys P, int L)
+// As k_adj_fin, one workgroup per row (G = FG, blk the row table) or per FG
+// rows of a cluster (G = 1, blk = pblk); gm0[2c], gm0[2c + 1] of cluster c.
+template <int G>
+__global__ __launch_bounds__(FWG) void k_ens_adj_fin(const ARec* __restrict__ rec,
+                                                    const double* __restrict__ y,
+                                                    const double* __restrict__ mu,
+                                                    const double* __restrict__ m,
+                                                    const int* __restrict__ coff,
+                                                    const int* __restrict__ crow,
+                                                    const EBlk* __restrict__ blk,
+                                                    const double* __restrict__ apart,
+                                                    const long long* __restrict__ aoff,
+                                                    const double* __restrict__ sums, AdjAdd z,
+                                                    double* out, double* __restrict__ gm0,
+                                                    double* __restrict__ rows,
+                                                    unsigned int* __restrict__ ticket, Phys P,
+                                                    int L)
 {
     const EBlk b = blk[blockIdx.x];
     const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
-    const int li = b.first + (int)threadIdx.x;
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    if (li < nst) {
-        const int p = off + 1 + li;
-        const ABH B = load_abh(y, mu, m, P.cap, off);
-        double g[NADJ1];
-        adj_star_grad(rec[p], B, P.eps, P.eps2, P.lam, g);
-        const double* base = apart + aoff[b.c] + li;
-        const int S = ens_nchunks(nst, L), nIb = (nst + WG - 1) / WG;
-        for (int s = 0; s < S; ++s) {
-#pragma unroll
-            for (int k = 0; k < NADJ1; ++k) g[k] += base[(size_t)(s * NADJ1 + k) * nst];
-        }
-        const double* pj = base + (size_t)S * NADJ1 * nst;
-        for (int ib = 0; ib < nIb; ++ib) {
-#pragma unroll
-            for (int k = 0; k < NADJ2; ++k) g[k] += pj[(size_t)(ib * NADJ2 + k) * nst];
-        }
-        adj_store(g, mu, out, (size_t)P.cap, p, t);
-    }
-    block_sum<4>(t, ablk + (size_t)blockIdx.x * 4);
-}
-
-// One workgroup per cluster: its BH's rows and its m0 derivative
-// (gm0[2c + 1] this evaluation, added to gm0[2c]).
-__global__ __launch_bounds__(WG) void k_ens_adj_bh(const double* __restrict__ ablk,
-                                                  const int* __restrict__ cblk,
-                                                  const int* __restrict__ coff,
-                                                  const double* __restrict__ mu,
-                                                  double* __restrict__ out,
-                                                  double* __restrict__ gm0, Phys P)
-{
-    const int c = blockIdx.x;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = cblk[c] + (int)threadIdx.x; b < cblk[c + 1]; b += WG)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[k] += ablk[(size_t)b * 4 + k];
-    __shared__ double tot[4];
-    block_sum<4>(s, tot);
-    if (threadIdx.x == 0) {
-        const size_t cap = (size_t)P.cap;
-        const int b0 = coff[c];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            out[(size_t)k * cap + b0] = -tot[k];
-            out[(size_t)(3 + k) * cap + b0] = mu[(size_t)k * cap + b0];
-        }
-        gm0[2 * c + 1] = tot[3];
-        gm0[2 * c] += tot[3];
-    }
+    const int r0 = crow[b.c], r1 = crow[b.c + 1];
+    const int li = b.first + (int)(G == 1 ? threadIdx.x : threadIdx.x & 63);
+    const int row = r0 + li / RB;
+    if (G > 1 || row < r1)
+        adj_fin_row<G>(rec, y, mu, m, apart + aoff[b.c], nst > 0 ? ens_nchunks(nst, L) : 0,
+                       (nst + WG - 1) / WG, (size_t)nst, (size_t)max(min(li, nst - 1), 0),
+                       off + 1 + li, li < nst, off, sums + (size_t)b.c * RV, z, out, rows, row,
+                       P);
+    if (last_block(ticket + b.c, (unsigned)(G == 1 ? (r1 - r0 + FG - 1) / FG : r1 - r0)))
+        adj_close(rows, r0, r1, off, mu, z, out, gm0 + 2 * (size_t)b.c, (size_t)P.cap);
 }
 
 }  // namespace pn1dev
 
 struct pn1_ens_adj {
     double *mu = nullptr, *out = nullptr, *L = nullptr, *LY1 = nullptr, *LY2 = nullptr;
-    double *T = nullptr, *ablk = nullptr, *gm0 = nullptr;
+    double *gm0 = nullptr, *sums = nullptr;
     ARec* rec = nullptr;
+    double* jd = nullptr;         // the pair kernel's records (RevD), [REVD_F][cap]
     double* ckpt = nullptr;
     double* seg = nullptr;        // per step of a segment: s, Y1, Y2 (6 x cap each)
-    int nck_cap = 0, seg_cap = 0, ablk_cap = 0;
+    int nck_cap = 0, seg_cap = 0;
     int grid = 0;                 // resident workgroups of k_ens_adj_rev
     double* apart = nullptr;      // pair kernel partials, apart_n doubles
     size_t apart_n = 0;
@@ -520,7 +485,7 @@ void ens_adj_free(pn1_ens* e)
 {
     pn1_ens_adj* a = e ? e->adj : nullptr;
     if (!a) return;
-    void* bufs[] = {a->mu, a->out, a->L, a->LY1, a->LY2, a->T, a->ablk, a->gm0, a->rec,
+    void* bufs[] = {a->mu, a->out, a->L, a->LY1, a->LY2, a->gm0, a->sums, a->rec, a->jd,
                     a->ckpt, a->seg, a->apart, a->aoff};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -566,8 +531,9 @@ int ens_adj_get(pn1_ens* e, pn1_ens_adj** out)
         if (!rc) rc = ealloc_adj(e, &a->L, s6);
         if (!rc) rc = ealloc_adj(e, &a->LY1, s6);
         if (!rc) rc = ealloc_adj(e, &a->LY2, s6);
-        if (!rc) rc = ealloc_adj(e, &a->T, s6);
         if (!rc) rc = ealloc_adj(e, &a->gm0, 2 * (size_t)e->capc);
+        if (!rc) rc = ealloc_adj(e, &a->sums, (size_t)RV * e->capc);
+        if (!rc) rc = ealloc_adj(e, &a->jd, (size_t)REVD_F * e->cap);
         if (!rc) rc = ealloc_adj(e, &a->rec, (size_t)e->cap + 2);
         if (!rc) rc = ealloc_adj(e, &a->aoff, (size_t)e->capc);
         if (!rc) rc = adj_resident_grid(e, k_ens_adj_rev, &a->grid);
@@ -577,14 +543,6 @@ int ens_adj_get(pn1_ens* e, pn1_ens_adj** out)
         }
     }
     pn1_ens_adj* a = e->adj;
-    if (e->nb > a->ablk_cap) {          // per-block partials follow the block table
-        if (a->ablk) (void)hipFree(a->ablk);
-        a->ablk = nullptr;
-        a->ablk_cap = 0;
-        int rc = ealloc_adj(e, &a->ablk, (size_t)e->nb * 4);
-        if (rc) return rc;
-        a->ablk_cap = e->nb;
-    }
     if (a->tab_L != e->L || a->tab_gen != e->gen) {   // partial layout of the clusters
         std::vector<long long> aoff(e->nc > 0 ? e->nc : 1, 0);
         size_t tot = 0;
@@ -614,34 +572,26 @@ int ens_adj_get(pn1_ens* e, pn1_ens_adj** out)
     return PN1_OK;
 }
 
-int ens_enqueue_vjp(pn1_ens* e, pn1_ens_adj* a, const double* y, const double* mu,
-                    double* out, const Phys& P)
+int ens_enqueue_vjp(pn1_ens* e, pn1_ens_adj* a, const double* y, const AdjLin& l,
+                    const AdjAdd& z, double* out, const Phys& P)
 {
-    if (e->nb)
-        hipLaunchKernelGGL(k_ens_adj_prep, dim3(e->nb), dim3(WG), 0, e->st, y, mu, e->m, e->coff,
-                           e->blk, P, a->rec);
-    if (e->nitems) {
-        hipLaunchKernelGGL(k_ens_adj_reset, dim3(1), dim3(64), 0, e->st, e->counter);
+    hipLaunchKernelGGL(k_ens_adj_prep, dim3(e->npblk), dim3(FWG), 0, e->st, y, l, a->mu, e->m,
+                       e->coff, e->crow, e->pblk, P, a->rec, a->jd, e->rows, a->sums, e->ticket,
+                       e->counter);
+    if (e->nitems)
         hipLaunchKernelGGL(k_ens_adj_rev, dim3(std::min(a->grid, e->nitems)), dim3(WG), 0, e->st,
-                           a->rec, y, mu, e->m, a->apart, a->aoff, e->items, e->counter, e->qoff,
-                           P, e->L);
-    }
-    if (e->nb)
-        hipLaunchKernelGGL(k_ens_adj_fin, dim3(e->nb), dim3(WG), 0, e->st, a->rec, y, mu, e->m,
-                           e->coff, e->blk, (const double*)a->apart, a->aoff, out, a->ablk, P,
-                           e->L);
-    hipLaunchKernelGGL(k_ens_adj_bh, dim3(e->nc), dim3(WG), 0, e->st, a->ablk, e->cblk, e->coff,
-                       mu, out, a->gm0, P);
+                           a->rec, a->jd, y, a->mu, e->m, a->apart, a->aoff, e->items,
+                           e->counter, e->qoff, P, e->L);
+    if (e->nrow <= ADJ_FIN_ROWS)
+        hipLaunchKernelGGL(k_ens_adj_fin<FG>, dim3(e->nrow), dim3(FWG), 0, e->st, a->rec, y, a->mu,
+                           e->m, e->coff, e->crow, e->row, (const double*)a->apart, a->aoff,
+                           a->sums, z, out, a->gm0, e->rows, e->ticket, P, e->L);
+    else
+        hipLaunchKernelGGL(k_ens_adj_fin<1>, dim3(e->npblk), dim3(FWG), 0, e->st, a->rec, y, a->mu,
+                           e->m, e->coff, e->crow, e->pblk, (const double*)a->apart, a->aoff,
+                           a->sums, z, out, a->gm0, e->rows, e->ticket, P, e->L);
     EHIPCHK(e, hipGetLastError());
     return PN1_OK;
-}
-
-void ens_lin(pn1_ens* e, double* out, double ca, const double* A, double cb = 0.0,
-             const double* B = nullptr, double cc = 0.0, const double* C = nullptr,
-             double cd = 0.0, const double* D = nullptr)
-{
-    hipLaunchKernelGGL(k_adj_lin, dim3((e->n + WG - 1) / WG), dim3(WG), 0, e->st, out, e->n,
-                       e->cap, ca, A, cb, B, cc, C, cd, D);
 }
 
 int ens_put6(pn1_ens* e, const double* hx, const double* hv, double* dst)
@@ -707,9 +657,10 @@ int pn1_ens_force_vjp(pn1_ens* e, const double* u, double* gx, double* gv, doubl
     pn1_ens_adj* a;
     if ((rc = ens_adj_get(e, &a))) return rc;
     const Phys P = ens_phys(e);
-    if ((rc = ens_put6(e, nullptr, u, a->mu))) return rc;
+    if ((rc = ens_put6(e, nullptr, u, a->L))) return rc;
     EHIPCHK(e, hipMemsetAsync(a->gm0, 0, 2 * (size_t)e->nc * sizeof(double), e->st));
-    if ((rc = ens_enqueue_vjp(e, a, e->X, a->mu, a->out, P))) return rc;
+    const AdjLin mu = {a->L, nullptr, 1.0, 0.0};
+    if ((rc = ens_enqueue_vjp(e, a, e->X, mu, AdjAdd{}, a->out, P))) return rc;
     const size_t cap = (size_t)e->cap;
     if ((rc = ens_fetch3(e, a->out, gx))) return rc;
     if ((rc = ens_fetch3(e, a->out + 3 * cap, gv))) return rc;
@@ -792,13 +743,13 @@ int pn1_ens_adjoint_backward(pn1_ens* e, const double* gx, const double* gv, dou
         }
         for (int t = t1 - 1; t >= t0; --t) {
             const double* st = a->seg + 3 * (size_t)(t - t0) * s6;
-            ens_lin(e, a->mu, dt / 6.0, a->L);
-            if ((rc = ens_enqueue_vjp(e, a, st + 2 * s6, a->mu, a->LY2, P))) return rc;
-            ens_lin(e, a->mu, dt / 6.0, a->L, dt / 2.0, a->LY2);
-            if ((rc = ens_enqueue_vjp(e, a, st + s6, a->mu, a->LY1, P))) return rc;
-            ens_lin(e, a->mu, dt / 6.0, a->L, dt / 2.0, a->LY1);
-            if ((rc = ens_enqueue_vjp(e, a, st, a->mu, a->T, P))) return rc;
-            ens_lin(e, a->L, 1.0, a->L, 1.0, a->LY2, 1.0, a->LY1, 1.0, a->T);
+            const AdjLin m2 = {a->L, nullptr, dt / 6.0, 0.0};
+            const AdjLin m1 = {a->L, a->LY2, dt / 6.0, dt / 2.0};
+            const AdjLin m0 = {a->L, a->LY1, dt / 6.0, dt / 2.0};
+            const AdjAdd sum = {a->L, a->LY2, a->LY1};
+            if ((rc = ens_enqueue_vjp(e, a, st + 2 * s6, m2, AdjAdd{}, a->LY2, P))) return rc;
+            if ((rc = ens_enqueue_vjp(e, a, st + s6, m1, AdjAdd{}, a->LY1, P))) return rc;
+            if ((rc = ens_enqueue_vjp(e, a, st, m0, sum, a->L, P))) return rc;
         }
     }
     if ((rc = ens_copy6(e, e->X, a->ckpt))) return rc;      // leave the initial state

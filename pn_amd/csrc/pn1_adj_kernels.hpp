@@ -170,35 +170,6 @@ __host__ __device__ __forceinline__ auto adj_star_psi(const T (&vi)[3], const T 
     return newton + lam * (t3 + t4 - t5 + t6 + t7 - t8);
 }
 
-// Record of star p (BH at b0) of the state y (SoA, stride cap) with
-// cotangent u = mu_v.
-__device__ __forceinline__ void adj_prep_star(const double* __restrict__ y,
-                                              const double* __restrict__ mu,
-                                              const double* __restrict__ m, size_t cap,
-                                              double eps2, int p, int b0,
-                                              ARec* __restrict__ rec)
-{
-    ARec r;
-    r.x = y[p]; r.y = y[cap + p]; r.z = y[2 * cap + p];
-    r.vx = y[3 * cap + p]; r.vy = y[4 * cap + p]; r.vz = y[5 * cap + p];
-    r.ux = mu[3 * cap + p]; r.uy = mu[4 * cap + p]; r.uz = mu[5 * cap + p];
-    r.m = m[p];
-    r.dx = r.x - y[b0]; r.dy = r.y - y[cap + b0]; r.dz = r.z - y[2 * cap + b0];
-    r.D2 = r.dx * r.dx + r.dy * r.dy + r.dz * r.dz;
-    r.e = rsq64(r.D2 + eps2);
-    r.pad = 0.0;
-    rec[p] = r;
-}
-
-__global__ __launch_bounds__(WG) void k_adj_prep(const double* __restrict__ y,
-                                                const double* __restrict__ mu,
-                                                const double* __restrict__ m, Phys P,
-                                                ARec* __restrict__ rec)
-{
-    const int p = blockIdx.x * WG + threadIdx.x + 1;
-    if (p < P.n) adj_prep_star(y, mu, m, (size_t)P.cap, P.eps2, p, 0, rec);
-}
-
 // d (psi_i + phi_ii) / d(x_i, v_i, m0) for star i with record `me`.  The
 // self pair phi_ii is taken with both sides on the same variables: r = 0
 // and its tangents cancel exactly, as in the reference's own sum.
@@ -221,99 +192,6 @@ __device__ __forceinline__ void adj_star_grad(const ARec& me, const ABH& B, doub
                                 me.m, me.m, m0, im0, ume, B.u0, eps2, lam);
 #pragma unroll
     for (int k = 0; k < NADJ1; ++k) g[k] = psi.d[k] + self.d[k];
-}
-
-// out_x = g_x, out_v = mu_x + g_v for particle p; t = {g_x, d/dm0}.
-__device__ __forceinline__ void adj_store(const double (&g)[NADJ1], const double* __restrict__ mu,
-                                          double* __restrict__ out, size_t cap, int p,
-                                          double (&t)[4])
-{
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        out[(size_t)k * cap + p] = g[k];
-        out[(size_t)(3 + k) * cap + p] = mu[(size_t)k * cap + p] + g[3 + k];
-        t[k] = g[k];
-    }
-    t[3] = g[6];
-}
-
-// Per star: the pair kernel's partials plus the star terms.  part holds S
-// rows of NADJ1 i-side sums (one per j chunk) and then nIb rows of NADJ2
-// j-side sums (one per 256-star i block), each row of stride cap.  Writes
-// out_x = g_x and out_v = mu_x + g_v (the VJP of the stage function
-// (x, v) -> (v, a)), and per-block partials {sum g_x, sum d/dm0}.
-__global__ __launch_bounds__(WG) void k_adj_fin(const ARec* __restrict__ rec,
-                                               const double* __restrict__ y,
-                                               const double* __restrict__ mu,
-                                               const double* __restrict__ m,
-                                               const double* __restrict__ part, int S, int nIb,
-                                               double* __restrict__ out,
-                                               double* __restrict__ blk, Phys P)
-{
-    const int p = blockIdx.x * WG + threadIdx.x + 1;
-    const size_t cap = (size_t)P.cap;
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    if (p < P.n) {
-        const ABH B = load_abh(y, mu, m, P.cap, 0);
-        double g[NADJ1];
-        adj_star_grad(rec[p], B, P.eps, P.eps2, P.lam, g);
-        for (int s = 0; s < S; ++s) {
-#pragma unroll
-            for (int k = 0; k < NADJ1; ++k) g[k] += part[(size_t)(s * NADJ1 + k) * cap + p];
-        }
-        const double* pj = part + (size_t)S * NADJ1 * cap;
-        for (int b = 0; b < nIb; ++b) {
-#pragma unroll
-            for (int k = 0; k < NADJ2; ++k) g[k] += pj[(size_t)(b * NADJ2 + k) * cap + p];
-        }
-        adj_store(g, mu, out, cap, p, t);
-    }
-    block_sum<4>(t, blk + (size_t)blockIdx.x * 4);
-}
-
-// BH: out_x[0] = -(sum of the stars' g_x), out_v[0] = mu_x[0]; the m0
-// derivative of this evaluation goes to gm0[1] and is added to gm0[0].
-__global__ __launch_bounds__(WG) void k_adj_bh(const double* __restrict__ blk, int nblk,
-                                              const double* __restrict__ mu,
-                                              double* __restrict__ out,
-                                              double* __restrict__ gm0, Phys P)
-{
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblk; b += WG)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) s[k] += blk[(size_t)b * 4 + k];
-    __shared__ double tot[4];
-    block_sum<4>(s, tot);
-    if (threadIdx.x == 0) {
-        const size_t cap = (size_t)P.cap;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            out[(size_t)k * cap] = -tot[k];
-            out[(size_t)(3 + k) * cap] = mu[(size_t)k * cap];
-        }
-        gm0[1] = tot[3];
-        gm0[0] += tot[3];
-    }
-}
-
-// out = a A + b B + c C + d D over the 6 rows of n particles (stride cap);
-// a null operand is skipped.  out may alias an operand.
-__global__ __launch_bounds__(WG) void k_adj_lin(double* out, int n, int cap, double a,
-                                               const double* A, double b, const double* B,
-                                               double c, const double* C, double d,
-                                               const double* D)
-{
-    const int p = blockIdx.x * WG + threadIdx.x;
-    if (p >= n) return;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const size_t i = (size_t)k * cap + p;
-        double r = a * A[i];
-        if (B) r += b * B[i];
-        if (C) r += c * C[i];
-        if (D) r += d * D[i];
-        out[i] = r;
-    }
 }
 
 }  // namespace pn1dev

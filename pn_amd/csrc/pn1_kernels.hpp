@@ -32,6 +32,7 @@
 // that are not templates are therefore declared inline.
 #pragma once
 #include "pn1_common.hpp"
+#include "pn1_rows.hpp"
 
 namespace pn1dev {
 // What the stage update of the reference's RK driver (Limit-sticky9.c:853-891)
@@ -109,134 +110,6 @@ __device__ __forceinline__ void stage_update(int p, int cap, const StageIn& s, i
         X[ix] = nx;
         X[iv] = nv;
     }
-}
-
-// ---------------------------------------------------------------------
-// rows: the O(n) kernels take the stars in rows of 64 (one per lane of a
-// wave), FG waves to a workgroup
-// ---------------------------------------------------------------------
-constexpr int RB = 64;
-constexpr int FG = 8;
-constexpr int FWG = FG * RB;
-// A row's share of the sums over all stars: RV doubles, the BH's 1PN
-// acceleration (3), then the NGS separable sums of the next evaluation.
-constexpr int RV = 16;
-constexpr int RV_G = 3;
-static_assert(RV_G + NGS <= RV, "a row's values");
-
-// Sum over the wave, in every lane (xor butterfly: the same bits in each).
-__device__ __forceinline__ double wave_sum(double t)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-    return t;
-}
-
-// lo = {a in the lower half (G = 32) or the even rows of 16 (G = 16), b's
-// other half moved there}, and hi the rest: adding both sums a over lane
-// pairs l, l ^ G in the lanes without that bit and b in the others.
-template <int G>
-__device__ __forceinline__ double swap_sum(double a, double b)
-{
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    const unsigned long long ua = (unsigned long long)__double_as_longlong(a);
-    const unsigned long long ub = (unsigned long long)__double_as_longlong(b);
-    u32x2 l, h;
-    if (G == 32) {
-        l = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
-        h = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
-    } else {
-        l = __builtin_amdgcn_permlane16_swap((unsigned)ua, (unsigned)ub, false, false);
-        h = __builtin_amdgcn_permlane16_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
-    }
-    const double x = __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0]));
-    const double y = __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
-    return x + y;
-}
-
-// The wave's sums of 16 values: lane l gets the sum of v[l >> 2] over all
-// lanes.  Halving the values at each exchange takes 15 of them instead of
-// the 16 x 6 of one butterfly per value, and half the code, which in kernels
-// that run each instruction once is most of their time.
-__device__ __forceinline__ double wave_sums16(const double (&v)[16])
-{
-    const int lane = threadIdx.x & 63;
-    double a[8], b[4], c[2];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) a[k] = swap_sum<32>(v[k], v[8 + k]);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) b[k] = swap_sum<16>(a[k], a[4 + k]);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const bool up = lane & 8;
-        const double keep = up ? b[2 + k] : b[k], send = up ? b[k] : b[2 + k];
-        c[k] = keep + __shfl_xor(send, 8, 64);
-    }
-    const bool up = lane & 4;
-    double t = (up ? c[1] : c[0]) + __shfl_xor(up ? c[0] : c[1], 4, 64);
-    t += __shfl_xor(t, 2, 64);
-    t += __shfl_xor(t, 1, 64);
-    return t;
-}
-
-// Values that one workgroup hands to another within a launch (the rows' sums
-// and masks, to the last workgroup): stored and loaded at device scope, past
-// the XCD's own L2.  A release fence would do the same for ordinary stores,
-// but it writes back every dirty line of that L2, per workgroup (measured on
-// MI355X: 0.14 us each, 1.4 ms of an ensemble's 9864 workgroups).
-template <typename T>
-__device__ __forceinline__ void hand_over(T* p, T v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ T take_over(const T* p)
-{
-    return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Fixed-order sums of rows [b0, b1), by a workgroup of FWG threads, into
-// tot[RV] (LDS), for every thread of it: thread t adds value t % RV of rows
-// t / RV, t / RV + FWG / RV, ...
-__device__ __forceinline__ void rows_total(const double* rows, int b0, int b1, double* tot)
-{
-    __shared__ double sh[FG][RV];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    double t = 0.0;
-#pragma unroll 8
-    for (int b = b0 + (int)threadIdx.x / RV; b < b1; b += FWG / RV)
-        t += take_over(&rows[(size_t)b * RV + (threadIdx.x & (RV - 1))]);
-    t += __shfl_xor(t, 16, 64);
-    t += __shfl_xor(t, 32, 64);
-    if (lane < RV) sh[wid][lane] = t;
-    __syncthreads();
-    if (threadIdx.x < RV) {
-        t = sh[0][threadIdx.x];
-#pragma unroll
-        for (int w = 1; w < FG; ++w) t += sh[w][threadIdx.x];
-        tot[threadIdx.x] = t;
-    }
-    __syncthreads();
-}
-
-// Whether this workgroup is the last of `nblk` to get here (the counter goes
-// back to 0 for the next launch).  What the others handed over before is
-// visible to it: every wave waits for its own stores to complete before the
-// workgroup takes its ticket, and the last ticket is taken after all others.
-// Every thread of the workgroup calls it.
-__device__ __forceinline__ bool last_block(unsigned int* cnt, unsigned int nblk)
-{
-    __shared__ bool s_last;
-    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned int t =
-            __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_last = t == nblk - 1;
-        if (s_last) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    return s_last;
 }
 
 // ---------------------------------------------------------------------
