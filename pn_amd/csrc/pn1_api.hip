@@ -59,8 +59,6 @@ int dalloc(pn1_ctx* c, T** p, size_t count)
     return PN1_OK;
 }
 
-int nblocks(int nst) { return nst > 0 ? (nst + WG - 1) / WG : 1; }
-
 Phys make_phys(const pn1_ctx* c)
 {
     Phys P;
@@ -87,8 +85,8 @@ double flag_threshold(double dmax)
     return PN1_FLAG_ETA / (6.0 * 0x1p-24 * 2.0 * dmax);
 }
 
-// j split of the 256-star kernels where none is set explicitly (i shards,
-// energy): many short rounds of workgroups, chunks of at least 64 records.
+// j split of the 256-star kernels where none is set explicitly (i shards):
+// many short rounds of workgroups, chunks of at least 64 records.
 int auto_split(int nst)
 {
     const int nib = nst > 0 ? (nst + WG - 1) / WG : 0;
@@ -119,7 +117,6 @@ int auto_slots(int nst)
 void plan(pn1_ctx* c)
 {
     const int nst = c->n - 1;
-    c->nblk = nblocks(nst);
     c->nrow = nst > 0 ? (nst + RB - 1) / RB : 1;
     c->nIblk = nst > 0 ? (nst + WG - 1) / WG : 0;
     c->slots = 0;
@@ -139,11 +136,8 @@ size_t part_need(const pn1_ctx* c, int slots = 0)
 {
     const size_t cap = (size_t)c->cap;
     const size_t S = (size_t)(slots > 0 ? slots : c->slots ? c->slots : c->S);
-    const size_t SE = (size_t)std::max(c->slots ? auto_split(c->n - 1) : c->S, 1);
     size_t need = S * NACC * cap * sizeof(double);
-    const size_t needE = SE * NACCE * cap * sizeof(double);
     const size_t need32 = S * MROWS * cap * sizeof(float);
-    if (needE > need) need = needE;
     if (need32 > need) need = need32;
     return need;
 }
@@ -513,7 +507,6 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
         return PN1_EDEVICE;
     }
     const size_t cap = (size_t)capacity;
-    const size_t nb = (size_t)nblocks(capacity) + 1;
     const size_t nr = (cap + RB - 1) / RB + 1;          // rows of 64 stars
     int rc = PN1_OK;
     if (!rc) rc = dalloc(c, &c->X, 6 * cap);
@@ -524,7 +517,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->acc, 3 * cap);
     if (!rc) rc = dalloc(c, &c->rows, nr * RV);
     if (!rc) rc = dalloc(c, &c->gs, 16);
-    if (!rc) rc = dalloc(c, &c->eblk, nb * NEB);
+    if (!rc) rc = dalloc(c, &c->eblk, nr * ECHUNK * EV);
     if (!rc) rc = dalloc(c, &c->eout, 8);
     // two records more than particles: the pair loops fetch up to jr[j + 2]
     if (!rc) rc = dalloc(c, &c->j64, 3 * (cap + 2));
@@ -730,14 +723,9 @@ int pn1_energy(pn1_ctx* c, pn1_energy_t* out)
     if (!out) return seterr(c, PN1_EINVAL, "null output");
     const Phys P = make_phys(c);
     if ((rc = prep_x(c, P, true))) return rc;
-    const int S = c->slots ? auto_split(c->n - 1) : c->S;
-    if (c->n > 1)
-        hipLaunchKernelGGL(k_epair64, dim3(pair_grid(S, c->nIblk)), dim3(WG), 0, c->st, c->j64,
-                           c->X, (double*)c->part, P, S, c->nIblk);
-    hipLaunchKernelGGL(k_efin, dim3(c->nblk), dim3(WG), 0, c->st, c->X, c->m,
-                       (const double*)c->part, c->n > 1 ? S : 0, c->gs, c->eblk, P);
-    hipLaunchKernelGGL(k_ered, dim3(1), dim3(WG), 0, c->st, c->eblk, c->nblk, c->X, c->m, c->gs,
-                       c->eout, P);
+    hipLaunchKernelGGL(k_energy, dim3(c->nrow, energy_chunks(c->n - 1)), dim3(PW * RB), 0, c->st,
+                       (const JRec64*)rec_buf(c, 0), (const double*)c->X, (const double*)c->gs,
+                       c->eblk, c->eout, c->ticket, P);
     HIPCHK(c, hipGetLastError());
     double e[5];
     HIPCHK(c, hipMemcpyAsync(e, c->eout, sizeof e, hipMemcpyDeviceToHost, c->st));

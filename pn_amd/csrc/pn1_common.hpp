@@ -8,9 +8,7 @@ namespace pn1dev {
 
 constexpr int WG = 256;     // threads per workgroup (4 waves of 64)
 constexpr int NACC = 16;    // force pair accumulators
-constexpr int NACCE = 5;    // energy pair accumulators
 constexpr int NGS = 7;      // separable O(n) sums
-constexpr int NEB = 4;      // energy per-block partials
 
 // sqrt(3/2): stored velocities are pre-scaled by it, so that the pair term
 // 1.5 (v_j.r)^2 w^2 is a plain square of (s_j.r) w with s_j = sqrt(3/2) v_j.
@@ -50,8 +48,6 @@ enum { A_NX, A_NY, A_NZ, A_RX, A_RY, A_RZ, A_UX, A_UY, A_UZ, A_TX, A_TY, A_TZ,
 constexpr int A_TS = NACC;
 constexpr int NACC32 = NACC + 1;
 constexpr int MROWS = NACC32 + 3;
-// energy pair accumulators: phi, sum m_j w s_j, sum m_j w^3 (r.v_i)(r.s_j)
-enum { E_PHI, E_PVX, E_PVY, E_PVZ, E_GAM };
 // separable sums over stars: sum m e, sum m e^3 d, sum m v
 enum { G_G1, G_M1X, G_M1Y, G_M1Z, G_PX, G_PY, G_PZ };
 
@@ -61,8 +57,9 @@ enum { G_G1, G_M1X, G_M1Y, G_M1Z, G_PX, G_PY, G_PZ };
 //   A            1.25 m0 e - 2 |v|^2       B = 0.25 m0 e^3
 //   MB = m B     Qd = Q d, Q = 3.5 m0 m e^3 (the pair term Q w d is then one FMA
 //                per component)            e = (|d|^2 + eps^2)^-1/2
+//   Ae = 1.5 |v|^2 + m0 e (the energy's pair term)
 struct __align__(16) JRec64 {
-    double x, y, z, sx, sy, sz, m, D2, A, B, MB, Qdx, Qdy, Qdz, e, pad;
+    double x, y, z, sx, sy, sz, m, D2, A, B, MB, Qdx, Qdy, Qdz, e, Ae;
 };
 // j-record, mixed form: double-single position (hi, lo), the rest rounded
 // to FP32, and Qd = Q d (the pair term Q w d is then one FMA per component).

@@ -27,7 +27,7 @@ struct pn1_ctx {
     // launch plan for the current n
     // j split (S parts); slots: partials per star of the automatic plan's pair
     // kernels, which give each PW parts (0: the explicit split's kernels)
-    int S = 1, slots = 0, nIblk = 0, nblk = 1, tile = 64;
+    int S = 1, slots = 0, nIblk = 0, tile = 64;
     // device buffers
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr;
     double *m = nullptr, *acc = nullptr, *rows = nullptr, *gs = nullptr;

@@ -6,9 +6,8 @@
 //   coff[nc + 1]   first particle of each cluster
 //   cm0[nc]        BH mass of each cluster
 //   cmmax[nc]      largest star mass of each cluster
-//   blk[nb], cblk[nc + 1]   256-star blocks, per cluster (energy, adjoint)
-//   row[nrow], crow[nc + 1]   64-star rows of the force's O(n) kernels, per
-//                  cluster; pblk[npblk]: groups of FG of them (k_ens_prep)
+//   row[nrow], crow[nc + 1]   64-star rows of the O(n) kernels, per
+//                  cluster; pblk[npblk]: groups of FG of them
 //   items[nitems]  pair work items in 8 per-XCD queues (qoff[9]): whole
 //                  clusters go to the least-loaded queue, largest first;
 //                  each queue is sorted by decreasing pair count
@@ -57,17 +56,17 @@ struct pn1_ens {
     // three buffers of cap + 2 records, as in pn1_ctx
     pn1dev::JRec64* j64 = nullptr;
     pn1dev::JRec32* j32 = nullptr;
-    int *coff = nullptr, *cblk = nullptr, *qoff = nullptr;
-    pn1dev::EBlk* blk = nullptr;
+    int *coff = nullptr, *qoff = nullptr;
     pn1dev::EItem* items = nullptr;
     long long* poff = nullptr;
     unsigned int* counter = nullptr;
-    int nb = 0, nitems = 0, nb_cap = 0, items_cap = 0;
+    int nitems = 0, items_cap = 0;
+    int echunks = 1;                // largest energy_chunks of a cluster
     long long slots = 0;
     void* part = nullptr;
     size_t part_bytes = 0;
     double* h_stage = nullptr;
-    int grid64[2] = {0, 0}, grid32[4] = {0, 0, 0, 0}, gride = 0;   // per kernel variant
+    int grid64[2] = {0, 0}, grid32[4] = {0, 0, 0, 0};   // per kernel variant
     hipGraphExec_t gexec = nullptr;
     bool prof = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;

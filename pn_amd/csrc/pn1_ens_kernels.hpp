@@ -275,112 +275,34 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
         fin_close<MODE, STAGE>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P);
 }
 
-// One workgroup per cluster: rows [cblk[c], cblk[c+1]) of `rows` (N wide).
-template <int N>
-__device__ __forceinline__ void cluster_rows_sum(const double* __restrict__ rows,
-                                                 const int* __restrict__ cblk, int c,
-                                                 double (&g)[N])
-{
-#pragma unroll
-    for (int k = 0; k < N; ++k) g[k] = 0.0;
-    for (int b = cblk[c] + (int)threadIdx.x; b < cblk[c + 1]; b += WG)
-#pragma unroll
-        for (int k = 0; k < N; ++k) g[k] += rows[(size_t)b * N + k];
-}
-
 // ---------------------------------------------------------------------
 // ensemble energies (FP64)
 // ---------------------------------------------------------------------
-inline __global__ __launch_bounds__(WG) void k_ens_epair64(const JRec64* __restrict__ jr,
-                                                   const double* __restrict__ st,
-                                                   double* __restrict__ part,
-                                                   const EItem* __restrict__ items,
-                                                   unsigned int* __restrict__ counter,
-                                                   const int* __restrict__ qoff, Phys P)
+// As k_energy, workgroup (row of the ensemble, chunk); a cluster uses
+// energy_chunks of the grid's chunks, the others leave at once.  Its last
+// workgroup writes its energies to out[5 c].
+inline __global__ __launch_bounds__(PW * RB)
+void k_ens_energy(const JRec64* __restrict__ jr, const double* __restrict__ st, EnsBufs E,
+                  const EBlk* __restrict__ rowt, const double* __restrict__ gs,
+                  double* __restrict__ eb, double* __restrict__ out,
+                  unsigned int* __restrict__ ticket, Phys P)
 {
-    int q = 0;
-    for (;;) {
-        const int it = ens_take(counter, qoff, q);
-        if (it < 0) break;
-        const EItem w = items[it];
-        const EGeom g = ens_geom(w);
-        IE64 I;
-        I.x = jr[g.i].x; I.y = jr[g.i].y; I.z = jr[g.i].z;
-        I.ux = st[3 * P.cap + g.i] / PN1_SQ15;
-        I.uy = st[4 * P.cap + g.i] / PN1_SQ15;
-        I.uz = st[5 * P.cap + g.i] / PN1_SQ15;
-        double a[NACCE];
-#pragma unroll
-        for (int k = 0; k < NACCE; ++k) a[k] = 0.0;
-        if (g.w0 < g.w1) {
-            erun64<false>(jr, w.j0, g.w0, g.i, I, a, P.eps2);
-            erun64<true>(jr, g.w0, g.w1, g.i, I, a, P.eps2);
-            erun64<false>(jr, g.w1, w.j1, g.i, I, a, P.eps2);
-        } else {
-            erun64<false>(jr, w.j0, w.j1, g.i, I, a, P.eps2);
-        }
-        if (g.li < w.nst) {
-            double* pp = part + w.pslot * NACCE + g.li;
-#pragma unroll
-            for (int k = 0; k < NACCE; ++k) stream_out(a[k], &pp[(size_t)k * w.nst]);
-        }
-    }
-}
-
-inline __global__ __launch_bounds__(WG) void k_ens_efin(const double* __restrict__ st,
-                                                const double* __restrict__ m,
-                                                const double* __restrict__ cm0,
-                                                const int* __restrict__ coff,
-                                                const EBlk* __restrict__ blk,
-                                                const double* __restrict__ part,
-                                                const long long* __restrict__ poff,
-                                                const double* __restrict__ gs,
-                                                double* __restrict__ eblk, Phys P, EConst E)
-{
-    const EBlk b = blk[blockIdx.x];
-    const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
-    const int li = b.first + (int)threadIdx.x;
-    double t[NEB] = {0.0, 0.0, 0.0, 0.0};
-    if (li < nst) {
-        const double* pp = part + poff[b.c] * NACCE + li;
-        double A[NACCE] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        const int S = ens_nchunks(nst, E.L);
-        for (int s = 0; s < S; ++s)
-#pragma unroll
-            for (int k = 0; k < NACCE; ++k) A[k] += pp[(size_t)(s * NACCE + k) * nst];
-        efin_star(st, m, P.cap, off + 1 + li, off, cm0[b.c], P.eps2, A,
-                  gs[(size_t)b.c * NGS + G_G1], t);
-    }
-    block_sum<NEB>(t, eblk + (size_t)blockIdx.x * NEB);
-}
-
-// out[c] = {kin, pot, pot_pn/c^2, pot_pn2/c^2, total} of cluster c
-inline __global__ __launch_bounds__(WG) void k_ens_ered(const double* __restrict__ eblk,
-                                                const int* __restrict__ cblk,
-                                                const int* __restrict__ coff,
-                                                const double* __restrict__ st,
-                                                const double* __restrict__ m,
-                                                const double* __restrict__ gs,
-                                                double* __restrict__ out, Phys P)
-{
-    const int c = blockIdx.x;
-    double s[NEB];
-    cluster_rows_sum<NEB>(eblk, cblk, c, s);
-    __shared__ double tot[NEB];
-    block_sum<NEB>(s, tot);
-    if (threadIdx.x == 0) {
-        const int b0 = coff[c], cap = P.cap;
-        const double v0x = st[3 * cap + b0], v0y = st[4 * cap + b0], v0z = st[5 * cap + b0];
-        const double kin = 0.5 * (m[b0] * (v0x * v0x + v0y * v0y + v0z * v0z) + tot[0]);
-        const double pot = tot[1] - m[b0] * gs[(size_t)c * NGS + G_G1];
-        const double pn = P.lam * tot[2], pn2 = P.lam * tot[3];
-        double* o = out + (size_t)c * 5;
-        o[0] = kin;
-        o[1] = pot;
-        o[2] = pn;
-        o[3] = pn2;
-        o[4] = kin + pot + pn + pn2;
-    }
+    __shared__ double t[EV];
+    const int2 w = energy_item();
+    const int r = w.x, s = w.y, c = rowt[r].c;
+    const int off = E.coff[c], nst = E.coff[c + 1] - off - 1;
+    const int S = energy_chunks(nst), r0 = E.crow[c], nrow = E.crow[c + 1] - r0;
+    if (s >= S) return;
+    const double m0 = E.cm0[c], G1 = gs[(size_t)c * NGS + G_G1];
+    if (nst > 0)
+        energy_row(jr, st, P.cap, off, nst, nrow, r - r0, s, S, m0, G1, P.eps2, t);
+    else if (threadIdx.x < EV)
+        t[threadIdx.x] = 0.0;
+    if (threadIdx.x < EV)
+        hand_over(&eb[((size_t)r * ECHUNK + s) * EV + threadIdx.x], t[threadIdx.x]);
+    if (last_block(ticket + c, (unsigned)(nrow * S)))
+        energy_total(eb + (size_t)r0 * ECHUNK * EV, nrow * S, S, ECHUNK, st, P.cap, off, m0, G1,
+                     P.lam, out + (size_t)c * 5);
 }
 
 }  // namespace pn1dev

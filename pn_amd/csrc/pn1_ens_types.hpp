@@ -18,17 +18,12 @@ struct __align__(32) EItem {
     long long pslot;
 };
 
-// Star block of the O(n) kernels: cluster and first local star index.
+// Row (or group of rows) of the O(n) kernels: cluster and first local star.
 // Partial sums of cluster c start at slot poff[c] (a slot is one chunk of
 // one star; slots of c: nchunks(c) x its star count) times the number of
-// values a kernel keeps per slot (NACC, NACC + 3 or NACCE).
+// values a kernel keeps per slot (NACC or MROWS).
 struct __align__(8) EBlk {
     int c, first;
-};
-
-// Ensemble launch constants: chunk length L (j-records per item).
-struct EConst {
-    int nitems, L, nclusters;
 };
 
 __device__ __forceinline__ int ens_nchunks(int nst, int L) { return (nst + L - 1) / L; }

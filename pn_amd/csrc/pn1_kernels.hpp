@@ -180,7 +180,7 @@ __device__ __forceinline__ bool prep_star(const double (&xp)[3], const double (&
     const double Q = 3.5 * m0 * q;
     r.MB = mp * r.B;
     r.Qdx = Q * dx; r.Qdy = Q * dy; r.Qdz = Q * dz;
-    r.e = e; r.pad = 0.0;
+    r.e = e; r.Ae = 1.5 * V2 + m0 * e;
     j64[p] = r;
     g[G_G1] = mp * e;
     g[G_M1X] = q * dx; g[G_M1Y] = q * dy; g[G_M1Z] = q * dz;
@@ -1473,155 +1473,202 @@ inline __global__ __launch_bounds__(FWG) void k_bh(FinBufs F, RowBufs R, int nro
 }
 
 // ---------------------------------------------------------------------
-// energy: pair sums (FP64 in both modes), per-star terms, totals
+// energy (FP64 in both modes)
 // ---------------------------------------------------------------------
-// Energy pair body.  The record holds s_j = sqrt(3/2) v_j; the lane's
-// velocity is pre-divided by sqrt(3/2) so that (r.v_i)(r.s_j) needs no
-// rescaling, and k_efin divides sum m_j w s_j by sqrt(3/2).
+// The energy needs totals only (Limit-sticky9.c:452-550), so each unordered
+// pair is evaluated once:
+//   pot  -= m_i m_j w
+//   pn2  += m_i m_j [w (Ae_i + Ae_j - 3.5 v_i.v_j) - 0.5 w^3 (r.v_i)(r.v_j)]
+// with Ae = 1.5 |v|^2 + m0 e from the records.  Row a of 64 stars (one per
+// lane) meets the stars of the next half of the rows, cyclically: rows a + 1
+// .. a + h, h = nrow / 2 (a row less for the upper half of the rows when nrow
+// is even), and its own stars above each lane's.  That list is split in S
+// chunks of PW waves, which work as k_pair64w's.  Against all ordered pairs
+// with five sums per star it is half the rsqrts and no partials: n = 65537,
+// 4.17 -> 2.24 ms on MI355X (31 issue slots per pair: 2.17 ms at the FP64
+// rate of 3.1e13 lanes/s).
+// Chunks per row: 16, fewer while a wave's part would hold fewer than 4
+// records (each meets half of the stars).
+__host__ __device__ inline int energy_chunks(int nst)
+{
+    int s = 16;
+    while (s > 1 && nst < 8 * s * PW) s >>= 1;
+    return s;
+}
+constexpr int ECHUNK = 16;
+
+// Per-lane constants of star i: position, p = -3.5 / sqrt(3/2) v, q = -0.5 /
+// sqrt(3/2) v (the records hold s = sqrt(3/2) v).
 struct IE64 {
-    double x, y, z, ux, uy, uz;
+    double x, y, z, px, py, pz, qx, qy, qz;
 };
 
-template <bool MASK>
-__device__ __forceinline__ void ebody64(const JRec64& J, int j, int i, const IE64& I,
-                                        double (&a)[NACCE], double eps2)
+// One pair: a += m_j w, b += m_j [w (Ae_j - 3.5 v_i.v_j) - 0.5 w^3 (r.v_i)(r.v_j)].
+__device__ __forceinline__ void ebody64(const JRec64& J, double mj, const IE64& I, double& a,
+                                        double& b, double eps2)
 {
-    double mj = J.m;
-    if (MASK) mj = (j == i) ? 0.0 : mj;
     const double rx = J.x - I.x, ry = J.y - I.y, rz = J.z - I.z;
     const double R2e = __builtin_fma(rx, rx, __builtin_fma(ry, ry, __builtin_fma(rz, rz, eps2)));
     const double w = rsq64(R2e);
-    const double mw = mj * w;
-    a[E_PHI] += mw;
-    a[E_PVX] = __builtin_fma(mw, J.sx, a[E_PVX]);
-    a[E_PVY] = __builtin_fma(mw, J.sy, a[E_PVY]);
-    a[E_PVZ] = __builtin_fma(mw, J.sz, a[E_PVZ]);
-    const double rvi = __builtin_fma(I.ux, rx, __builtin_fma(I.uy, ry, I.uz * rz));
+    const double rvi = __builtin_fma(I.qx, rx, __builtin_fma(I.qy, ry, I.qz * rz));
     const double rvj = __builtin_fma(J.sx, rx, __builtin_fma(J.sy, ry, J.sz * rz));
-    a[E_GAM] = __builtin_fma(mw * (w * w), rvi * rvj, a[E_GAM]);
+    double t = __builtin_fma(I.px, J.sx, __builtin_fma(I.py, J.sy, __builtin_fma(I.pz, J.sz, J.Ae)));
+    t = __builtin_fma(w * w, rvi * rvj, t);
+    const double mw = mj * w;
+    a += mw;
+    b = __builtin_fma(mw, t, b);
 }
 
-template <bool MASK>
-__device__ __forceinline__ void erun64(const JRec64* __restrict__ jr, int j0, int j1, int i,
-                                       const IE64& I, double (&a)[NACCE], double eps2)
+// Row `row` (of nrow) of a cluster's stars off + 1 .. off + nst, chunk s of S:
+// its four sums {m v^2, -m m w, the pot_pn terms, the pot_pn2 terms} in out
+// (LDS); the sums over single stars with chunk 0.  m0: the BH's mass, G1 =
+// sum m e.  Every thread of the workgroup (PW waves) calls it.
+constexpr int EV = 4;
+__device__ __forceinline__ void energy_row(const JRec64* __restrict__ jr,
+                                           const double* __restrict__ st, int cap, int off,
+                                           int nst, int nrow, int row, int s, int S, double m0,
+                                           double G1, double eps2, double* out)
 {
-    if (j0 >= j1) return;
-    JRec64 cur = jr[j0];
-    for (int j = j0; j < j1; ++j) {
-        const JRec64 nxt = jr[j + 1];
-        ebody64<MASK>(cur, j, i, I, a, eps2);
-        cur = nxt;
-    }
-}
-
-inline __global__ __launch_bounds__(WG) void k_epair64(const JRec64* __restrict__ jr,
-                                               const double* __restrict__ st,
-                                               double* __restrict__ part, Phys P, int S,
-                                               int nIblk)
-{
-    int s, ib;
-    map_block(blockIdx.x, S, nIblk, s, ib);
-    if (ib >= nIblk) return;
-    const int n = P.n, cap = P.cap;
-    const int li = ib * WG + threadIdx.x + 1;
-    const int i = li < n ? li : n - 1;
+    __shared__ double sh[PW][EV];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int li = row * RB + lane, p1 = off + 1;
+    const bool ok = li < nst;
+    const int i = p1 + (ok ? li : row * RB);
+    const JRec64 me = jr[i];
+    const double v[3] = {st[3 * cap + i], st[4 * cap + i], st[5 * cap + i]};
     IE64 I;
-    I.x = jr[i].x; I.y = jr[i].y; I.z = jr[i].z;
-    I.ux = st[3 * cap + i] / PN1_SQ15;
-    I.uy = st[4 * cap + i] / PN1_SQ15;
-    I.uz = st[5 * cap + i] / PN1_SQ15;
-    const JRange R = j_range(s, S, n, ib);
-    const double eps2 = P.eps2;
-    double a[NACCE];
-#pragma unroll
-    for (int k = 0; k < NACCE; ++k) a[k] = 0.0;
-    if (R.w0 < R.w1) {
-        erun64<false>(jr, R.j0, R.w0, i, I, a, eps2);
-        erun64<true>(jr, R.w0, R.w1, i, I, a, eps2);
-        erun64<false>(jr, R.w1, R.j1, i, I, a, eps2);
-    } else {
-        erun64<false>(jr, R.j0, R.j1, i, I, a, eps2);
+    I.x = me.x; I.y = me.y; I.z = me.z;
+    I.px = -3.5 * PN1_ISQ15 * v[0]; I.py = -3.5 * PN1_ISQ15 * v[1]; I.pz = -3.5 * PN1_ISQ15 * v[2];
+    I.qx = -0.5 * PN1_ISQ15 * v[0]; I.qy = -0.5 * PN1_ISQ15 * v[1]; I.qz = -0.5 * PN1_ISQ15 * v[2];
+    // the list: stars [first, first + len) modulo nst
+    const int h = nrow / 2 - ((nrow & 1) == 0 && row >= nrow / 2 ? 1 : 0);
+    const int first = row + 1 < nrow ? (row + 1) * RB : 0, last = row + h;      // row of the end
+    const int len = h <= 0 ? 0
+                    : last < nrow ? min(nst, (last + 1) * RB) - (row + 1) * RB
+                                  : max(nst - (row + 1) * RB, 0) + min(nst, (last - nrow + 1) * RB);
+    const int part = (len + S * PW - 1) / (S * PW);
+    const int q0 = min(len, (s * PW + wave) * part), q1 = min(len, q0 + part);
+    double a = 0.0, b = 0.0;
+    for (int j = first + q0; j < min(nst, first + q1); ++j) {
+        const JRec64& J = jr[p1 + j];
+        ebody64(J, J.m, I, a, b, eps2);
     }
-    if (li < n) {
-#pragma unroll
-        for (int k = 0; k < NACCE; ++k) stream_out(a[k], &part[(size_t)(s * NACCE + k) * cap + li]);
+    for (int j = max(first + q0 - nst, 0); j < first + q1 - nst; ++j) {
+        const JRec64& J = jr[p1 + j];
+        ebody64(J, J.m, I, a, b, eps2);
     }
+    double t[EV] = {0.0, 0.0, 0.0, 0.0};
+    if (s == 0) {
+        // the row's own pairs, wave w taking records w, w + PW, ...
+        for (int j = row * RB + wave; j < min(nst, row * RB + RB); j += PW) {
+            const JRec64& J = jr[p1 + j];
+            ebody64(J, j > li ? J.m : 0.0, I, a, b, eps2);
+        }
+        if (wave == 0) {
+            // single-star terms of Limit-sticky9.c:452-550
+            const double e = me.e, mp = me.m;
+            double d[3], v0[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                d[k] = st[(size_t)k * cap + i] - st[(size_t)k * cap + off];
+                v0[k] = st[(size_t)(3 + k) * cap + off];
+            }
+            const double V2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+            const double v0v = v0[0] * v[0] + v0[1] * v[1] + v0[2] * v[2];
+            const double dv0 = d[0] * v0[0] + d[1] * v0[1] + d[2] * v0[2];
+            const double dv = d[0] * v[0] + d[1] * v[1] + d[2] * v[2];
+            t[0] = mp * V2;
+            t[2] = 0.375 * mp * V2 * V2 + 1.5 * m0 * e * mp * V2 + 0.5 * m0 * m0 * e * e * mp
+                   + 0.5 * m0 * e * mp * (3.0 * V2 - 7.0 * v0v - dv0 * dv * e * e);
+            t[3] = mp * (0.5 * m0 * e * (G1 - mp * e));
+        }
+    }
+    t[1] = -me.m * a;
+    t[3] += me.m * __builtin_fma(me.Ae, a, b);
+#pragma unroll
+    for (int k = 0; k < EV; ++k) {
+        const double u = wave_sum(ok ? t[k] : 0.0);
+        if (lane == 0) sh[wave][k] = u;
+    }
+    __syncthreads();
+    if (threadIdx.x < EV) {
+        double u = sh[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < PW; ++w) u += sh[w][threadIdx.x];
+        out[threadIdx.x] = u;
+    }
+    __syncthreads();
 }
 
-// Per-star energy terms of Limit-sticky9.c:452-550 with the self pair
-// excluded, for star p of the cluster whose BH is at b0, from its energy
-// pair sums A: {m v^2, -1/2 m phi, pot_pn term, pot_pn2 term}.
-__device__ __forceinline__ void efin_star(const double* __restrict__ st,
-                                          const double* __restrict__ m, int cap, int p, int b0,
-                                          double m0, double eps2, const double (&A)[NACCE],
-                                          double G1, double (&t)[NEB])
+// The energy {kin, pot, pot_pn / c^2, pot_pn2 / c^2, total} of the cluster
+// with its BH at off from the sums of its `cnt` workgroups (EV values each, S
+// per row, rows `stride` workgroups apart), by a workgroup of PW waves.
+__device__ __forceinline__ void energy_total(const double* eb, int cnt, int S, int stride,
+                                             const double* __restrict__ st, int cap, int off,
+                                             double m0, double G1, double lam,
+                                             double* __restrict__ out)
 {
-    const double mp = m[p];
-    const double x[3] = {st[p], st[cap + p], st[2 * cap + p]};
-    const double v[3] = {st[3 * cap + p], st[4 * cap + p], st[5 * cap + p]};
-    const double v0[3] = {st[3 * cap + b0], st[4 * cap + b0], st[5 * cap + b0]};
-    double d[3], e;
-    {
-#pragma clang fp contract(off)
-        for (int k = 0; k < 3; ++k) d[k] = x[k] - st[(size_t)k * cap + b0];
-        e = 1.0 / sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + eps2);
-    }
-    const double V2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-    const double v0v = v0[0] * v[0] + v0[1] * v[1] + v0[2] * v[2];
-    const double dv0 = d[0] * v0[0] + d[1] * v0[1] + d[2] * v0[2];
-    const double dv = d[0] * v[0] + d[1] * v[1] + d[2] * v[2];
-    const double vPhv = (v[0] * A[E_PVX] + v[1] * A[E_PVY] + v[2] * A[E_PVZ]) / PN1_SQ15;
-    t[0] = mp * V2;
-    t[1] = -0.5 * mp * A[E_PHI];
-    t[2] = 0.375 * mp * V2 * V2 + 1.5 * m0 * e * mp * V2 + 0.5 * m0 * m0 * e * e * mp
-           + 0.5 * m0 * e * mp * (3.0 * V2 - 7.0 * v0v - dv0 * dv * e * e);
-    t[3] = mp * (0.25 * (6.0 * V2 * A[E_PHI] - 7.0 * vPhv - A[E_GAM]) + m0 * e * A[E_PHI]
-                 + 0.5 * m0 * e * (G1 - mp * e));
-}
-
-inline __global__ __launch_bounds__(WG) void k_efin(const double* __restrict__ st,
-                                            const double* __restrict__ m,
-                                            const double* __restrict__ part, int S,
-                                            const double* __restrict__ gs,
-                                            double* __restrict__ eblk, Phys P)
-{
-    const int p = blockIdx.x * WG + threadIdx.x + 1;
-    double t[NEB] = {0.0, 0.0, 0.0, 0.0};
-    if (p < P.n) {
-        double A[NACCE] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        for (int s = 0; s < S; ++s)
+    __shared__ double sh[PW][EV], tot[EV];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double t = 0.0;
+#pragma unroll 8
+    for (int k = (int)threadIdx.x / EV; k < cnt; k += PW * RB / EV)
+        t += take_over(&eb[((size_t)(k / S) * stride + k % S) * EV + (threadIdx.x & (EV - 1))]);
 #pragma unroll
-            for (int k = 0; k < NACCE; ++k) A[k] += part[(size_t)(s * NACCE + k) * P.cap + p];
-        efin_star(st, m, P.cap, p, 0, P.m0, P.eps2, A, gs[G_G1], t);
-    }
-    block_sum<NEB>(t, eblk + (size_t)blockIdx.x * NEB);
-}
-
-// out = {kin, pot, pot_pn/c^2, pot_pn2/c^2, total}
-inline __global__ __launch_bounds__(WG) void k_ered(const double* __restrict__ eblk, int nblk,
-                                            const double* __restrict__ st,
-                                            const double* __restrict__ m,
-                                            const double* __restrict__ gs,
-                                            double* __restrict__ out, Phys P)
-{
-    double s[NEB] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblk; b += WG)
+    for (int off2 = EV; off2 < 64; off2 <<= 1) t += __shfl_xor(t, off2, 64);
+    if (lane < EV) sh[wave][lane] = t;
+    __syncthreads();
+    if (threadIdx.x < EV) {
+        t = sh[0][threadIdx.x];
 #pragma unroll
-        for (int k = 0; k < NEB; ++k) s[k] += eblk[(size_t)b * NEB + k];
-    __shared__ double tot[NEB];
-    block_sum<NEB>(s, tot);
+        for (int w = 1; w < PW; ++w) t += sh[w][threadIdx.x];
+        tot[threadIdx.x] = t;
+    }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        const int cap = P.cap;
-        const double v0x = st[3 * cap], v0y = st[4 * cap], v0z = st[5 * cap];
-        const double kin = 0.5 * (m[0] * (v0x * v0x + v0y * v0y + v0z * v0z) + tot[0]);
-        const double pot = tot[1] - P.m0 * gs[G_G1];
-        const double pn = P.lam * tot[2], pn2 = P.lam * tot[3];
+        const double v0x = st[3 * cap + off], v0y = st[4 * cap + off], v0z = st[5 * cap + off];
+        const double kin = 0.5 * (m0 * (v0x * v0x + v0y * v0y + v0z * v0z) + tot[0]);
+        const double pot = tot[1] - m0 * G1;
+        const double pn = lam * tot[2], pn2 = lam * tot[3];
         out[0] = kin;
         out[1] = pot;
         out[2] = pn;
         out[3] = pn2;
         out[4] = kin + pot + pn + pn2;
     }
+}
+
+// Row and chunk of this workgroup of a grid of (rows, chunks): consecutive
+// workgroups take the chunks of one row, so that an XCD's share of the
+// resident ones reads two of a row's chunks and not all records (n = 65537:
+// 2.24 ms, 2.44 with consecutive rows).  The grid is two-dimensional because a
+// dimension holds less than 2^32 threads.
+__device__ __forceinline__ int2 energy_item()
+{
+    const unsigned k = blockIdx.y * gridDim.x + blockIdx.x;
+    return make_int2((int)(k / gridDim.y), (int)(k % gridDim.y));
+}
+
+// One workgroup per (row, chunk), the last one adds them up.  The
+// BH mass is m0, the separable sums gs as k_prep left them.
+inline __global__ __launch_bounds__(PW * RB)
+void k_energy(const JRec64* __restrict__ jr, const double* __restrict__ st,
+              const double* __restrict__ gs, double* __restrict__ eb, double* __restrict__ out,
+              unsigned int* __restrict__ ticket, Phys P)
+{
+    __shared__ double t[EV];
+    const int nrow = (int)gridDim.x, S = (int)gridDim.y;
+    const int2 w = energy_item();
+    const double G1 = gs[G_G1];
+    if (P.n > 1)
+        energy_row(jr, st, P.cap, 0, P.n - 1, nrow, w.x, w.y, S, P.m0, G1, P.eps2, t);
+    else if (threadIdx.x < EV)
+        t[threadIdx.x] = 0.0;
+    if (threadIdx.x < EV)
+        hand_over(&eb[((size_t)w.x * S + w.y) * EV + threadIdx.x], t[threadIdx.x]);
+    if (last_block(ticket, (unsigned)(nrow * S)))
+        energy_total(eb, nrow * S, S, S, st, P.cap, 0, P.m0, G1, P.lam, out);
 }
 
 }  // namespace pn1dev
