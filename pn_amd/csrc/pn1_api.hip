@@ -105,11 +105,13 @@ int auto_split(int nst)
 //   n = 2049    35/41 23.3/28.7  23.5/23.7                 27/26      37/34
 //   n = 10241         178/128    177/111      178/108      182/113    201/130
 //   n = 131073                   24850/12860  24808/12715
+// Above 2^22 stars the rows alone are over a hundred workgroups per CU, and
+// the split only bounds the partials: at most 2^26 of them (7 GB).
 int auto_slots(int nst)
 {
-    if (nst >= 8192) return TLONG + TSHORT;
+    if (nst >= 8192 && nst < (1 << 22)) return TLONG + TSHORT;
     int s = TLONG;
-    while (s > 1 && nst < 4 * s * PW) s >>= 1;
+    while (s > 1 && (nst < 4 * s * PW || (long)nst * s > (1L << 26))) s >>= 1;
     return s;
 }
 
@@ -158,6 +160,19 @@ int ensure_part(pn1_ctx* c, int slots = 0)
     c->part = p;
     c->part_bytes = need;
     return PN1_OK;
+}
+
+// Plan and partials of the current n.  Where the automatic plan's partials are
+// refused (a capacity far above n: they are laid out by capacity), the
+// 256-star kernels' split takes its place, which at large n needs fewer.
+int plan_parts(pn1_ctx* c)
+{
+    plan(c);
+    const int rc = ensure_part(c);
+    if (!rc || !c->slots) return rc;
+    c->slots = 0;
+    c->S = auto_split(c->n - 1);
+    return ensure_part(c);
 }
 
 // Kernel form in use: the requested one, or per mode the faster one
@@ -577,13 +592,12 @@ int pn1_set_tuning(pn1_ctx* c, int jsplit, int tile, int variant)
     if (!c->have_state) return PN1_OK;
     HIPCHK(c, hipSetDevice(c->dev));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    plan(c);
-    const int rc = ensure_part(c);
+    const int rc = plan_parts(c);
     if (rc) {                           // refused: the shape in use before stays
         c->jsplit_req = keep_S;
         c->tile_req = keep_tile;
         c->variant_req = keep_var;
-        plan(c);
+        (void)plan_parts(c);
     }
     return rc;
 }
@@ -643,8 +657,7 @@ int pn1_upload(pn1_ctx* c, const double* x, const double* v, const double* m, in
     c->tauf = flag_threshold(std::sqrt(dmax2));
     c->acc_ok = false;
     c->have_state = true;
-    plan(c);
-    return ensure_part(c);
+    return plan_parts(c);
 }
 
 int pn1_download(pn1_ctx* c, double* x, double* v)
@@ -851,8 +864,7 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
         c->jsplit_req = S;
         c->variant_req = S ? var : -1;
         c->tile_req = keep_tile;
-        plan(c);
-        int r = ensure_part(c);
+        int r = plan_parts(c);
         if (!r) r = enqueue_force(c, P);                         // warm-up
         if (!r && hipEventRecord(ea, c->st) != hipSuccess) r = seterr(c, PN1_EDEVICE, "hipEventRecord failed");
         for (int k = 0; k < reps && !r; ++k) r = enqueue_force(c, P);
@@ -881,15 +893,13 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
     if (rc) {                              // leave the shape the caller had
         c->jsplit_req = keep_S;
         c->variant_req = keep_var;
-        plan(c);
-        (void)ensure_part(c);
+        (void)plan_parts(c);
         return rc;
     }
     c->jsplit_req = bS;
     c->variant_req = bV;
     drop_graph(c);
-    plan(c);
-    if ((rc = ensure_part(c))) return rc;
+    if ((rc = plan_parts(c))) return rc;
     if (jsplit) *jsplit = c->S;
     if (variant) *variant = kernel_variant(c);
     if (best_ms) *best_ms = best;
