@@ -212,12 +212,13 @@ int  pn1_adjoint_backward(pn1_ctx *ctx, const double *gx, const double *gv,
 /* ====================================================================== */
 /* Cluster c is particles [offsets[c], offsets[c+1]) of the AoS arrays;
  * its first particle is its BH.  All clusters share eps, c, dt and mode.
- * One force evaluation of the ensemble is one persistent pair-kernel
- * launch: workgroups take (cluster, 256-star block, j chunk) items from
- * eight per-XCD queues (whole clusters per queue, balanced by cost;
- * largest items first; idle workgroups take from the other queues); each
- * item writes its own partial sums, so results do not depend on the order
- * items run in. */
+ * One force evaluation of the ensemble is one pair-kernel launch over
+ * (cluster, row of 64 stars, j chunk) items; with an explicit chunk or
+ * variant, and in the adjoint, a persistent launch whose workgroups take
+ * (cluster, 256-star block, j chunk) items from eight per-XCD queues (whole
+ * clusters per queue, balanced by cost; largest items first; idle workgroups
+ * take from the other queues).  Each item writes its own partial sums, so
+ * results do not depend on the order items run in. */
 typedef struct pn1_ens pn1_ens;
 
 /* Up to `capacity` particles in total (at most PN1_MAX_CAPACITY) in up to
@@ -241,15 +242,16 @@ int  pn1_ens_energy(pn1_ens *ens, double *out);
 int  pn1_ens_step(pn1_ens *ens, int steps);
 int  pn1_ens_sync(pn1_ens *ens);
 const char *pn1_ens_last_error(const pn1_ens *ens);
-/* Work-item shape: j chunk length `chunk` (records per item; 0 = chosen
- * at upload so that each persistent workgroup takes about 8 items; applies
- * from the next upload), mixed compensation interval `tile` and kernel
- * `variant` as pn1_set_tuning. */
+/* Shape of the 256-star items: j chunk length `chunk` (records per item; 0 =
+ * chosen at upload so that each persistent workgroup takes about 8 items;
+ * applies from the next upload), mixed compensation interval `tile` and kernel
+ * `variant` as pn1_set_tuning.  With chunk 0 and variant -1 the force and
+ * steps use rows of 64 stars, in chunks of their own. */
 int  pn1_ens_set_tuning(pn1_ens *ens, int chunk, int tile, int variant);
 int  pn1_ens_get_tuning(const pn1_ens *ens, int *chunk, int *tile,
                         int *variant);
 /* Autotuner of the ensemble, as pn1_autotune, over chunk lengths
- * 256 ... 1024 and the j loop variant; applies at once (the work tables
+ * 256 ... 1024, the j loop variant and the automatic plan; applies at once (the work tables
  * are rebuilt) and invalidates a pending adjoint. */
 int  pn1_ens_autotune(pn1_ens *ens, int reps, int *chunk, int *variant,
                       double *best_ms);

@@ -543,6 +543,7 @@ int ens_adj_get(pn1_ens* e, pn1_ens_adj** out)
         }
     }
     pn1_ens_adj* a = e->adj;
+    if (int rc = ens_items(e)) return rc;
     if (a->tab_L != e->L || a->tab_gen != e->gen) {   // partial layout of the clusters
         std::vector<long long> aoff(e->nc > 0 ? e->nc : 1, 0);
         size_t tot = 0;
@@ -652,7 +653,7 @@ extern "C" {
 int pn1_ens_force_vjp(pn1_ens* e, const double* u, double* gx, double* gv, double* gm0)
 {
     int rc;
-    if (!ens_ready(e, &rc)) return rc;
+    if (!ens_force_ready(e, &rc)) return rc;
     if (!u || !gx || !gv) return eerr(e, PN1_EINVAL, "null argument");
     pn1_ens_adj* a;
     if ((rc = ens_adj_get(e, &a))) return rc;
@@ -670,7 +671,7 @@ int pn1_ens_force_vjp(pn1_ens* e, const double* u, double* gx, double* gv, doubl
 int pn1_ens_adjoint_forward(pn1_ens* e, int steps, int interval)
 {
     int rc;
-    if (!ens_ready(e, &rc)) return rc;
+    if (!ens_force_ready(e, &rc)) return rc;
     if (steps < 1 || interval < 1)
         return eerr(e, PN1_EINVAL, "steps (%d) and interval (%d) must be >= 1", steps, interval);
     pn1_ens_adj* a;
@@ -714,7 +715,7 @@ int pn1_ens_adjoint_backward(pn1_ens* e, const double* gx, const double* gv, dou
                              double* gv0, double* gm0)
 {
     int rc;
-    if (!ens_ready(e, &rc)) return rc;
+    if (!ens_force_ready(e, &rc)) return rc;
     if (!gx || !gv || !gx0 || !gv0) return eerr(e, PN1_EINVAL, "null argument");
     pn1_ens_adj* a = e->adj;
     if (!a || !a->have_fwd)

@@ -8,9 +8,13 @@
 //   cmmax[nc]      largest star mass of each cluster
 //   row[nrow], crow[nc + 1]   64-star rows of the O(n) kernels, per
 //                  cluster; pblk[npblk]: groups of FG of them
-//   items[nitems]  pair work items in 8 per-XCD queues (qoff[9]): whole
+//   parts[nparts]  the automatic plan's pair work items (row, chunk), filled
+//                  on the device from place[nc]
+//   items[nitems]  the 256-star items of an explicit chunk or variant and of
+//                  the adjoint, in 8 per-XCD queues (qoff[9]): whole
 //                  clusters go to the least-loaded queue, largest first;
-//                  each queue is sorted by decreasing pair count
+//                  each queue is sorted by decreasing pair count; built when
+//                  first needed
 //   poff[nc]       first partial-sum slot of each cluster
 #pragma once
 #include <hip/hip_runtime.h>
@@ -61,6 +65,13 @@ struct pn1_ens {
     long long* poff = nullptr;
     unsigned int* counter = nullptr;
     int nitems = 0, items_cap = 0;
+    bool have_items = false;      // items, qoff are those of this state and L
+    pn1dev::EPart* parts = nullptr;
+    pn1dev::EPlace* place = nullptr;
+    int nparts = 0, parts_cap = 0;
+    bool autoplan = true;         // no explicit chunk at the last upload
+    bool tab_auto = false;        // the tables are the automatic plan's
+    int Lf = 512;                 // the force's chunk: L, or the plan's own
     int echunks = 1;                // largest energy_chunks of a cluster
     long long slots = 0;
     void* part = nullptr;
@@ -89,6 +100,10 @@ int ens_enqueue_eval(pn1_ens* e, int stage, const pn1dev::Phys& P);
 int ens_ensure_prev_acc(pn1_ens* e, const pn1dev::Phys& P);
 int ens_fetch3(pn1_ens* e, const double* dsrc, double* out);
 bool ens_ready(pn1_ens* e, int* rc);
+// ens_ready, and the tables are those of the force's present plan.
+bool ens_force_ready(pn1_ens* e, int* rc);
+// items and qoff for the present state and L, if they are not there.
+int ens_items(pn1_ens* e);
 void edrop_graph(pn1_ens* e);
 void ens_adj_free(pn1_ens* e);   // pn1_adj.hip
 

@@ -8,7 +8,10 @@
 //   k_ens_prep   per-star j-records and the clusters' separable sums;
 //                workgroups come from a table, each inside one cluster, and
 //                a cluster's last one adds its sums (a ticket per cluster)
-//   k_ens_pair*  ONE persistent launch for all clusters: workgroups take
+//   k_ens_pair*w one launch for all clusters, a workgroup of PW waves per
+//                (cluster, row of 64 stars, j chunk) of the automatic plan
+//   k_ens_pair*  with an explicit chunk length or kernel variant: one
+//                persistent launch for all clusters: workgroups take
 //                (cluster, 256-star i-block, j-chunk) items from per-XCD
 //                queues (atomic counters), items sorted by decreasing cost
 //                on the host; every item writes its partial sums to its own
@@ -178,6 +181,93 @@ void k_ens_pair32x(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64
                    const double* __restrict__ cmmax, Phys P, int tile)
 {
     ens_pair32<PP, TS, EQ>(jr, j64, thr, st, part, items, counter, qoff, cmmax, P, tile);
+}
+
+// ---------------------------------------------------------------------
+// the automatic plan: k_pair64w and k_pair32w over a table of (cluster, row,
+// chunk)
+// ---------------------------------------------------------------------
+// Item k of queue q is workgroup sum_q' min(k, len q') + (queues before q with
+// more than k items): the queues side by side, so that workgroup b, which the
+// dispatcher gives to XCD b % 8, takes an item of queue b % 8 until the
+// shortest queue ends.  A queue holds whole clusters, those with the longest
+// parts first.  A workgroup per cluster.
+inline __global__ __launch_bounds__(WG) void k_ens_parts(const EPlace* __restrict__ place,
+                                                        const int* __restrict__ crow, QLen len,
+                                                        EPart* __restrict__ parts)
+{
+    const int c = blockIdx.x;
+    const EPlace w = place[c];
+    const int cnt = (crow[c + 1] - crow[c]) * w.S;       // S = 0: no star
+    for (int t = threadIdx.x; t < cnt; t += WG) {
+        const int k = w.k0 + t;
+        int b = 0;
+#pragma unroll
+        for (int q = 0; q < NXCD; ++q) b += min(k, len.n[q]) + (q < w.q && len.n[q] > k ? 1 : 0);
+        parts[b] = EPart{c, t / w.S, t % w.S, w.S};
+    }
+}
+
+// The item's cluster (BH at off, nst stars), its lane's star li (particle i,
+// clamped) and wave's records R.
+struct EWave {
+    int off, nst, li, i;
+    JRange R;
+};
+
+__device__ __forceinline__ EWave ens_wave(const EPart& w, const int* __restrict__ coff, int wave,
+                                          int lane)
+{
+    EWave g;
+    g.off = coff[w.c];
+    g.nst = coff[w.c + 1] - g.off - 1;
+    g.li = w.ig * RB + lane;
+    g.i = g.off + 1 + min(g.li, g.nst - 1);
+    const int len = (g.nst + w.S * PW - 1) / (w.S * PW), j0 = g.off + 1;
+    g.R.j0 = j0 + min(g.nst, (w.s * PW + wave) * len);
+    g.R.j1 = j0 + min(g.nst, (w.s * PW + wave + 1) * len);
+    g.R.w0 = max(g.R.j0, j0 + w.ig * RB);
+    g.R.w1 = min(g.R.j1, j0 + w.ig * RB + RB);
+    return g;
+}
+
+inline __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(7, 8)))
+void k_ens_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
+                   double* __restrict__ part, const EPart* __restrict__ parts,
+                   const int* __restrict__ coff, const long long* __restrict__ poff, Phys P)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const EPart w = parts[blockIdx.x];
+    const EWave g = ens_wave(w, coff, wave, lane);
+    const I64 I = load_i64(jr, st, P.cap, g.i, P.eps2);
+    double a[NACC];
+    part64(jr, g.R, g.i, I, a, P.eps2);
+    waves_total(a, wave, lane);
+    if (wave == 0 && g.li < g.nst) {
+        double* pp = part + (poff[w.c] + (long long)w.s * g.nst) * NACC + g.li;
+#pragma unroll
+        for (int k = 0; k < NACC; ++k) stream_out(a[k], &pp[(size_t)k * g.nst]);
+    }
+}
+
+template <bool TS, bool EQ>
+__global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void k_ens_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
+                   const Thr* __restrict__ thr, const double* __restrict__ st,
+                   float* __restrict__ part, const EPart* __restrict__ parts,
+                   const int* __restrict__ coff, const long long* __restrict__ poff,
+                   const double* __restrict__ cmmax, Phys P, int tile)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const EPart w = parts[blockIdx.x];
+    const EWave g = ens_wave(w, coff, wave, lane);
+    const I32 I = load_i32(j64, thr, st, P.cap, g.i, g.off, P.eps2);
+    float a[NACC32], sumN[3], cmpN[3];
+    part32<TS, EQ>(jr, j64, g.R, g.i, I, P.eps2f, P.eps2, 1.0 / cmmax[w.c], tile, a, sumN, cmpN);
+    put_part32<TS>(a, sumN, cmpN, wave, lane, g.li < g.nst,
+                   part + (poff[w.c] + (long long)w.s * g.nst) * MROWS + g.li, (size_t)g.nst);
 }
 
 // Per-cluster buffers.  Cluster c's rows of 64 stars are [crow[c],

@@ -18,6 +18,18 @@ struct __align__(32) EItem {
     long long pslot;
 };
 
+// A pair work item of the automatic plan: row ig of 64 stars of cluster c
+// against chunk s of its S chunks.
+struct __align__(16) EPart {
+    int c, ig, s, S;
+};
+
+// Where cluster c's items of the automatic plan go: queue q, from its
+// position k0 on, S chunks per row.
+struct __align__(16) EPlace {
+    int q, k0, S, pad;
+};
+
 // Row (or group of rows) of the O(n) kernels: cluster and first local star.
 // Partial sums of cluster c start at slot poff[c] (a slot is one chunk of
 // one star; slots of c: nchunks(c) x its star count) times the number of
@@ -38,6 +50,11 @@ __device__ __forceinline__ int ens_nchunks(int nst, int L) { return (nst + L - 1
 // workgroup work on one item, so they read the same j-record stream
 // (through the scalar cache) in step.
 constexpr int NXCD = 8;
+
+// Items of each queue.
+struct QLen {
+    int n[NXCD];
+};
 
 // The next work item for this workgroup, identical in every lane (and
 // known to the compiler as uniform); -1 when every queue is empty.  `k`

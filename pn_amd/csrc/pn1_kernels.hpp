@@ -567,6 +567,21 @@ __device__ __forceinline__ void waves_total(double (&v)[N], int wave, int lane)
     }
 }
 
+// A wave's sums a for star i over records [R.j0, R.j1).
+__device__ __forceinline__ void part64(const JRec64* __restrict__ jr, const JRange& R, int i,
+                                       const I64& I, double (&a)[NACC], double eps2)
+{
+#pragma unroll
+    for (int k = 0; k < NACC; ++k) a[k] = 0.0;
+    if (R.w0 < R.w1) {
+        run64<false, 0>(jr, R.j0, R.w0, i, I, a, eps2);
+        run64<true, 0>(jr, R.w0, R.w1, i, I, a, eps2);
+        run64<false, 0>(jr, R.w1, R.j1, i, I, a, eps2);
+    } else {
+        run64<false, 0>(jr, R.j0, R.j1, i, I, a, eps2);
+    }
+}
+
 // Held to k_pair64's 7 waves per SIMD (72 VGPRs; 80 otherwise).
 inline __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(7, 8)))
 void k_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
@@ -578,17 +593,8 @@ void k_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
     const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
     const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
     const I64 I = load_i64(jr, st, P.cap, i, P.eps2);
-    const double eps2 = P.eps2;
     double a[NACC];
-#pragma unroll
-    for (int k = 0; k < NACC; ++k) a[k] = 0.0;
-    if (R.w0 < R.w1) {
-        run64<false, 0>(jr, R.j0, R.w0, i, I, a, eps2);
-        run64<true, 0>(jr, R.w0, R.w1, i, I, a, eps2);
-        run64<false, 0>(jr, R.w1, R.j1, i, I, a, eps2);
-    } else {
-        run64<false, 0>(jr, R.j0, R.j1, i, I, a, eps2);
-    }
+    part64(jr, R, i, I, a, P.eps2);
     waves_total(a, wave, lane);
     if (wave == 0 && li < n) {
 #pragma unroll
@@ -1006,25 +1012,15 @@ void k_pair32q(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
     }
 }
 
-// k_pair64w's form of the mixed kernel.  The waves' sums are added in FP64:
-// the Newtonian totals s - c are written as a hi/lo float pair (s = hi,
-// c = -lo, so that k_fin's s - c is the FP64 total to ~2^-48), the other sums
-// rounded once to FP32.
+// A wave's sums for star i over records [R.j0, R.j1): a, and the Newtonian
+// ones as sumN - cmpN (rscale: 1 / the records' mass scale).
 template <bool TS, bool EQ>
-__global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
-void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
-               const Thr* __restrict__ thr, const double* __restrict__ st,
-               float* __restrict__ part, Phys P, int S, int nrow, int tile)
+__device__ __forceinline__ void part32(const JRec32* __restrict__ jr,
+                                       const JRec64* __restrict__ j64, const JRange R, int i,
+                                       const I32& I, float eps2, double eps2d, double rscale,
+                                       int tile, float (&a)[NACC32], float (&sumN)[3],
+                                       float (&cmpN)[3])
 {
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63;
-    int s, ig;
-    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
-    const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
-    const I32 I = load_i32(j64, thr, st, P.cap, i, 0, P.eps2);
-    const float eps2 = P.eps2f;
-    const double eps2d = P.eps2, rscale = 1.0 / P.mmax;
-    float a[NACC32], sumN[3], cmpN[3];
 #pragma unroll
     for (int k = 0; k < NACC32; ++k) a[k] = 0.0f;
 #pragma unroll
@@ -1038,22 +1034,50 @@ void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
         run32<false, 0, TS, EQ>(jr, j64, R.j0, R.j1, i, I, a, eps2, eps2d, rscale, sumN, cmpN, tile, cnt);
     }
     fold_newton(a, sumN, cmpN);
+}
+
+// The sums of the workgroup's waves, added in FP64, as partials (rows of
+// `stride` floats from ps): the Newtonian totals as a hi/lo float pair (s = hi,
+// c = -lo, so that k_fin's s - c is the FP64 total to ~2^-48), the others
+// rounded once to FP32.  ok: the lane has a star.
+template <bool TS>
+__device__ __forceinline__ void put_part32(const float (&a)[NACC32], const float (&sumN)[3],
+                                           const float (&cmpN)[3], int wave, int lane, bool ok,
+                                           float* __restrict__ ps, size_t stride)
+{
     constexpr int NV = TS ? NACC32 : NACC;
     double v[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k)
         v[k] = k <= A_NZ ? (double)sumN[k] - (double)cmpN[k] : (double)a[k];
     waves_total(v, wave, lane);
-    if (wave == 0 && li < n) {
-        const size_t cap = (size_t)P.cap;
-        float* ps = part + (size_t)s * MROWS * cap + li;
+    if (wave == 0 && ok) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             const float hi = (float)v[k];
-            stream_out(hi, &ps[k * cap]);
-            if (k <= A_NZ) stream_out(-(float)(v[k] - (double)hi), &ps[(NACC32 + k) * cap]);
+            stream_out(hi, &ps[k * stride]);
+            if (k <= A_NZ) stream_out(-(float)(v[k] - (double)hi), &ps[(NACC32 + k) * stride]);
         }
     }
+}
+
+// k_pair64w's form of the mixed kernel.
+template <bool TS, bool EQ>
+__global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
+void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
+               const Thr* __restrict__ thr, const double* __restrict__ st,
+               float* __restrict__ part, Phys P, int S, int nrow, int tile)
+{
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    int s, ig;
+    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
+    const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
+    const I32 I = load_i32(j64, thr, st, P.cap, i, 0, P.eps2);
+    float a[NACC32], sumN[3], cmpN[3];
+    part32<TS, EQ>(jr, j64, R, i, I, P.eps2f, P.eps2, 1.0 / P.mmax, tile, a, sumN, cmpN);
+    put_part32<TS>(a, sumN, cmpN, wave, lane, li < n, part + (size_t)s * MROWS * P.cap + li,
+                   (size_t)P.cap);
 }
 
 // ---------------------------------------------------------------------

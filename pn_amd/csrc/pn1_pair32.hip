@@ -59,6 +59,14 @@ void ens_launch32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P
                            P, e->tile);
 }
 
+template <bool TS, bool EQ>
+void ens_launch32w(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P)
+{
+    hipLaunchKernelGGL((k_ens_pair32w<TS, EQ>), dim3(e->nparts), dim3(PW * RB), 0, e->st, e->j32,
+                       j64, e->thr, in, (float*)e->part, e->parts, e->coff, e->poff, e->cmmax, P,
+                       e->tile);
+}
+
 using EnsLaunch32 = void (*)(pn1_ens*, const JRec64*, const double*, const Phys&, dim3);
 const EnsLaunch32 k_ens_launch32[16] = {
     ens_launch32<0, false, false>, ens_launch32<0, false, true>, ens_launch32<0, true, false>,
@@ -89,6 +97,14 @@ void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Ph
                        int form)
 {
     k_ens_launch32[form & 15](e, j64, in, P, g);
+}
+
+void launch_ens_pair32w(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, bool ts)
+{
+    if (ts)
+        (e->eqm ? ens_launch32w<true, true> : ens_launch32w<true, false>)(e, j64, in, P);
+    else
+        (e->eqm ? ens_launch32w<false, true> : ens_launch32w<false, false>)(e, j64, in, P);
 }
 
 hipError_t ens_pair32_occupancy(int var, int* per_cu)

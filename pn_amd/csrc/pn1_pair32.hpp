@@ -28,6 +28,9 @@ void launch_pair32w(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
 // Ensemble: one persistent launch of grid g over the work queues.
 void launch_ens_pair32(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
                        const pn1dev::Phys& P, dim3 g, int form);
+// Its automatic plan's form.
+void launch_ens_pair32w(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
+                        const pn1dev::Phys& P, bool ts);
 // Resident workgroups per CU of the ensemble kernel of loop variant var
 // (0..3), in its form with the cancellation sums (the one with the most
 // registers).

@@ -30,3 +30,55 @@ def test_automatic_plan_against_explicit_split(stars, mode, bound):
         ctx.set_tuning(16, 0, -1)
         b = ctx.force()
     assert (np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)).max() <= bound
+
+
+@pytest.mark.parametrize("mode,bound", [(pn.FP64, 1e-12), (pn.MIXED, 2e-6)])
+def test_ensemble_plan_against_items(mode, bound):
+    """The ensemble's automatic plan (rows of 64 stars) against its 256-star
+    items: an explicit chunk, and a variant set and taken back after the upload,
+    which changes the tables under a captured step.  Sizes at the edges of rows,
+    chunks and parts, and a cluster without stars."""
+    sizes = [1, 63, 64, 65, 255, 256, 257, 511, 513, 1025, 4097]
+    cl = []
+    for k in sizes:
+        x, v, m = cluster(k, 500 + k)
+        x[1:] += (0.5, 0.25, -0.125)          # one star alone is at the BH's place
+        cl.append((x, v, m))
+    cl.insert(3, (np.zeros((1, 3)), np.ones((1, 3)), np.array([2.0])))
+    n = sum(len(m) for _, _, m in cl)
+
+    def worst(a, b):
+        return max((np.linalg.norm(p - q, axis=1) / np.maximum(np.linalg.norm(q, axis=1), 1e-300)).max()
+                   for p, q in zip(a, b))
+
+    with pn.Ensemble(n, len(cl)) as ens:
+        ens.set_params(1e-2, 50.0, 2.0**-10, mode)
+        ens.upload(cl)
+        a = ens.force()
+        ens.step(2)
+        x0, v0 = ens.download()
+        ens.set_tuning(0, 0, 0)               # 256-star items from here on
+        ens.upload(cl)
+        b = ens.force()
+        ens.set_tuning(0, 0, -1)
+        a2 = ens.force()
+        ens.set_tuning(0, 0, 1)
+        b2 = ens.force()
+        ens.set_tuning(0, 0, -1)
+        ens.upload(cl)
+        assert all(np.array_equal(p, q) for p, q in zip(ens.force(), a))
+        ens.step(1)
+        ens.set_tuning(0, 0, 0)
+        ens.force()
+        ens.set_tuning(0, 0, -1)
+        ens.step(1)
+        x1, v1 = ens.download()
+        ens.set_tuning(128, 0, -1)
+        ens.upload(cl)
+        d = ens.force()
+    for other in (b, a2, b2, d):
+        assert worst(other, a) <= bound
+    # FP64: the same step from the same state; mixed: its first evaluation's
+    # pair thresholds come from another evaluation of the same accuracy
+    for p, q in zip(x0 + v0, x1 + v1):
+        assert np.abs(p - q).max() <= (1e-12 if mode == pn.FP64 else 1e-6) * max(1.0, np.abs(q).max())
