@@ -170,38 +170,30 @@ int enqueue_vjp(pn1_ctx* c, pn1_adj* a, const double* y, const AdjLin& l, const 
     return PN1_OK;
 }
 
-// AoS host [n][3] pair (x part, v part) -> SoA device 6 x cap.
-int put6(pn1_ctx* c, const double* hx, const double* hv, double* dst)
-{
-    const size_t cap = (size_t)c->cap;
-    double* h = c->h_stage;
-    for (int i = 0; i < c->n; ++i)
-        for (int k = 0; k < 3; ++k) {
-            h[k * cap + i] = hx ? hx[3 * i + k] : 0.0;
-            h[(3 + k) * cap + i] = hv ? hv[3 * i + k] : 0.0;
-        }
-    for (int k = 0; k < 6; ++k)
-        HIPCHK(c, hipMemcpyAsync(dst + k * cap, h + k * cap, c->n * sizeof(double),
-                                 hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    return PN1_OK;
-}
-
-int copy6(pn1_ctx* c, double* dst, const double* src)
-{
-    const size_t cap = (size_t)c->cap;
-    for (int k = 0; k < 6; ++k)
-        HIPCHK(c, hipMemcpyAsync(dst + k * cap, src + k * cap, c->n * sizeof(double),
-                                 hipMemcpyDeviceToDevice, c->st));
-    return PN1_OK;
-}
-
 // The adjoint runs the FP64 kernels whatever the context's mode.
 struct Fp64Scope {
     pn1_ctx* c;
     int mode;
     explicit Fp64Scope(pn1_ctx* cc) : c(cc), mode(cc->mode) { c->mode = PN1_FP64; }
     ~Fp64Scope() { c->mode = mode; }
+};
+
+// Stages 1 and 2 of a step written to Y1 and Y2 (6 x cap each) instead of the
+// stage states H1 and H2.
+template <class C>
+struct StageScope {
+    C* c;
+    double *h1, *h2;
+    StageScope(C* cc, double* Y1, double* Y2) : c(cc), h1(cc->H1), h2(cc->H2)
+    {
+        c->H1 = Y1;
+        c->H2 = Y2;
+    }
+    ~StageScope()
+    {
+        c->H1 = h1;
+        c->H2 = h2;
+    }
 };
 
 // The first `last` evaluations of a step, the first of them prepared.
@@ -226,18 +218,12 @@ int pn1_force_vjp(pn1_ctx* c, const double* u, double* gx, double* gv, double* g
     pn1_adj* a;
     if ((rc = adj_get(c, &a))) return rc;
     const Phys P = make_phys(c);
-    if ((rc = put6(c, nullptr, u, a->L))) return rc;
-    HIPCHK(c, hipMemsetAsync(a->gm0, 0, 2 * sizeof(double), c->st));
+    if ((rc = put6(c, nullptr, u, a->L, a->gm0, 2))) return rc;
     const AdjLin mu = {a->L, nullptr, 1.0, 0.0};
     if ((rc = enqueue_vjp(c, a, c->X, mu, AdjAdd{}, a->out, P))) return rc;
-    const size_t cap = (size_t)c->cap;
-    if ((rc = fetch3(c, a->out, gx))) return rc;
-    if ((rc = fetch3(c, a->out + 3 * cap, gv))) return rc;
-    if (gm0) {
-        double h[2];
-        HIPCHK(c, hipMemcpy(h, a->gm0, sizeof h, hipMemcpyDeviceToHost));
-        *gm0 = h[1];
-    }
+    double h[2];
+    if ((rc = fetch(c, a->out, c->n, gx, gv, a->gm0, 2, h))) return rc;
+    if (gm0) *gm0 = h[1];
     return PN1_OK;
 }
 
@@ -274,8 +260,8 @@ int pn1_adjoint_forward(pn1_ctx* c, int steps, int interval)
     const Phys P = make_phys(c);
     if ((rc = enqueue_prep(c, P))) return rc;
     for (int t = 0; t < steps; ++t) {
-        if (t % interval == 0 && (rc = copy6(c, a->ckpt + (size_t)(t / interval) * s6, c->X)))
-            return rc;
+        if (t % interval == 0)
+            HIPCHK(c, copy6(c->st, a->ckpt + (size_t)(t / interval) * s6, c->X, c->n, c->cap));
         if ((rc = enqueue_stages(c, 3, P))) return rc;
     }
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -301,21 +287,19 @@ int pn1_adjoint_backward(pn1_ctx* c, const double* gx, const double* gv, double*
     const Phys P = make_phys(c);
     const double dt = c->dt;
     const size_t s6 = 6 * (size_t)c->cap;
-    if ((rc = put6(c, gx, gv, a->L))) return rc;
-    HIPCHK(c, hipMemsetAsync(a->gm0, 0, 2 * sizeof(double), c->st));
+    if ((rc = put6(c, gx, gv, a->L, a->gm0, 2))) return rc;
     const int nck = (a->steps + a->interval - 1) / a->interval;
     for (int k = nck - 1; k >= 0; --k) {
         const int t0 = k * a->interval, t1 = std::min(a->steps, t0 + a->interval);
         // the segment's states: per step s, Y1 = H1 and Y2 = H2 (the last
         // step runs two stages only: its end state is not needed)
-        if ((rc = copy6(c, c->X, a->ckpt + (size_t)k * s6))) return rc;
+        HIPCHK(c, copy6(c->st, c->X, a->ckpt + (size_t)k * s6, c->n, c->cap));
         if ((rc = enqueue_prep(c, P))) return rc;
         for (int t = t0; t < t1; ++t) {
             double* st = a->seg + 3 * (size_t)(t - t0) * s6;
-            if ((rc = copy6(c, st, c->X))) return rc;
+            HIPCHK(c, copy6(c->st, st, c->X, c->n, c->cap));
+            const StageScope<pn1_ctx> keep(c, st + s6, st + 2 * s6);
             if ((rc = enqueue_stages(c, t + 1 < t1 ? 3 : 2, P))) return rc;
-            if ((rc = copy6(c, st + s6, c->H1))) return rc;
-            if ((rc = copy6(c, st + 2 * s6, c->H2))) return rc;
         }
         for (int t = t1 - 1; t >= t0; --t) {
             const double* st = a->seg + 3 * (size_t)(t - t0) * s6;
@@ -328,16 +312,10 @@ int pn1_adjoint_backward(pn1_ctx* c, const double* gx, const double* gv, double*
             if ((rc = enqueue_vjp(c, a, st, m0, sum, a->L, P))) return rc;
         }
     }
-    if ((rc = copy6(c, c->X, a->ckpt))) return rc;          // leave the initial state
-    HIPCHK(c, hipGetLastError());
-    const size_t cap = (size_t)c->cap;
-    if ((rc = fetch3(c, a->L, gx0))) return rc;
-    if ((rc = fetch3(c, a->L + 3 * cap, gv0))) return rc;
-    if (gm0) {
-        double h[2];
-        HIPCHK(c, hipMemcpy(h, a->gm0, sizeof h, hipMemcpyDeviceToHost));
-        *gm0 = h[0];
-    }
+    HIPCHK(c, copy6(c->st, c->X, a->ckpt, c->n, c->cap));    // leave the initial state
+    double h[2];
+    if ((rc = fetch(c, a->L, c->n, gx0, gv0, a->gm0, 2, h))) return rc;
+    if (gm0) *gm0 = h[0];
     return PN1_OK;
 }
 
@@ -595,38 +573,14 @@ int ens_enqueue_vjp(pn1_ens* e, pn1_ens_adj* a, const double* y, const AdjLin& l
     return PN1_OK;
 }
 
-int ens_put6(pn1_ens* e, const double* hx, const double* hv, double* dst)
-{
-    const size_t cap = (size_t)e->cap;
-    double* h = e->h_stage;
-    for (int i = 0; i < e->n; ++i)
-        for (int k = 0; k < 3; ++k) {
-            h[k * cap + i] = hx ? hx[3 * i + k] : 0.0;
-            h[(3 + k) * cap + i] = hv ? hv[3 * i + k] : 0.0;
-        }
-    for (int k = 0; k < 6; ++k)
-        EHIPCHK(e, hipMemcpyAsync(dst + k * cap, h + k * cap, e->n * sizeof(double),
-                                  hipMemcpyHostToDevice, e->st));
-    EHIPCHK(e, hipStreamSynchronize(e->st));
-    return PN1_OK;
-}
-
-int ens_copy6(pn1_ens* e, double* dst, const double* src)
-{
-    const size_t cap = (size_t)e->cap;
-    for (int k = 0; k < 6; ++k)
-        EHIPCHK(e, hipMemcpyAsync(dst + k * cap, src + k * cap, e->n * sizeof(double),
-                                  hipMemcpyDeviceToDevice, e->st));
-    return PN1_OK;
-}
-
-int ens_get_gm0(pn1_ens* e, pn1_ens_adj* a, int which, double* gm0)
+// Fetches src (6 x cap) to ox, ov and value `which` of each cluster's gm0 pair.
+int ens_get(pn1_ens* e, pn1_ens_adj* a, const double* src, double* ox, double* ov, int which,
+            double* gm0)
 {
     std::vector<double> h(2 * (size_t)e->nc);
-    EHIPCHK(e, hipMemcpyAsync(h.data(), a->gm0, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                              e->st));
-    EHIPCHK(e, hipStreamSynchronize(e->st));
-    for (int c = 0; c < e->nc; ++c) gm0[c] = h[2 * (size_t)c + which];
+    const int rc = ens_fetch(e, src, ox, ov, a->gm0, h.size(), h.data());
+    if (rc) return rc;
+    for (int c = 0; gm0 && c < e->nc; ++c) gm0[c] = h[2 * (size_t)c + which];
     return PN1_OK;
 }
 
@@ -658,14 +612,10 @@ int pn1_ens_force_vjp(pn1_ens* e, const double* u, double* gx, double* gv, doubl
     pn1_ens_adj* a;
     if ((rc = ens_adj_get(e, &a))) return rc;
     const Phys P = ens_phys(e);
-    if ((rc = ens_put6(e, nullptr, u, a->L))) return rc;
-    EHIPCHK(e, hipMemsetAsync(a->gm0, 0, 2 * (size_t)e->nc * sizeof(double), e->st));
+    if ((rc = ens_put6(e, nullptr, u, a->L, a->gm0, 2 * (size_t)e->nc))) return rc;
     const AdjLin mu = {a->L, nullptr, 1.0, 0.0};
     if ((rc = ens_enqueue_vjp(e, a, e->X, mu, AdjAdd{}, a->out, P))) return rc;
-    const size_t cap = (size_t)e->cap;
-    if ((rc = ens_fetch3(e, a->out, gx))) return rc;
-    if ((rc = ens_fetch3(e, a->out + 3 * cap, gv))) return rc;
-    return gm0 ? ens_get_gm0(e, a, 1, gm0) : PN1_OK;
+    return ens_get(e, a, a->out, gx, gv, 1, gm0);
 }
 
 int pn1_ens_adjoint_forward(pn1_ens* e, int steps, int interval)
@@ -699,8 +649,8 @@ int pn1_ens_adjoint_forward(pn1_ens* e, int steps, int interval)
     const Phys P = ens_phys(e);
     if ((rc = ens_enqueue_prep(e, P))) return rc;
     for (int t = 0; t < steps; ++t) {
-        if (t % interval == 0 && (rc = ens_copy6(e, a->ckpt + (size_t)(t / interval) * s6, e->X)))
-            return rc;
+        if (t % interval == 0)
+            EHIPCHK(e, copy6(e->st, a->ckpt + (size_t)(t / interval) * s6, e->X, e->n, e->cap));
         if ((rc = ens_stages(e, 3, P))) return rc;
     }
     EHIPCHK(e, hipStreamSynchronize(e->st));
@@ -728,19 +678,17 @@ int pn1_ens_adjoint_backward(pn1_ens* e, const double* gx, const double* gv, dou
     const Phys P = ens_phys(e);
     const double dt = e->dt;
     const size_t s6 = 6 * (size_t)e->cap;
-    if ((rc = ens_put6(e, gx, gv, a->L))) return rc;
-    EHIPCHK(e, hipMemsetAsync(a->gm0, 0, 2 * (size_t)e->nc * sizeof(double), e->st));
+    if ((rc = ens_put6(e, gx, gv, a->L, a->gm0, 2 * (size_t)e->nc))) return rc;
     const int nck = (a->steps + a->interval - 1) / a->interval;
     for (int k = nck - 1; k >= 0; --k) {
         const int t0 = k * a->interval, t1 = std::min(a->steps, t0 + a->interval);
-        if ((rc = ens_copy6(e, e->X, a->ckpt + (size_t)k * s6))) return rc;
+        EHIPCHK(e, copy6(e->st, e->X, a->ckpt + (size_t)k * s6, e->n, e->cap));
         if ((rc = ens_enqueue_prep(e, P))) return rc;
         for (int t = t0; t < t1; ++t) {
             double* st = a->seg + 3 * (size_t)(t - t0) * s6;
-            if ((rc = ens_copy6(e, st, e->X))) return rc;
+            EHIPCHK(e, copy6(e->st, st, e->X, e->n, e->cap));
+            const StageScope<pn1_ens> keep(e, st + s6, st + 2 * s6);
             if ((rc = ens_stages(e, t + 1 < t1 ? 3 : 2, P))) return rc;
-            if ((rc = ens_copy6(e, st + s6, e->H1))) return rc;
-            if ((rc = ens_copy6(e, st + 2 * s6, e->H2))) return rc;
         }
         for (int t = t1 - 1; t >= t0; --t) {
             const double* st = a->seg + 3 * (size_t)(t - t0) * s6;
@@ -753,12 +701,8 @@ int pn1_ens_adjoint_backward(pn1_ens* e, const double* gx, const double* gv, dou
             if ((rc = ens_enqueue_vjp(e, a, st, m0, sum, a->L, P))) return rc;
         }
     }
-    if ((rc = ens_copy6(e, e->X, a->ckpt))) return rc;      // leave the initial state
-    EHIPCHK(e, hipGetLastError());
-    const size_t cap = (size_t)e->cap;
-    if ((rc = ens_fetch3(e, a->L, gx0))) return rc;
-    if ((rc = ens_fetch3(e, a->L + 3 * cap, gv0))) return rc;
-    return gm0 ? ens_get_gm0(e, a, 0, gm0) : PN1_OK;
+    EHIPCHK(e, copy6(e->st, e->X, a->ckpt, e->n, e->cap));  // leave the initial state
+    return ens_get(e, a, a->L, gx0, gv0, 0, gm0);
 }
 
 }  // extern "C"

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -31,6 +32,7 @@
 #include "pn1_ctx.hpp"
 #include "pn1_ens.hpp"
 #include "pn1_ens_kernels.hpp"
+#include "pn1_io.hpp"
 #include "pn1_kernels.hpp"
 #include "pn1_pair32.hpp"
 
@@ -394,17 +396,95 @@ int enqueue_step(pn1_ctx* c, const Phys& P)
     return PN1_OK;
 }
 
-// SoA device [k][cap] -> AoS host [n][3] for k in 0..2, through the stage.
-int fetch3(pn1_ctx* c, const double* dsrc, double* out)
+// ---- between AoS host arrays and SoA device buffers -----------------------
+// The finite test adds the exponent's lowest bit to the magnitude's bits,
+// which reaches the sign bit for infinities and NaN alone.
+static uint64_t copy_finite(const double* a, size_t n, double* out)
 {
-    const size_t cap = (size_t)c->cap;
-    for (int k = 0; k < 3; ++k)
-        HIPCHK(c, hipMemcpyAsync(c->h_stage + k * cap, dsrc + k * cap, c->n * sizeof(double),
-                                 hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    for (int i = 0; i < c->n; ++i)
-        for (int k = 0; k < 3; ++k) out[3 * i + k] = c->h_stage[k * cap + i];
+    uint64_t bad = 0;
+    for (size_t k = 0; k < n; ++k) {
+        uint64_t b;
+        std::memcpy(&b, a + k, sizeof b);
+        bad |= (b & 0x7fffffffffffffffull) + 0x0010000000000000ull;
+        std::memcpy(out + k, &b, sizeof b);
+    }
+    return bad >> 63;
+}
+
+bool stage_cluster(const double* x, const double* v, const double* m, int n, double* sx,
+                   double* sv, double* sm, StarScan* scan)
+{
+    uint64_t bad = copy_finite(x, 3 * (size_t)n, sx);
+    bad |= copy_finite(v, 3 * (size_t)n, sv);
+    bad |= copy_finite(m, (size_t)n, sm);
+    double mmax = 0.0, dmax2 = 0.0, dmin2 = HUGE_VAL;
+    bool differ = false;
+    for (int i = 1; i < n; ++i) {
+        double d2 = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            const double d = x[3 * (size_t)i + k] - x[k];
+            d2 += d * d;
+        }
+        dmax2 = d2 > dmax2 ? d2 : dmax2;
+        dmin2 = d2 < dmin2 ? d2 : dmin2;
+        const double a = std::fabs(m[i]);
+        mmax = a > mmax ? a : mmax;
+        differ |= m[i] != m[1];
+    }
+    scan->mmax = mmax;
+    scan->dmax2 = dmax2;
+    scan->eqm = n < 2 || (!differ && m[1] > 0.0);
+    return !bad && m[0] > 0.0 && (n < 2 || dmin2 > 0.0);
+}
+
+// Results to the caller's array, large ones 2 KB at a time: their pages are
+// often new, and one memcpy faulting them in takes twice as long (3 MB: 660
+// us, 330 in pieces; 40 and 45 into pages that are there).
+static void copy_out(double* out, const double* stage, size_t n)
+{
+    const size_t piece = n < (1u << 17) ? n : 256;
+    for (size_t k = 0; k < n; k += piece)
+        std::memcpy(out + k, stage + k, std::min(piece, n - k) * sizeof(double));
+}
+
+// Workgroups of WG threads for cnt values, two each.
+static dim3 io_grid(size_t cnt)
+{
+    return dim3((unsigned)std::max<size_t>(1, (cnt + 2 * WG - 1) / (2 * WG)));
+}
+
+int put6(pn1_ctx* c, const double* hx, const double* hv, double* dst, double* zero, size_t nz)
+{
+    HIPCHK(c, hipStreamSynchronize(c->st));              // the stage is free
+    const size_t n3 = 3 * (size_t)c->n;
+    if (hx) std::memcpy(c->h_stage, hx, n3 * sizeof(double));
+    std::memcpy(c->h_stage + n3, hv, n3 * sizeof(double));
+    hipLaunchKernelGGL(k_put, io_grid(std::max(2 * n3, nz)), dim3(WG), 0, c->st, (const double2*)c->h_stage, c->n,
+                       (size_t)c->cap, !hx, dst, (double*)nullptr, zero, nz);
+    HIPCHK(c, hipGetLastError());
     return PN1_OK;
+}
+
+int fetch(pn1_ctx* c, const double* src, int cnt, double* out0, double* out1,
+          const double* extra, size_t ne, double* oute)
+{
+    const size_t n3 = 3 * (size_t)cnt;
+    const int nv = out1 ? 2 : 1;
+    hipLaunchKernelGGL(k_get, io_grid(nv * n3 + ne), dim3(WG), 0, c->st, src, cnt, (size_t)c->cap,
+                       nv, extra, ne, (double2*)c->h_stage);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    copy_out(out0, c->h_stage, n3);
+    if (out1) copy_out(out1, c->h_stage + n3, n3);
+    if (ne) std::memcpy(oute, c->h_stage + nv * n3, ne * sizeof(double));
+    return PN1_OK;
+}
+
+hipError_t copy6(hipStream_t st, double* dst, const double* src, int n, int cap)
+{
+    hipLaunchKernelGGL(k_copy6, dim3((n + WG - 1) / WG, 6), dim3(WG), 0, st, src, n, (size_t)cap,
+                       dst);
+    return hipGetLastError();
 }
 
 // ---- scratch of pn1_force_noalloc -----------------------------------------
@@ -482,7 +562,7 @@ void pn1_destroy(pn1_ctx* c)
         (void)hipEventDestroy(e.first);
         (void)hipEventDestroy(e.second);
     }
-    double* bufs[] = {c->X, c->Y, c->H1, c->H2, c->m, c->acc, c->rows, c->gs, c->eblk, c->eout};
+    double* bufs[] = {c->X, c->Y, c->H1, c->H2, c->m, c->acc, c->rows, c->gs, c->eblk};
     for (double* b : bufs)
         if (b) (void)hipFree(b);
     if (c->j64) (void)hipFree(c->j64);
@@ -533,7 +613,6 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->rows, nr * RV);
     if (!rc) rc = dalloc(c, &c->gs, 16);
     if (!rc) rc = dalloc(c, &c->eblk, nr * ECHUNK * EV);
-    if (!rc) rc = dalloc(c, &c->eout, 8);
     // two records more than particles: the pair loops fetch up to jr[j + 2]
     if (!rc) rc = dalloc(c, &c->j64, 3 * (cap + 2));
     if (!rc) rc = dalloc(c, &c->j32, cap + 2);
@@ -547,7 +626,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->ticket, 1);
     if (!rc && hipMemsetAsync(c->ticket, 0, sizeof(unsigned int), c->st) != hipSuccess)
         rc = PN1_EDEVICE;
-    if (!rc && host_malloc((void**)&c->h_stage, 7 * cap * sizeof(double)) != hipSuccess) {
+    if (!rc && host_malloc((void**)&c->h_stage, stage_doubles(cap, 1) * sizeof(double)) != hipSuccess) {
         c->h_stage = nullptr;
         rc = PN1_ENOMEM;
     }
@@ -615,25 +694,22 @@ int pn1_upload(pn1_ctx* c, const double* x, const double* v, const double* m, in
 {
     if (!c) return PN1_EINVAL;
     char msg[256];
-    int rc = pn1_check_input(x, v, m, n, c->eps, msg, sizeof msg);
-    if (rc) return seterr(c, rc, "%s", msg);
-    if (n > c->cap) return seterr(c, PN1_EINVAL, "n = %d exceeds capacity %d", n, c->cap);
+    if (n < 1 || !x || !v || !m || n > c->cap) {
+        const int rc = pn1_check_input(x, v, m, n, c->eps, msg, sizeof msg);
+        if (rc) return seterr(c, rc, "%s", msg);
+        return seterr(c, PN1_EINVAL, "n = %d exceeds capacity %d", n, c->cap);
+    }
     HIPCHK(c, hipSetDevice(c->dev));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    const size_t cap = (size_t)c->cap;
     double* h = c->h_stage;
-    for (int i = 0; i < n; ++i) {
-        for (int k = 0; k < 3; ++k) {
-            h[k * cap + i] = x[3 * i + k];
-            h[(3 + k) * cap + i] = v[3 * i + k];
-        }
-        h[6 * cap + i] = m[i];
+    StarScan scan;
+    if (!stage_cluster(x, v, m, n, h, h + 3 * (size_t)n, h + 6 * (size_t)n, &scan)) {
+        const int rc = pn1_check_input(x, v, m, n, c->eps, msg, sizeof msg);
+        if (rc) return seterr(c, rc, "%s", msg);
     }
-    for (int k = 0; k < 6; ++k)
-        HIPCHK(c, hipMemcpyAsync(c->X + k * cap, h + k * cap, n * sizeof(double),
-                                 hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->m, h + 6 * cap, n * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    hipLaunchKernelGGL(k_put, io_grid(7 * (size_t)n), dim3(WG), 0, c->st, (const double2*)h, n, (size_t)c->cap,
+                       false, c->X, c->m, (double*)nullptr, (size_t)0);
+    HIPCHK(c, hipGetLastError());
     // a captured step holds this state's launch constants (n, the BH mass,
     // the mixed form's mass scale, equal-mass kernels, BH-close threshold)
     drop_graph(c);
@@ -644,17 +720,9 @@ int pn1_upload(pn1_ctx* c, const double* x, const double* v, const double* m, in
     // every star is massless: their records then have mass 0, and no pair
     // needs a threshold); the equal-mass kernels take unit record masses,
     // so only for stars of one positive mass
-    c->mmax = 0.0;
-    c->eqm = n > 1 && m[1] > 0.0;
-    double dmax2 = 0.0;
-    for (int i = 1; i < n; ++i) {
-        c->mmax = std::max(c->mmax, std::fabs(m[i]));
-        c->eqm = c->eqm && m[i] == m[1];
-        double d2 = 0.0;
-        for (int k = 0; k < 3; ++k) d2 += (x[3 * i + k] - x[k]) * (x[3 * i + k] - x[k]);
-        dmax2 = std::max(dmax2, d2);
-    }
-    c->tauf = flag_threshold(std::sqrt(dmax2));
+    c->mmax = scan.mmax;
+    c->eqm = n > 1 && scan.eqm;
+    c->tauf = flag_threshold(std::sqrt(scan.dmax2));
     c->acc_ok = false;
     c->have_state = true;
     return plan_parts(c);
@@ -665,9 +733,7 @@ int pn1_download(pn1_ctx* c, double* x, double* v)
     int rc;
     if (!ready(c, &rc)) return rc;
     if (!x || !v) return seterr(c, PN1_EINVAL, "null output");
-    const size_t cap = (size_t)c->cap;
-    if ((rc = fetch3(c, c->X, x))) return rc;
-    return fetch3(c, c->X + 3 * cap, v);
+    return fetch(c, c->X, c->n, x, v);
 }
 
 int pn1_force(pn1_ctx* c, double* a)
@@ -678,7 +744,7 @@ int pn1_force(pn1_ctx* c, double* a)
     const Phys P = make_phys(c);
     if ((rc = ensure_prev_acc(c, P))) return rc;
     if ((rc = enqueue_force(c, P))) return rc;
-    return fetch3(c, c->acc, a);
+    return fetch(c, c->acc, c->n, a, nullptr);
 }
 
 int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
@@ -719,14 +785,7 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
         launch_fin<0, 0>(c, in, P, part_slots(c, S), i0, i1, false);
     if (!mixed) c->acc_ok = false;
     HIPCHK(c, hipGetLastError());
-    const size_t cap = (size_t)c->cap, cnt = (size_t)(i1 - i0);
-    for (int k = 0; k < 3; ++k)
-        HIPCHK(c, hipMemcpyAsync(c->h_stage + k * cap, c->acc + k * cap + i0,
-                                 cnt * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    for (size_t i = 0; i < cnt; ++i)
-        for (int k = 0; k < 3; ++k) a[3 * i + k] = c->h_stage[k * cap + i];
-    return PN1_OK;
+    return fetch(c, c->acc + i0, i1 - i0, a, nullptr);
 }
 
 int pn1_energy(pn1_ctx* c, pn1_energy_t* out)
@@ -738,11 +797,10 @@ int pn1_energy(pn1_ctx* c, pn1_energy_t* out)
     if ((rc = prep_x(c, P, true))) return rc;
     hipLaunchKernelGGL(k_energy, dim3(c->nrow, energy_chunks(c->n - 1)), dim3(PW * RB), 0, c->st,
                        (const JRec64*)rec_buf(c, 0), (const double*)c->X, (const double*)c->gs,
-                       c->eblk, c->eout, c->ticket, P);
+                       c->eblk, c->h_stage, c->ticket, P);
     HIPCHK(c, hipGetLastError());
-    double e[5];
-    HIPCHK(c, hipMemcpyAsync(e, c->eout, sizeof e, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
+    const double* e = c->h_stage;
     out->kin = e[0];
     out->pot = e[1];
     out->pot_pn = e[2];
@@ -1005,8 +1063,8 @@ static pn1_ctx* legacy_ctx(const char* what, const double* x, const double* v, c
                            int n, double eps, int mode)
 {
     char msg[256];
-    if (pn1_check_input(x, v, m, n, eps, msg, sizeof msg) != PN1_OK) die(what, msg);
     if (!g_ctx || g_ctx->cap < n) {
+        if (pn1_check_input(x, v, m, n, eps, msg, sizeof msg) != PN1_OK) die(what, msg);
         pn1_destroy(g_ctx);
         g_ctx = nullptr;
         int cap = n < 1024 ? 1024 : n;
@@ -1017,8 +1075,10 @@ static pn1_ctx* legacy_ctx(const char* what, const double* x, const double* v, c
         }
     }
     if (pn1_set_params(g_ctx, eps, g_c, g_ctx->dt, mode) != PN1_OK ||
-        pn1_upload(g_ctx, x, v, m, n) != PN1_OK)
+        pn1_upload(g_ctx, x, v, m, n) != PN1_OK) {
+        if (pn1_check_input(x, v, m, n, eps, msg, sizeof msg) != PN1_OK) die(what, msg);
         die(what, g_ctx->err);
+    }
     return g_ctx;
 }
 

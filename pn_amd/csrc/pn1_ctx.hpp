@@ -31,7 +31,7 @@ struct pn1_ctx {
     // device buffers
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr;
     double *m = nullptr, *acc = nullptr, *rows = nullptr, *gs = nullptr;
-    double *eblk = nullptr, *eout = nullptr;
+    double* eblk = nullptr;
     // three buffers of cap + 2 records: each of a step's evaluations reads
     // one and prepares the next
     pn1dev::JRec64* j64 = nullptr;
@@ -52,7 +52,7 @@ struct pn1_ctx {
     bool acc_ok = false;
     void* part = nullptr;
     size_t part_bytes = 0;
-    double* h_stage = nullptr;  // pinned, 7 * cap doubles
+    double* h_stage = nullptr;  // pinned, stage_doubles(cap, 1)
     hipGraphExec_t gexec = nullptr;
     bool prof = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
@@ -76,8 +76,32 @@ int enqueue_eval(pn1_ctx* c, int stage, const pn1dev::Phys& P);
 // Mixed form after an upload: one evaluation with the pair thresholds off
 // (no previous accelerations yet), so that the next has them.
 int ensure_prev_acc(pn1_ctx* c, const pn1dev::Phys& P);
-// SoA device [k][cap] -> AoS host [n][3] for k in 0..2, through the stage.
-int fetch3(pn1_ctx* c, const double* dsrc, double* out);
+// ---- between AoS host arrays and SoA device buffers (pn1_io.hpp)
+// Doubles of the stage of a context or ensemble: a state, and per cluster
+// what is fetched with it (gm0) or instead of it (the energies).
+// (an even number: the kernels take double2)
+inline size_t stage_doubles(size_t cap, size_t clusters)
+{
+    return (7 * cap + 8 * clusters + 1) / 2 * 2;
+}
+// What the launches need of a cluster's stars: the largest |m|, the largest
+// squared distance to the BH, whether all have one positive mass.
+struct StarScan {
+    double mmax = 0.0, dmax2 = 0.0;
+    bool eqm = true;
+};
+// Copies a cluster (BH first) to sx, sv, sm and scans its stars.  False if
+// pn1_check_input might refuse it (it then says).
+bool stage_cluster(const double* x, const double* v, const double* m, int n, double* sx,
+                   double* sv, double* sm, StarScan* scan);
+// The caller's arrays hx (null: zeros) and hv into the stage and on to dst (6
+// x cap); clears zero[0, nz).
+int put6(pn1_ctx* c, const double* hx, const double* hv, double* dst, double* zero, size_t nz);
+// src (SoA, cnt stars from its first) to out0 and, if not null, src + 3 cap to
+// out1, AoS; also extra[0, ne) to oute.  Waits for the stream.
+int fetch(pn1_ctx* c, const double* src, int cnt, double* out0, double* out1,
+          const double* extra = nullptr, size_t ne = 0, double* oute = nullptr);
+hipError_t copy6(hipStream_t st, double* dst, const double* src, int n, int cap);
 // Checks that a state is resident and makes the context's device current;
 // *rc is PN1_OK, or the error when it returns false.
 bool ready(pn1_ctx* c, int* rc);

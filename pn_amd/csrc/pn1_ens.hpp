@@ -37,7 +37,11 @@ struct pn1_ens {
     int L_req = 0, tile_req = 0, variant_req = -1;
     int L = 512, tile = 64;
     double *X = nullptr, *Y = nullptr, *H1 = nullptr, *H2 = nullptr, *m = nullptr, *acc = nullptr;
-    double *rows = nullptr, *gs = nullptr, *eblk = nullptr, *eout = nullptr;
+    double *rows = nullptr, *gs = nullptr, *eblk = nullptr;
+    // the tables of the upload, one device block (tab) and its pinned source
+    // (h_tab): cm0 ... place below point into it
+    char *tab = nullptr, *h_tab = nullptr;
+    size_t tab_bytes = 0;
     double* cm0 = nullptr;
     double* cmmax = nullptr;      // each cluster's largest star mass
     pn1dev::Thr* thr = nullptr;   // mixed form's per-star pair thresholds
@@ -55,7 +59,7 @@ struct pn1_ens {
     pn1dev::EBlk *row = nullptr, *pblk = nullptr;
     int* crow = nullptr;
     int nrow = 0, npblk = 0;
-    int fmask_cap = 0, hmask_cap = 0, row_cap = 0, pblk_cap = 0;
+    int fmask_cap = 0, hmask_cap = 0;
     int rows_cap = 0, eblk_cap = 0;
     // three buffers of cap + 2 records, as in pn1_ctx
     pn1dev::JRec64* j64 = nullptr;
@@ -76,7 +80,7 @@ struct pn1_ens {
     long long slots = 0;
     void* part = nullptr;
     size_t part_bytes = 0;
-    double* h_stage = nullptr;
+    double* h_stage = nullptr;    // pinned, stage_doubles(cap, capc)
     int grid64[2] = {0, 0}, grid32[4] = {0, 0, 0, 0};   // per kernel variant
     hipGraphExec_t gexec = nullptr;
     bool prof = false;
@@ -85,7 +89,8 @@ struct pn1_ens {
     double prof_ms = 0.0;
     pn1_ens_adj* adj = nullptr;   // allocated by the first adjoint call
     unsigned gen = 0;             // bumped when the state or eps, c, dt change
-    std::vector<int> off_h;       // host copy of the cluster offsets
+    std::vector<int> off_h;       // host copies: cluster offsets, and per cluster
+    std::vector<double> m0_h, mmax_h, tauf_h;   // the values of cm0, cmmax, ctauf
     char err[512] = {0};
 };
 
@@ -98,7 +103,11 @@ int ens_enqueue_prep(pn1_ens* e, const pn1dev::Phys& P);
 int ens_enqueue_eval(pn1_ens* e, int stage, const pn1dev::Phys& P);
 // Mixed form after an upload: one evaluation with the pair thresholds off.
 int ens_ensure_prev_acc(pn1_ens* e, const pn1dev::Phys& P);
-int ens_fetch3(pn1_ens* e, const double* dsrc, double* out);
+// As put6 and fetch (pn1_ctx.hpp), all particles.
+int ens_put6(pn1_ens* e, const double* hx, const double* hv, double* dst, double* zero,
+             size_t nz);
+int ens_fetch(pn1_ens* e, const double* src, double* out0, double* out1,
+              const double* extra = nullptr, size_t ne = 0, double* oute = nullptr);
 bool ens_ready(pn1_ens* e, int* rc);
 // ens_ready, and the tables are those of the force's present plan.
 bool ens_force_ready(pn1_ens* e, int* rc);
