@@ -114,7 +114,7 @@ int  pn1_force_range(pn1_ctx *ctx, int i0, int i1, double *a);
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): the FP64 force of pn1_force on a state
  * that already lies in device memory.  It allocates nothing: every
- * intermediate lives in a fixed scratch area of the library, 69 MB on each
+ * intermediate lives in a fixed scratch area of the library, 36 MB on each
  * GPU it runs on, held from the library's load there until the process
  * ends.
  *   st      device, 6 rows of n doubles: x, y, z, vx, vy, vz (SoA)
@@ -148,10 +148,11 @@ const char *pn1_last_error(const pn1_ctx *ctx);
 /* Launch shape of the pair kernels: the j range is split into `jsplit`
  * chunks, one per 256-star workgroup (0 = automatic: up to 192 parts, eight
  * of them to a workgroup of 64 stars, which adds their sums; `variant` then
- * stays -1, else the split is an automatic one of the 256-star kernels).  A
- * split of 32 or more, a multiple of 8, ends in 16 chunks an eighth as long
- * as the others, which the launch runs last, so that it does not wait long
- * on its last workgroups.  The mixed kernel compensates its FP32 sums every
+ * stays -1, else the split is an automatic one of the 256-star kernels;
+ * splits of 2 to 32 without a `variant` run as up to 16 chunks of that row
+ * form).  A split of the 256-star kernels of 32 or more, a multiple of 8,
+ * ends in 16 chunks an eighth as long as the others, which the launch runs
+ * last, so that it does not wait long on its last workgroups.  The mixed kernel compensates its FP32 sums every
  * `tile` pairs (0 = default), and `variant` picks the kernel form (-1 =
  * automatic per mode): bit 0 the j loop (clear: one j-record at a time,
  * set: two in flight), bit 1 (mixed form) one Newton step on the FP32

@@ -117,6 +117,22 @@ int auto_slots(int nst)
     return s;
 }
 
+// Partials per star of an explicit split in S chunks where the row kernels take
+// it, else 0: from 2 chunks on (one stays one serial sum per star, as an
+// ensemble's unsplit chunk is) to 32, as far as a launch holds them, in up to
+// 16 chunks of PW parts.  Measured on MI355X, evaluation with the 256-star
+// kernels' S chunks / with these, FP64 and mixed, us:
+//   n = 129, S = 2    24.9 / 15.8  31.6 / 20.5
+//   n = 1025, S = 16  28.9 / 18.9  31.7 / 20.9
+//   n = 4097, S = 32  67.0 / 44.6  96.8 / 37.4
+//   n = 16384, S = 32  429 / 418    324 / 241
+int explicit_slots(int S, int nst)
+{
+    if (S < 2 || S > 32) return 0;
+    const int s = std::min(S, TLONG);
+    return (long)s * ((nst + RB - 1) / RB) <= (1L << 22) ? s : 0;
+}
+
 // Launch plan of the pair kernels for the current n.
 void plan(pn1_ctx* c)
 {
@@ -126,6 +142,7 @@ void plan(pn1_ctx* c)
     c->slots = 0;
     if (c->jsplit_req > 0) {
         c->S = std::max(1, std::min(c->jsplit_req, std::max(nst, 1)));
+        if (c->variant_req < 0 && nst > 0) c->slots = explicit_slots(c->S, nst);
     } else if (c->variant_req >= 0 || nst < 1) {
         c->S = auto_split(nst);
     } else {
@@ -171,7 +188,7 @@ int plan_parts(pn1_ctx* c)
 {
     plan(c);
     const int rc = ensure_part(c);
-    if (!rc || !c->slots) return rc;
+    if (!rc || !c->slots || c->jsplit_req > 0) return rc;
     c->slots = 0;
     c->S = auto_split(c->n - 1);
     return ensure_part(c);
@@ -239,8 +256,7 @@ bool ready(pn1_ctx* c, int* rc)
 // ---- one force evaluation (+ stage update) ------------------------------
 JRec64* rec_buf(const pn1_ctx* c, int k) { return c->j64 + (size_t)k * ((size_t)c->cap + 2); }
 
-// ticket false: the sums over the rows are left to k_gsum / k_bh, or not
-// needed (an i shard).
+// ticket false: the sums over the rows are not needed (an i shard).
 RowBufs row_bufs(const pn1_ctx* c, bool ticket = true)
 {
     RowBufs R;
@@ -251,6 +267,7 @@ RowBufs row_bufs(const pn1_ctx* c, bool ticket = true)
     R.flist = c->flist;
     R.fn = c->fn;
     R.ticket = ticket ? c->ticket : nullptr;
+    R.clear = nullptr;
     return R;
 }
 
@@ -318,6 +335,17 @@ void launch_pair(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P,
     }
 }
 
+// The same by the row kernels, rows row0 .. row0 + nrow - 1, the plan's slots.
+void launch_pairw(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int row0,
+                  int nrow, bool ts)
+{
+    if (c->mode == PN1_MIXED)
+        launch_pair32w(c, j64, in, P, c->slots, row0, nrow, ts);
+    else
+        hipLaunchKernelGGL(k_pair64w, dim3(c->slots * nrow), dim3(PW * RB), 0, c->st, j64, in,
+                           (double*)c->part, P, c->slots, nrow, c->slots * row0);
+}
+
 // The records and sums of an evaluation on X; FP64: whatever the mode, the
 // FP64 form's only (energy).
 int prep_x(pn1_ctx* c, const Phys& P, bool fp64)
@@ -344,13 +372,10 @@ int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
         hipEvent_t e1 = nullptr;
         if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
         const JRec64* j64 = rec_buf(c, stage <= 1 ? 0 : stage - 1);
-        if (!c->slots)
-            launch_pair(c, j64, in, P, 0, c->nIblk, c->S, stage <= 1);
-        else if (mixed)
-            launch_pair32w(c, j64, in, P, c->slots, stage <= 1);
+        if (c->slots)
+            launch_pairw(c, j64, in, P, 0, c->nrow, stage <= 1);
         else
-            hipLaunchKernelGGL(k_pair64w, dim3(c->slots * c->nrow), dim3(PW * RB), 0, c->st, j64,
-                               in, (double*)c->part, P, c->slots, c->nrow);
+            launch_pair(c, j64, in, P, 0, c->nIblk, c->S, stage <= 1);
         if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     }
     switch (stage * 2 + (mixed ? 1 : 0)) {
@@ -488,18 +513,19 @@ hipError_t copy6(hipStream_t st, double* dst, const double* src, int n, int cap)
 }
 
 // ---- scratch of pn1_force_noalloc -----------------------------------------
-// Sized for n <= PN1_NOALLOC_MAX_N and a j split of at most NA_MAXS chunks:
-// j-records, pair partials, the rows' values and the separable sums of one FP64 force evaluation, each part 256-byte
-// aligned (offsets in doubles).
+// Sized for n <= PN1_NOALLOC_MAX_N and the explicit_slots of a j split of at
+// most NA_MAXS chunks: j-records, pair partials, the rows' values of k_prep and of k_fin_na and its
+// counter, each part 256-byte aligned (offsets in doubles).
 constexpr int NA_MAXS = 32;
 constexpr int NA_MAXB = (PN1_NOALLOC_MAX_N + RB - 1) / RB;
 constexpr size_t na_round(size_t d) { return (d + 31) & ~(size_t)31; }
 constexpr size_t NA_J64 = 0;
 constexpr size_t NA_PART =
     NA_J64 + na_round((size_t)PN1_NOALLOC_MAX_N * (sizeof(JRec64) / sizeof(double)));
-constexpr size_t NA_ROWS = NA_PART + na_round((size_t)NA_MAXS * NACC * PN1_NOALLOC_MAX_N);
-constexpr size_t NA_GS = NA_ROWS + na_round((size_t)NA_MAXB * RV);
-constexpr size_t NA_TOTAL = NA_GS + na_round(NGS);
+constexpr size_t NA_PROWS = NA_PART + na_round((size_t)TLONG * NACC * PN1_NOALLOC_MAX_N);
+constexpr size_t NA_ROWS = NA_PROWS + na_round((size_t)NA_MAXB * RV);
+constexpr size_t NA_TICKET = NA_ROWS + na_round((size_t)NA_MAXB * RV);
+constexpr size_t NA_TOTAL = NA_TICKET + na_round(1);
 static_assert(sizeof(JRec64) % sizeof(double) == 0, "JRec64 in doubles");
 
 // j split of pn1_force_noalloc: NA_MAXS chunks, halved while a chunk would
@@ -771,18 +797,23 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
         while (S < 512 && (long)S * nib < 16384 && (nst + 2 * S - 1) / (2 * S) >= 64) S *= 2;
     }
     if ((rc = ensure_prev_acc(c, P))) return rc;
-    if ((rc = ensure_part(c, S))) return rc;
+    const bool rowk = c->jsplit_req > 0 && c->slots;
+    const int slots = rowk ? c->slots : part_slots(c, S);
+    if ((rc = ensure_part(c, rowk ? 0 : S))) return rc;
     // every star's j-record and the separable sums: what a sharded run would
     // all-gather and all-reduce before its pair kernel
     if ((rc = enqueue_prep(c, P))) return rc;
     hipEvent_t e1 = nullptr;
     if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
-    launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
+    if (rowk)
+        launch_pairw(c, rec_buf(c, 0), in, P, (i0 - 1) / RB, (i1 - i0 + RB - 1) / RB, true);
+    else
+        launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     if (mixed)
-        launch_fin<1, 0>(c, in, P, part_slots(c, S), i0, i1, false);
+        launch_fin<1, 0>(c, in, P, slots, i0, i1, false);
     else
-        launch_fin<0, 0>(c, in, P, part_slots(c, S), i0, i1, false);
+        launch_fin<0, 0>(c, in, P, slots, i0, i1, false);
     if (!mixed) c->acc_ok = false;
     HIPCHK(c, hipGetLastError());
     return fetch(c, c->acc + i0, i1 - i0, a, nullptr);
@@ -970,8 +1001,11 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
 // The FP64 force of pn1_force on a state the caller holds in device memory,
 // with every intermediate in this GPU's scratch: the same kernels, the j
 // split na_split(n - 1).  Enqueues only (no hipMalloc, hipFree, memset or
-// synchronisation); nothing in the scratch needs clearing, every value read
-// is written earlier in the same call.
+// synchronisation); nothing in the scratch needs clearing beforehand, every
+// value read is written earlier in the same call, the counter too (a call that
+// overlapped another one against the contract leaves nothing behind).  Three
+// launches: n = 4097, 103 us with the wait -> 62 (256-star kernels, five
+// launches before), n = 257, 45 -> 31.
 int pn1_force_noalloc(const double* st, const double* m, int n, double eps, double c,
                       double* acc, void* stream)
 {
@@ -999,9 +1033,8 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
     JRec64* j64 = (JRec64*)(base + NA_J64);
     double* part = base + NA_PART;
     RowBufs R = {};
-    R.rows = base + NA_ROWS;
-    R.gs = base + NA_GS;
-    MixPrep M = {};
+    R.rows = base + NA_PROWS;
+    R.clear = (unsigned int*)(base + NA_TICKET);
     FinBufs F = {};
     F.in = st;
     F.m = m;
@@ -1010,25 +1043,21 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
     const int nst = n - 1, nib = (nst + WG - 1) / WG;
     const int nrow = nst > 0 ? (nst + RB - 1) / RB : 1;
     const int S = na_split(nst);
-    // no ticket counter here: a call that overlapped another one against the
-    // contract would leave it wrong for every later call
+    // (the rows hold fewer than 2^22 / 16 stars here: S = 1 alone is not theirs)
+    const int slots = explicit_slots(S, nst);
     hipLaunchKernelGGL(k_prep, dim3((nrow + FG - 1) / FG), dim3(FWG), 0, s, st, m, P, nrow, j64, R,
-                       M, (const double*)nullptr, (const float*)nullptr);
-    hipLaunchKernelGGL(k_gsum, dim3(1), dim3(FWG), 0, s, R, nrow);
-    // The two-in-flight form gives the same sums; with few waves per SIMD it
-    // hides more of its loads' latency, and above 8192 stars the one-record
-    // form's 7 waves make two rounds of the grid (measured on MI355X, pair
-    // launch, one record / two: n = 4097 58/60 us, 12000 287/268, 16384
-    // 482/438).
-    if (nst > 8192)
-        hipLaunchKernelGGL(k_pair64<1>, dim3(pair_grid(S, nib)), dim3(WG), 0, s,
-                           (const JRec64*)j64, st, part, P, S, nib, 0);
+                       MixPrep{}, (const double*)nullptr, (const float*)nullptr);
+    if (slots)
+        hipLaunchKernelGGL(k_pair64w, dim3(slots * nrow), dim3(PW * RB), 0, s, (const JRec64*)j64,
+                           st, part, P, slots, nrow, 0);
     else if (nst > 0)
         hipLaunchKernelGGL(k_pair64<0>, dim3(pair_grid(S, nib)), dim3(WG), 0, s,
                            (const JRec64*)j64, st, part, P, S, nib, 0);
-    hipLaunchKernelGGL((k_fin<0, 0, FG>), dim3(nrow), dim3(FWG), 0, s, F, R, (const void*)part, S,
-                       M, P, 0, n, nrow);
-    hipLaunchKernelGGL(k_bh, dim3(1), dim3(FWG), 0, s, F, R, nrow, P);
+    R.rows = base + NA_ROWS;
+    R.ticket = (unsigned int*)(base + NA_TICKET);
+    hipLaunchKernelGGL(k_fin_na, dim3(nrow), dim3(FWG), 0, s, F, R,
+                       (const double*)(base + NA_PROWS), (const void*)part, slots ? slots : S, P,
+                       nrow);
     return hipGetLastError() == hipSuccess ? PN1_OK : PN1_EDEVICE;
 }
 

@@ -303,8 +303,10 @@ struct RowBufs {
     unsigned long long *fmask, *hmask;     // per row: BH-close and hard stars
     double* gs;                            // separable sums of the evaluation
     int *flist, *fn;                       // its BH-close stars and their number
-    unsigned int* ticket;                  // last_block's counter (null: the sums are
-                                           // added by k_gsum and k_bh instead)
+    unsigned int* ticket;                  // last_block's counter (k_prep: null if the
+                                           // sums are left to k_fin_na; k_fin: null for
+                                           // an i shard)
+    unsigned int* clear;                   // a counter that k_prep sets to 0, or null
 };
 
 // After the last row of a prep: the separable sums, and the BH-close list of
@@ -329,6 +331,7 @@ inline __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ 
                                              const double* __restrict__ aprev,
                                              const float* __restrict__ kprev)
 {
+    if (R.clear && blockIdx.x == 0 && threadIdx.x == 0) *R.clear = 0u;
     const int lane = threadIdx.x & 63;
     const int row = blockIdx.x * FG + (int)(threadIdx.x >> 6);
     const int p = 1 + row * RB + lane;
@@ -357,12 +360,6 @@ inline __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ 
     }
     if (R.ticket && last_block(R.ticket, gridDim.x))
         close_prep(R, M.j32 != nullptr, 0, nrow, 1, R.gs, R.flist, R.fn);
-}
-
-// The separable sums of the rows (one workgroup), where k_prep leaves them.
-inline __global__ __launch_bounds__(FWG) void k_gsum(RowBufs R, int nrow)
-{
-    close_prep(R, false, 0, nrow, 1, R.gs, R.flist, R.fn);
 }
 
 // ---------------------------------------------------------------------
@@ -510,9 +507,10 @@ constexpr int PW = 8;
 
 // Workgroup -> chunk s of S and row ig of 64 stars, and the bounds of wave
 // w's part of the chunk with the window that can contain j == i.  A split of
-// TLONG + TSHORT chunks is tapered: the last TSHORT are an eighth as long
-// and run after all others, so that the launch does not wait long on its last
-// workgroups.
+// TLONG + TSHORT chunks is tapered: the last TSHORT are an eighth as long and
+// run after all others, so that the launch does not wait long on its last
+// workgroups.  (A launch of some rows only starts at workgroup bid0 = S times
+// the first row; it is never tapered.)
 constexpr int TLONG = 16, TSHORT = 8;
 __device__ __forceinline__ JRange j_part(int bid, int S, int nrow, int wave, int n, int& s,
                                          int& ig)
@@ -585,12 +583,12 @@ __device__ __forceinline__ void part64(const JRec64* __restrict__ jr, const JRan
 // Held to k_pair64's 7 waves per SIMD (72 VGPRs; 80 otherwise).
 inline __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(7, 8)))
 void k_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
-               double* __restrict__ part, Phys P, int S, int nrow)
+               double* __restrict__ part, Phys P, int S, int nrow, int bid0)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     int s, ig;
-    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
+    const JRange R = j_part(bid0 + (int)blockIdx.x, S, nrow, wave, P.n, s, ig);
     const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
     const I64 I = load_i64(jr, st, P.cap, i, P.eps2);
     double a[NACC];
@@ -1066,12 +1064,12 @@ template <bool TS, bool EQ>
 __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
                const Thr* __restrict__ thr, const double* __restrict__ st,
-               float* __restrict__ part, Phys P, int S, int nrow, int tile)
+               float* __restrict__ part, Phys P, int S, int nrow, int bid0, int tile)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     int s, ig;
-    const JRange R = j_part(blockIdx.x, S, nrow, wave, P.n, s, ig);
+    const JRange R = j_part(bid0 + (int)blockIdx.x, S, nrow, wave, P.n, s, ig);
     const int n = P.n, li = ig * RB + lane + 1, i = li < n ? li : n - 1;
     const I32 I = load_i32(j64, thr, st, P.cap, i, 0, P.eps2);
     float a[NACC32], sumN[3], cmpN[3];
@@ -1490,10 +1488,24 @@ void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M
         fin_close<MODE, STAGE>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P);
 }
 
-// The BH from the rows' shares (one workgroup), where k_fin leaves it.
-inline __global__ __launch_bounds__(FWG) void k_bh(FinBufs F, RowBufs R, int nrow, Phys P)
+// k_fin of pn1_force_noalloc (FP64, G = FG): every workgroup adds the separable
+// sums from k_prep's rows (prows, FWG threads: the order of k_prep's last
+// workgroup) for itself, so that only one counter, R.ticket, is left, which
+// k_prep clears in the same call.
+inline __global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void k_fin_na(FinBufs F, RowBufs R, const double* __restrict__ prows,
+              const void* __restrict__ part, int S, Phys P, int nrow)
 {
-    fin_close<0, 0>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P);
+    __shared__ double tot[RV];
+    rows_total(prows, 0, nrow, tot);
+    const Row q = {0, P.n - 1, (int)blockIdx.x * RB, (int)blockIdx.x};
+    if (P.n > 1)
+        fin_rows<0, 0, FG>(F, R, q, part, S, (size_t)P.cap, 1, tot + RV_G, nullptr, nullptr,
+                           F.m[0], MixPrep{}, P);
+    else
+        empty_row(R, 0, false);
+    if (last_block(R.ticket, gridDim.x))
+        fin_close<0, 0>(F, R, 0, nrow, 0, tot + RV_G, nullptr, nullptr, P);
 }
 
 // ---------------------------------------------------------------------

@@ -40,10 +40,12 @@ const Launch32 k_launch32[16] = {
     launch32<3, true, true>};
 
 template <bool TS, bool EQ>
-void launch32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots)
+void launch32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots, int row0,
+               int nrow)
 {
-    hipLaunchKernelGGL((k_pair32w<TS, EQ>), dim3(slots * c->nrow), dim3(PW * RB), 0, c->st, c->j32,
-                       j64, c->thr, in, (float*)c->part, P, slots, c->nrow, c->tile);
+    hipLaunchKernelGGL((k_pair32w<TS, EQ>), dim3(slots * nrow), dim3(PW * RB), 0, c->st, c->j32,
+                       j64, c->thr, in, (float*)c->part, P, slots, nrow, slots * row0,
+                       c->tile);
 }
 
 template <int PP, bool TS, bool EQ>
@@ -85,12 +87,13 @@ void launch_pair32(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& 
 }
 
 void launch_pair32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots,
-                    bool ts)
+                    int row0, int nrow, bool ts)
 {
     if (ts)
-        (c->eqm ? launch32w<true, true> : launch32w<true, false>)(c, j64, in, P, slots);
+        (c->eqm ? launch32w<true, true> : launch32w<true, false>)(c, j64, in, P, slots, row0, nrow);
     else
-        (c->eqm ? launch32w<false, true> : launch32w<false, false>)(c, j64, in, P, slots);
+        (c->eqm ? launch32w<false, true> : launch32w<false, false>)(c, j64, in, P, slots, row0,
+                                                                    nrow);
 }
 
 void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g,

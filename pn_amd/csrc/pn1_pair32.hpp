@@ -22,9 +22,9 @@ inline int pair32_form(int variant, bool ts, bool eqm)
 // range split in S chunks (pn1_pair32.hip).
 void launch_pair32(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
                    const pn1dev::Phys& P, int ib0, int nib, int S, int form);
-// The automatic plan's form: every star, `slots` partials each.
+// The row kernels' form: nrow rows from row0 on, `slots` partials per star.
 void launch_pair32w(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
-                    const pn1dev::Phys& P, int slots, bool ts);
+                    const pn1dev::Phys& P, int slots, int row0, int nrow, bool ts);
 // Ensemble: one persistent launch of grid g over the work queues.
 void launch_ens_pair32(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
                        const pn1dev::Phys& P, dim3 g, int form);

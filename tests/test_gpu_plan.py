@@ -82,3 +82,22 @@ def test_ensemble_plan_against_items(mode, bound):
     # pair thresholds come from another evaluation of the same accuracy
     for p, q in zip(x0 + v0, x1 + v1):
         assert np.abs(p - q).max() <= (1e-12 if mode == pn.FP64 else 1e-6) * max(1.0, np.abs(q).max())
+
+
+@pytest.mark.parametrize("mode,bound", [(pn.FP64, 1e-12), (pn.MIXED, 2e-6)])
+@pytest.mark.parametrize("stars", [2, 64, 65, 700, 2049])
+def test_explicit_splits(stars, mode, bound):
+    """Splits at the edges of the row kernels' range (2 to 32, at most one chunk
+    per star) against the 256-star kernels of the same split."""
+    x, v, m = cluster(stars, 600 + stars)
+    with pn.Context(stars + 1) as ctx:
+        ctx.set_params(1e-2, 50.0, 2.0**-10, mode)
+        for split in (1, 2, 15, 16, 17, 24, 32, 33):
+            print(f"case: {stars} stars, split {split}, mode {mode}", flush=True)
+            ctx.set_tuning(split, 0, -1)
+            ctx.upload(x, v, m)
+            a = ctx.force()
+            ctx.set_tuning(split, 0, 0)
+            b = ctx.force()
+            err = np.linalg.norm(a - b, axis=1) / np.linalg.norm(b, axis=1)
+            assert err.max() <= bound, (split, err.max())
