@@ -243,11 +243,13 @@ void k_ens_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
     const I64 I = load_i64(jr, st, P.cap, g.i, P.eps2);
     double a[NACC];
     part64(jr, g.R, g.i, I, a, P.eps2);
-    waves_total(a, wave, lane);
-    if (wave == 0 && g.li < g.nst) {
+    double t[NSHARE<NACC>];
+    waves_share(a, wave, lane, t);
+    if (g.li < g.nst) {
         double* pp = part + (poff[w.c] + (long long)w.s * g.nst) * NACC + g.li;
 #pragma unroll
-        for (int k = 0; k < NACC; ++k) stream_out(a[k], &pp[(size_t)k * g.nst]);
+        for (int q = 0; q < NSHARE<NACC>; ++q)
+            stream_out(t[q], &pp[(size_t)(q * PW + wave) * g.nst]);
     }
 }
 
@@ -352,17 +354,22 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
         M.mmax = E.cmmax[b.c];
         M.tauf = E.ctauf[b.c];
     }
+    StageIn bh = {};
     if (nst > 0) {
         const void* base = MODE == 0 ? (const void*)((const double*)part + poff[b.c] * NACC)
                                      : (const void*)((const float*)part + poff[b.c] * MROWS);
         fin_rows<MODE, STAGE, G>(F, R, q, base, ens_nchunks(nst, L), (size_t)nst, 0, gs,
-                                 R.flist + off, R.fn + b.c, E.cm0[b.c], M, P);
+                                 R.flist + off, R.fn + b.c, E.cm0[b.c], M, P, bh);
     } else {
         empty_row(R, q.row, MODE == 1);
     }
     const unsigned nblk = (unsigned)(G == 1 ? (r1 - r0 + FG - 1) / FG : r1 - r0);
-    if (last_block(R.ticket + b.c, nblk))
-        fin_close<MODE, STAGE>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P);
+    if (last_block(R.ticket + b.c, nblk)) {
+        if (G > 1 && nst > 0)
+            fin_close<MODE, STAGE, true>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
+        else
+            fin_close<MODE, STAGE, false>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
+    }
 }
 
 // ---------------------------------------------------------------------

@@ -546,22 +546,35 @@ __device__ __forceinline__ JRange j_part(int bid, int S, int nrow, int wave, int
     return R;
 }
 
-// Adds the PW waves' v pairwise in a fixed order; the sums are in wave 0.
-// Every thread of the workgroup calls it.
+// Adds the waves' v pairwise in a fixed order; value q PW + w's sum goes to
+// t[q] of wave w.  Each round passes PW values through LDS, so all waves add (a
+// tree over the waves left most of them idle: 600 cycles more of the 10000 of
+// a workgroup at n = 1025 on MI355X).  Every thread of the workgroup (PW waves) calls it.
 template <int N>
-__device__ __forceinline__ void waves_total(double (&v)[N], int wave, int lane)
+constexpr int NSHARE = (N + PW - 1) / PW;
+template <int N>
+__device__ __forceinline__ void waves_share(const double (&v)[N], int wave, int lane,
+                                            double (&t)[NSHARE<N>])
 {
-    __shared__ double sh[PW / 2][N][RB];
+    __shared__ double sh[PW][PW][RB];
 #pragma unroll
-    for (int h = PW / 2; h >= 1; h >>= 1) {
-        if (wave >= h && wave < 2 * h)
+    for (int q = 0; q < NSHARE<N>; ++q) {
+        if (q > 0) __syncthreads();
 #pragma unroll
-            for (int k = 0; k < N; ++k) sh[wave - h][k][lane] = v[k];
+        for (int k = 0; k < PW; ++k)
+            if (q * PW + k < N) sh[k][wave][lane] = v[q * PW + k];
         __syncthreads();
-        if (wave < h)
+        t[q] = 0.0;
+        if (q * PW + wave < N) {
+            double u[PW];
 #pragma unroll
-            for (int k = 0; k < N; ++k) v[k] += sh[wave][k][lane];
-        if (h > 1) __syncthreads();
+            for (int k = 0; k < PW; ++k) u[k] = sh[wave][k][lane];
+#pragma unroll
+            for (int h = PW / 2; h >= 1; h >>= 1)
+#pragma unroll
+                for (int k = 0; k < h; ++k) u[k] += u[k + h];
+            t[q] = u[0];
+        }
     }
 }
 
@@ -593,10 +606,12 @@ void k_pair64w(const JRec64* __restrict__ jr, const double* __restrict__ st,
     const I64 I = load_i64(jr, st, P.cap, i, P.eps2);
     double a[NACC];
     part64(jr, R, i, I, a, P.eps2);
-    waves_total(a, wave, lane);
-    if (wave == 0 && li < n) {
+    double t[NSHARE<NACC>];
+    waves_share(a, wave, lane, t);
+    if (li < n) {
 #pragma unroll
-        for (int k = 0; k < NACC; ++k) stream_out(a[k], &part[(size_t)(s * NACC + k) * P.cap + li]);
+        for (int q = 0; q < NSHARE<NACC>; ++q)
+            stream_out(t[q], &part[(size_t)(s * NACC + q * PW + wave) * P.cap + li]);
     }
 }
 
@@ -1048,13 +1063,16 @@ __device__ __forceinline__ void put_part32(const float (&a)[NACC32], const float
 #pragma unroll
     for (int k = 0; k < NV; ++k)
         v[k] = k <= A_NZ ? (double)sumN[k] - (double)cmpN[k] : (double)a[k];
-    waves_total(v, wave, lane);
-    if (wave == 0 && ok) {
+    double t[NSHARE<NV>];
+    waves_share(v, wave, lane, t);
+    if (ok) {
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-            const float hi = (float)v[k];
+        for (int q = 0; q < NSHARE<NV>; ++q) {
+            const int k = q * PW + wave;
+            if (k >= NV) break;
+            const float hi = (float)t[q];
             stream_out(hi, &ps[k * stride]);
-            if (k <= A_NZ) stream_out(-(float)(v[k] - (double)hi), &ps[(NACC32 + k) * stride]);
+            if (k <= A_NZ) stream_out(-(float)(t[q] - (double)hi), &ps[(NACC32 + k) * stride]);
         }
     }
 }
@@ -1160,60 +1178,80 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
 // NACC32 sums, then the Newtonian Kahan compensations), whose sums built
 // from the record's mass m_j / mscale are scaled back by mscale; A[NACC] is
 // the mixed form's A_TS sum (TS: the stages whose pair kernels write it).
+// Two chunks' loads are in flight at once: a partial comes from another XCD,
+// 1.1 us away, and few waves run here.
+template <int MODE, bool TS>
+struct Chunk {
+    static constexpr int NV = MODE == 1 && TS ? NACC + 1 : NACC;
+    double L64[MODE == 0 ? NV : 1];
+    float L32[MODE == 1 ? NV : 1], C[MODE == 1 ? 3 : 1];
+    __device__ __forceinline__ void load(const void* __restrict__ part, int s, size_t stride,
+                                         size_t idx)
+    {
+        if (MODE == 0) {
+            const double* pp = (const double*)part + (size_t)s * NACC * stride + idx;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) L64[k] = __builtin_nontemporal_load(&pp[k * stride]);
+        } else {
+            const float* ps = (const float*)part + (size_t)s * MROWS * stride + idx;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) L32[k] = __builtin_nontemporal_load(&ps[k * stride]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                C[k] = __builtin_nontemporal_load(&ps[(NACC32 + k) * stride]);
+        }
+    }
+    __device__ __forceinline__ void add(double (&A)[NACC + 1]) const
+    {
+#pragma unroll
+        for (int k = 0; k < NV; ++k) A[k] += MODE == 0 ? L64[k] : (double)L32[k];
+        if (MODE == 1)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) A[A_NX + k] -= (double)C[k];
+    }
+};
+
 template <int MODE, bool TS, int G>
 __device__ __forceinline__ void gather_row(const void* __restrict__ part, int S, size_t stride,
                                            size_t idx, double mscale, double (&A)[NACC + 1])
 {
-    constexpr int NV = MODE == 1 && TS ? NACC + 1 : NACC;
+    constexpr int NV = Chunk<MODE, TS>::NV;
     const int lane = threadIdx.x & 63;
     const int g = G == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 #pragma unroll
     for (int k = 0; k <= NACC; ++k) A[k] = 0.0;
-    if (MODE == 0) {
-        const double* pp = (const double*)part;
-        for (int s = g; s < S; s += G) {
-            double L[NACC];
-#pragma unroll
-            for (int k = 0; k < NACC; ++k)
-                L[k] = __builtin_nontemporal_load(&pp[(size_t)(s * NACC + k) * stride + idx]);
-            __builtin_amdgcn_sched_barrier(0);       // all of a chunk's loads in flight
-#pragma unroll
-            for (int k = 0; k < NACC; ++k) A[k] += L[k];
+    Chunk<MODE, TS> c0, c1;
+    int s = g;
+    if (G > 1)
+        for (; s + G < S; s += 2 * G) {
+            c0.load(part, s, stride, idx);
+            c1.load(part, s + G, stride, idx);
+            __builtin_amdgcn_sched_barrier(0);       // all of their loads in flight
+            c0.add(A);
+            c1.add(A);
         }
-    } else {
-        const float* pp = (const float*)part;
-        for (int s = g; s < S; s += G) {
-            const float* ps = pp + (size_t)s * MROWS * stride + idx;
-            float L[NV], C[3];
-#pragma unroll
-            for (int k = 0; k < NV; ++k)
-                L[k] = __builtin_nontemporal_load(&ps[(size_t)k * stride]);
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                C[k] = __builtin_nontemporal_load(&ps[(size_t)(NACC32 + k) * stride]);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int k = 0; k < NV; ++k) A[k] += (double)L[k];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) A[A_NX + k] -= (double)C[k];
-        }
+    for (; s < S; s += G) {
+        c0.load(part, s, stride, idx);
+        __builtin_amdgcn_sched_barrier(0);
+        c0.add(A);
+    }
+    if (MODE == 1)
 #pragma unroll
         for (int k = 0; k < NV; ++k)
             if (k <= A_UZ || k == A_KS || k == A_PHI || k == A_W3 || k == A_TS) A[k] *= mscale;
-    }
     if (G > 1) {
-        __shared__ double sh[G > 1 ? G / 2 : 1][NV][RB];
+        __shared__ double sum[G > 1 ? NV : 1][RB];
+        double v[NV], t[NSHARE<NV>];
 #pragma unroll
-        for (int h = G / 2; h >= 1; h >>= 1) {
-            if (g >= h && g < 2 * h)
+        for (int k = 0; k < NV; ++k) v[k] = A[k];
+        waves_share(v, g, lane, t);
 #pragma unroll
-                for (int k = 0; k < NV; ++k) sh[g - h][k][lane] = A[k];
-            __syncthreads();
-            if (g < h)
+        for (int q = 0; q < NSHARE<NV>; ++q)
+            if (q * PW + g < NV) sum[G > 1 ? q * PW + g : 0][lane] = t[q];
+        __syncthreads();
+        if (g == 0)
 #pragma unroll
-                for (int k = 0; k < NV; ++k) A[k] += sh[g][k][lane];
-            __syncthreads();
-        }
+            for (int k = 0; k < NV; ++k) A[k] = sum[G > 1 ? k : 0][lane];
     }
 }
 
@@ -1347,6 +1385,9 @@ struct Row {
 // inside a step (STAGE 1..3), the records and row sums of the driver's next
 // evaluation on the state the stage update gives.  Every thread calls this.
 //
+// bh (G = FG): lane k < 3 of the last wave gets the BH's component k, which
+// fin_close takes from there.
+//
 // G = FG is for few rows: one wave adding all S chunks of its stars leaves
 // most of the chip idle (at n = 10241, S = 128 that took as long as the pair
 // kernel).  With many rows the chip is full either way, and the star part
@@ -1357,7 +1398,7 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
                                          size_t idx0, const double* __restrict__ gsp,
                                          const int* __restrict__ flist,
                                          const int* __restrict__ fn, double m0, const MixPrep& M,
-                                         const Phys& P)
+                                         const Phys& P, StageIn& bh)
 {
     constexpr bool TS = STAGE <= 1;
     const int lane = threadIdx.x & 63, cap = P.cap;
@@ -1371,7 +1412,9 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
     const bool star = G == 1 ? lf < q.nst : wid == 0;   // this wave runs the star part
     int nf = 0;
     bool is_hard = false;
-    if (MODE == 1) {
+    // the BH-close and hard stars, if any
+    auto rare = [&]() {
+        if (MODE == 0) return;
         nf = *fn;
         unsigned long long any = 0ull;
 #pragma unroll
@@ -1384,23 +1427,95 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         if (nf > 0 || any)
             rare_rows(F.j64, F.in, cap, P.eps2, q.off, q.nst, q.first, G == 1 ? FG : 1,
                       R.hmask + q.row, flist, nf, F.xr);
-    }
+    };
     // everything the star part reads, requested ahead of the partial sums
-    StageIn st, b0;
-    double gs[NGS], mp = 0.0, D2 = 0.0, e = 0.0;
+    StageIn st;
+    double gs[NGS], mp = 0.0, D2 = 0.0, e = 0.0, x0[3], x0n[3];
     float kr = 0.0f;
-    if (star) {
-        D2 = F.j64[p].D2;
-        e = F.j64[p].e;
-        st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, p);
-        b0 = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, q.off);
-        mp = F.m[p];
-#pragma unroll
-        for (int k = 0; k < NGS; ++k) gs[k] = gsp[k];
-        if (MODE == 1 && !TS) kr = F.kr[p];
-    }
     double A[NACC + 1];
-    if (G > 1 || star) gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+    if (G == 1) {
+        rare();
+        if (star) {
+            D2 = F.j64[p].D2;
+            e = F.j64[p].e;
+            st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, p);
+            const StageIn b0 = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, q.off);
+            mp = F.m[p];
+#pragma unroll
+            for (int k = 0; k < NGS; ++k) gs[k] = gsp[k];
+            if (MODE == 1 && !TS) kr = F.kr[p];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                x0[k] = b0.x[k];
+                x0n[k] = stage_pos<STAGE>(b0, P.dt, k);
+            }
+            gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+        }
+    } else {
+        // Row r of what the star part reads of its star: components of in, X,
+        // H1 and H2 as the stage needs them, the mass, D2 and e.  Wave w
+        // fetches rows w, w + FG, ... beside its partial sums, the last wave
+        // also the BH's state and the separable sums (by lane: as scalar loads
+        // they would queue, one line each, behind one another), all through
+        // LDS; one trip to memory in all.
+        constexpr int NST = STAGE == 3 ? 24 : STAGE == 2 ? 12 : 6, NR = NST + 3;
+        constexpr int NL = (NR + FG - 1) / FG;
+        __shared__ double pre[NR][RB], uni[6 + NGS];
+        double ld[NL], g0 = 0.0;
+#pragma unroll
+        for (int t = 0; t < NL; ++t) {
+            const int r = wid + t * FG;
+            ld[t] = 0.0;
+            if (r < NST) {
+                const double* b = r < 6 ? F.in : r < 12 ? F.X : r < 18 ? F.H1 : F.H2;
+                ld[t] = b[(size_t)(r % 6) * cap + p];
+            } else if (r < NR) {
+                const double* b = r == NST ? F.m + p
+                                           : r == NST + 1 ? &F.j64[p].D2 : &F.j64[p].e;
+                ld[t] = *b;
+            }
+        }
+        if (MODE == 1 && !TS && wid == 0) kr = F.kr[p];
+        if (wid == FG - 1) {
+            if (lane < 3) bh = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, cap, q.off, lane, 1);
+            if (lane < NGS) g0 = gsp[lane];
+        }
+        rare();
+        gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+#pragma unroll
+        for (int t = 0; t < NL; ++t)
+            if (wid + t * FG < NR) pre[wid + t * FG][lane] = ld[t];
+        if (wid == FG - 1) {
+            if (lane < 3) {
+                uni[lane] = bh.x[0];
+                uni[3 + lane] = stage_pos<STAGE>(bh, P.dt, 0);
+            }
+            if (lane < NGS) uni[6 + lane] = g0;
+        }
+        __syncthreads();
+        if (star) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                st.x[k] = pre[k][lane];
+                st.v[k] = pre[3 + k][lane];
+                if (STAGE >= 2) {
+                    st.X[k] = pre[STAGE >= 2 ? 6 + k : 0][lane];
+                    st.V[k] = pre[STAGE >= 2 ? 9 + k : 0][lane];
+                }
+                if (STAGE == 3) {
+                    st.hx[k] = pre[STAGE == 3 ? 12 + k : 0][lane] + pre[STAGE == 3 ? 18 + k : 0][lane];
+                    st.hv[k] = pre[STAGE == 3 ? 15 + k : 0][lane] + pre[STAGE == 3 ? 21 + k : 0][lane];
+                }
+                x0[k] = to_scalar(uni[k]);
+                x0n[k] = to_scalar(uni[3 + k]);
+            }
+            mp = pre[NST][lane];
+            D2 = pre[NST + 1][lane];
+            e = pre[NST + 2][lane];
+#pragma unroll
+            for (int k = 0; k < NGS; ++k) gs[k] = to_scalar(uni[6 + k]);
+        }
+    }
     if (MODE == 1 && star && ok && (is_hard || nf > 0)) {
         // a hard star: its FP64 row instead of the gathered sums; another
         // one: plus its pairs with the BH-close stars
@@ -1412,16 +1527,14 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
     double cb[3] = {0.0, 0.0, 0.0}, a[3], nx[3], nv[3], g[NGS];
     bool f = false, hard = false;
     if (ok) {
-        fin_star<STAGE>(st, b0.x, mp, D2, e, F.X, F.Y, F.H1, F.H2, cap, p, A, gs,
+        fin_star<STAGE>(st, x0, mp, D2, e, F.X, F.Y, F.H1, F.H2, cap, p, A, gs,
                         fin_consts(P, m0), F.acc, cb, a, nx, nv);
         if (MODE == 1 && TS) {
             kr = cancel_ratio(A[NACC], a);
             F.kr[p] = kr;
         }
         if (STAGE > 0) {
-            const double x0[3] = {stage_pos<STAGE>(b0, P.dt, 0), stage_pos<STAGE>(b0, P.dt, 1),
-                                  stage_pos<STAGE>(b0, P.dt, 2)};
-            f = prep_star(nx, nv, x0, mp, p, m0, P.eps2, F.jnext, g, M, true, a, kr, hard);
+            f = prep_star(nx, nv, x0n, mp, p, m0, P.eps2, F.jnext, g, M, true, a, kr, hard);
         }
     }
     put_row<true, (STAGE > 0)>(q.row + mine, ok, cb, g, R.rows, MODE == 1, f, hard, R.fmask,
@@ -1440,24 +1553,24 @@ __device__ __forceinline__ void empty_row(const RowBufs& R, int row, bool mixed)
 
 // After the last row of an evaluation: the BH at b0, its acceleration Newton
 // sum_j m_j e_j^3 d_j plus lam times the rows' shares and its stage update
-// (thread k: component k), and the next evaluation's separable sums and
-// BH-close list.
-template <int MODE, int STAGE>
+// (lane k of a wave: component k), and the next evaluation's separable sums and
+// BH-close list.  PRE: the last wave holds the BH's state already (bh).
+template <int MODE, int STAGE, bool PRE>
 __device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, int b0row,
                                           int b1row, int b0, double* __restrict__ gs,
                                           int* __restrict__ flist, int* __restrict__ fn,
-                                          const Phys& P)
+                                          const Phys& P, const StageIn& bh)
 {
     __shared__ double tot[RV];
-    const int t = threadIdx.x;
-    StageIn st;
+    const int t = (int)threadIdx.x - (PRE ? (FG - 1) * 64 : 0);
+    StageIn st = bh;
     double nwt = 0.0;
-    if (t < 3) {
-        st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, P.cap, b0, t, 1);
+    if (t >= 0 && t < 3) {
+        if (!PRE) st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, P.cap, b0, t, 1);
         nwt = gs[G_M1X + t];
     }
     rows_total(R.rows, b0row, b1row, tot);
-    if (t < 3) {
+    if (t >= 0 && t < 3) {
         double nx, nv;
         const double a = nwt + P.lam * tot[t];
         F.acc[(size_t)t * P.cap + b0] = a;
@@ -1465,7 +1578,7 @@ __device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, in
     }
     if (STAGE > 0) {
         __syncthreads();                       // gs has been read
-        if (t < NGS) gs[t] = tot[RV_G + t];
+        if (threadIdx.x < NGS) gs[threadIdx.x] = tot[RV_G + threadIdx.x];
         if (MODE == 1) list_flagged(R.fmask, b0row, b1row, b0 + 1, flist, fn);
     }
 }
@@ -1479,13 +1592,18 @@ void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M
 {
     const int row = row0 + (int)blockIdx.x * (G == 1 ? FG : 1);
     const Row q = {0, p1 - 1, row * RB, row};
+    StageIn bh = {};
     if (P.n > 1)
         fin_rows<MODE, STAGE, G>(F, R, q, part, S, (size_t)P.cap, 1, R.gs, R.flist, R.fn, F.m[0],
-                                 M, P);
+                                 M, P, bh);
     else
         empty_row(R, 0, MODE == 1);
-    if (R.ticket && last_block(R.ticket, gridDim.x))
-        fin_close<MODE, STAGE>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P);
+    if (R.ticket && last_block(R.ticket, gridDim.x)) {
+        if (G > 1 && P.n > 1)
+            fin_close<MODE, STAGE, true>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
+        else
+            fin_close<MODE, STAGE, false>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
+    }
 }
 
 // k_fin of pn1_force_noalloc (FP64, G = FG): every workgroup adds the separable
@@ -1499,13 +1617,14 @@ void k_fin_na(FinBufs F, RowBufs R, const double* __restrict__ prows,
     __shared__ double tot[RV];
     rows_total(prows, 0, nrow, tot);
     const Row q = {0, P.n - 1, (int)blockIdx.x * RB, (int)blockIdx.x};
+    StageIn bh = {};
     if (P.n > 1)
         fin_rows<0, 0, FG>(F, R, q, part, S, (size_t)P.cap, 1, tot + RV_G, nullptr, nullptr,
-                           F.m[0], MixPrep{}, P);
+                           F.m[0], MixPrep{}, P, bh);
     else
         empty_row(R, 0, false);
     if (last_block(R.ticket, gridDim.x))
-        fin_close<0, 0>(F, R, 0, nrow, 0, tot + RV_G, nullptr, nullptr, P);
+        fin_close<0, 0, false>(F, R, 0, nrow, 0, tot + RV_G, nullptr, nullptr, P, bh);
 }
 
 // ---------------------------------------------------------------------

@@ -49,6 +49,34 @@ __device__ __forceinline__ double swap_sum(double a, double b)
     return x + y;
 }
 
+// A value that is the same in all lanes, in scalar registers.
+__device__ __forceinline__ double to_scalar(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// v of lane l ^ X, X = 1, 2, 4 or 8, by DPP (a ds_bpermute shuffle takes over 100 cycles).
+template <int X>
+__device__ __forceinline__ int lane_xor(int v)
+{
+    if (X == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);      // quad 1 0 3 2
+    if (X == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);      // quad 2 3 0 1
+    if (X == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);     // row_ror 8
+    v = __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);                    // l ^ 7, then
+    return __builtin_amdgcn_mov_dpp(v, 0x1B, 0xF, 0xF, true);                  // quad 3 2 1 0
+}
+template <int X>
+__device__ __forceinline__ double lane_xor(double v)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = (unsigned)lane_xor<X>((int)(unsigned)u);
+    const unsigned hi = (unsigned)lane_xor<X>((int)(unsigned)(u >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // The wave's sums of 16 values: lane l gets the sum of v[l >> 2] over all
 // lanes.  Halving the values at each exchange takes 15 of them instead of
 // the 16 x 6 of one butterfly per value, and half the code, which in kernels
@@ -65,12 +93,12 @@ __device__ __forceinline__ double wave_sums16(const double (&v)[16])
     for (int k = 0; k < 2; ++k) {
         const bool up = lane & 8;
         const double keep = up ? b[2 + k] : b[k], send = up ? b[k] : b[2 + k];
-        c[k] = keep + __shfl_xor(send, 8, 64);
+        c[k] = keep + lane_xor<8>(send);
     }
     const bool up = lane & 4;
-    double t = (up ? c[1] : c[0]) + __shfl_xor(up ? c[0] : c[1], 4, 64);
-    t += __shfl_xor(t, 2, 64);
-    t += __shfl_xor(t, 1, 64);
+    double t = (up ? c[1] : c[0]) + lane_xor<4>(up ? c[0] : c[1]);
+    t += lane_xor<2>(t);
+    t += lane_xor<1>(t);
     return t;
 }
 
