@@ -215,6 +215,9 @@ bool quad_pairs(const pn1_ctx* c, int S)
 // Partials per star of a launch of the 256-star kernels split in S chunks.
 int part_slots(const pn1_ctx* c, int S) { return quad_pairs(c, S) ? S / QSUB : S; }
 
+// The plan's.
+int plan_slots(const pn1_ctx* c) { return c->slots ? c->slots : part_slots(c, c->S); }
+
 // Workgroups of a pair launch over nib i blocks with `slots` chunks each
 // (map_block's arrangement when slots divides 8).
 int pair_grid(int slots, int nib)
@@ -284,9 +287,17 @@ MixPrep mix_prep(const pn1_ctx* c, const Phys& P)
     return M;
 }
 
-// Waves per row of k_fin: FG up to FIN_ROWS rows, which one wave per row
-// would leave most of the chip idle on; 1 above.
-constexpr int FIN_ROWS = 1024;
+// k_fin's form: a workgroup per row up to FIN_ROWS rows, per FG rows above (see
+// fin_rows); per group of 16 stars where few rows have many partials each.
+// Measured on MI355X, evaluation with a workgroup per row / per group, FP64
+// and mixed, us:
+//   n = 33 (1 partial)  11.3 / 12.2  14.7 / 16.1
+//   n = 257 (8)         14.4 / 13.4  17.5 / 16.6
+//   n = 1025 (16)       17.6 / 16.0  19.5 / 19.6
+//   n = 2049 (16)       23.6 / 23.2  23.7 / 24.0
+//   n = 8193 (24)       120.4 / 123.4  77.9 / 84.5
+constexpr int FIN_ROWS = 1024, FIN_SUB = 16;
+bool fin_sub(int nst, int nrow, int slots) { return nst > 0 && nrow <= FIN_SUB && slots >= FG; }
 
 // Stars i0 .. i1 - 1 (all: every star and the BH), `slots` partials each.
 template <int MODE, int STAGE>
@@ -306,13 +317,16 @@ void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, 
     F.jnext = rec_buf(c, STAGE % 3);
     const int row0 = (i0 - 1) / RB, rows = std::max(1, (i1 - i0 + RB - 1) / RB);
     const RowBufs R = row_bufs(c, all);
-    if (c->nrow <= FIN_ROWS)
-        hipLaunchKernelGGL((k_fin<MODE, STAGE, FG>), dim3(rows), dim3(FWG), 0, c->st, F, R,
-                           (const void*)c->part, slots, mix_prep(c, P), P, row0, i1, c->nrow);
+    auto launch = [&](auto kernel, int wgs) {
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(FWG), 0, c->st, F, R, (const void*)c->part,
+                           slots, mix_prep(c, P), P, row0, i1, c->nrow);
+    };
+    if (fin_sub(c->n - 1, c->nrow, slots))
+        launch(k_fin<MODE, STAGE, FG, 4>, 4 * rows);
+    else if (c->nrow <= FIN_ROWS)
+        launch(k_fin<MODE, STAGE, FG, 1>, rows);
     else
-        hipLaunchKernelGGL((k_fin<MODE, STAGE, 1>), dim3((rows + FG - 1) / FG), dim3(FWG), 0,
-                           c->st, F, R, (const void*)c->part, slots, mix_prep(c, P), P, row0, i1,
-                           c->nrow);
+        launch(k_fin<MODE, STAGE, 1, 1>, (rows + FG - 1) / FG);
 }
 
 // The pair kernel over i blocks ib0 .. ib0 + nib - 1 against every star,
@@ -353,9 +367,12 @@ int prep_x(pn1_ctx* c, const Phys& P, bool fp64)
     MixPrep M = mix_prep(c, P);
     if (fp64) M.j32 = nullptr;
     const bool prev = M.j32 && c->acc_ok;
-    hipLaunchKernelGGL(k_prep, dim3((c->nrow + FG - 1) / FG), dim3(FWG), 0, c->st,
-                       (const double*)c->X, c->m, P, c->nrow, rec_buf(c, 0), row_bufs(c), M,
-                       prev ? (const double*)c->acc : nullptr, prev ? (const float*)c->kr : nullptr);
+    // (the energy's sums do not depend on the plan)
+    const bool sub = !fp64 && fin_sub(c->n - 1, c->nrow, plan_slots(c));
+    hipLaunchKernelGGL(sub ? k_prep<4> : k_prep<1>, dim3((c->nrow + FG - 1) / FG), dim3(FWG), 0,
+                       c->st, (const double*)c->X, (const double*)c->m, P, c->nrow, rec_buf(c, 0),
+                       row_bufs(c), M, prev ? (const double*)c->acc : nullptr,
+                       prev ? (const float*)c->kr : nullptr);
     HIPCHK(c, hipGetLastError());
     return PN1_OK;
 }
@@ -367,7 +384,7 @@ int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
 {
     const double* in = stage <= 1 ? c->X : c->Y;
     const bool mixed = c->mode == PN1_MIXED;
-    const int slots = c->slots ? c->slots : part_slots(c, c->S);
+    const int slots = plan_slots(c);
     if (c->n > 1) {
         hipEvent_t e1 = nullptr;
         if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
@@ -523,8 +540,9 @@ constexpr size_t NA_J64 = 0;
 constexpr size_t NA_PART =
     NA_J64 + na_round((size_t)PN1_NOALLOC_MAX_N * (sizeof(JRec64) / sizeof(double)));
 constexpr size_t NA_PROWS = NA_PART + na_round((size_t)TLONG * NACC * PN1_NOALLOC_MAX_N);
-constexpr size_t NA_ROWS = NA_PROWS + na_round((size_t)NA_MAXB * RV);
-constexpr size_t NA_TICKET = NA_ROWS + na_round((size_t)NA_MAXB * RV);
+constexpr size_t NA_ROWV = na_round((size_t)std::max(NA_MAXB, 4 * FIN_SUB) * RV);
+constexpr size_t NA_ROWS = NA_PROWS + NA_ROWV;
+constexpr size_t NA_TICKET = NA_ROWS + NA_ROWV;
 constexpr size_t NA_TOTAL = NA_TICKET + na_round(1);
 static_assert(sizeof(JRec64) % sizeof(double) == 0, "JRec64 in doubles");
 
@@ -636,7 +654,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->H2, 6 * cap);
     if (!rc) rc = dalloc(c, &c->m, cap);
     if (!rc) rc = dalloc(c, &c->acc, 3 * cap);
-    if (!rc) rc = dalloc(c, &c->rows, nr * RV);
+    if (!rc) rc = dalloc(c, &c->rows, std::max(nr, (size_t)4 * FIN_SUB) * RV);
     if (!rc) rc = dalloc(c, &c->gs, 16);
     if (!rc) rc = dalloc(c, &c->eblk, nr * ECHUNK * EV);
     // two records more than particles: the pair loops fetch up to jr[j + 2]
@@ -1045,8 +1063,11 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
     const int S = na_split(nst);
     // (the rows hold fewer than 2^22 / 16 stars here: S = 1 alone is not theirs)
     const int slots = explicit_slots(S, nst);
-    hipLaunchKernelGGL(k_prep, dim3((nrow + FG - 1) / FG), dim3(FWG), 0, s, st, m, P, nrow, j64, R,
-                       MixPrep{}, (const double*)nullptr, (const float*)nullptr);
+    const int parts = slots ? slots : S;
+    const bool sub = fin_sub(nst, nrow, parts);
+    hipLaunchKernelGGL(sub ? k_prep<4> : k_prep<1>, dim3((nrow + FG - 1) / FG), dim3(FWG), 0, s,
+                       st, m, P, nrow, j64, R, MixPrep{}, (const double*)nullptr,
+                       (const float*)nullptr);
     if (slots)
         hipLaunchKernelGGL(k_pair64w, dim3(slots * nrow), dim3(PW * RB), 0, s, (const JRec64*)j64,
                            st, part, P, slots, nrow, 0);
@@ -1055,8 +1076,8 @@ int pn1_force_noalloc(const double* st, const double* m, int n, double eps, doub
                            (const JRec64*)j64, st, part, P, S, nib, 0);
     R.rows = base + NA_ROWS;
     R.ticket = (unsigned int*)(base + NA_TICKET);
-    hipLaunchKernelGGL(k_fin_na, dim3(nrow), dim3(FWG), 0, s, F, R,
-                       (const double*)(base + NA_PROWS), (const void*)part, slots ? slots : S, P,
+    hipLaunchKernelGGL(sub ? k_fin_na<4> : k_fin_na<1>, dim3(sub ? 4 * nrow : nrow), dim3(FWG), 0,
+                       s, F, R, (const double*)(base + NA_PROWS), (const void*)part, parts, P,
                        nrow);
     return hipGetLastError() == hipSuccess ? PN1_OK : PN1_EDEVICE;
 }

@@ -328,7 +328,7 @@ inline __global__ __launch_bounds__(FWG) void k_ens_prep(const double* __restric
                           kr, hard);
         }
         const double cb[3] = {0.0, 0.0, 0.0};
-        put_row<false, true>(row, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
+        put_row<false, true>(row, 0, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
                              R.hmask);
     }
     if (last_block(R.ticket + b.c, (unsigned)((r1 - r0 + FG - 1) / FG)))
@@ -358,17 +358,17 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
     if (nst > 0) {
         const void* base = MODE == 0 ? (const void*)((const double*)part + poff[b.c] * NACC)
                                      : (const void*)((const float*)part + poff[b.c] * MROWS);
-        fin_rows<MODE, STAGE, G>(F, R, q, base, ens_nchunks(nst, L), (size_t)nst, 0, gs,
-                                 R.flist + off, R.fn + b.c, E.cm0[b.c], M, P, bh);
+        fin_rows<MODE, STAGE, G, 1>(F, R, q, base, ens_nchunks(nst, L), (size_t)nst, 0, gs,
+                                 R.flist + off, R.fn + b.c, E.cm0[b.c], M, P, bh, 0);
     } else {
-        empty_row(R, q.row, MODE == 1);
+        empty_row<1>(R, q.row, MODE == 1);
     }
     const unsigned nblk = (unsigned)(G == 1 ? (r1 - r0 + FG - 1) / FG : r1 - r0);
     if (last_block(R.ticket + b.c, nblk)) {
         if (G > 1 && nst > 0)
-            fin_close<MODE, STAGE, true>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
+            fin_close<MODE, STAGE, true, 1>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
         else
-            fin_close<MODE, STAGE, false>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
+            fin_close<MODE, STAGE, false, 1>(F, R, r0, r1, off, gs, R.flist + off, R.fn + b.c, P, bh);
     }
 }
 

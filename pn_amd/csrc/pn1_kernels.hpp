@@ -218,8 +218,10 @@ __device__ __forceinline__ bool prep_star(const double (&xp)[3], const double (&
 // One row of stars' share of the sums over all stars, by its wave (ok: the
 // lane holds a star): the BH shares cb (BH) and the separable sums g (NEXT),
 // and, in the mixed form, the bit masks of its BH-close and its hard stars.
-template <bool BH, bool NEXT>
-__device__ __forceinline__ void put_row(int row, bool ok, const double (&cb)[3],
+// Q = 4: the share of each of its groups of 16 stars apart; `sub` >= 0: of that
+// group only, which lanes 0 .. 15 hold.
+template <bool BH, bool NEXT, int Q = 1>
+__device__ __forceinline__ void put_row(int row, int sub, bool ok, const double (&cb)[3],
                                         const double (&g)[NGS], double* __restrict__ rows,
                                         bool mixed, bool flagged, bool hard,
                                         unsigned long long* __restrict__ fmask,
@@ -237,14 +239,26 @@ __device__ __forceinline__ void put_row(int row, bool ok, const double (&cb)[3],
 #pragma unroll
             for (int k = 0; k < NGS; ++k) v[RV_G + k] = g[k];
     }
-    const double t = wave_sums16(v);
-    if ((lane & 3) == 0) hand_over(&rows[(size_t)row * RV + (lane >> 2)], t);
+    if (Q == 1) {
+        const double t = wave_sums16(v);
+        if ((lane & 3) == 0) hand_over(&rows[(size_t)row * RV + (lane >> 2)], t);
+    } else {
+        const double t = group_sums16(v);
+        const int grp = sub < 0 ? lane / RV : sub;
+        if (sub < 0 || lane < RV)
+            hand_over(&rows[((size_t)row * Q + grp) * RV + (lane & (RV - 1))], t);
+    }
     if (NEXT && mixed) {
         const unsigned long long f = __builtin_amdgcn_ballot_w64(ok && flagged);
         const unsigned long long h = __builtin_amdgcn_ballot_w64(ok && hard);
         if (lane == 0) {
-            hand_over(&fmask[row], f);
-            hmask[row] = h;
+            if (Q == 1 || sub < 0) {
+                hand_over(&fmask[row], f);
+                hmask[row] = h;
+            } else {
+                hand_over((unsigned short*)&fmask[row] + sub, (unsigned short)f);
+                ((unsigned short*)&hmask[row])[sub] = (unsigned short)h;
+            }
         }
     }
 }
@@ -311,12 +325,13 @@ struct RowBufs {
 
 // After the last row of a prep: the separable sums, and the BH-close list of
 // rows [b0, b1) (p0: row b0's first star).
+template <int Q = 1>
 __device__ __forceinline__ void close_prep(const RowBufs& R, bool mixed, int b0, int b1, int p0,
                                            double* __restrict__ gs, int* __restrict__ flist,
                                            int* __restrict__ fn)
 {
     __shared__ double tot[RV];
-    rows_total(R.rows, b0, b1, tot);
+    rows_total<Q>(R.rows, b0, b1, tot);
     if (threadIdx.x < NGS) gs[threadIdx.x] = tot[RV_G + threadIdx.x];
     if (mixed) list_flagged(R.fmask, b0, b1, p0, flist, fn);
 }
@@ -324,8 +339,10 @@ __device__ __forceinline__ void close_prep(const RowBufs& R, bool mixed, int b0,
 // Records, separable sums and (mixed form) thresholds, BH-close and hard
 // stars of the state st.  aprev, kprev (mixed form): each star's previous
 // acceleration (SoA [3][cap]) and cancellation ratio, null after an upload.
-// The BH mass is m[0].
-inline __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ st,
+// The BH mass is m[0].  Q: the groups whose sums k_fin adds up (one order in
+// both, so that a step call continues another bit for bit).
+template <int Q>
+__global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ st,
                                              const double* __restrict__ m, Phys P, int nrow,
                                              JRec64* __restrict__ j64, RowBufs R, MixPrep M,
                                              const double* __restrict__ aprev,
@@ -355,11 +372,11 @@ inline __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ 
                           hard);
         }
         const double cb[3] = {0.0, 0.0, 0.0};
-        put_row<false, true>(row, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
+        put_row<false, true, Q>(row, -1, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
                              R.hmask);
     }
     if (R.ticket && last_block(R.ticket, gridDim.x))
-        close_prep(R, M.j32 != nullptr, 0, nrow, 1, R.gs, R.flist, R.fn);
+        close_prep<Q>(R, M.j32 != nullptr, 0, nrow, 1, R.gs, R.flist, R.fn);
 }
 
 // ---------------------------------------------------------------------
@@ -1116,6 +1133,8 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
                                                     double eps2, int off, int nst, int first,
                                                     int nrow,
                                                     const unsigned long long* __restrict__ hmask,
+                                                    int shift, unsigned long long width,
+                                                    int nall,
                                                     const int* __restrict__ flist, int nf,
                                                     double* __restrict__ x)
 {
@@ -1142,7 +1161,7 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
         x[(size_t)NACC * cap + i] = ts;
     }
     for (int r = 0; r < nrow && first + r * RB < nst; ++r) {
-        unsigned long long hm = hmask[r];
+        unsigned long long hm = (hmask[r] >> shift) & width;
         while (hm) {
             const int h = r * RB + __builtin_ctzll(hm), i = off + 1 + first + h;
             hm &= hm - 1;
@@ -1150,7 +1169,7 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
             ts = 0.0;
 #pragma unroll
             for (int k = 0; k < NACC; ++k) a[k] = 0.0;
-            for (int j = off + 1 + (int)threadIdx.x; j <= off + nst; j += FWG) pair(j, i, I);
+            for (int j = off + 1 + (int)threadIdx.x; j <= off + nall; j += FWG) pair(j, i, I);
 #pragma unroll
             for (int k = 0; k <= NACC; ++k) {
                 const double t = wave_sum(k < NACC ? a[k] : ts);
@@ -1253,6 +1272,56 @@ __device__ __forceinline__ void gather_row(const void* __restrict__ part, int S,
 #pragma unroll
             for (int k = 0; k < NV; ++k) A[k] = sum[G > 1 ? k : 0][lane];
     }
+}
+
+// The same for 16 stars by the FG waves of a workgroup: lane l has star l % 16,
+// and its quarter of wave w adds chunks 4 w + l / 16, ... + 4 FG, ...; the
+// sums over chunks are in every quarter of wave 0.
+template <int MODE, bool TS>
+__device__ __forceinline__ void gather_sub(const void* __restrict__ part, int S, size_t stride,
+                                           size_t idx, double mscale, double (&A)[NACC + 1])
+{
+    constexpr int NV = Chunk<MODE, TS>::NV, RS = 16;
+    __shared__ double sh[FG][NV][RS], sum[NV][RS];
+    const int lane = threadIdx.x & 63, ls = lane % RS;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nw = min(FG, (S + 3) / 4);             // waves with a chunk
+#pragma unroll
+    for (int k = 0; k <= NACC; ++k) A[k] = 0.0;
+    if (wid < nw) {
+        for (int s = wid * 4 + lane / RS; s < S; s += 4 * FG) {
+            Chunk<MODE, TS> c;
+            c.load(part, s, stride, idx);
+            __builtin_amdgcn_sched_barrier(0);
+            c.add(A);
+        }
+        // quarter q of the wave: values 8 (q / 2) + 4 (q % 2) + 0 .. 3
+        double a[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) a[k] = swap_sum<32>(A[k], A[8 + k]);
+        const int v0 = 8 * (lane >> 5) + 4 * ((lane >> 4) & 1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sh[wid][v0 + k][ls] = swap_sum<16>(a[k], a[4 + k]);
+        if (NV > NACC) {
+            double t = A[NACC];
+            t += __shfl_xor(t, 32, 64);
+            t += __shfl_xor(t, 16, 64);
+            if (lane < RS) sh[wid][NV - 1][ls] = t;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < NV * RS) {
+        const int k = threadIdx.x / RS;
+        double t = sh[0][k][ls];
+        for (int w = 1; w < nw; ++w) t += sh[w][k][ls];
+        if (MODE == 1)
+            if (k <= A_UZ || k == A_KS || k == A_PHI || k == A_W3 || k == A_TS) t *= mscale;
+        sum[k][ls] = t;
+    }
+    __syncthreads();
+    if (wid == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) A[k] = sum[k][ls];
 }
 
 // Mixed form: the star's cancellation ratio for the next evaluation's
@@ -1388,26 +1457,31 @@ struct Row {
 // bh (G = FG): lane k < 3 of the last wave gets the BH's component k, which
 // fin_close takes from there.
 //
+// Q = 4 (with G = FG): group `sub` of 16 stars of row q.row only.  At n = 1025
+// a row's 16 chunks of partials are 131 KB, which one CU reads in 4 us of
+// k_fin's 9.5 (MI355X, by its clock); its four quarters go to four CUs.
+//
 // G = FG is for few rows: one wave adding all S chunks of its stars leaves
 // most of the chip idle (at n = 10241, S = 128 that took as long as the pair
 // kernel).  With many rows the chip is full either way, and the star part
 // behind the gather, which one wave runs, counts: G = 1 keeps all FG busy.
-template <int MODE, int STAGE, int G>
+template <int MODE, int STAGE, int G, int Q>
 __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, const Row& q,
                                          const void* __restrict__ part, int S, size_t stride,
                                          size_t idx0, const double* __restrict__ gsp,
                                          const int* __restrict__ flist,
                                          const int* __restrict__ fn, double m0, const MixPrep& M,
-                                         const Phys& P, StageIn& bh)
+                                         const Phys& P, StageIn& bh, int sub)
 {
     constexpr bool TS = STAGE <= 1;
+    constexpr int RS = RB / Q;                      // stars per wave of the star part
     const int lane = threadIdx.x & 63, cap = P.cap;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int mine = G == 1 ? wid : 0;              // this wave's row of the workgroup's
-    const int lf = q.first + mine * RB;             // its first star
-    const int li = lf + lane;
-    const bool ok = li < q.nst;
-    const int lc = ok ? li : min(q.first, q.nst - 1);
+    const int lf = q.first + mine * RB + sub * RS;  // its first star
+    const int li = lf + lane % RS;
+    const bool ok = li < q.nst && lane < RS;
+    const int lc = li < q.nst ? li : min(q.first, q.nst - 1);
     const int p = q.off + 1 + lc;
     const bool star = G == 1 ? lf < q.nst : wid == 0;   // this wave runs the star part
     int nf = 0;
@@ -1420,13 +1494,15 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
 #pragma unroll
         for (int r = 0; r < (G == 1 ? FG : 1); ++r)
             if (q.first + r * RB < q.nst) {
-                const unsigned long long hm = R.hmask[q.row + r];
+                unsigned long long hm = R.hmask[q.row + r];
+                if (Q > 1) hm = (hm >> (sub * RS)) & 0xffffu;
                 any |= hm;
                 if (r == mine) is_hard = (hm >> lane) & 1;
             }
         if (nf > 0 || any)
-            rare_rows(F.j64, F.in, cap, P.eps2, q.off, q.nst, q.first, G == 1 ? FG : 1,
-                      R.hmask + q.row, flist, nf, F.xr);
+            rare_rows(F.j64, F.in, cap, P.eps2, q.off, Q > 1 ? min(q.nst, lf + RS) : q.nst,
+                      Q > 1 ? lf : q.first, G == 1 ? FG : 1, R.hmask + q.row, sub * RS,
+                      Q > 1 ? 0xffffull : ~0ull, q.nst, flist, nf, F.xr);
     };
     // everything the star part reads, requested ahead of the partial sums
     StageIn st;
@@ -1459,12 +1535,13 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         // they would queue, one line each, behind one another), all through
         // LDS; one trip to memory in all.
         constexpr int NST = STAGE == 3 ? 24 : STAGE == 2 ? 12 : 6, NR = NST + 3;
-        constexpr int NL = (NR + FG - 1) / FG;
-        __shared__ double pre[NR][RB], uni[6 + NGS];
+        constexpr int H = FG * Q, NL = (NR + H - 1) / H;
+        const int h = wid * Q + (Q == 1 ? 0 : lane / RS);
+        __shared__ double pre[NR][RS], uni[6 + NGS];
         double ld[NL], g0 = 0.0;
 #pragma unroll
         for (int t = 0; t < NL; ++t) {
-            const int r = wid + t * FG;
+            const int r = h + t * H;
             ld[t] = 0.0;
             if (r < NST) {
                 const double* b = r < 6 ? F.in : r < 12 ? F.X : r < 18 ? F.H1 : F.H2;
@@ -1481,10 +1558,14 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
             if (lane < NGS) g0 = gsp[lane];
         }
         rare();
-        gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+        if (Q == 1)
+            gather_row<MODE, TS, G>(part, S, stride, idx0 + lc, M.mmax, A);
+        else
+            gather_sub<MODE, TS>(part, S, stride, idx0 + lc, M.mmax, A);
+        const int ls = Q == 1 ? lane : lane % RS;
 #pragma unroll
         for (int t = 0; t < NL; ++t)
-            if (wid + t * FG < NR) pre[wid + t * FG][lane] = ld[t];
+            if (h + t * H < NR) pre[h + t * H][ls] = ld[t];
         if (wid == FG - 1) {
             if (lane < 3) {
                 uni[lane] = bh.x[0];
@@ -1496,22 +1577,22 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         if (star) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                st.x[k] = pre[k][lane];
-                st.v[k] = pre[3 + k][lane];
+                st.x[k] = pre[k][ls];
+                st.v[k] = pre[3 + k][ls];
                 if (STAGE >= 2) {
-                    st.X[k] = pre[STAGE >= 2 ? 6 + k : 0][lane];
-                    st.V[k] = pre[STAGE >= 2 ? 9 + k : 0][lane];
+                    st.X[k] = pre[STAGE >= 2 ? 6 + k : 0][ls];
+                    st.V[k] = pre[STAGE >= 2 ? 9 + k : 0][ls];
                 }
                 if (STAGE == 3) {
-                    st.hx[k] = pre[STAGE == 3 ? 12 + k : 0][lane] + pre[STAGE == 3 ? 18 + k : 0][lane];
-                    st.hv[k] = pre[STAGE == 3 ? 15 + k : 0][lane] + pre[STAGE == 3 ? 21 + k : 0][lane];
+                    st.hx[k] = pre[STAGE == 3 ? 12 + k : 0][ls] + pre[STAGE == 3 ? 18 + k : 0][ls];
+                    st.hv[k] = pre[STAGE == 3 ? 15 + k : 0][ls] + pre[STAGE == 3 ? 21 + k : 0][ls];
                 }
                 x0[k] = to_scalar(uni[k]);
                 x0n[k] = to_scalar(uni[3 + k]);
             }
-            mp = pre[NST][lane];
-            D2 = pre[NST + 1][lane];
-            e = pre[NST + 2][lane];
+            mp = pre[NST][ls];
+            D2 = pre[NST + 1][ls];
+            e = pre[NST + 2][ls];
 #pragma unroll
             for (int k = 0; k < NGS; ++k) gs[k] = to_scalar(uni[6 + k]);
         }
@@ -1537,14 +1618,15 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
             f = prep_star(nx, nv, x0n, mp, p, m0, P.eps2, F.jnext, g, M, true, a, kr, hard);
         }
     }
-    put_row<true, (STAGE > 0)>(q.row + mine, ok, cb, g, R.rows, MODE == 1, f, hard, R.fmask,
+    put_row<true, (STAGE > 0), Q>(q.row + mine, sub, ok, cb, g, R.rows, MODE == 1, f, hard, R.fmask,
                                R.hmask);
 }
 
-// A cluster without stars: its one row of zeros.
+// A cluster without stars: its one row of zeros (all Q groups of it).
+template <int Q>
 __device__ __forceinline__ void empty_row(const RowBufs& R, int row, bool mixed)
 {
-    if (threadIdx.x < RV) hand_over(&R.rows[(size_t)row * RV + threadIdx.x], 0.0);
+    if (threadIdx.x < RV * Q) hand_over(&R.rows[(size_t)row * Q * RV + threadIdx.x], 0.0);
     if (mixed && threadIdx.x == 0) {
         hand_over(&R.fmask[row], 0ull);
         R.hmask[row] = 0ull;
@@ -1555,7 +1637,7 @@ __device__ __forceinline__ void empty_row(const RowBufs& R, int row, bool mixed)
 // sum_j m_j e_j^3 d_j plus lam times the rows' shares and its stage update
 // (lane k of a wave: component k), and the next evaluation's separable sums and
 // BH-close list.  PRE: the last wave holds the BH's state already (bh).
-template <int MODE, int STAGE, bool PRE>
+template <int MODE, int STAGE, bool PRE, int Q>
 __device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, int b0row,
                                           int b1row, int b0, double* __restrict__ gs,
                                           int* __restrict__ flist, int* __restrict__ fn,
@@ -1569,7 +1651,7 @@ __device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, in
         if (!PRE) st = stage_load<STAGE>(F.in, F.X, F.H1, F.H2, P.cap, b0, t, 1);
         nwt = gs[G_M1X + t];
     }
-    rows_total(R.rows, b0row, b1row, tot);
+    rows_total<Q>(R.rows, b0row, b1row, tot);
     if (t >= 0 && t < 3) {
         double nx, nv;
         const double a = nwt + P.lam * tot[t];
@@ -1584,25 +1666,26 @@ __device__ __forceinline__ void fin_close(const FinBufs& F, const RowBufs& R, in
 }
 
 // Rows from row0 on, up to star p1 (all: the BH too, by the last workgroup;
-// a sub-range is one i shard of a plain evaluation); the BH mass is m[0].
-template <int MODE, int STAGE, int G>
+// a sub-range is one i shard of a plain evaluation); the BH mass is m[0].  A
+// workgroup per row and group of it (G = FG) or per FG rows (G = 1).
+template <int MODE, int STAGE, int G, int Q>
 __global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M, Phys P,
            int row0, int p1, int nrow)
 {
-    const int row = row0 + (int)blockIdx.x * (G == 1 ? FG : 1);
+    const int row = row0 + (G == 1 ? (int)blockIdx.x * FG : (int)blockIdx.x / Q);
     const Row q = {0, p1 - 1, row * RB, row};
     StageIn bh = {};
     if (P.n > 1)
-        fin_rows<MODE, STAGE, G>(F, R, q, part, S, (size_t)P.cap, 1, R.gs, R.flist, R.fn, F.m[0],
-                                 M, P, bh);
+        fin_rows<MODE, STAGE, G, Q>(F, R, q, part, S, (size_t)P.cap, 1, R.gs, R.flist, R.fn,
+                                    F.m[0], M, P, bh, (int)blockIdx.x % Q);
     else
-        empty_row(R, 0, MODE == 1);
+        empty_row<Q>(R, 0, MODE == 1);
     if (R.ticket && last_block(R.ticket, gridDim.x)) {
         if (G > 1 && P.n > 1)
-            fin_close<MODE, STAGE, true>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
+            fin_close<MODE, STAGE, true, Q>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
         else
-            fin_close<MODE, STAGE, false>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
+            fin_close<MODE, STAGE, false, Q>(F, R, 0, nrow, 0, R.gs, R.flist, R.fn, P, bh);
     }
 }
 
@@ -1610,21 +1693,23 @@ void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M
 // sums from k_prep's rows (prows, FWG threads: the order of k_prep's last
 // workgroup) for itself, so that only one counter, R.ticket, is left, which
 // k_prep clears in the same call.
-inline __global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
+template <int Q>
+__global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_fin_na(FinBufs F, RowBufs R, const double* __restrict__ prows,
               const void* __restrict__ part, int S, Phys P, int nrow)
 {
     __shared__ double tot[RV];
-    rows_total(prows, 0, nrow, tot);
-    const Row q = {0, P.n - 1, (int)blockIdx.x * RB, (int)blockIdx.x};
+    rows_total<Q>(prows, 0, nrow, tot);
+    const int row = (int)blockIdx.x / Q;
+    const Row q = {0, P.n - 1, row * RB, row};
     StageIn bh = {};
     if (P.n > 1)
-        fin_rows<0, 0, FG>(F, R, q, part, S, (size_t)P.cap, 1, tot + RV_G, nullptr, nullptr,
-                           F.m[0], MixPrep{}, P, bh);
+        fin_rows<0, 0, FG, Q>(F, R, q, part, S, (size_t)P.cap, 1, tot + RV_G, nullptr, nullptr,
+                              F.m[0], MixPrep{}, P, bh, (int)blockIdx.x % Q);
     else
-        empty_row(R, 0, false);
+        empty_row<Q>(R, 0, false);
     if (last_block(R.ticket, gridDim.x))
-        fin_close<0, 0, false>(F, R, 0, nrow, 0, tot + RV_G, nullptr, nullptr, P, bh);
+        fin_close<0, 0, false, Q>(F, R, 0, nrow, 0, tot + RV_G, nullptr, nullptr, P, bh);
 }
 
 // ---------------------------------------------------------------------

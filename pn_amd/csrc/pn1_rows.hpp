@@ -102,6 +102,27 @@ __device__ __forceinline__ double wave_sums16(const double (&v)[16])
     return t;
 }
 
+// The same over the lower 16 lanes: lane l < 16 gets the sum of v[l].
+template <int X, int N>
+__device__ __forceinline__ void halve(const double (&v)[2 * N], double (&o)[N])
+{
+    const bool up = threadIdx.x & X;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double keep = up ? v[N + k] : v[k], send = up ? v[k] : v[N + k];
+        o[k] = keep + lane_xor<X>(send);
+    }
+}
+__device__ __forceinline__ double group_sums16(const double (&v)[16])
+{
+    double a[8], b[4], c[2], d[1];
+    halve<8>(v, a);
+    halve<4>(a, b);
+    halve<2>(b, c);
+    halve<1>(c, d);
+    return d[0];
+}
+
 // Values that one workgroup hands to another within a launch (the rows' sums
 // and masks, to the last workgroup): stored and loaded at device scope, past
 // the XCD's own L2.  A release fence would do the same for ordinary stores,
@@ -120,15 +141,25 @@ __device__ __forceinline__ T take_over(const T* p)
 
 // Fixed-order sums of rows [b0, b1), by a workgroup of FWG threads, into
 // tot[RV] (LDS), for every thread of it: thread t adds value t % RV of rows
-// t / RV, t / RV + FWG / RV, ...
+// t / RV, t / RV + FWG / RV, ...  Q: the values are those of a row's Q groups
+// of 16 stars.
+template <int Q = 1>
 __device__ __forceinline__ void rows_total(const double* rows, int b0, int b1, double* tot)
 {
     __shared__ double sh[FG][RV];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     double t = 0.0;
+    if (Q == 1) {
 #pragma unroll 8
-    for (int b = b0 + (int)threadIdx.x / RV; b < b1; b += FWG / RV)
-        t += take_over(&rows[(size_t)b * RV + (threadIdx.x & (RV - 1))]);
+        for (int b = b0 + (int)threadIdx.x / RV; b < b1; b += FWG / RV)
+            t += take_over(&rows[(size_t)b * RV + (threadIdx.x & (RV - 1))]);
+    } else {
+#pragma unroll 2
+        for (int b = b0 + (int)threadIdx.x / RV; b < b1; b += FWG / RV) {
+            const double* r = &rows[(size_t)b * 4 * RV + (threadIdx.x & (RV - 1))];
+            t += (take_over(r) + take_over(r + RV)) + (take_over(r + 2 * RV) + take_over(r + 3 * RV));
+        }
+    }
     t += __shfl_xor(t, 16, 64);
     t += __shfl_xor(t, 32, 64);
     if (lane < RV) sh[wid][lane] = t;
