@@ -348,7 +348,7 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
     const EBlk b = blk[blockIdx.x];
     const int off = E.coff[b.c], nst = E.coff[b.c + 1] - off - 1;
     const int r0 = E.crow[b.c], r1 = E.crow[b.c + 1];
-    const Row q = {off, nst, b.first, r0 + b.first / RB};
+    const Row q = {off, nst, b.first, r0 + b.first / RB, nst};
     double* gs = R.gs + (size_t)b.c * NGS;
     if (MODE == 1) {
         M.mmax = E.cmmax[b.c];

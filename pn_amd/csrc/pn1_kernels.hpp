@@ -1442,10 +1442,11 @@ struct FinBufs {
                          // still read this evaluation's)
 };
 
-// One row of a cluster's stars: local stars first .. first + 63 of nst, BH
-// at index off, its rows from row0 on; row: this one's index among all rows.
+// One row of a cluster's stars: local stars first .. first + 63 of the nst to
+// be done (of the cluster's nall: fewer in an i shard), BH at index off; row:
+// this one's index among all rows.
 struct Row {
-    int off, nst, first, row;
+    int off, nst, first, row, nall;
 };
 
 // The workgroup's rows of a cluster: row q.row by all FG waves (G = FG), or
@@ -1502,7 +1503,7 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         if (nf > 0 || any)
             rare_rows(F.j64, F.in, cap, P.eps2, q.off, Q > 1 ? min(q.nst, lf + RS) : q.nst,
                       Q > 1 ? lf : q.first, G == 1 ? FG : 1, R.hmask + q.row, sub * RS,
-                      Q > 1 ? 0xffffull : ~0ull, q.nst, flist, nf, F.xr);
+                      Q > 1 ? 0xffffull : ~0ull, q.nall, flist, nf, F.xr);
     };
     // everything the star part reads, requested ahead of the partial sums
     StageIn st;
@@ -1674,7 +1675,7 @@ void k_fin(FinBufs F, RowBufs R, const void* __restrict__ part, int S, MixPrep M
            int row0, int p1, int nrow)
 {
     const int row = row0 + (G == 1 ? (int)blockIdx.x * FG : (int)blockIdx.x / Q);
-    const Row q = {0, p1 - 1, row * RB, row};
+    const Row q = {0, p1 - 1, row * RB, row, P.n - 1};
     StageIn bh = {};
     if (P.n > 1)
         fin_rows<MODE, STAGE, G, Q>(F, R, q, part, S, (size_t)P.cap, 1, R.gs, R.flist, R.fn,
@@ -1701,7 +1702,7 @@ void k_fin_na(FinBufs F, RowBufs R, const double* __restrict__ prows,
     __shared__ double tot[RV];
     rows_total<Q>(prows, 0, nrow, tot);
     const int row = (int)blockIdx.x / Q;
-    const Row q = {0, P.n - 1, row * RB, row};
+    const Row q = {0, P.n - 1, row * RB, row, P.n - 1};
     StageIn bh = {};
     if (P.n > 1)
         fin_rows<0, 0, FG, Q>(F, R, q, part, S, (size_t)P.cap, 1, tot + RV_G, nullptr, nullptr,
