@@ -299,9 +299,11 @@ MixPrep mix_prep(const pn1_ctx* c, const Phys& P)
 constexpr int FIN_ROWS = 1024, FIN_SUB = 16;
 bool fin_sub(int nst, int nrow, int slots) { return nst > 0 && nrow <= FIN_SUB && slots >= FG; }
 
-// Stars i0 .. i1 - 1 (all: every star and the BH), `slots` partials each.
+// Stars i0 .. i1 - 1 (all: every star and the BH), `slots` partials each; rowk:
+// by the row kernels.
 template <int MODE, int STAGE>
-void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, int i1, bool all)
+void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, int i1, bool all,
+                bool rowk)
 {
     FinBufs F;
     F.in = in;
@@ -313,6 +315,7 @@ void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, 
     F.acc = c->acc;
     F.kr = c->kr;
     F.xr = c->xr;
+    F.hp = rowk && c->nrow <= HROWS ? c->hpart : nullptr;
     F.j64 = rec_buf(c, STAGE <= 1 ? 0 : STAGE - 1);
     F.jnext = rec_buf(c, STAGE % 3);
     const int row0 = (i0 - 1) / RB, rows = std::max(1, (i1 - i0 + RB - 1) / RB);
@@ -396,14 +399,14 @@ int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
         if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     }
     switch (stage * 2 + (mixed ? 1 : 0)) {
-    case 0: launch_fin<0, 0>(c, in, P, slots, 1, c->n, true); break;
-    case 1: launch_fin<1, 0>(c, in, P, slots, 1, c->n, true); break;
-    case 2: launch_fin<0, 1>(c, in, P, slots, 1, c->n, true); break;
-    case 3: launch_fin<1, 1>(c, in, P, slots, 1, c->n, true); break;
-    case 4: launch_fin<0, 2>(c, in, P, slots, 1, c->n, true); break;
-    case 5: launch_fin<1, 2>(c, in, P, slots, 1, c->n, true); break;
-    case 6: launch_fin<0, 3>(c, in, P, slots, 1, c->n, true); break;
-    default: launch_fin<1, 3>(c, in, P, slots, 1, c->n, true); break;
+    case 0: launch_fin<0, 0>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 1: launch_fin<1, 0>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 2: launch_fin<0, 1>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 3: launch_fin<1, 1>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 4: launch_fin<0, 2>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 5: launch_fin<1, 2>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    case 6: launch_fin<0, 3>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
+    default: launch_fin<1, 3>(c, in, P, slots, 1, c->n, true, c->slots > 0); break;
     }
     HIPCHK(c, hipGetLastError());
     c->acc_ok = mixed;
@@ -613,7 +616,7 @@ void pn1_destroy(pn1_ctx* c)
     if (c->j32) (void)hipFree(c->j32);
     if (c->thr) (void)hipFree(c->thr);
     if (c->kr) (void)hipFree(c->kr);
-    void* fbufs[] = {c->fmask, c->hmask, c->flist, c->fn, c->ticket, c->xr};
+    void* fbufs[] = {c->fmask, c->hmask, c->flist, c->fn, c->ticket, c->xr, c->hpart};
     for (void* b : fbufs)
         if (b) (void)hipFree(b);
     if (c->part) (void)hipFree(c->part);
@@ -665,6 +668,9 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->fmask, nr);
     if (!rc) rc = dalloc(c, &c->hmask, nr);
     if (!rc) rc = dalloc(c, &c->xr, (size_t)(NACC + 1) * cap);
+    if (!rc)
+        rc = dalloc(c, &c->hpart,
+                    std::min(nr, (size_t)HROWS) * HSLOT * HCHUNK * (NACC + 1));
     if (!rc) rc = dalloc(c, &c->flist, cap);
     if (!rc) rc = dalloc(c, &c->fn, 4);
     if (!rc) rc = dalloc(c, &c->ticket, 1);
@@ -829,9 +835,9 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
         launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     if (mixed)
-        launch_fin<1, 0>(c, in, P, slots, i0, i1, false);
+        launch_fin<1, 0>(c, in, P, slots, i0, i1, false, rowk);
     else
-        launch_fin<0, 0>(c, in, P, slots, i0, i1, false);
+        launch_fin<0, 0>(c, in, P, slots, i0, i1, false, rowk);
     if (!mixed) c->acc_ok = false;
     HIPCHK(c, hipGetLastError());
     return fetch(c, c->acc + i0, i1 - i0, a, nullptr);

@@ -46,6 +46,7 @@ struct pn1_ctx {
     int *flist = nullptr, *fn = nullptr;
     unsigned int* ticket = nullptr;
     double* xr = nullptr;       // FP64 sums for hard stars and BH-close pairs [NACC + 1][cap]
+    double* hpart = nullptr;    // hard stars' sums of the row kernels, [rows][HSLOT][HCHUNK][NACC + 1]
     // acc and kr hold the last mixed evaluation of the uploaded run (cleared
     // by pn1_upload and by FP64 evaluations): the mixed form's thresholds
     // read them

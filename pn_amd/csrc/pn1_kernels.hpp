@@ -1094,12 +1094,73 @@ __device__ __forceinline__ void put_part32(const float (&a)[NACC32], const float
     }
 }
 
+// Hard stars (PN1_HARD_K) of the row kernels: the FP64 sums of a row's first
+// HSLOT of them over chunk [j0, j1), one record per lane, NACC sums and sum m_j
+// w^2 each, to out + slot HCHUNK (NACC + 1); k_fin adds the chunks' (hard_sum).
+// By k_fin's one workgroup for the row (rare_rows) a star takes 15 us at n =
+// 10241 on MI355X while the rest of the chip waits; here its chunks run beside
+// other rows' work.  Not inlined, and held to the pair kernel's registers: the
+// call is rare.  With one hard star, evaluation: n = 10241, 135 -> 122 us, n =
+// 12289, 197 -> 162, n = 16385, 271 -> 239.  Every thread of the workgroup calls
+// it.
+constexpr int HSLOT = 2, HCHUNK = TLONG + TSHORT;
+constexpr int HROWS = 4096;                  // rows with room for them
+__attribute__((noinline)) __device__ void
+hard_part(const JRec64* __restrict__ jr, const double* __restrict__ st, int cap, double eps2,
+          int i0, unsigned long long hm, int j0, int j1, double* __restrict__ out)
+{
+    __shared__ double wsum[NACC + 1][PW];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    for (int slot = 0; slot < HSLOT && hm; ++slot) {
+        const int i = i0 + __builtin_ctzll(hm);
+        hm &= hm - 1;
+        const I64 I = load_i64(jr, st, cap, i, eps2);
+        double a[NACC], ts = 0.0;
+#pragma unroll
+        for (int k = 0; k < NACC; ++k) a[k] = 0.0;
+        for (int j = j0 + (int)threadIdx.x; j < j1; j += PW * RB) {
+            const JRec64& J = jr[j];
+            body64<true>(J, j, i, I, a, eps2);
+            if (j != i) {
+                const double rx = J.x - I.x, ry = J.y - I.y, rz = J.z - I.z;
+                ts += J.m / (rx * rx + ry * ry + rz * rz + eps2);
+            }
+        }
+        const double u = wave_sums16(a), w = wave_sum(ts);
+        if ((lane & 3) == 0) wsum[lane >> 2][wid] = u;
+        if (lane == 0) wsum[NACC][wid] = w;
+        __syncthreads();
+        if (threadIdx.x <= NACC) {
+            double t = 0.0;
+#pragma unroll
+            for (int k = 0; k < PW; ++k) t += wsum[threadIdx.x][k];
+            out[(size_t)slot * HCHUNK * (NACC + 1) + threadIdx.x] = t;
+        }
+        __syncthreads();
+    }
+}
+
+// A hard star's sums over its S chunks hp: lane k <= NACC gets value k.
+__device__ __forceinline__ double hard_sum(const double* __restrict__ hp, int S)
+{
+    constexpr int N = NACC + 1;
+    const int lane = threadIdx.x & 63, v = lane % N, g = lane / N;
+    double t = 0.0;
+    if (g < 3) {
+#pragma unroll 8
+        for (int s = g; s < S; s += 3) t += hp[s * N + v];
+    }
+    const double b = __shfl(t, min(lane + N, 63), 64), c = __shfl(t, min(lane + 2 * N, 63), 64);
+    return (t + b) + c;
+}
+
 // k_pair64w's form of the mixed kernel.
 template <bool TS, bool EQ>
 __global__ __launch_bounds__(PW * RB) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
                const Thr* __restrict__ thr, const double* __restrict__ st,
-               float* __restrict__ part, Phys P, int S, int nrow, int bid0, int tile)
+               float* __restrict__ part, Phys P, int S, int nrow, int bid0, int tile,
+               const unsigned long long* __restrict__ hmask, double* __restrict__ hpart)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -1111,6 +1172,17 @@ void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
     part32<TS, EQ>(jr, j64, R, i, I, P.eps2f, P.eps2, 1.0 / P.mmax, tile, a, sumN, cmpN);
     put_part32<TS>(a, sumN, cmpN, wave, lane, li < n, part + (size_t)s * MROWS * P.cap + li,
                    (size_t)P.cap);
+    if (hpart) {
+        const unsigned long long hm = hmask[ig];
+        if (hm) {
+            // the whole chunk: from wave 0's part to the last wave's
+            int s0, g0;
+            const JRange A = j_part(bid0 + (int)blockIdx.x, S, nrow, 0, n, s0, g0);
+            const JRange B = j_part(bid0 + (int)blockIdx.x, S, nrow, PW - 1, n, s0, g0);
+            hard_part(j64, st, P.cap, P.eps2, 1 + ig * RB, hm, A.j0, B.j1,
+                      hpart + ((size_t)ig * HSLOT * HCHUNK + s) * (NACC + 1));
+        }
+    }
 }
 
 // ---------------------------------------------------------------------
@@ -1120,7 +1192,8 @@ void k_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64,
 // stars) whose sums need more than the FP32 pass gave, mixed form: x at the
 // star's index gets, [NACC + 1][cap] (the NACC sums and sum m_j w^2, from the
 // FP64 form's body),
-//   a hard star (hmask of the rows, see PN1_HARD_K): its whole row over the
+//   a hard star (hmask of the rows, see PN1_HARD_K; but for each row's first
+//     `skip`, which hard_part has done): its whole row over the
 //     cluster's records (BH-close stars included, with their full records),
 //     reduced over the workgroup's FWG lanes in a fixed order;
 //   any other star: its pairs with the nf BH-close stars (flist, see
@@ -1134,7 +1207,7 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
                                                     int nrow,
                                                     const unsigned long long* __restrict__ hmask,
                                                     int shift, unsigned long long width,
-                                                    int nall,
+                                                    int nall, int skip,
                                                     const int* __restrict__ flist, int nf,
                                                     double* __restrict__ x)
 {
@@ -1161,7 +1234,9 @@ __attribute__((noinline)) __device__ void rare_rows(const JRec64* __restrict__ j
         x[(size_t)NACC * cap + i] = ts;
     }
     for (int r = 0; r < nrow && first + r * RB < nst; ++r) {
-        unsigned long long hm = (hmask[r] >> shift) & width;
+        unsigned long long hm = hmask[r];
+        for (int k = 0; k < skip; ++k) hm &= hm - 1;      // those of hard_part
+        hm = (hm >> shift) & width;
         while (hm) {
             const int h = r * RB + __builtin_ctzll(hm), i = off + 1 + first + h;
             hm &= hm - 1;
@@ -1437,6 +1512,7 @@ struct FinBufs {
     double* acc;
     float* kr;
     double* xr;          // rare_rows' sums (mixed form)
+    const double* hp;    // hard_part's, or null if the pair kernel has none
     const JRec64* j64;   // this evaluation's records
     JRec64* jnext;       // the next one's (another buffer: other rows may
                          // still read this evaluation's)
@@ -1485,9 +1561,10 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
     const int lc = li < q.nst ? li : min(q.first, q.nst - 1);
     const int p = q.off + 1 + lc;
     const bool star = G == 1 ? lf < q.nst : wid == 0;   // this wave runs the star part
-    int nf = 0;
+    int nf = 0, hslot = -1;      // the lane's star: hard_part's slot of it
     bool is_hard = false;
     // the BH-close and hard stars, if any
+    __shared__ double hx[MODE == 1 ? (G == 1 ? FG : 1) : 1][HSLOT][MODE == 1 ? NACC + 1 : 1];
     auto rare = [&]() {
         if (MODE == 0) return;
         nf = *fn;
@@ -1495,16 +1572,37 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
 #pragma unroll
         for (int r = 0; r < (G == 1 ? FG : 1); ++r)
             if (q.first + r * RB < q.nst) {
-                unsigned long long hm = R.hmask[q.row + r];
-                if (Q > 1) hm = (hm >> (sub * RS)) & 0xffffu;
-                any |= hm;
-                if (r == mine) is_hard = (hm >> lane) & 1;
+                const unsigned long long hm = R.hmask[q.row + r];
+                unsigned long long rest = hm;
+                if (F.hp) {
+                    rest &= rest - 1;
+                    rest &= rest - 1;
+                }
+                if (Q > 1) rest = (rest >> (sub * RS)) & 0xffffu;
+                any |= rest;
+                if (r != mine) continue;
+                const int bit = sub * RS + lane % RS;
+                is_hard = (hm >> bit) & 1;
+                if (F.hp && is_hard) {
+                    const int before = __popcll(hm & ((1ull << bit) - 1ull));
+                    hslot = before < HSLOT ? before : -1;
+                }
+                // by a wave each of those that have no star part (G = 1: by
+                // the row's)
+                if (F.hp && hm)
+                    for (int k = 0; k < HSLOT && k < __popcll(hm); ++k)
+                        if (G == 1 || wid == 1 + k) {
+                            const double t =
+                                hard_sum(F.hp + ((size_t)(q.row + r) * HSLOT + k) * HCHUNK * (NACC + 1), S);
+                            if (MODE == 1 && lane <= NACC) hx[G == 1 ? wid : 0][k][lane] = t;
+                        }
             }
         if (nf > 0 || any)
             rare_rows(F.j64, F.in, cap, P.eps2, q.off, Q > 1 ? min(q.nst, lf + RS) : q.nst,
                       Q > 1 ? lf : q.first, G == 1 ? FG : 1, R.hmask + q.row, sub * RS,
-                      Q > 1 ? 0xffffull : ~0ull, q.nall, flist, nf, F.xr);
+                      Q > 1 ? 0xffffull : ~0ull, q.nall, F.hp ? HSLOT : 0, flist, nf, F.xr);
     };
+    static_assert(HSLOT == 2, "two bits cleared above");
     // everything the star part reads, requested ahead of the partial sums
     StageIn st;
     double gs[NGS], mp = 0.0, D2 = 0.0, e = 0.0, x0[3], x0n[3];
@@ -1603,7 +1701,8 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         // one: plus its pairs with the BH-close stars
 #pragma unroll
         for (int k = 0; k <= NACC; ++k)
-            A[k] = (is_hard ? 0.0 : A[k]) + F.xr[(size_t)k * cap + p];
+            A[k] = hslot >= 0 ? hx[G == 1 ? wid : 0][hslot & (HSLOT - 1)][k]
+                              : (is_hard ? 0.0 : A[k]) + F.xr[(size_t)k * cap + p];
     }
     if (!star) return;
     double cb[3] = {0.0, 0.0, 0.0}, a[3], nx[3], nv[3], g[NGS];

@@ -45,7 +45,7 @@ void launch32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, i
 {
     hipLaunchKernelGGL((k_pair32w<TS, EQ>), dim3(slots * nrow), dim3(PW * RB), 0, c->st, c->j32,
                        j64, c->thr, in, (float*)c->part, P, slots, nrow, slots * row0,
-                       c->tile);
+                       c->tile, c->hmask, c->nrow <= HROWS ? c->hpart : nullptr);
 }
 
 template <int PP, bool TS, bool EQ>

@@ -1,4 +1,5 @@
-"""Stars whose pair terms cancel (PN1_HARD_K) take their sums in FP64.  Massless
+"""Stars whose pair terms cancel (PN1_HARD_K) take their sums in FP64: the first
+two of a row of 64 in the pair kernel's chunks, any more in k_fin.  Massless
 stars at and around the centre of a point-symmetric cluster, one to four to a
 row, over k_fin's three forms, and shards, which must equal the full rows."""
 import numpy as np
