@@ -56,6 +56,8 @@ struct pn1_ens {
     int *flist = nullptr, *fn = nullptr;
     unsigned int* ticket = nullptr;
     double* xr = nullptr;         // as in pn1_ctx
+    double* hpart = nullptr;      // as in pn1_ctx, by the ensemble's rows
+    int hpart_cap = 0;
     pn1dev::EBlk *row = nullptr, *pblk = nullptr;
     int* crow = nullptr;
     int nrow = 0, npblk = 0;

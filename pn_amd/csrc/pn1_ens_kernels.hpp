@@ -259,7 +259,9 @@ void k_ens_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64
                    const Thr* __restrict__ thr, const double* __restrict__ st,
                    float* __restrict__ part, const EPart* __restrict__ parts,
                    const int* __restrict__ coff, const long long* __restrict__ poff,
-                   const double* __restrict__ cmmax, Phys P, int tile)
+                   const double* __restrict__ cmmax, Phys P, int tile,
+                   const int* __restrict__ crow, const unsigned long long* __restrict__ hmask,
+                   double* __restrict__ hpart)
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -270,6 +272,15 @@ void k_ens_pair32w(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64
     part32<TS, EQ>(jr, j64, g.R, g.i, I, P.eps2f, P.eps2, 1.0 / cmmax[w.c], tile, a, sumN, cmpN);
     put_part32<TS>(a, sumN, cmpN, wave, lane, g.li < g.nst,
                    part + (poff[w.c] + (long long)w.s * g.nst) * MROWS + g.li, (size_t)g.nst);
+    if (hpart && w.S <= HCHUNK) {
+        const int row = crow[w.c] + w.ig;
+        const unsigned long long hm = hmask[row];
+        if (hm) {
+            const EWave a = ens_wave(w, coff, 0, lane), b = ens_wave(w, coff, PW - 1, lane);
+            hard_part(j64, st, P.cap, P.eps2, g.off + 1 + w.ig * RB, hm, a.R.j0, b.R.j1,
+                      hpart + ((size_t)row * HSLOT * HCHUNK + w.s) * (NACC + 1));
+        }
+    }
 }
 
 // Per-cluster buffers.  Cluster c's rows of 64 stars are [crow[c],
@@ -356,6 +367,7 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
     }
     StageIn bh = {};
     if (nst > 0) {
+        if (ens_nchunks(nst, L) > HCHUNK) F.hp = nullptr;
         const void* base = MODE == 0 ? (const void*)((const double*)part + poff[b.c] * NACC)
                                      : (const void*)((const float*)part + poff[b.c] * MROWS);
         fin_rows<MODE, STAGE, G, 1>(F, R, q, base, ens_nchunks(nst, L), (size_t)nst, 0, gs,

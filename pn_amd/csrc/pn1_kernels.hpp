@@ -1104,7 +1104,7 @@ __device__ __forceinline__ void put_part32(const float (&a)[NACC32], const float
 // 12289, 197 -> 162, n = 16385, 271 -> 239.  Every thread of the workgroup calls
 // it.
 constexpr int HSLOT = 2, HCHUNK = TLONG + TSHORT;
-constexpr int HROWS = 4096;                  // rows with room for them
+constexpr int HROWS = 4096, EHROWS = 16384;  // rows with room for them (EHROWS: of an ensemble)
 __attribute__((noinline)) __device__ void
 hard_part(const JRec64* __restrict__ jr, const double* __restrict__ st, int cap, double eps2,
           int i0, unsigned long long hm, int j0, int j1, double* __restrict__ out)

@@ -66,7 +66,7 @@ void ens_launch32w(pn1_ens* e, const JRec64* j64, const double* in, const Phys& 
 {
     hipLaunchKernelGGL((k_ens_pair32w<TS, EQ>), dim3(e->nparts), dim3(PW * RB), 0, e->st, e->j32,
                        j64, e->thr, in, (float*)e->part, e->parts, e->coff, e->poff, e->cmmax, P,
-                       e->tile);
+                       e->tile, e->crow, e->hmask, e->nrow <= EHROWS ? e->hpart : nullptr);
 }
 
 using EnsLaunch32 = void (*)(pn1_ens*, const JRec64*, const double*, const Phys&, dim3);

@@ -71,3 +71,21 @@ def test_hard_stars(stars):
             err = rel(ctx.force_range(a, b), exact[a:b])
             inside = hard[(hard >= a) & (hard < b)] - a
             assert err.max() <= 1e-6 and (err[inside] <= 1e-9).all()
+
+
+def test_hard_stars_of_an_ensemble():
+    """The automatic plan of clusters of one and of several chunks, against each
+    cluster's FP64 forces, as above."""
+    cl = [state(k) for k in (300, 10240, 700, 3000)]
+    exact = []
+    with pn.Ensemble(sum(len(c[2]) for c in cl), len(cl)) as ens:
+        ens.set_params(1e-3, 50.0, 2.0**-10, pn.FP64)
+        ens.upload([c[:3] for c in cl])
+        exact = ens.force()
+        ens.set_params(1e-3, 50.0, 2.0**-10, pn.MIXED)
+        ens.upload([c[:3] for c in cl])
+        for _ in range(2):
+            for a, e, c in zip(ens.force(), exact, cl):
+                err = rel(a, e)
+                assert err[1:].max() <= 1e-6
+                assert err[c[3]].max() <= 1e-9, err[c[3]]
