@@ -517,7 +517,7 @@ __global__ __launch_bounds__(WG) void k_pair64(const JRec64* __restrict__ jr,
 // Measured on MI355X, FP64 / mixed evaluation (pair and k_fin), us:
 //   n         65    257   1025  2049  4097  8193     10241    32769
 //   256 stars 23/31 25/29 28/31 43/60 55/56 147/98   209/130  1683/903
-//   this form 13/15 15/18 18/20 24/24 44/35 121/81   176/111  1578/841
+//   this form 12/16 13/17 16/20 24/24 44/35 120/78   181/112  1612/852
 // PW = 4 and 16 were within 3% up to n = 2049; above, 16 waves leave a
 // compute unit idle between workgroups (up to +30%).
 constexpr int PW = 8;
