@@ -257,15 +257,27 @@ bool ready(pn1_ctx* c, int* rc)
 }
 
 // ---- one force evaluation (+ stage update) ------------------------------
+// The records and hard stars of a step's evaluations are each in a buffer of
+// their own: evaluation `stage` reads buffer eval_buf(stage) while its k_fin
+// writes that of the next one, next_buf(stage).
+int eval_buf(int stage) { return stage <= 1 ? 0 : stage - 1; }
+int next_buf(int stage) { return stage % 3; }
+size_t rows_of(size_t cap) { return (cap + RB - 1) / RB + 1; }
 JRec64* rec_buf(const pn1_ctx* c, int k) { return c->j64 + (size_t)k * ((size_t)c->cap + 2); }
+unsigned long long* hard_buf(const pn1_ctx* c, int k)
+{
+    return c->hmask + (size_t)k * rows_of((size_t)c->cap);
+}
 
-// ticket false: the sums over the rows are not needed (an i shard).
-RowBufs row_bufs(const pn1_ctx* c, bool ticket = true)
+// For k_prep, or the k_fin of an evaluation.  ticket false: the sums over the
+// rows are not needed (an i shard).
+RowBufs row_bufs(const pn1_ctx* c, int stage = 0, bool ticket = true)
 {
     RowBufs R;
     R.rows = c->rows;
     R.fmask = c->fmask;
-    R.hmask = c->hmask;
+    R.hmask = hard_buf(c, eval_buf(stage));
+    R.hnext = hard_buf(c, next_buf(stage));
     R.gs = c->gs;
     R.flist = c->flist;
     R.fn = c->fn;
@@ -316,10 +328,10 @@ void launch_fin(pn1_ctx* c, const double* in, const Phys& P, int slots, int i0, 
     F.kr = c->kr;
     F.xr = c->xr;
     F.hp = rowk && c->nrow <= HROWS ? c->hpart : nullptr;
-    F.j64 = rec_buf(c, STAGE <= 1 ? 0 : STAGE - 1);
-    F.jnext = rec_buf(c, STAGE % 3);
+    F.j64 = rec_buf(c, eval_buf(STAGE));
+    F.jnext = rec_buf(c, next_buf(STAGE));
     const int row0 = (i0 - 1) / RB, rows = std::max(1, (i1 - i0 + RB - 1) / RB);
-    const RowBufs R = row_bufs(c, all);
+    const RowBufs R = row_bufs(c, STAGE, all);
     auto launch = [&](auto kernel, int wgs) {
         hipLaunchKernelGGL(kernel, dim3(wgs), dim3(FWG), 0, c->st, F, R, (const void*)c->part,
                            slots, mix_prep(c, P), P, row0, i1, c->nrow);
@@ -352,12 +364,13 @@ void launch_pair(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P,
     }
 }
 
-// The same by the row kernels, rows row0 .. row0 + nrow - 1, the plan's slots.
-void launch_pairw(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int row0,
-                  int nrow, bool ts)
+// The same by the row kernels, rows row0 .. row0 + nrow - 1, the plan's slots,
+// with the records (and hard stars) of buffer k.
+void launch_pairw(pn1_ctx* c, int k, const double* in, const Phys& P, int row0, int nrow, bool ts)
 {
+    const JRec64* j64 = rec_buf(c, k);
     if (c->mode == PN1_MIXED)
-        launch_pair32w(c, j64, in, P, c->slots, row0, nrow, ts);
+        launch_pair32w(c, j64, hard_buf(c, k), in, P, c->slots, row0, nrow, ts);
     else
         hipLaunchKernelGGL(k_pair64w, dim3(c->slots * nrow), dim3(PW * RB), 0, c->st, j64, in,
                            (double*)c->part, P, c->slots, nrow, c->slots * row0);
@@ -391,11 +404,11 @@ int enqueue_eval(pn1_ctx* c, int stage, const Phys& P)
     if (c->n > 1) {
         hipEvent_t e1 = nullptr;
         if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
-        const JRec64* j64 = rec_buf(c, stage <= 1 ? 0 : stage - 1);
+        const int k = eval_buf(stage);
         if (c->slots)
-            launch_pairw(c, j64, in, P, 0, c->nrow, stage <= 1);
+            launch_pairw(c, k, in, P, 0, c->nrow, stage <= 1);
         else
-            launch_pair(c, j64, in, P, 0, c->nIblk, c->S, stage <= 1);
+            launch_pair(c, rec_buf(c, k), in, P, 0, c->nIblk, c->S, stage <= 1);
         if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     }
     switch (stage * 2 + (mixed ? 1 : 0)) {
@@ -649,7 +662,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
         return PN1_EDEVICE;
     }
     const size_t cap = (size_t)capacity;
-    const size_t nr = (cap + RB - 1) / RB + 1;          // rows of 64 stars
+    const size_t nr = rows_of(cap);                     // rows of 64 stars
     int rc = PN1_OK;
     if (!rc) rc = dalloc(c, &c->X, 6 * cap);
     if (!rc) rc = dalloc(c, &c->Y, 6 * cap);
@@ -666,7 +679,7 @@ int pn1_create(pn1_ctx** out, int capacity, int device)
     if (!rc) rc = dalloc(c, &c->thr, cap);
     if (!rc) rc = dalloc(c, &c->kr, cap);
     if (!rc) rc = dalloc(c, &c->fmask, nr);
-    if (!rc) rc = dalloc(c, &c->hmask, nr);
+    if (!rc) rc = dalloc(c, &c->hmask, 3 * nr);
     if (!rc) rc = dalloc(c, &c->xr, (size_t)(NACC + 1) * cap);
     if (!rc)
         rc = dalloc(c, &c->hpart,
@@ -830,7 +843,7 @@ int pn1_force_range(pn1_ctx* c, int i0, int i1, double* a)
     hipEvent_t e1 = nullptr;
     if (c->prof) HIPCHK(c, prof_open(c->ev, c->st, &e1));
     if (rowk)
-        launch_pairw(c, rec_buf(c, 0), in, P, (i0 - 1) / RB, (i1 - i0 + RB - 1) / RB, true);
+        launch_pairw(c, 0, in, P, (i0 - 1) / RB, (i1 - i0 + RB - 1) / RB, true);
     else
         launch_pair(c, rec_buf(c, 0), in, P, (i0 - 1) / WG, nib, S, true);
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));

@@ -39,8 +39,9 @@ struct pn1_ctx {
     pn1dev::Thr* thr = nullptr; // mixed form's per-star pair thresholds
     float* kr = nullptr;        // mixed form's per-star cancellation ratios
     // per row of 64 stars: its values of the sums over all stars (rows) and,
-    // mixed form, the masks of its BH-close and hard stars; the list of
-    // BH-close stars and its length; the O(n) kernels' ticket counter
+    // mixed form, the masks of its BH-close and hard stars (hmask: three of
+    // rows_of(cap), one to each record buffer); the list of BH-close stars and
+    // its length; the O(n) kernels' ticket counter
     int nrow = 1;
     unsigned long long *fmask = nullptr, *hmask = nullptr;
     int *flist = nullptr, *fn = nullptr;

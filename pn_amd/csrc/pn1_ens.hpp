@@ -50,7 +50,8 @@ struct pn1_ens {
     bool eqm = false;             // each cluster's stars have one mass
     double* ctauf = nullptr;      // each cluster's BH-close threshold (PN1_FLAG_ETA)
     // per row: its values of the sums over all stars (rows) and, mixed form,
-    // the masks of its BH-close and hard stars; BH-close stars (lists at each
+    // the masks of its BH-close and hard stars (hmask: three of nrow, one to
+    // each record buffer); BH-close stars (lists at each
     // cluster's offset, per-cluster numbers); the O(n) kernels' tickets
     unsigned long long *fmask = nullptr, *hmask = nullptr;
     int *flist = nullptr, *fn = nullptr;

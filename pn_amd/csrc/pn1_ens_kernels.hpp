@@ -340,7 +340,7 @@ inline __global__ __launch_bounds__(FWG) void k_ens_prep(const double* __restric
         }
         const double cb[3] = {0.0, 0.0, 0.0};
         put_row<false, true>(row, 0, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
-                             R.hmask);
+                             R.hnext);
     }
     if (last_block(R.ticket + b.c, (unsigned)((r1 - r0 + FG - 1) / FG)))
         close_prep(R, M.j32 != nullptr, r0, r1, off + 1, R.gs + (size_t)b.c * NGS, R.flist + off,

@@ -225,7 +225,7 @@ __device__ __forceinline__ void put_row(int row, int sub, bool ok, const double 
                                         const double (&g)[NGS], double* __restrict__ rows,
                                         bool mixed, bool flagged, bool hard,
                                         unsigned long long* __restrict__ fmask,
-                                        unsigned long long* __restrict__ hmask)
+                                        unsigned long long* __restrict__ hnext)
 {
     const int lane = threadIdx.x & 63;
     double v[RV];
@@ -254,10 +254,10 @@ __device__ __forceinline__ void put_row(int row, int sub, bool ok, const double 
         if (lane == 0) {
             if (Q == 1 || sub < 0) {
                 hand_over(&fmask[row], f);
-                hmask[row] = h;
+                hnext[row] = h;
             } else {
                 hand_over((unsigned short*)&fmask[row] + sub, (unsigned short)f);
-                ((unsigned short*)&hmask[row])[sub] = (unsigned short)h;
+                ((unsigned short*)&hnext[row])[sub] = (unsigned short)h;
             }
         }
     }
@@ -314,7 +314,10 @@ __device__ __forceinline__ void list_flagged(const unsigned long long* mask, int
 // The buffers of the O(n) kernels' sums over all stars.
 struct RowBufs {
     double* rows;                          // per row: its RV values
-    unsigned long long *fmask, *hmask;     // per row: BH-close and hard stars
+    unsigned long long* fmask;             // per row: the BH-close stars of the state prepared
+    const unsigned long long* hmask;       // per row: the hard stars of this evaluation
+    unsigned long long* hnext;             // those of the state prepared: another buffer, because
+                                           // other waves and workgroups may still read hmask
     double* gs;                            // separable sums of the evaluation
     int *flist, *fn;                       // its BH-close stars and their number
     unsigned int* ticket;                  // last_block's counter (k_prep: null if the
@@ -373,7 +376,7 @@ __global__ __launch_bounds__(FWG) void k_prep(const double* __restrict__ st,
         }
         const double cb[3] = {0.0, 0.0, 0.0};
         put_row<false, true, Q>(row, -1, ok, cb, g, R.rows, M.j32 != nullptr, f, hard, R.fmask,
-                             R.hmask);
+                             R.hnext);
     }
     if (R.ticket && last_block(R.ticket, gridDim.x))
         close_prep<Q>(R, M.j32 != nullptr, 0, nrow, 1, R.gs, R.flist, R.fn);
@@ -1719,7 +1722,7 @@ __device__ __forceinline__ void fin_rows(const FinBufs& F, const RowBufs& R, con
         }
     }
     put_row<true, (STAGE > 0), Q>(q.row + mine, sub, ok, cb, g, R.rows, MODE == 1, f, hard, R.fmask,
-                               R.hmask);
+                               R.hnext);
 }
 
 // A cluster without stars: its one row of zeros (all Q groups of it).
@@ -1729,7 +1732,7 @@ __device__ __forceinline__ void empty_row(const RowBufs& R, int row, bool mixed)
     if (threadIdx.x < RV * Q) hand_over(&R.rows[(size_t)row * Q * RV + threadIdx.x], 0.0);
     if (mixed && threadIdx.x == 0) {
         hand_over(&R.fmask[row], 0ull);
-        R.hmask[row] = 0ull;
+        R.hnext[row] = 0ull;
     }
 }
 

@@ -40,12 +40,12 @@ const Launch32 k_launch32[16] = {
     launch32<3, true, true>};
 
 template <bool TS, bool EQ>
-void launch32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots, int row0,
-               int nrow)
+void launch32w(pn1_ctx* c, const JRec64* j64, const unsigned long long* hmask, const double* in,
+               const Phys& P, int slots, int row0, int nrow)
 {
     hipLaunchKernelGGL((k_pair32w<TS, EQ>), dim3(slots * nrow), dim3(PW * RB), 0, c->st, c->j32,
                        j64, c->thr, in, (float*)c->part, P, slots, nrow, slots * row0,
-                       c->tile, c->hmask, c->nrow <= HROWS ? c->hpart : nullptr);
+                       c->tile, hmask, c->nrow <= HROWS ? c->hpart : nullptr);
 }
 
 template <int PP, bool TS, bool EQ>
@@ -62,11 +62,12 @@ void ens_launch32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P
 }
 
 template <bool TS, bool EQ>
-void ens_launch32w(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P)
+void ens_launch32w(pn1_ens* e, const JRec64* j64, const unsigned long long* hmask,
+                   const double* in, const Phys& P)
 {
     hipLaunchKernelGGL((k_ens_pair32w<TS, EQ>), dim3(e->nparts), dim3(PW * RB), 0, e->st, e->j32,
                        j64, e->thr, in, (float*)e->part, e->parts, e->coff, e->poff, e->cmmax, P,
-                       e->tile, e->crow, e->hmask, e->nrow <= EHROWS ? e->hpart : nullptr);
+                       e->tile, e->crow, hmask, e->nrow <= EHROWS ? e->hpart : nullptr);
 }
 
 using EnsLaunch32 = void (*)(pn1_ens*, const JRec64*, const double*, const Phys&, dim3);
@@ -86,14 +87,15 @@ void launch_pair32(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& 
     k_launch32[form & 15](c, j64, in, P, ib0, nib, S);
 }
 
-void launch_pair32w(pn1_ctx* c, const JRec64* j64, const double* in, const Phys& P, int slots,
-                    int row0, int nrow, bool ts)
+void launch_pair32w(pn1_ctx* c, const JRec64* j64, const unsigned long long* hmask,
+                    const double* in, const Phys& P, int slots, int row0, int nrow, bool ts)
 {
     if (ts)
-        (c->eqm ? launch32w<true, true> : launch32w<true, false>)(c, j64, in, P, slots, row0, nrow);
+        (c->eqm ? launch32w<true, true> : launch32w<true, false>)(c, j64, hmask, in, P, slots,
+                                                                  row0, nrow);
     else
-        (c->eqm ? launch32w<false, true> : launch32w<false, false>)(c, j64, in, P, slots, row0,
-                                                                    nrow);
+        (c->eqm ? launch32w<false, true> : launch32w<false, false>)(c, j64, hmask, in, P, slots,
+                                                                    row0, nrow);
 }
 
 void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, dim3 g,
@@ -102,12 +104,13 @@ void launch_ens_pair32(pn1_ens* e, const JRec64* j64, const double* in, const Ph
     k_ens_launch32[form & 15](e, j64, in, P, g);
 }
 
-void launch_ens_pair32w(pn1_ens* e, const JRec64* j64, const double* in, const Phys& P, bool ts)
+void launch_ens_pair32w(pn1_ens* e, const JRec64* j64, const unsigned long long* hmask,
+                        const double* in, const Phys& P, bool ts)
 {
     if (ts)
-        (e->eqm ? ens_launch32w<true, true> : ens_launch32w<true, false>)(e, j64, in, P);
+        (e->eqm ? ens_launch32w<true, true> : ens_launch32w<true, false>)(e, j64, hmask, in, P);
     else
-        (e->eqm ? ens_launch32w<false, true> : ens_launch32w<false, false>)(e, j64, in, P);
+        (e->eqm ? ens_launch32w<false, true> : ens_launch32w<false, false>)(e, j64, hmask, in, P);
 }
 
 hipError_t ens_pair32_occupancy(int var, int* per_cu)

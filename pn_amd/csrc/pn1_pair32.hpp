@@ -22,15 +22,17 @@ inline int pair32_form(int variant, bool ts, bool eqm)
 // range split in S chunks (pn1_pair32.hip).
 void launch_pair32(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
                    const pn1dev::Phys& P, int ib0, int nib, int S, int form);
-// The row kernels' form: nrow rows from row0 on, `slots` partials per star.
-void launch_pair32w(pn1_ctx* c, const pn1dev::JRec64* j64, const double* in,
-                    const pn1dev::Phys& P, int slots, int row0, int nrow, bool ts);
+// The row kernels' form: nrow rows from row0 on, `slots` partials per star;
+// hmask: the evaluation's hard stars.
+void launch_pair32w(pn1_ctx* c, const pn1dev::JRec64* j64, const unsigned long long* hmask,
+                    const double* in, const pn1dev::Phys& P, int slots, int row0, int nrow,
+                    bool ts);
 // Ensemble: one persistent launch of grid g over the work queues.
 void launch_ens_pair32(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
                        const pn1dev::Phys& P, dim3 g, int form);
 // Its automatic plan's form.
-void launch_ens_pair32w(pn1_ens* e, const pn1dev::JRec64* j64, const double* in,
-                        const pn1dev::Phys& P, bool ts);
+void launch_ens_pair32w(pn1_ens* e, const pn1dev::JRec64* j64, const unsigned long long* hmask,
+                        const double* in, const pn1dev::Phys& P, bool ts);
 // Resident workgroups per CU of the ensemble kernel of loop variant var
 // (0..3), in its form with the cancellation sums (the one with the most
 // registers).
