@@ -336,7 +336,8 @@ __global__ __launch_bounds__(FWG) void k_ens_adj_prep(const double* __restrict__
                                                      const double* __restrict__ m,
                                                      const int* __restrict__ coff,
                                                      const int* __restrict__ crow,
-                                                     const EBlk* __restrict__ pblk, Phys P,
+                                                     const EBlk* __restrict__ pblk, int npblk,
+                                                     Phys P,
                                                      ARec* __restrict__ rec,
                                                      double* __restrict__ jd,
                                                      double* __restrict__ rows,
@@ -345,8 +346,10 @@ __global__ __launch_bounds__(FWG) void k_ens_adj_prep(const double* __restrict__
                                                      unsigned int* __restrict__ counter)
 {
     __shared__ double tot[RV];
-    if (blockIdx.x == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
-    const EBlk b = pblk[blockIdx.x];
+    const int wg = ens_block();
+    if (wg == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
+    if (wg >= npblk) return;
+    const EBlk b = pblk[wg];
     const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
     const int r0 = crow[b.c], r1 = crow[b.c + 1];
     const int row = r0 + b.first / RB + (int)(threadIdx.x >> 6);
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(FWG) void k_ens_adj_fin(const ARec* __restrict__ re
                                                     const double* __restrict__ m,
                                                     const int* __restrict__ coff,
                                                     const int* __restrict__ crow,
-                                                    const EBlk* __restrict__ blk,
+                                                    const EBlk* __restrict__ blk, int n,
                                                     const double* __restrict__ apart,
                                                     const long long* __restrict__ aoff,
                                                     const double* __restrict__ sums, AdjAdd z,
@@ -422,7 +425,9 @@ __global__ __launch_bounds__(FWG) void k_ens_adj_fin(const ARec* __restrict__ re
                                                     unsigned int* __restrict__ ticket, Phys P,
                                                     int L)
 {
-    const EBlk b = blk[blockIdx.x];
+    const int wg = ens_block();
+    if (wg >= n) return;
+    const EBlk b = blk[wg];
     const int off = coff[b.c], nst = coff[b.c + 1] - off - 1;
     const int r0 = crow[b.c], r1 = crow[b.c + 1];
     const int li = b.first + (int)(G == 1 ? threadIdx.x : threadIdx.x & 63);
@@ -554,8 +559,8 @@ int ens_adj_get(pn1_ens* e, pn1_ens_adj** out)
 int ens_enqueue_vjp(pn1_ens* e, pn1_ens_adj* a, const double* y, const AdjLin& l,
                     const AdjAdd& z, double* out, const Phys& P)
 {
-    hipLaunchKernelGGL(k_ens_adj_prep, dim3(e->npblk), dim3(FWG), 0, e->st, y, l, a->mu, e->m,
-                       e->coff, e->crow, e->pblk, P, a->rec, a->jd, e->rows, a->sums, e->ticket,
+    hipLaunchKernelGGL(k_ens_adj_prep, ens_grid(e->npblk), dim3(FWG), 0, e->st, y, l, a->mu, e->m,
+                       e->coff, e->crow, e->pblk, e->npblk, P, a->rec, a->jd, e->rows, a->sums, e->ticket,
                        e->counter);
     if (e->nitems)
         hipLaunchKernelGGL(k_ens_adj_rev, dim3(std::min(a->grid, e->nitems)), dim3(WG), 0, e->st,
@@ -563,11 +568,12 @@ int ens_enqueue_vjp(pn1_ens* e, pn1_ens_adj* a, const double* y, const AdjLin& l
                            e->counter, e->qoff, P, e->L);
     if (e->nrow <= ADJ_FIN_ROWS)
         hipLaunchKernelGGL(k_ens_adj_fin<FG>, dim3(e->nrow), dim3(FWG), 0, e->st, a->rec, y, a->mu,
-                           e->m, e->coff, e->crow, e->row, (const double*)a->apart, a->aoff,
+                           e->m, e->coff, e->crow, e->row, e->nrow, (const double*)a->apart, a->aoff,
                            a->sums, z, out, a->gm0, e->rows, e->ticket, P, e->L);
     else
-        hipLaunchKernelGGL(k_ens_adj_fin<1>, dim3(e->npblk), dim3(FWG), 0, e->st, a->rec, y, a->mu,
-                           e->m, e->coff, e->crow, e->pblk, (const double*)a->apart, a->aoff,
+        hipLaunchKernelGGL(k_ens_adj_fin<1>, ens_grid(e->npblk), dim3(FWG), 0, e->st, a->rec, y,
+                           a->mu, e->m, e->coff, e->crow, e->pblk, e->npblk,
+                           (const double*)a->apart, a->aoff,
                            a->sums, z, out, a->gm0, e->rows, e->ticket, P, e->L);
     EHIPCHK(e, hipGetLastError());
     return PN1_OK;

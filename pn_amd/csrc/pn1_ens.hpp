@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "pn1.h"
+#include "pn1_ens_plan.hpp"
 #include "pn1_ens_types.hpp"
 
 struct pn1_ens_adj;   // adjoint buffers (pn1_adj.hip)
@@ -58,12 +59,11 @@ struct pn1_ens {
     unsigned int* ticket = nullptr;
     double* xr = nullptr;         // as in pn1_ctx
     double* hpart = nullptr;      // as in pn1_ctx, by the ensemble's rows
-    int hpart_cap = 0;
+    size_t hpart_cap = 0;
     pn1dev::EBlk *row = nullptr, *pblk = nullptr;
     int* crow = nullptr;
     int nrow = 0, npblk = 0;
-    int fmask_cap = 0, hmask_cap = 0;
-    int rows_cap = 0, eblk_cap = 0;
+    size_t fmask_cap = 0, hmask_cap = 0, rows_cap = 0, eblk_cap = 0;
     // three buffers of cap + 2 records, as in pn1_ctx
     pn1dev::JRec64* j64 = nullptr;
     pn1dev::JRec32* j32 = nullptr;
@@ -71,14 +71,17 @@ struct pn1_ens {
     pn1dev::EItem* items = nullptr;
     long long* poff = nullptr;
     unsigned int* counter = nullptr;
-    int nitems = 0, items_cap = 0;
+    int nitems = 0;
+    size_t items_cap = 0;
     bool have_items = false;      // items, qoff are those of this state and L
     pn1dev::EPart* parts = nullptr;
     pn1dev::EPlace* place = nullptr;
-    int nparts = 0, parts_cap = 0;
+    int nparts = 0;
+    size_t parts_cap = 0;
     bool autoplan = true;         // no explicit chunk at the last upload
+    int L_auto = 0;               // the automatic plan's chunk; 0: it does not take this state
     bool tab_auto = false;        // the tables are the automatic plan's
-    int Lf = 512;                 // the force's chunk: L, or the plan's own
+    int Lf = 512;                 // the force's chunk: L or L_auto
     int echunks = 1;                // largest energy_chunks of a cluster
     long long slots = 0;
     void* part = nullptr;
@@ -101,6 +104,8 @@ namespace pn1host {
 
 int eerr(pn1_ens* e, int code, const char* fmt, ...);
 pn1dev::Phys ens_phys(const pn1_ens* e);
+// Grid of n workgroups whose index is ens_block.
+dim3 ens_grid(int n);
 // As enqueue_prep and enqueue_eval, for every cluster.
 int ens_enqueue_prep(pn1_ens* e, const pn1dev::Phys& P);
 int ens_enqueue_eval(pn1_ens* e, int stage, const pn1dev::Phys& P);

@@ -192,11 +192,12 @@ void k_ens_pair32x(const JRec32* __restrict__ jr, const JRec64* __restrict__ j64
 // dispatcher gives to XCD b % 8, takes an item of queue b % 8 until the
 // shortest queue ends.  A queue holds whole clusters, those with the longest
 // parts first.  A workgroup per cluster.
-inline __global__ __launch_bounds__(WG) void k_ens_parts(const EPlace* __restrict__ place,
+inline __global__ __launch_bounds__(WG) void k_ens_parts(const EPlace* __restrict__ place, int nc,
                                                         const int* __restrict__ crow, QLen len,
                                                         EPart* __restrict__ parts)
 {
-    const int c = blockIdx.x;
+    const int c = ens_block();
+    if (c >= nc) return;
     const EPlace w = place[c];
     const int cnt = (crow[c + 1] - crow[c]) * w.S;       // S = 0: no star
     for (int t = threadIdx.x; t < cnt; t += WG) {
@@ -295,7 +296,7 @@ struct EnsBufs {
 
 __device__ __forceinline__ void reset_queues(unsigned int* counter)
 {
-    if (blockIdx.x == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
+    if (ens_block() == 0 && threadIdx.x < NXCD) counter[threadIdx.x] = 0u;
 }
 
 // As k_prep, one workgroup per FG rows of a cluster (pblk: its cluster and
@@ -303,13 +304,15 @@ __device__ __forceinline__ void reset_queues(unsigned int* counter)
 // R.fn: one entry (or NGS) per cluster.
 inline __global__ __launch_bounds__(FWG) void k_ens_prep(const double* __restrict__ st,
                                                 const double* __restrict__ m, Phys P, EnsBufs E,
-                                                const EBlk* __restrict__ pblk,
+                                                const EBlk* __restrict__ pblk, int npblk,
                                                 JRec64* __restrict__ j64, RowBufs R, MixPrep M,
                                                 const double* __restrict__ aprev,
                                                 const float* __restrict__ kprev)
 {
     reset_queues(E.counter);
-    const EBlk b = pblk[blockIdx.x];
+    const int wg = ens_block();
+    if (wg >= npblk) return;
+    const EBlk b = pblk[wg];
     const int off = E.coff[b.c], nst = E.coff[b.c + 1] - off - 1;
     const int r0 = E.crow[b.c], r1 = E.crow[b.c + 1];
     const int row = r0 + b.first / RB + (int)(threadIdx.x >> 6);
@@ -348,15 +351,17 @@ inline __global__ __launch_bounds__(FWG) void k_ens_prep(const double* __restric
 }
 
 // As k_fin: one workgroup per row of the ensemble (G = FG, blk the row
-// table) or per FG rows of a cluster (G = 1, blk = pblk).
+// table) or per FG rows of a cluster (G = 1, blk = pblk), n in all.
 template <int MODE, int STAGE, int G>
 __global__ __launch_bounds__(FWG) __attribute__((amdgpu_waves_per_eu(4, 8)))
-void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
+void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk, int n,
                const void* __restrict__ part, const long long* __restrict__ poff, int L,
                MixPrep M, Phys P)
 {
     reset_queues(E.counter);
-    const EBlk b = blk[blockIdx.x];
+    const int wg = ens_block();
+    if (wg >= n) return;
+    const EBlk b = blk[wg];
     const int off = E.coff[b.c], nst = E.coff[b.c + 1] - off - 1;
     const int r0 = E.crow[b.c], r1 = E.crow[b.c + 1];
     const Row q = {off, nst, b.first, r0 + b.first / RB, nst};
@@ -388,17 +393,19 @@ void k_ens_fin(FinBufs F, RowBufs R, EnsBufs E, const EBlk* __restrict__ blk,
 // ensemble energies (FP64)
 // ---------------------------------------------------------------------
 // As k_energy, workgroup (row of the ensemble, chunk); a cluster uses
-// energy_chunks of the grid's chunks, the others leave at once.  Its last
-// workgroup writes its energies to out[5 c].
+// energy_chunks of the grid's chunks, the others leave at once (the grid's third
+// dimension: further rows).  Its last workgroup writes its energies to out[5 c].
 inline __global__ __launch_bounds__(PW * RB)
 void k_ens_energy(const JRec64* __restrict__ jr, const double* __restrict__ st, EnsBufs E,
-                  const EBlk* __restrict__ rowt, const double* __restrict__ gs,
+                  const EBlk* __restrict__ rowt, int nrows, const double* __restrict__ gs,
                   double* __restrict__ eb, double* __restrict__ out,
                   unsigned int* __restrict__ ticket, Phys P)
 {
     __shared__ double t[EV];
     const int2 w = energy_item();
-    const int r = w.x, s = w.y, c = rowt[r].c;
+    const int r = (int)(blockIdx.z * gridDim.x) + w.x, s = w.y;
+    if (r >= nrows) return;
+    const int c = rowt[r].c;
     const int off = E.coff[c], nst = E.coff[c + 1] - off - 1;
     const int S = energy_chunks(nst), r0 = E.crow[c], nrow = E.crow[c + 1] - r0;
     if (s >= S) return;

@@ -38,6 +38,9 @@ struct __align__(8) EBlk {
     int c, first;
 };
 
+// Index of this workgroup in a grid of ens_grid.
+__device__ __forceinline__ int ens_block() { return (int)(blockIdx.y * gridDim.x + blockIdx.x); }
+
 __device__ __forceinline__ int ens_nchunks(int nst, int L) { return (nst + L - 1) / L; }
 
 // Work queues, one per XCD.  The dispatcher deals workgroup ids to the 8
