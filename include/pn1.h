@@ -146,29 +146,31 @@ int  pn1_sync(pn1_ctx *ctx);
 const char *pn1_last_error(const pn1_ctx *ctx);
 
 /* Launch shape of the pair kernels: the j range is split into `jsplit`
- * chunks, one per 256-star workgroup (0 = automatic: up to 192 parts, eight
- * of them to a workgroup of 64 stars, which adds their sums; `variant` then
- * stays -1, else the split is an automatic one of the 256-star kernels;
- * splits of 2 to 32 without a `variant` run as up to 16 chunks of that row
- * form).  A split of the 256-star kernels of 32 or more, a multiple of 8,
- * ends in 16 chunks an eighth as long as the others, which the launch runs
- * last, so that it does not wait long on its last workgroups.  The mixed kernel compensates its FP32 sums every
- * `tile` pairs (0 = default), and `variant` picks the kernel form (-1 =
+ * chunks, one per 256-star workgroup (0 = automatic: with variant -1 up to
+ * 192 parts, eight of them to a workgroup of 64 stars, which adds their
+ * sums, with another variant a split of the 256-star kernels; splits of 2 to
+ * 32 with variant -1 run as up to 16 chunks of that row form).  A split of
+ * the 256-star kernels of 32 or more, a multiple of 8, ends in 16 chunks an
+ * eighth as long as the others, which the launch runs last, so that it does
+ * not wait long on its last workgroups.  The mixed kernel compensates its
+ * FP32 sums every `tile` pairs (0 = default), and `variant` picks the kernel form (-1 =
  * automatic per mode): bit 0 the j loop (clear: one j-record at a time,
  * set: two in flight), bit 1 (mixed form) one Newton step on the FP32
  * rsqrt, bit 2 (mixed form, splits into a multiple of 4 chunks) four
  * chunks per 1024-thread workgroup combined in LDS instead of one chunk
  * per 256-thread workgroup: a quarter of the partial sums written, ~1.6%
  * more pair-kernel time.
- * pn1_get_tuning reports the values in use.  Used by the tuner. */
+ * pn1_get_tuning reports the values in use, in a form that pn1_set_tuning
+ * takes back: jsplit 0 and variant -1 for the automatic plan, variant -1 for
+ * splits in the row form.  Used by the tuner. */
 int  pn1_set_tuning(pn1_ctx *ctx, int jsplit, int tile, int variant);
 int  pn1_get_tuning(const pn1_ctx *ctx, int *jsplit, int *tile, int *variant);
 /* Autotuner: times `reps` whole force evaluations of the resident state
  * (every kernel, so the cost of reducing the split's partial sums counts)
  * for each j split (automatic, 8 ... 256) and j loop variant, keeps the
- * fastest (as pn1_set_tuning would) and reports it with its time per
- * evaluation in ms (any output may be NULL).  The mixed form's compensation interval is
- * not changed: it trades accuracy.  No counterpart in the reference. */
+ * fastest (as pn1_set_tuning would) and reports it, as pn1_get_tuning
+ * does, with its time per evaluation in ms (any output may be NULL).  The
+ * mixed form's compensation interval is not changed: it trades accuracy.  No counterpart in the reference. */
 int  pn1_autotune(pn1_ctx *ctx, int reps, int *jsplit, int *variant,
                   double *best_ms);
 
@@ -246,8 +248,10 @@ const char *pn1_ens_last_error(const pn1_ens *ens);
 /* Shape of the 256-star items: j chunk length `chunk` (records per item; 0 =
  * chosen at upload so that each persistent workgroup takes about 8 items;
  * applies from the next upload), mixed compensation interval `tile` and kernel
- * `variant` as pn1_set_tuning.  With chunk 0 and variant -1 the force and
- * steps use rows of 64 stars, in chunks of their own. */
+ * `variant` as pn1_set_tuning.  With variant -1 and chunk 0, or the very
+ * chunk that 0 would choose, the force and steps use rows of 64 stars, in
+ * chunks of their own.  pn1_ens_get_tuning reports the items' chunk all the
+ * same, with variant -1; set again, its values give the same kernels. */
 int  pn1_ens_set_tuning(pn1_ens *ens, int chunk, int tile, int variant);
 int  pn1_ens_get_tuning(const pn1_ens *ens, int *chunk, int *tile,
                         int *variant);

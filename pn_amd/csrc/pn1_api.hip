@@ -747,9 +747,12 @@ int pn1_set_tuning(pn1_ctx* c, int jsplit, int tile, int variant)
 int pn1_get_tuning(const pn1_ctx* c, int* jsplit, int* tile, int* variant)
 {
     if (!c) return PN1_EINVAL;
-    if (jsplit) *jsplit = c->S;
+    // the row kernels run without a variant alone, the automatic plan's splits
+    // of them without a split too
+    const bool automatic = c->jsplit_req <= 0 && c->variant_req < 0;
+    if (jsplit) *jsplit = automatic ? 0 : c->S;
     if (tile) *tile = c->tile;
-    if (variant) *variant = kernel_variant(c);
+    if (variant) *variant = automatic || c->slots ? -1 : kernel_variant(c);
     return PN1_OK;
 }
 
@@ -1026,10 +1029,8 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
     c->variant_req = bV;
     drop_graph(c);
     if ((rc = plan_parts(c))) return rc;
-    if (jsplit) *jsplit = c->S;
-    if (variant) *variant = kernel_variant(c);
     if (best_ms) *best_ms = best;
-    return PN1_OK;
+    return pn1_get_tuning(c, jsplit, nullptr, variant);
 }
 
 // =========================================================================
