@@ -3,7 +3,8 @@ from one evaluation to the next.  k_fin reads this evaluation's hard stars while
 it writes the next one's, and a star's FP64 sums are found by counting the hard
 stars before it in its row: the two must not share memory.  Massless stars cross
 the threshold inwards and outwards near the centre of a point-symmetric cluster,
-six to a row in all of its groups of 16, over k_fin's three forms."""
+six to a row in all of its groups of 16, over k_fin's three forms, with the sums
+in the pair kernel's chunks (the automatic plan) and in k_fin (variant 0)."""
 import numpy as np
 import pytest
 
@@ -64,8 +65,10 @@ def bound(a):
     return STEPS * DT * 1e-6 * np.linalg.norm(a[1:], axis=1).max()
 
 
-@pytest.mark.parametrize("stars", [300, 1024, 3000, 70000])
-def test_hard_stars_change_between_steps(stars):
+@pytest.mark.parametrize("stars,tuning", [(300, (0, 0, -1)), (1024, (0, 0, -1)), (3000, (0, 0, -1)),
+                                          (70000, (0, 0, -1)), (1024, (16, 0, 0)), (3000, (16, 0, 0)),
+                                          (70000, (32, 0, 0))])
+def test_hard_stars_change_between_steps(stars, tuning):
     x, v, m, near = state(stars)
     n = len(m)
     with pn.Context(n) as ctx:
@@ -81,6 +84,7 @@ def test_hard_stars_change_between_steps(stars):
         assert ins >= 2 and outs >= 2
         tol = bound(seen[0][1])
         ctx.set_params(EPS, 50.0, DT, pn.MIXED)
+        ctx.set_tuning(*tuning)
         runs = []
         for calls in ([STEPS], [STEPS], [1] * STEPS):
             ctx.upload(x, v, m)
@@ -93,8 +97,8 @@ def test_hard_stars_change_between_steps(stars):
         assert np.array_equal(xs, runs[0][0]) and np.array_equal(vs, runs[0][1])
 
 
-@pytest.mark.parametrize("clusters", [6, 220])
-def test_hard_stars_of_an_ensemble_change_between_steps(clusters):
+@pytest.mark.parametrize("clusters,variant", [(6, -1), (220, -1), (6, 0), (220, 0)])
+def test_hard_stars_of_an_ensemble_change_between_steps(clusters, variant):
     """A workgroup per row, and a wave per row (more than 1024 rows)."""
     cl = [state(300 + 32 * (k % 3), k) for k in range(clusters)]
     with pn.Ensemble(sum(len(c[2]) for c in cl), clusters) as ens:
@@ -110,6 +114,7 @@ def test_hard_stars_of_an_ensemble_change_between_steps(clusters):
         print(f"case: {clusters} clusters, crossings {cross}", flush=True)
         assert all(i >= 1 and o >= 1 for i, o, _ in cross)
         ens.set_params(EPS, 50.0, DT, pn.MIXED)
+        ens.set_tuning(0, 0, variant)
         runs = []
         for _ in range(2):
             ens.upload([c[:3] for c in cl])
