@@ -167,7 +167,8 @@ int  pn1_set_tuning(pn1_ctx *ctx, int jsplit, int tile, int variant);
 int  pn1_get_tuning(const pn1_ctx *ctx, int *jsplit, int *tile, int *variant);
 /* Autotuner: times `reps` whole force evaluations of the resident state
  * (every kernel, so the cost of reducing the split's partial sums counts)
- * for each j split (automatic, 8 ... 256) and j loop variant, keeps the
+ * for each j split (automatic, 8 ... 256) and j loop variant, those near the
+ * best twice (the first ones run on a clock still rising), keeps the
  * fastest (as pn1_set_tuning would) and reports it, as pn1_get_tuning
  * does, with its time per evaluation in ms (any output may be NULL).  The
  * mixed form's compensation interval is not changed: it trades accuracy.  No counterpart in the reference. */

@@ -962,7 +962,12 @@ int pn1_profile_read(pn1_ctx* c, int* launches, double* total_ms)
 // Autotuner: times the pair kernel of `reps` force evaluations on the
 // resident state per candidate shape (j split x kernel variant; the mixed
 // form's compensation interval is left alone: it trades accuracy), after
-// one warm-up evaluation, and keeps the fastest.
+// one warm-up evaluation, and keeps the fastest.  Shapes within TUNE_MARGIN of
+// the fastest are timed a second time, each keeping its better one: the first
+// shapes run on a clock that is still rising (measured on MI355X, 256 clusters
+// of 256-8192 stars, mixed: the automatic plan 2.29 ms first, 2.03 later, the
+// next best 2.26).
+constexpr double TUNE_MARGIN = 1.25;
 int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_ms)
 {
     int rc;
@@ -1004,17 +1009,24 @@ int pn1_autotune(pn1_ctx* c, int reps, int* jsplit, int* variant, double* best_m
         *avg = (double)ms / reps;
         return r;
     };
-    for (int S : splits) {
-        for (int var = 0; var < (S ? 2 : 1) && !rc; ++var) {
-            double avg = 0.0;
-            rc = time_shape(S, var, &avg);
-            if (!rc && avg < best) {
-                best = avg;
-                bS = S;
+    struct Shape {
+        int S, var;
+        double ms;
+    };
+    std::vector<Shape> shapes;
+    for (int S : splits)
+        for (int var = 0; var < (S ? 2 : 1); ++var) shapes.push_back(Shape{S, var, 0.0});
+    for (int round = 0; round < 2 && !rc; ++round) {
+        const double limit = TUNE_MARGIN * best;
+        for (Shape& s : shapes) {
+            if (round > 0 && s.ms > limit) continue;
+            if ((rc = time_shape(s.S, s.var, &s.ms))) break;
+            if (s.ms < best) {
+                best = s.ms;
+                bS = s.S;
                 bV = c->variant_req;
             }
         }
-        if (rc) break;
     }
     (void)hipEventDestroy(ea);
     (void)hipEventDestroy(eb);
