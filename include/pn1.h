@@ -37,7 +37,8 @@ extern "C" {
 
 /* Largest capacity a context or ensemble accepts: the kernels index the
  * six state rows of `capacity` doubles with 32-bit offsets (6 x 2^28 <
- * 2^31); at ~0.5 KB of device state per particle it is also ~130 GB. */
+ * 2^31); at ~0.83 KB of device state per particle it is also ~220 GB,
+ * and 34 GB of pair partials at that size. */
 #define PN1_MAX_CAPACITY (1 << 28)
 
 /* ====================================================================== */
@@ -104,7 +105,8 @@ int  pn1_force(pn1_ctx *ctx, double *a);
  * over every star, is not evaluated.  i0 - 1 and i1 - 1 must be multiples
  * of 256 (or i1 = n); a is AoS [i1 - i0][3].  With an explicit j split
  * (pn1_set_tuning, pn1_autotune) it equals rows i0 .. i1 - 1 of pn1_force
- * bit for bit; otherwise the shard gets a split of its own (more chunks
+ * bit for bit (mixed form: of a pn1_force after the same evaluation, whose
+ * accelerations set the pair thresholds); otherwise the shard gets a split of its own (more chunks
  * for its smaller grid) and agrees to rounding.  No counterpart in the
  * reference, which runs on one processor. */
 int  pn1_force_range(pn1_ctx *ctx, int i0, int i1, double *a);

@@ -108,7 +108,9 @@ int auto_split(int nst)
 //   n = 10241         178/128    177/111      178/108      182/113    201/130
 //   n = 131073                   24850/12860  24808/12715
 // Above 2^22 stars the rows alone are over a hundred workgroups per CU, and
-// the split only bounds the partials: at most 2^26 of them (7 GB).
+// the split only bounds the partials (128 bytes each): at most 2^26 (8.6 GB),
+// while a star has more than one; with one, up to 34 GB at 2^28 stars.  Just
+// below 2^22 stars the 24 are 12.9 GB.
 int auto_slots(int nst)
 {
     if (nst >= 8192 && nst < (1 << 22)) return TLONG + TSHORT;

@@ -106,10 +106,11 @@ struct Phys {
 // pair terms cancel to 1/30 of their magnitudes or less) takes every pair in
 // FP64: the FP32 rounding of the terms, ~0.1 u of their magnitudes once
 // averaged, would otherwise near 1e-6 of |a|.  Its whole row is evaluated in
-// FP64 by k_fin, in the workgroup that finishes the star, and its FP32 lane
-// does no extra work (rc2 = dn2 = 0).  An FP64 branch in the lane for every
-// pair instead would make its whole wave several times slower than the
-// others.
+// FP64: a row of 64 stars' first two by the row kernels' workgroups, chunk by
+// chunk (hard_part), further ones and those of the 256-star kernels by k_fin,
+// in the workgroup that finishes the star (rare_rows).  Its FP32 lane does no
+// extra work (rc2 = dn2 = 0); an FP64 branch in the lane for every pair would
+// make its whole wave several times slower than the others.
 // Without a previous evaluation (after an upload) the thresholds are
 // rc2 = 0 and dn2 = FLT_MAX: no FP64 pairs, lo parts everywhere.
 #define PN1_CLOSE_KAPPA 0.25
@@ -161,32 +162,6 @@ __host__ __device__ __forceinline__ double rsq64(double x)
 #else
     return 1.0 / __builtin_sqrt(x);
 #endif
-}
-
-// Fixed-order workgroup sum of N doubles; thread 0 writes out[0..N).
-// Wave level: xor butterfly (every lane ends with the same bits); then the
-// four wave totals are added in wave order.
-template <int N>
-__device__ __forceinline__ void block_sum(double (&v)[N], double* out)
-{
-    __shared__ double sh[N][WG / 64];
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        double t = v[k];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-        v[k] = t;
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < N; ++k) sh[k][wid] = v[k];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < N; ++k) out[k] = ((sh[k][0] + sh[k][1]) + sh[k][2]) + sh[k][3];
-    }
 }
 
 // Store of a pair kernel's partial sum, read once by the finishing kernel:
