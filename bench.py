@@ -314,7 +314,7 @@ def run_ensemble(steps, warmup, chunk=0, tile=0, variant=-1, eager=False, adj_st
     """The batched workload: 256 seeded Plummer clusters (star counts
     log-uniform in [256, 8192], BH masses uniform in [0.005, 0.05], c = 100,
     eps = 1e-3, dt = 2^-10), all advanced by one pn1_ens_step per step (one
-    persistent pair launch per force evaluation, graph-captured steps),
+    pair launch per force evaluation, graph-captured steps),
     against the same clusters advanced one after another through a single
     context (pn1_step, also graph-captured)."""
     W = workloads.ENSEMBLE
@@ -335,7 +335,7 @@ def run_ensemble(steps, warmup, chunk=0, tile=0, variant=-1, eager=False, adj_st
             e0 = ens.energy()
             wall = time_steps(ens, steps, warmup, eager)
             e1 = ens.energy()
-            # pair-kernel time: HIP events around each persistent pair launch
+            # pair-kernel time: HIP events around each pair launch
             # of 3 steps (9 launches), after one untimed step
             ens.upload(cl)                          # keeps the tuned shape
             ens.step(1)
